@@ -541,6 +541,18 @@ static int workspace_for(int dev, hipStream_t stream, Workspace* out) {
     return HFRK_SUCCESS;
 }
 
+int stream_workspace(hipStream_t stream, float** ws, size_t* ws_bytes, int** counters) {
+    int dev = 0;
+    HFRK_HIP_TRY(hipGetDevice(&dev));
+    Workspace w;
+    const int rc = workspace_for(dev, stream, &w);
+    if (rc != HFRK_SUCCESS) return rc;
+    *ws = w.ws;
+    *ws_bytes = kWsFloats * sizeof(float);
+    *counters = w.counters;
+    return HFRK_SUCCESS;
+}
+
 // ---- the allocation-free entry point's scratch: one array per device, part of the code object -----------------------------
 // First kStaticWsBytes: fp32 partial sums; then kStaticCounters arrival counters.
 constexpr size_t kStaticWsBytes = (size_t)16 << 20;

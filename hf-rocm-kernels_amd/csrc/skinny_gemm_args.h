@@ -61,6 +61,10 @@ struct GemmArgs {
     int* counters;           // arrival counters, zero between launches
 };
 
+// The split-K workspace of `stream` on the current device: fp32 partial sums (kWsFloats) and kMaxPanels arrival counters, zero
+// between launches (skinny_gemm.hip).
+int stream_workspace(hipStream_t stream, float** ws, size_t* ws_bytes, int** counters);
+
 // wave-stream kernel (m <= 32), skinny_gemm_stream.hip: act_loads = ceil(m/4) 16-byte activation loads per lane and
 // chunk, row_tiles = 16-row weight tiles per chunk (1: act_loads 1..4; 2: act_loads 3..8)
 // swiglu: the weight holds gate rows [0, n/2) and up rows [n/2, n); a chunk pairs gate tile t with up tile t

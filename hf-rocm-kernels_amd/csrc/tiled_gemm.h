@@ -1,0 +1,54 @@
+// Launch arguments and tile shapes of the tiled GEMM (calls with more rows than the skinny kernels take).
+#pragma once
+
+#include "skinny_gemm_args.h"
+
+#include <type_traits>
+
+namespace hfrk {
+
+struct TiledGemmArgs {
+    const uint8_t* A;
+    const uint8_t* B;
+    void* D;
+    const void* base;  // 16-bit addend or null
+    int base_stride;   // elements between its rows; 0: one row for all (a bias)
+    const float* scale_a;
+    const float* scale_b;
+    int sa_stride, sb_stride;
+    int m, n, k, b_stride;
+    int d_dtype;
+    int vec;                      // rows of D and base are 16-byte aligned
+    int tiles_m, tiles_n, group_m;
+    int stages_q, stages_r;       // k stages per split, the first stages_r splits one more
+    int splits;
+    float* ws;
+    uint32_t ws_bytes;
+    int* counters;
+};
+
+constexpr int kTiledStage = 128;    // bytes of k per pipeline stage
+constexpr int kTiledThreads = 256;  // four waves
+
+// TM x TN matrix tiles of 32 x 32 per wave, WM x WN waves, NST stages of operands in LDS, WGS workgroups per compute unit.
+// X(index, TM, TN, WM, WN, NST, WGS)
+#define HFRK_TILED_SHAPES(X) \
+    X(0, 4, 4, 2, 2, 2, 1)   \
+    X(1, 4, 2, 2, 2, 3, 1)   \
+    X(2, 2, 2, 2, 2, 5, 1)   \
+    X(3, 2, 1, 2, 2, 3, 2)   \
+    X(4, 1, 1, 2, 2, 8, 1)
+
+struct TiledShape {
+    int bm, bn, stages, per_cu;
+};
+#define HFRK_TILED_ROW(I, TM, TN, WM, WN, NST, WGS) {32 * TM * WM, 32 * TN * WN, NST, WGS},
+constexpr TiledShape kTiledShapes[] = {HFRK_TILED_SHAPES(HFRK_TILED_ROW)};
+#undef HFRK_TILED_ROW
+constexpr int kTiledShapeCount = sizeof(kTiledShapes) / sizeof(kTiledShapes[0]);
+constexpr int tiled_lds_bytes(const TiledShape& s) { return (s.bm + s.bn) * kTiledStage * s.stages; }
+
+int launch_tiled_rowmajor(const TiledGemmArgs& args, int shape, hipStream_t stream);  // tiled_gemm_rowmajor.hip
+int launch_tiled_packed(const TiledGemmArgs& args, int shape, hipStream_t stream);    // tiled_gemm_packed.hip
+
+}  // namespace hfrk

@@ -1,0 +1,143 @@
+// Host side of the tiled GEMM: plan and entry points (the kernel is in tiled_gemm_kernel.h).
+#include <math.h>
+
+#include "tiled_gemm.h"
+
+namespace hfrk {
+
+static int div_up(long a, long b) { return (int)((a + b - 1) / b); }
+
+static bool tiled_size_ok(int m, int n, int k) {
+    // every offset the kernel forms inside one tile's buffers stays below 2^31, every tile count and workspace index in 32 bits
+    constexpr int kMost = 1 << 21;
+    return m >= 1 && n >= 1 && k >= 1 && m <= (1 << 24) && n <= kMost && k <= kMost &&
+           (long)div_up(m, 64) * div_up(n, 64) < (1L << 24);
+}
+
+static size_t tiled_ws_bytes(const TiledShape& s, int m, int n, int splits) {
+    return splits <= 1 ? 0 : (size_t)div_up(m, s.bm) * div_up(n, s.bn) * splits * s.bm * s.bn * sizeof(float);
+}
+
+static int check_tiled_plan(int m, int n, int k, const hfrk_tiled_plan& p) {
+    if (p.shape < 0 || p.shape >= kTiledShapeCount || p.splits < 1 || p.group_m < 1) return HFRK_INVALID_CONFIG;
+    const TiledShape& s = kTiledShapes[p.shape];
+    const long tiles = (long)div_up(m, s.bm) * div_up(n, s.bn);
+    if (p.splits > div_up(k, kTiledStage) || p.group_m > div_up(m, s.bm)) return HFRK_INVALID_CONFIG;
+    if (p.splits > 1 && (tiled_ws_bytes(s, m, n, p.splits) > kWsFloats * sizeof(float) || tiles > kMaxPanels)) return HFRK_INVALID_CONFIG;
+    return HFRK_SUCCESS;
+}
+
+// The shape and the number of k splits with the smallest predicted time, in us.  The constants are a least-squares fit of this very
+// expression to 4100 measured calls (11 weights from 1024 x 4096 to 8192 x 28672, 15 row counts from 65 to 4096, every shape and
+// 1..8 splits); over those 158 sizes the choice is 1.4 % slower than the best measured plan in the geometric mean, 10 % or more on 6.
+static float tiled_cost(int m, int n, int k, int shape, int splits) {
+    struct Shape { float fixed, stage; };  // a workgroup's prologue and epilogue; one stage of 128 bytes of k on an idle chip
+    static constexpr Shape kShape[kTiledShapeCount] = {{13.6f, 1.31f}, {7.9f, .67f}, {4.8f, .40f}, {1.4f, .32f}, {2.0f, .225f}};
+    constexpr float kL2 = 18.1e6f, kHbm = 4.16e6f, kShares = 7.4e6f;  // bytes per us: operands into LDS, weights, partial sums
+    constexpr float kPairFixed = 1.3f, kPairStage = 1.6f;             // two workgroups on a compute unit against one
+    const TiledShape& s = kTiledShapes[shape];
+    const long wgs = (long)div_up(m, s.bm) * div_up(n, s.bn) * splits, slots = (long)kNumCU * s.per_cu;
+    const float stages = (float)div_up(k, kTiledStage) / splits;
+    auto round_us = [&](long count) {
+        if (count == 0) return 0.f;
+        const bool pair = count > kNumCU;
+        const float own = kShape[shape].stage * (pair ? kPairStage : 1.f), traffic = count * (float)((m < s.bm ? m : s.bm) + s.bn) * kTiledStage / kL2;
+        return kShape[shape].fixed * (pair ? kPairFixed : 1.f) + stages * (own > traffic ? own : traffic);
+    };
+    float t = (float)(wgs / slots) * round_us(slots) + round_us(wgs % slots);
+    const float stream = (float)n * k / kHbm;
+    if (t < stream) t = stream;
+    if (splits > 1) t += .93f + .76f * splits + (float)wgs * s.bm * s.bn * 8.f / kShares;
+    return t;
+}
+
+static void make_tiled_plan(int m, int n, int k, hfrk_tiled_plan* plan) {
+    float best = INFINITY;
+    const int stages = div_up(k, kTiledStage);
+    for (int shape = 0; shape < kTiledShapeCount; ++shape) {
+        const TiledShape& s = kTiledShapes[shape];
+        const int tiles_m = div_up(m, s.bm);
+        const long tiles = (long)tiles_m * div_up(n, s.bn);
+        for (int splits = 1; splits <= 8 && splits <= stages; ++splits) {
+            // a split keeps at least two stages and the launch at most two workgroups per compute unit
+            if (splits > 1 && (tiles * splits > 2 * kNumCU || stages < 2 * splits)) break;
+            const float t = tiled_cost(m, n, k, shape, splits);
+            if (t < best) {
+                best = t;
+                plan->shape = shape;
+                plan->splits = splits;
+                // the 32 workgroups of an XCD cover about as many rows as columns of D
+                const int square = (int)lroundf(sqrtf(32.f * s.bn / s.bm));
+                plan->group_m = tiles_m < square ? tiles_m : square;
+            }
+        }
+    }
+}
+
+}  // namespace hfrk
+
+extern "C" {
+
+int hfrk_tiled_gemm_plan(int m, int n, int k, hfrk_tiled_plan* plan) {
+    if (!plan || !hfrk::tiled_size_ok(m, n, k)) return HFRK_BAD_SHAPE;
+    if (k % 16 != 0) return HFRK_K_NOT_DIVISIBLE_BY_WARPTILE_K;
+    hfrk::make_tiled_plan(m, n, k, plan);
+    return HFRK_SUCCESS;
+}
+
+int hfrk_tiled_gemm(const void* A, const void* B, int packed, void* D, const void* base, int base_stride, const float* scale_a,
+                    int sa_stride, const float* scale_b, int sb_stride, int m, int n, int k, int b_stride, int d_dtype,
+                    const hfrk_tiled_plan* plan, void* stream) {
+    using namespace hfrk;
+    if (packed) b_stride = k;
+    if (!tiled_size_ok(m, n, k) || b_stride < k || b_stride > (1 << 21)) return HFRK_BAD_SHAPE;
+    if (k % 16 != 0 || (packed && k % 256 != 0)) return HFRK_K_NOT_DIVISIBLE_BY_WARPTILE_K;
+    if (d_dtype != HFRK_F16 && d_dtype != HFRK_BF16) return HFRK_BAD_DTYPE;
+    if (!A || !B || !D || !scale_a) return HFRK_BAD_SHAPE;
+    if ((sa_stride != 0 && sa_stride != 1) || (sb_stride != 0 && sb_stride != 1)) return HFRK_BAD_SHAPE;
+    if (base && base_stride != 0 && (base_stride < n || base_stride > (1 << 21))) return HFRK_BAD_SHAPE;
+    if ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) & 15 || (b_stride & 15)) return HFRK_BAD_ALIGNMENT;
+    if ((reinterpret_cast<uintptr_t>(D) | reinterpret_cast<uintptr_t>(base)) & 1) return HFRK_BAD_ALIGNMENT;
+    hfrk_tiled_plan p;
+    if (plan) {
+        p = *plan;
+        const int rc = check_tiled_plan(m, n, k, p);
+        if (rc != HFRK_SUCCESS) return rc;
+    } else {
+        make_tiled_plan(m, n, k, &p);
+    }
+    const TiledShape& s = kTiledShapes[p.shape];
+    TiledGemmArgs args{};
+    args.A = static_cast<const uint8_t*>(A);
+    args.B = static_cast<const uint8_t*>(B);
+    args.D = D;
+    args.base = base;
+    args.base_stride = base ? base_stride : 0;
+    args.scale_a = scale_a;
+    args.scale_b = scale_b;
+    args.sa_stride = sa_stride;
+    args.sb_stride = sb_stride;
+    args.m = m;
+    args.n = n;
+    args.k = k;
+    args.b_stride = b_stride;
+    args.d_dtype = d_dtype;
+    args.vec = n % 8 == 0 && args.base_stride % 8 == 0 && ((reinterpret_cast<uintptr_t>(D) | reinterpret_cast<uintptr_t>(base)) & 15) == 0;
+    args.tiles_m = div_up(m, s.bm);
+    args.tiles_n = div_up(n, s.bn);
+    args.group_m = p.group_m;
+    const int stages = div_up(k, kTiledStage);
+    args.splits = p.splits;
+    args.stages_q = stages / p.splits;
+    args.stages_r = stages % p.splits;
+    if (p.splits > 1) {
+        size_t bytes = 0;
+        const int rc = stream_workspace(static_cast<hipStream_t>(stream), &args.ws, &bytes, &args.counters);
+        if (rc != HFRK_SUCCESS) return rc;
+        args.ws_bytes = (uint32_t)bytes;
+    }
+    return packed ? launch_tiled_packed(args, p.shape, static_cast<hipStream_t>(stream))
+                  : launch_tiled_rowmajor(args, p.shape, static_cast<hipStream_t>(stream));
+}
+
+}  // extern "C"

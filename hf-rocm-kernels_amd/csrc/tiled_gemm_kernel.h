@@ -1,0 +1,418 @@
+// Tiled FP8 (OCP e4m3fn) GEMM for more rows than the skinny kernels take:
+//   D[m,n] = (base ? base[m,n] : 0) + sa[m] * sb[n] * sum_k A[m,k] * W[n,k]
+// No counterpart in the reference, whose kernel stops at 32 rows (skinny_gemm_caller.cu:33-60); the linear layer ran such calls
+// as one skinny launch per 64 rows, each of which streamed the whole weight again.
+//
+//  * Bound: the matrix cores on the large tiles (v_mfma_f32_32x32x64_f8f6f4, 64 cycles each), L2 -> LDS traffic on the small
+//    ones.  A workgroup is four waves, one per SIMD; a wave owns TM x TN matrix tiles of 32 x 32.  On the largest tile
+//    (256 x 256, 128 x 128 per wave) an operand byte read from LDS feeds 128 multiply-adds, so the LDS pipe is half busy when the
+//    matrix cores are fully busy; accumulators fill the 256 accumulation registers, operands are double buffered in the others.
+//  * Operands go from memory to LDS without passing registers (buffer_load_dwordx4 ... lds), NST stages of 128 bytes of k deep, the
+//    stage NST ahead being requested behind the barrier that frees its slot.  One barrier per stage: a wave reads the operands of
+//    k step s + 1 (64 bytes) while it multiplies those of step s, so nothing in a step waits for LDS but its first instruction.
+//  * Such a load fills LDS in lane order, so the swizzle that keeps operand reads free of bank conflicts is applied to the memory
+//    side: the lane that fills slot c of row r fetches piece c ^ f(r) of that row (a permutation within one 128-byte line).
+//    Measured conflicts: none (SQ_LDS_BANK_CONFLICT = 0).  A packed weight is fetched as 512-byte runs into the same kind of layout.
+//  * Rows and columns past the edge, and the part of the last stage past k, are outside the buffers' ranges and read as zero.
+//  * Weights are the matrix instruction's A operand with their rows permuted so that a lane's 16 results of a tile are consecutive
+//    columns; results go through LDS in fp32 and leave as whole rows, scaled, added to their addend and rounded once.
+//  * Workgroup ids are dealt to the XCDs in contiguous ranges and walk the tiles in column-major groups of group_m rows of tiles, so
+//    that the workgroups of one L2 share both operands.
+//  * Few tiles and a long k: k is cut between `splits` workgroups.  Partial tiles are written through to memory, the last arriver
+//    adds them in split order (bit-reproducible), as in the skinny workgroup kernel.
+//
+// Measured (row-major / packed, us, bf16 out): 4096 x 28672 x 4096 412 / 395 (2.3 / 2.4 PFLOP/s; 1550 as 64 skinny launches; a loop that
+// stays resident clocks at 1.8 - 2.0 GHz, so the matrix cores' power bounds it before their issue rate does), 512 x 4096 x 14336
+// 38 / 37 (150), 201 x 6144 x 4096 13.2 / 13.1 (46), 65 x 4096 x 4096 10.5 / 9.9 (16).  The epilogue is written with little code on
+// purpose: with a branch per value for NaN and 64-bit addresses it took 18 us of a 256 x 256 tile, now 7.
+#pragma once
+
+#include "tiled_gemm.h"
+
+namespace hfrk {
+
+typedef float v16f __attribute__((ext_vector_type(16)));
+
+// One 16-byte-per-lane load from memory straight into LDS: lane l's piece lands at lds_base + 16 l.  As inline assembly because the
+// compiler, when it knows of such a load, waits for it before every LDS read that follows; the waits are placed by hand here.
+__device__ __forceinline__ void load_to_lds(const v4i& rsrc, int voffset, uint32_t lds_base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds_base), "v"(voffset), "s"(rsrc) : "memory");
+}
+
+// All but the COUNT youngest loads of this wave have landed, and its LDS reads are done.
+template <int COUNT>
+__device__ __forceinline__ void wait_loads_and_lds() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(COUNT) : "memory");
+}
+
+__device__ __forceinline__ void workgroup_barrier() { asm volatile("s_barrier" ::: "memory"); }
+
+__device__ __forceinline__ v4i tile_rsrc(const uint8_t* base, uint32_t bytes) {
+    const uint64_t p = reinterpret_cast<uint64_t>(base);
+    return v4i{__builtin_amdgcn_readfirstlane((int)(uint32_t)p), __builtin_amdgcn_readfirstlane((int)((uint32_t)(p >> 32) & 0xffffu)),
+               __builtin_amdgcn_readfirstlane((int)bytes), 0x00020000};
+}
+
+// Two floats to two 16-bit values in one register, round to nearest even (v_cvt_pk_bf16_f32 / v_cvt_pk_f16_f32: no branch for NaN).
+template <int DT>
+__device__ __forceinline__ uint32_t pack_pair(float lo, float hi) {
+    typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+    typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+    if constexpr (DT == HFRK_BF16) return __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{lo, hi}, v2bf));
+    else return __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{lo, hi}, v2h));
+}
+
+template <int TM, int TN, int WM, int WN, int NST, int WGS, bool PACKED>
+__global__ void __launch_bounds__(kTiledThreads, WGS) tiled_gemm_kernel(const TiledGemmArgs a) {
+    static_assert(WM * WN == 4, "a workgroup is 4 waves");
+    constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN;
+    constexpr int KB = kTiledStage;
+    constexpr int A_BYTES = BM * KB, B_BYTES = BN * KB, STAGE = A_BYTES + B_BYTES;
+    constexpr int LA = A_BYTES / 4096, LB = B_BYTES / 4096;  // load instructions per wave and stage, 1 KB each
+    constexpr int NMMA = TM * TN;
+    constexpr int kOutside = 0x7ffffff0;  // beyond any tile's range
+
+    extern __shared__ __align__(16) uint8_t lds[];
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((int)(uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void*)lds));
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / WN, wn = wave % WN;
+    const int lr = lane & 31, lg = lane >> 5;
+
+    // ---- which tile, which part of k ---------------------------------------------------------------------------------
+    int id = blockIdx.x;
+    {
+        const int per = (int)gridDim.x >> 3, extra = (int)gridDim.x & 7, x = id & 7;  // XCD x works on one contiguous range of ids
+        id = x * per + min(x, extra) + (id >> 3);
+    }
+    const int tiles = a.tiles_m * a.tiles_n;
+    const int split = a.splits == 1 ? 0 : id / tiles, tile = id - split * tiles;  // neighbours work on the same part of k
+    const int group_tiles = a.group_m * a.tiles_n;
+    const int grp = tile / group_tiles, in_grp = tile - grp * group_tiles;
+    const int gm = min(a.group_m, a.tiles_m - grp * a.group_m);
+    const int tn = in_grp / gm, tm = grp * a.group_m + in_grp - tn * gm;
+    const int m0 = tm * BM, n0 = tn * BN;
+    const int s_begin = split * a.stages_q + min(split, a.stages_r), s_end = s_begin + a.stages_q + (split < a.stages_r ? 1 : 0);
+
+    // ---- operand streams ---------------------------------------------------------------------------------------------
+    // buffers over this tile's rows from the current stage on
+    const int rows_a = min(BM, a.m - m0);
+    v4i ra = tile_rsrc(a.A + (long)m0 * a.k + (long)s_begin * KB, (uint32_t)rows_a * (uint32_t)a.k - (uint32_t)(s_begin * KB));
+    v4i rb;
+    constexpr int kStepB = PACKED ? 2048 : KB;  // a stage of a packed 16-row tile is half of a 4 KB chunk
+    if constexpr (PACKED) {
+        const int tiles16 = min(BN / 16, (a.n + 15) / 16 - n0 / 16);
+        rb = tile_rsrc(a.B + (long)(n0 / 16) * a.k * 16 + (long)s_begin * kStepB, (uint32_t)tiles16 * (uint32_t)a.k * 16u - (uint32_t)(s_begin * kStepB));
+    } else {
+        const int rows_b = min(BN, a.n - n0);
+        rb = tile_rsrc(a.B + (long)n0 * a.b_stride + (long)s_begin * kStepB,
+                       (uint32_t)(rows_b - 1) * (uint32_t)a.b_stride + (uint32_t)a.k - (uint32_t)(s_begin * kStepB));
+    }
+    int va[LA], vb[LB];
+    int pa[LA], pb[LB];  // k byte of the lane's piece within its stage (for the last, partial stage)
+#pragma unroll
+    for (int q = 0; q < LA; ++q) {
+        const int row = (q * 4 + wave) * 8 + (lane >> 3);
+        pa[q] = ((lane & 7) ^ ((row >> 1) & 7)) * 16;
+        va[q] = row * a.k + pa[q];
+    }
+#pragma unroll
+    for (int q = 0; q < LB; ++q) {
+        if constexpr (PACKED) {
+            // LDS block (16-row tile, half of the stage): [piece j][k group][row slot], 1 KB
+            const int blk = q * 4 + wave, t16 = blk >> 1, s = blk & 1, group = (lane >> 4) & 1;
+            const int row = (lane & 15) ^ ((t16 & 1) << 3) ^ group << 2;
+            vb[q] = t16 * a.k * 16 + (lane >> 5) * 1024 + s * 512 + group * 256 + row * 16;
+            pb[q] = 0;
+        } else {
+            const int row = (q * 4 + wave) * 8 + (lane >> 3);
+            pb[q] = ((lane & 7) ^ (((row >> 1) & 3) | ((row >> 4) & 1) << 2)) * 16;
+            vb[q] = row * a.b_stride + pb[q];
+        }
+    }
+    int issued = s_begin;
+    uint32_t slot_issue = 0;
+    const int k_tail = a.k & (KB - 1), tail_stage = k_tail ? a.k / KB : -1;
+    auto issue_begin = [&]() __attribute__((always_inline)) {
+        if (issued >= s_end) { ra[2] = 0; rb[2] = 0; }  // past the end: as many loads as ever, nothing is read
+    };
+    auto issue_a = [&](int q) __attribute__((always_inline)) {
+        int off = va[q];
+        if (issued == tail_stage) off = pa[q] < k_tail ? off : kOutside;
+        load_to_lds(ra, off, lds0 + slot_issue + (uint32_t)(q * 4 + wave) * 1024u);
+    };
+    auto issue_b = [&](int q) __attribute__((always_inline)) {
+        int off = vb[q];
+        if (!PACKED && issued == tail_stage) off = pb[q] < k_tail ? off : kOutside;
+        load_to_lds(rb, off, lds0 + slot_issue + A_BYTES + (uint32_t)(q * 4 + wave) * 1024u);
+    };
+    auto issue_end = [&]() __attribute__((always_inline)) {
+        auto advance = [](v4i& r, uint32_t by) __attribute__((always_inline)) {
+            const uint64_t p = ((uint64_t)(uint32_t)r[1] << 32 | (uint32_t)r[0]) + by;
+            r[0] = (int)(uint32_t)p;
+            r[1] = (int)(uint32_t)(p >> 32);
+            r[2] -= (int)by;
+        };
+        if (issued < s_end) {
+            advance(ra, KB);
+            advance(rb, kStepB);
+        }
+        ++issued;
+        slot_issue = slot_issue + STAGE == NST * STAGE ? 0 : slot_issue + STAGE;
+    };
+
+    // ---- operand reads -----------------------------------------------------------------------------------------------
+    // matrix row r of a weight tile is weight row perm(r): a lane's 16 results of a tile are then 16 consecutive columns
+    const int perm = ((lr >> 2) & 1) * 16 + (lr >> 3) * 4 + (lr & 3);
+    const int fa = (lr >> 1) & 7, fb = ((perm >> 1) & 3) | ((perm >> 4) & 1) << 2;
+    const int a_row = (wm * TM * 32 + lr) * KB;
+    const int b_row = A_BYTES + (PACKED ? (wn * TN * 2 + (perm >> 4)) * 2048 + lg * 256 + ((perm & 15) ^ ((perm >> 4) << 3) ^ (lg << 2)) * 16
+                                        : (wn * TN * 32 + perm) * KB);
+    uint32_t slot_read = 0;
+    v8i fra[2][TM], frb[2][TN];
+    auto read16 = [&](int off) __attribute__((always_inline)) { return *reinterpret_cast<const v4i*>(lds + off); };
+    auto join = [](v4i lo, v4i hi) __attribute__((always_inline)) { return v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]}; };
+    auto read_a = [&](v8i& dst, int i, int s) __attribute__((always_inline)) {
+        const int off = (int)slot_read + a_row + (((2 * lg) ^ fa ^ (4 * s)) << 4);
+        dst = join(read16(off + i * 32 * KB), read16((off ^ 16) + i * 32 * KB));
+    };
+    auto read_b = [&](v8i& dst, int j, int s) __attribute__((always_inline)) {
+        if constexpr (PACKED) {
+            const int off = (int)slot_read + b_row + j * 4096 + s * 1024;
+            dst = join(read16(off), read16(off + 512));
+        } else {
+            const int off = (int)slot_read + b_row + (((2 * lg) ^ fb ^ (4 * s)) << 4);
+            dst = join(read16(off + j * 32 * KB), read16((off ^ 16) + j * 32 * KB));
+        }
+    };
+
+    v16f acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+
+    // Half a stage (64 bytes of k): multiply the operands read half a stage ago (register set S) while the next half's are read into
+    // the other set.  The second half reads from the next stage, so it opens with the wait for that stage and the barrier behind
+    // which this stage's slot is free and the stage NST ahead is requested into it.  The schedule is fixed: operand reads in front
+    // of the first three quarters of the matrix instructions, loads spread over all of them.
+    auto half = [&](auto sel) __attribute__((always_inline)) {
+        constexpr int S = decltype(sel)::value;
+        if constexpr (S == 1) {
+            wait_loads_and_lds<(NST - 2) * (LA + LB)>();
+            workgroup_barrier();
+            slot_read = slot_read + STAGE == NST * STAGE ? 0 : slot_read + STAGE;
+            issue_begin();
+        }
+        constexpr int READS = TM + TN, LOADS = S == 1 ? LA + LB : 0;
+        int reads = 0, loads = 0;
+#pragma unroll
+        for (int t = 0; t < NMMA; ++t) {
+            const int reads_to = NMMA <= 2 ? READS : min(READS, (t + 1) * READS * 4 / (3 * NMMA) + 1), loads_to = (t + 1) * LOADS / NMMA;
+#pragma unroll
+            for (int r = 0; r < READS; ++r)
+                if (r >= reads && r < reads_to) {
+                    if (r < TN) read_b(frb[S ^ 1][r], r, S ^ 1);
+                    else read_a(fra[S ^ 1][r - TN], r - TN, S ^ 1);
+                }
+#pragma unroll
+            for (int l = 0; l < LOADS; ++l)
+                if (l >= loads && l < loads_to) {
+                    if (l < LA) issue_a(l);
+                    else issue_b(l - LA);
+                }
+            reads = reads_to;
+            loads = loads_to;
+            acc[t / TN][t % TN] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(frb[S][t % TN], fra[S][t / TN], acc[t / TN][t % TN], 0, 0, 0, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (S == 1) issue_end();
+    };
+
+    // ---- main loop ---------------------------------------------------------------------------------------------------
+    asm volatile("s_nop 4" ::: "memory");  // scalars a vector instruction wrote are not read by a load at once
+#pragma unroll 1
+    for (int s = 0; s < NST; ++s) {
+        issue_begin();
+#pragma unroll
+        for (int q = 0; q < LA; ++q) issue_a(q);
+#pragma unroll
+        for (int q = 0; q < LB; ++q) issue_b(q);
+        issue_end();
+    }
+    wait_loads_and_lds<(NST - 1) * (LA + LB)>();
+    workgroup_barrier();
+#pragma unroll
+    for (int j = 0; j < TN; ++j) read_b(frb[0][j], j, 0);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) read_a(fra[0][i], i, 0);
+#pragma unroll 1
+    for (int s = s_begin; s < s_end; ++s) {
+        half(std::integral_constant<int, 0>{});
+        half(std::integral_constant<int, 1>{});
+    }
+    wait_loads_and_lds<0>();
+    workgroup_barrier();  // LDS is free: no wave reads operands any more, no load is under way
+
+    // ---- partial sums of a tile whose k is split -----------------------------------------------------------------------
+    if (a.splits > 1) {
+        const __amdgpu_buffer_rsrc_t ws = make_rsrc(a.ws, a.ws_bytes);
+        constexpr int kCoherent = 17;  // sc0 | sc1: written through to memory, read past the caches (the XCDs' L2s are not coherent)
+        auto ws_off = [&](int sp, int t, int p) __attribute__((always_inline)) {
+            return ((((tile * a.splits + sp) * 4 + wave) * NMMA + t) * 4 + p) * 1024 + lane * 16;
+        };
+#pragma unroll
+        for (int t = 0; t < NMMA; ++t)
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                const v16f& x = acc[t / TN][t % TN];
+                const v4f v = {x[4 * p], x[4 * p + 1], x[4 * p + 2], x[4 * p + 3]};
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i, v), ws, ws_off(split, t, p), 0, kCoherent);
+            }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        int* const flag = reinterpret_cast<int*>(lds);
+        if (tid == 0) {
+            const int seen = __hip_atomic_fetch_add(a.counters + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const int last = seen == a.splits - 1;
+            if (last) __hip_atomic_store(a.counters + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            *flag = last;
+        }
+        __syncthreads();
+        const int last = *flag;
+        __syncthreads();  // the epilogue writes where the flag lies
+        if (!last) return;
+        constexpr int CH = NMMA < 4 ? NMMA : 4;  // tiles whose shares are in flight together
+#pragma unroll
+        for (int t0 = 0; t0 < NMMA; t0 += CH) {
+            v4f sum[CH * 4];
+#pragma unroll
+            for (int p = 0; p < CH * 4; ++p) sum[p] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+            for (int sp = 0; sp < a.splits; ++sp) {
+                v4i share[CH * 4];
+#pragma unroll
+                for (int p = 0; p < CH * 4; ++p) share[p] = __builtin_amdgcn_raw_buffer_load_b128(ws, ws_off(sp, t0 + p / 4, p % 4), 0, kCoherent);
+#pragma unroll
+                for (int p = 0; p < CH * 4; ++p) sum[p] += __builtin_bit_cast(v4f, share[p]);
+            }
+#pragma unroll
+            for (int t = 0; t < CH; ++t)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[(t0 + t) / TN][(t0 + t) % TN][v] = sum[t * 4 + v / 4][v % 4];
+        }
+    }
+
+    // ---- epilogue ----------------------------------------------------------------------------------------------------
+    // acc[i][j][v] of a lane: row (wm TM + i) 32 + lr of the tile, column (wn TN + j) 32 + 16 lg + v.  32 rows at a time go through
+    // LDS so that memory sees whole rows (a lane holds 16 columns of one row: stored from there, every store would touch 64
+    // lines).  Each wave has a part of LDS of its own: no barrier.
+    constexpr int LPR = 4 * TN;            // lanes per row, 8 columns each
+    constexpr int RPI = 64 / LPR;          // rows per pass
+    constexpr int PASSES = 32 / RPI;
+    constexpr int RS = TN * 32 + 4;        // floats between rows: 16 rows of one column lie in different banks
+    static_assert(4 * 32 * RS * 4 <= NST * STAGE, "the staging fits in the operands' LDS");
+    float* const stage = reinterpret_cast<float*>(lds) + wave * (32 * RS);
+    const int row0 = wm * TM * 32, col = wn * TN * 32 + (lane % LPR) * 8;
+    // buffers over the tile's rows: what lies outside reads as zero and is not stored
+    const int outside = n0 + col < a.n ? 0 : kOutside;
+    const __amdgpu_buffer_rsrc_t rd = make_rsrc(static_cast<uint16_t*>(a.D) + (long)m0 * a.n, (uint32_t)rows_a * (uint32_t)a.n * 2u);
+    const __amdgpu_buffer_rsrc_t rbase = make_rsrc(static_cast<const uint16_t*>(a.base) + (long)m0 * a.base_stride,
+                                                   a.base ? (uint32_t)((rows_a - 1) * a.base_stride + a.n) * 2u : 0u);
+    const __amdgpu_buffer_rsrc_t rsa = make_rsrc(a.scale_a + (long)m0 * a.sa_stride, (uint32_t)((rows_a - 1) * a.sa_stride + 1) * 4u);
+    float sb[8];
+#pragma unroll
+    for (int v = 0; v < 8; ++v) sb[v] = a.scale_b ? a.scale_b[(long)min(n0 + col + v, a.n - 1) * a.sb_stride] : 1.0f;
+    auto write_back = [&](auto dt) __attribute__((always_inline)) {
+        constexpr int DT = decltype(dt)::value;
+        // The memory counter retires in order, so a load requested after stores waits for them: scales and addends of 32 rows
+        // are requested before the stores of the 32 rows in front.
+        v4i add[2][PASSES];
+        float sa[2][PASSES];
+        const int base_off = ((row0 + lane / LPR) * a.base_stride + n0 + col) * 2 | outside, base_step = RPI * a.base_stride * 2;
+        auto fetch = [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+            for (int r = 0; r < PASSES; ++r) {
+                sa[i & 1][r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsa, (row0 + i * 32 + r * RPI + lane / LPR) * a.sa_stride * 4, 0, 0));
+                add[i & 1][r] = __builtin_amdgcn_raw_buffer_load_b128(rbase, base_off + (i * PASSES + r) * base_step, 0, 0);
+            }
+        };
+        const int d_off = ((row0 + lane / LPR) * a.n + n0 + col) * 2 | outside, d_step = RPI * a.n * 2;
+        if (a.vec) fetch(0);
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int p = 0; p < 4; ++p)
+                    *reinterpret_cast<v4f*>(stage + lr * RS + j * 32 + lg * 16 + p * 4) =
+                        v4f{acc[i][j][4 * p], acc[i][j][4 * p + 1], acc[i][j][4 * p + 2], acc[i][j][4 * p + 3]};
+            if (a.vec && i + 1 < TM) fetch(i + 1);
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            if (a.vec) {
+#pragma unroll
+                for (int r = 0; r < PASSES; ++r) {
+                    const float* const src = stage + (r * RPI + lane / LPR) * RS + (lane % LPR) * 8;
+                    const v4f x0 = reinterpret_cast<const v4f*>(src)[0], x1 = reinterpret_cast<const v4f*>(src)[1];
+                    const float x[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
+                    v4i o;
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const uint32_t b = (uint32_t)add[i & 1][r][v];
+                        o[v] = (int)pack_pair<DT>(load16<DT>((uint16_t)(b & 0xffff)) + x[2 * v] * (sa[i & 1][r] * sb[2 * v]),
+                                               load16<DT>((uint16_t)(b >> 16)) + x[2 * v + 1] * (sa[i & 1][r] * sb[2 * v + 1]));
+                    }
+                    __builtin_amdgcn_raw_buffer_store_b128(o, rd, d_off + (i * PASSES + r) * d_step, 0, 0);
+                }
+            } else {  // rows of D or base that are not 16-byte aligned: one element per lane
+#pragma unroll 1
+                for (int e = lane; e < 32 * TN * 32; e += 64) {
+                    const int r = e / (TN * 32), c = e % (TN * 32);
+                    const int m = m0 + row0 + i * 32 + r, n = n0 + wn * TN * 32 + c;
+                    if (m >= a.m || n >= a.n) continue;
+                    float x = stage[r * RS + c] * (a.scale_a[(long)m * a.sa_stride] * (a.scale_b ? a.scale_b[(long)n * a.sb_stride] : 1.0f));
+                    if (a.base) x += load16<DT>(static_cast<const uint16_t*>(a.base)[(long)m * a.base_stride + n]);
+                    static_cast<uint16_t*>(a.D)[(long)m * a.n + n] = (uint16_t)pack_pair<DT>(x, 0.f);
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        }
+    };
+    if (a.d_dtype == HFRK_BF16) write_back(std::integral_constant<int, HFRK_BF16>{});
+    else write_back(std::integral_constant<int, HFRK_F16>{});
+}
+
+template <int TM, int TN, int WM, int WN, int NST, int WGS, bool PACKED>
+static int launch_tiled_shape(const TiledGemmArgs& args, int lds_bytes, hipStream_t stream) {
+    auto kern = tiled_gemm_kernel<TM, TN, WM, WN, NST, WGS, PACKED>;
+    static bool attr_done[kMaxDevices] = {};
+    int dev = 0;
+    HFRK_HIP_TRY(hipGetDevice(&dev));
+    if (dev < 0 || dev >= kMaxDevices || !attr_done[dev]) {
+        HFRK_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes));
+        if (dev >= 0 && dev < kMaxDevices) attr_done[dev] = true;
+    }
+    hipLaunchKernelGGL(kern, dim3(args.tiles_m * args.tiles_n * args.splits), dim3(kTiledThreads), lds_bytes, stream, args);
+    HFRK_HIP_TRY(hipGetLastError());
+    return HFRK_SUCCESS;
+}
+
+template <bool PACKED>
+static int launch_tiled(const TiledGemmArgs& args, int shape, hipStream_t stream) {
+    switch (shape) {
+#define HFRK_TILED_CASE(I, TM, TN, WM, WN, NST, WGS) \
+    case I: return launch_tiled_shape<TM, TN, WM, WN, NST, WGS, PACKED>(args, tiled_lds_bytes(kTiledShapes[I]), stream);
+        HFRK_TILED_SHAPES(HFRK_TILED_CASE)
+#undef HFRK_TILED_CASE
+    }
+    return HFRK_INVALID_CONFIG;
+}
+
+}  // namespace hfrk

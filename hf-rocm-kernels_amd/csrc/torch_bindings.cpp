@@ -406,6 +406,56 @@ int64_t skinny_gemm_packed(at::Tensor& A, at::Tensor& B_packed, int64_t n, at::T
     return gemm_fused_common(A, B_packed, true, n, D, base, scale_a, scale_b, out_scale, epilogue, intermediate_dtype);
 }
 
+// The linear layer's GEMM for any number of rows: D = base + scale_a x scale_b x A.B, base a [m, n] tensor or one [n] row.  Raises
+// on a non-zero status.  No reference counterpart (its kernel stops at 32 rows, skinny_gemm_caller.cu:33-60).
+void tiled_gemm(at::Tensor& A, at::Tensor& B, bool packed, int64_t n, at::Tensor& D, const std::optional<at::Tensor>& base,
+                at::Tensor& scale_a, const std::optional<at::Tensor>& scale_b) {
+    TORCH_CHECK(A.dim() == 2 && A.is_contiguous(), "A must be a contiguous [m, k] tensor");
+    check_fp8(A, "A");
+    check_fp8(B, "B");
+    const int64_t m = A.size(0), k = A.size(1);
+    TORCH_CHECK(n >= 1 && n < (int64_t(1) << 30) && m < (int64_t(1) << 30) && k < (int64_t(1) << 30), "m, n and k must fit 30 bits");
+    if (packed) {
+        const size_t plain = hfrk_packed_weight_bytes((int)n, (int)k), scaled = hfrk_packed_weight_bytes_scaled((int)n, (int)k);
+        TORCH_CHECK(B.is_contiguous() && B.numel() > 0 && ((size_t)B.numel() == plain || (size_t)B.numel() == scaled),
+                    "B must be the packed buffer of a [n, k] weight (pack_weight, pack_weight_scaled) with k = A.size(1)");
+    } else {
+        TORCH_CHECK(B.dim() == 2 && B.size(0) == k && B.size(1) == n && B.stride(0) == 1, "B must be [k, n] with unit stride along k");
+    }
+    TORCH_CHECK(D.dim() == 2 && D.size(0) == m && D.size(1) == n && D.is_contiguous(), "D must be a contiguous [m, n] tensor");
+    const int d_dtype = dtype16(D, "D");
+    TORCH_CHECK(scale_a.scalar_type() == at::kFloat && scale_a.is_contiguous() && (scale_a.numel() == 1 || scale_a.numel() == m),
+                "scale_a must be float32 with 1 or m elements");
+    check_same_device(A, B, "B");
+    check_same_device(A, D, "D");
+    check_same_device(A, scale_a, "scale_a");
+    const float* scale_b_ptr = nullptr;
+    int sb_stride = 0;
+    if (scale_b.has_value()) {
+        TORCH_CHECK(scale_b->scalar_type() == at::kFloat && scale_b->is_contiguous() && (scale_b->numel() == 1 || scale_b->numel() == n),
+                    "scale_b must be float32 with 1 or n elements");
+        check_same_device(A, *scale_b, "scale_b");
+        scale_b_ptr = scale_b->data_ptr<float>();
+        sb_stride = scale_b->numel() == 1 ? 0 : 1;
+    }
+    const void* base_ptr = nullptr;
+    int base_stride = 0;
+    if (base.has_value()) {
+        const bool row = base->dim() == 1;
+        TORCH_CHECK(base->is_contiguous() && base->scalar_type() == D.scalar_type() && (row ? base->size(0) == n : base->sizes() == D.sizes()),
+                    "base must be a contiguous [n] or [m, n] tensor of D's dtype");
+        check_same_device(A, *base, "base");
+        base_ptr = base->data_ptr();
+        base_stride = row ? 0 : (int)n;
+    }
+    if (m == 0) return;
+    DeviceScope scope(A);
+    raise_on(hfrk_tiled_gemm(A.data_ptr(), B.data_ptr(), packed ? 1 : 0, D.data_ptr(), base_ptr, base_stride, scale_a.data_ptr<float>(),
+                             scale_a.numel() == 1 ? 0 : 1, scale_b_ptr, sb_stride, (int)m, (int)n, (int)k, packed ? (int)k : (int)B.stride(1),
+                             d_dtype, nullptr, current_stream(A)),
+             "tiled_gemm");
+}
+
 bool is_byte_tensor(const at::Tensor& t) {
     return t.scalar_type() == at::kByte || t.scalar_type() == at::kFloat8_e4m3fn || t.scalar_type() == at::kFloat8_e4m3fnuz;
 }
@@ -512,6 +562,10 @@ TORCH_LIBRARY(_HFRK_C, ops) {
         "skinny_gemm_checked(Tensor A, Tensor B, bool packed, int n, Tensor! D, Tensor? base, Tensor scale_a, Tensor? scale_b, "
         "Tensor? out_scale, int epilogue, int intermediate_dtype) -> ()");
     ops.impl("skinny_gemm_checked", c10::kCUDA, &skinny_gemm_checked);
+
+    ops.def(
+        "tiled_gemm(Tensor A, Tensor B, bool packed, int n, Tensor! D, Tensor? base, Tensor scale_a, Tensor? scale_b) -> ()");
+    ops.impl("tiled_gemm", c10::kCUDA, &tiled_gemm);
 
     ops.def("pack_weight(Tensor src, Tensor! dst, int src_format) -> ()");
     ops.impl("pack_weight", c10::kCUDA, &pack_weight);

@@ -52,6 +52,11 @@ class GemmPlan(ctypes.Structure):
         return {name: getattr(self, name) for name, _ in self._fields_}
 
 
+class TiledPlan(ctypes.Structure):
+    """struct hfrk_tiled_plan"""
+    _fields_ = [(name, ctypes.c_int) for name in ("shape", "splits", "group_m")]
+
+
 _i, _p, _f = ctypes.c_int, ctypes.c_void_p, ctypes.c_float
 
 # name -> (restype, argtypes); every symbol the header declares
@@ -82,6 +87,8 @@ SIGNATURES = {
     "hfrk_pack_weight_scaled": (_i, [_p, _i, _i, _p, _p, _i, _i, _p]),
     "hfrk_packed_weight_scales": (_p, [_p, _i, _i]),
     "hfrk_skinny_gemm_packed": (_i, [_p, _p, _p, _p, _p, _i, _p, _i, _p, _i, _i, _i, _i, _i, ctypes.POINTER(GemmPlan), _p]),
+    "hfrk_tiled_gemm_plan": (_i, [_i, _i, _i, ctypes.POINTER(TiledPlan)]),
+    "hfrk_tiled_gemm": (_i, [_p, _p, _i, _p, _p, _i, _p, _i, _p, _i, _i, _i, _i, _i, _i, ctypes.POINTER(TiledPlan), _p]),
     "hfrk_residual_rms": (_i, [_p, _p, _p, _p, _f, _p, _p, _i, _i, _i, _i, _i, _i, _i, _p]),
     "hfrk_swiglu": (_i, [_p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _p]),
     "hfrk_residual_rms_dynamic": (_i, [_p, _p, _p, _f, _p, _p, _p, _i, _i, _i, _i, _p]),

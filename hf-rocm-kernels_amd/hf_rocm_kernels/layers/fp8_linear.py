@@ -4,10 +4,9 @@ The reference points to its vLLM integration for this (README.md:95-97); the hoo
 apply function for decode-sized batches.  This module is that hook without the vLLM dependency: a function with the
 usual (input, weight, weight_scale, input_scale, bias) signature, and an nn.Module that owns a quantised weight.
 
-Decode batches (up to 64 tokens) run as: one quantisation kernel (skipped when the caller already holds fp8
-activations and their scales, e.g. from `residual_rms_dynamic` / `swiglu_dynamic`) and one GEMM with the scales, the
-bias or residual folded into its epilogue.  Larger batches are cut into pieces of 64 rows; a prefill-sized batch
-belongs on a GEMM library and is only handled here so that the layer is always correct.
+A call runs as one quantisation kernel (skipped when the caller already holds fp8 activations and their scales, e.g. from
+`residual_rms_dynamic` / `swiglu_dynamic`) and one GEMM with the scales, the bias or residual folded into its epilogue: a
+skinny GEMM for decode batches (up to 64 tokens), the tiled GEMM for everything larger, up to whole prompts.
 """
 from typing import Optional, Sequence, Tuple, Union
 
@@ -17,6 +16,7 @@ from torch import Tensor
 from .. import _capi
 from ..operators.quantize import quantize_fp8
 from ..operators.skinny_gemm import skinny_gemm_add, skinny_gemm_scaled
+from ..operators.skinny_gemm.wrapped import skinny_gemm_checks
 from ..utils.fp8 import amax_scale, fp8_quantize
 from ..utils.weight_format import PackedWeight, pack_weight
 
@@ -67,6 +67,7 @@ def apply_fp8_linear(
     else:
         sb = weight_scale.reshape(-1)
     m = q.size(0)
+    tiled = m > _capi.GEMM_MAX_M
     base = None
     if residual is not None:
         base = residual.reshape(m, n)
@@ -74,15 +75,18 @@ def apply_fp8_linear(
             base = base + bias
         base = base.contiguous()
     elif bias is not None:
-        base = bias.to(out_dtype).expand(m, n).contiguous()
+        base = bias.to(out_dtype).contiguous() if tiled else bias.to(out_dtype).expand(m, n).contiguous()
     out = torch.empty((m, n), dtype=out_dtype, device=q.device)
-    for r0 in range(0, m, _capi.GEMM_MAX_M):
-        r1 = min(m, r0 + _capi.GEMM_MAX_M)
-        sa_part = sa if sa.numel() == 1 else sa[r0:r1]
-        if base is None:
-            skinny_gemm_scaled(q[r0:r1], w, sa_part, sb, output=out[r0:r1])
-        else:
-            skinny_gemm_add(q[r0:r1], w, sa_part, sb, base[r0:r1], output=out[r0:r1])
+    if tiled:
+        skinny_gemm_checks(q, w, sa[:1], out)
+        packed = isinstance(w, PackedWeight)
+        torch.ops._HFRK_C.tiled_gemm(q, w.data if packed else w, packed, n, out, base, sa.contiguous(), sb.contiguous())
+    elif m == 0:
+        pass
+    elif base is None:
+        skinny_gemm_scaled(q, w, sa, sb, output=out)
+    else:
+        skinny_gemm_add(q, w, sa, sb, base, output=out)
     return out.reshape(*lead, n)
 
 

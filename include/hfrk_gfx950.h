@@ -268,6 +268,31 @@ int hfrk_skinny_gemm_packed(const void* A, const void* B_packed, void* D, const 
                             int sa_stride, const float* scale_b, int sb_stride, const float* out_scale, int m, int n,
                             int k, int d_dtype, int epilogue, const hfrk_gemm_plan* plan, void* stream);
 
+/* How one tiled GEMM call is decomposed: an index into the library's tile shapes (0: 256 x 256, 1: 256 x 128, 2: 128 x 128,
+ * 3: 128 x 64, 4: 64 x 64 rows x columns of D per workgroup), how many workgroups share a tile's k, and how many rows of tiles
+ * the workgroups walk side by side. */
+typedef struct hfrk_tiled_plan {
+    int shape;
+    int splits;
+    int group_m;
+} hfrk_tiled_plan;
+
+/* The plan hfrk_tiled_gemm uses when none is passed.  Host only. */
+int hfrk_tiled_gemm_plan(int m, int n, int k, hfrk_tiled_plan* plan);
+
+/* D[i,j] = (base ? base[i*base_stride + j] : 0) + scale_a[i*sa_stride] * scale_b[j*sb_stride] * sum_k A[i,k] B[k,j] for any
+ * number of rows m (the skinny GEMMs stop at 64): the linear layer on more than one decode batch of rows.  No counterpart in the
+ * reference, whose kernel returns an error above 32 rows (csrc/op_src/skinny_gemm/skinny_gemm_caller.cu:33-60).
+ *   A  fp8 e4m3fn [m,k] row-major     B  the weight: row-major with row stride b_stride (packed == 0) or the buffer
+ *   D  16-bit [m,n] row-major            hfrk_pack_weight wrote (packed == 1, b_stride unused)
+ *   base  16-bit addend of D's type or NULL; base_stride elements between its rows, 0: one row for all (a bias)
+ * fp32 accumulation, one rounding, bit-reproducible.  k % 16 == 0 (256 for a packed weight); n, k and the strides at most 2^21.
+ * A and B 16-byte aligned, b_stride a multiple of 16; D and base may have any alignment, 16 bytes with n % 8 == 0 is the fast one.
+ * A plan whose k is split needs the stream's workspace like the skinny GEMMs (see hfrk_init). */
+int hfrk_tiled_gemm(const void* A, const void* B, int packed, void* D, const void* base, int base_stride, const float* scale_a,
+                    int sa_stride, const float* scale_b, int sb_stride, int m, int n, int k, int b_stride, int d_dtype,
+                    const hfrk_tiled_plan* plan, void* stream);
+
 /* residual <- input + residual (one 16-bit add); output <- rmsnorm(residual) * weight, optionally / scale -> fp8.
  * Replaces `void residual_rms(...)` at csrc/op_src/residual_rms/residual_rms_dispatch.cu:8-63.
  *   input, residual [rows,cols] io_dtype (f16/bf16) row-major; weight [cols] io_dtype

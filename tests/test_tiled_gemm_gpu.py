@@ -1,0 +1,90 @@
+"""GPU parity of the tiled GEMM (more rows than the skinny kernels take) against the CPU oracle, to the same bar as the skinny
+kernels: one output ulp plus 2^-16 of the sum of absolute products.  Every tile shape in both weight layouts, at sizes around
+the edges of tiles, stages and splits."""
+import ctypes
+
+import pytest
+import torch
+
+from test_gemm_gpu import oracle_checker
+
+pytestmark = pytest.mark.gpu
+
+
+def _operands(m, n, k, seed):
+    from hf_rocm_kernels.utils.fp8 import amax_scale, fp8_quantize
+    g = torch.Generator().manual_seed(seed)
+    a = torch.randn(m, k, generator=g)
+    a[m - 1] *= 20.0
+    w = torch.randn(n, k, generator=g) * 0.02
+    sa, sw = amax_scale(a, dim=1), amax_scale(w, dim=1)
+    return fp8_quantize(a, sa)[0], fp8_quantize(w, sw)[0], sa.reshape(-1), sw.reshape(-1)
+
+
+# (m, n, k, splits): one row; one tile and one stage; one row and eight columns past a tile, k past a stage and cut unevenly;
+# rows of D that are not 16-byte aligned; a last stage cut short; several groups of tiles; fewer stages than the pipeline is deep
+SIZES = [(1, 64, 256, 1), (64, 256, 128, 1), (257, 264, 1280, 3), (130, 203, 512, 2), (65, 136, 1008, 1), (600, 520, 768, 1), (200, 72, 16, 1)]
+
+
+@pytest.mark.parametrize("add", ["none", "bias", "residual"])
+@pytest.mark.parametrize("m,n,k,splits", SIZES)
+def test_every_tile_shape_matches_the_oracle(m, n, k, splits, add):
+    from hf_rocm_kernels import _capi
+    from hf_rocm_kernels.utils.weight_format import pack_weight
+    lib = _capi.load()
+    dtype = torch.float16 if add == "bias" else torch.bfloat16
+    a, w, sa, sw = _operands(m, n, k, seed=m + n + k)
+    g = torch.Generator().manual_seed(7)
+    base = {"none": None, "bias": torch.randn(n, generator=g).to(dtype), "residual": torch.randn(m, n, generator=g).to(dtype)}[add]
+    check = oracle_checker(a, w.t(), sa, sw, dtype, base=None if base is None else base.expand(m, n).contiguous())
+    dev = [t.cuda() for t in (a, w, sa, sw)]
+    dev_base = None if base is None else base.cuda()
+    layouts = [(0, dev[1])] + ([(1, pack_weight(dev[1]).data)] if k % 256 == 0 else [])
+    for shape in range(5):
+        first = None
+        for packed, weight in layouts:
+            for _ in range(2):
+                out = torch.full((m, n), float("nan"), dtype=dtype, device="cuda")
+                plan = _capi.TiledPlan(shape, splits, 2 if m > 256 else 1)
+                status = lib.hfrk_tiled_gemm(dev[0].data_ptr(), weight.data_ptr(), packed, out.data_ptr(), None if base is None else dev_base.data_ptr(),
+                                             n if add == "residual" else 0, dev[2].data_ptr(), 1, dev[3].data_ptr(), 1, m, n, k, k,
+                                             _capi.F16 if dtype == torch.float16 else _capi.BF16, ctypes.byref(plan),
+                                             torch.cuda.current_stream().cuda_stream)
+                _capi.check(status, "hfrk_tiled_gemm")
+                torch.cuda.synchronize()
+                if first is None:
+                    check(out)
+                    first = out
+                assert torch.equal(out, first), (shape, packed)  # the layouts and repeated launches give the same bits
+
+
+@pytest.mark.parametrize("m,n,k", [(65, 1000, 2048), (201, 1032, 1040), (300, 4096, 512)])
+def test_strided_weights_and_scalar_scales(m, n, k):
+    a, w, sa, sw = _operands(m, n, k, seed=3)
+    wide = torch.zeros(n, k + 48, dtype=torch.uint8)
+    wide[:, :k] = w.view(torch.uint8)
+    wide[:, k:] = 0x7F  # NaN beyond the row's end: never read into a sum
+    view = wide.cuda().view(torch.float8_e4m3fn)[:, :k]
+    out = torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
+    # Codes reach 448, so sum |a b| over k = 2048 is of the order of 3e6 and its fp32 error bound, 2^-16 of that, of the order of 50:
+    # a scale of 0.013 would make that 0.6, beyond the absolute 1e-2 of the check.  2e-6 brings results to order 1.
+    one = torch.tensor([2e-6])
+    torch.ops._HFRK_C.tiled_gemm(a.cuda(), view.t(), False, n, out, None, one.cuda(), None)
+    oracle_checker(a, w.t(), one, torch.ones(1), torch.bfloat16)(out)
+
+
+def test_argument_errors_and_plans():
+    from hf_rocm_kernels import _capi
+    lib = _capi.load()
+    buf = torch.zeros(1 << 16, dtype=torch.uint8, device="cuda")
+    p = buf.data_ptr()
+
+    def call(m=80, n=64, k=128, packed=0, stride=128, dtype=_capi.BF16, plan=None, a=p):
+        return lib.hfrk_tiled_gemm(a, p, packed, p + 32768, None, 0, p, 0, None, 0, m, n, k, stride, dtype, plan, None)
+
+    assert call(m=0) == _capi.BAD_SHAPE and call(stride=112) == _capi.BAD_SHAPE
+    assert call(k=120, stride=128) == _capi.K_NOT_DIVISIBLE_BY_WARPTILE_K and call(packed=1) == _capi.K_NOT_DIVISIBLE_BY_WARPTILE_K
+    assert call(dtype=_capi.FP8_E4M3FN) == _capi.BAD_DTYPE
+    assert call(a=p + 8) == _capi.BAD_ALIGNMENT
+    for bad in ((5, 1, 1), (-1, 1, 1), (0, 2, 1), (0, 1, 2), (4, 0, 1)):
+        assert call(plan=ctypes.byref(_capi.TiledPlan(*bad))) == _capi.INVALID_CONFIG, bad
