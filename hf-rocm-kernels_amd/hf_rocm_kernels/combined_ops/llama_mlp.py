@@ -119,6 +119,7 @@ class LlamaMlpGraph:
         args = (rms_weight, rms_epsilon, gate_up_weight, gate_up_input_scale, gate_up_output_scale, down_weight,
                 down_input_scale, down_output_scale)
         kwargs = dict(add_residual=add_residual, fused=fused)
+        self._operands = args  # the captured launches read their addresses: they live as long as the graph
         self._stream = torch.cuda.Stream(device)
         with torch.cuda.stream(self._stream):
             llama_mlp_combined_ops(self.attn_output, self.residual, *args, **kwargs)  # eager: workspace, code objects

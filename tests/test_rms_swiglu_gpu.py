@@ -384,6 +384,27 @@ def test_captured_mlp_block_replays_like_the_eager_block(packed):
 
 
 @pytest.mark.gpu
+def test_captured_mlp_block_keeps_its_operands_alive():
+    """A replay reads the weights and scales by address, so the block must own them: a caller that drops its own references (and a
+    cache that is emptied afterwards) must not take them away."""
+    import gc
+    import weakref
+    from hf_rocm_kernels.combined_ops.llama_mlp import LlamaMlpGraph
+    from hf_rocm_kernels.utils.weight_format import pack_weight
+    hidden, inter = 256, 512
+    one = torch.ones(1, device="cuda")
+    args = [torch.ones(hidden, dtype=torch.bfloat16, device="cuda"), 1e-5,
+            pack_weight(torch.zeros(2 * inter, hidden, device="cuda").to(torch.float8_e4m3fn)), one,
+            one.clone(), torch.zeros(hidden, inter, device="cuda").to(torch.float8_e4m3fn).t(), one.clone(), one.clone()]
+    refs = [weakref.ref(a) for a in args if not isinstance(a, float)]
+    block = LlamaMlpGraph(1, hidden, *args)
+    del args, one
+    gc.collect()
+    assert all(r() is not None for r in refs)
+    del block
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("fused", [False, True])
 def test_traced_mlp_block_equals_the_eager_block(fused):
     """The operators have shape-only implementations, so torch can trace the block as one graph (no graph break) and
