@@ -33,14 +33,13 @@ void set_last_hip_error(hipError_t e);
     } while (0)
 
 // ---- 16-bit <-> fp32, by dtype tag -------------------------------------------------------------------------
-// bf16: upper half of an fp32; conversion to bf16 rounds to nearest even (NaN kept quiet).
+// bf16: upper half of an fp32; conversion to bf16 rounds to nearest even (NaN kept quiet), by v_cvt_pk_bf16_f32.  Written out with
+// integer arithmetic it took a branch for NaN per value, in every epilogue and twice per element of the 16-bit residual add.
 __device__ __forceinline__ float bf16_bits_to_float(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
 
 __device__ __forceinline__ uint16_t float_to_bf16_bits(float f) {
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x0040u);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (uint16_t)(u >> 16);
+    typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+    return (uint16_t)__builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{f, f}, v2bf));
 }
 
 __device__ __forceinline__ float f16_bits_to_float(uint16_t b) {
