@@ -456,6 +456,149 @@ void tiled_gemm(at::Tensor& A, at::Tensor& B, bool packed, int64_t n, at::Tensor
              "tiled_gemm");
 }
 
+// ---- whole calls as one operator ------------------------------------------------------------------------------------------
+// What `Fp8Linear` and `skinny_gemm` do per call, allocations included.  A decode-sized call is a few microseconds of GPU work;
+// as Python (argument checks, two allocations, two operators) its host side took longer than that: Fp8Linear of 16 rows
+// 6144 x 4096 22.4 us per call against 11 us of kernels, skinny_gemm of 1 row 4096 x 4096 13.3 against 5.
+// Both take only what is certain to run and return an undefined tensor (None in Python) or false for everything else; the Python
+// wrapper then goes its general way, which converts, copies or raises.
+
+bool one_float(const at::Tensor& t, const at::Tensor& like) {
+    return t.numel() == 1 && t.scalar_type() == at::kFloat && t.device() == like.device();
+}
+
+bool float_vector(const at::Tensor& t, int64_t count, const at::Tensor& like) {
+    return (t.numel() == 1 || t.numel() == count) && t.scalar_type() == at::kFloat && t.is_contiguous() && t.device() == like.device();
+}
+
+bool is_16bit(at::ScalarType t) { return t == at::kBFloat16 || t == at::kHalf; }
+
+// input [..., k] 16-bit (quantised here: with input_scale, or per row when it is None) or fp8 with its scale(s); weight the
+// row-major [n, k] fp8 tensor (n = -1) or the packed buffer of a weight of n rows; D = bias or residual + input . weight^T.
+at::Tensor fp8_linear(const at::Tensor& input, const at::Tensor& weight, int64_t n, const std::optional<at::Tensor>& weight_scale,
+                      const std::optional<at::Tensor>& input_scale, const std::optional<at::Tensor>& bias,
+                      const std::optional<at::Tensor>& residual, std::optional<at::ScalarType> out_dtype) {
+    const bool packed = n >= 0, quantised = input.scalar_type() == at::kFloat8_e4m3fn;
+    if (!input.is_cuda() || input.dim() < 1 || input.numel() == 0 || !input.is_contiguous()) return {};
+    if (!quantised && !is_16bit(input.scalar_type())) return {};
+    if (weight.scalar_type() != at::kFloat8_e4m3fn || weight.device() != input.device()) return {};
+    const int64_t k = input.size(-1), m = input.numel() / k;
+    if (k >= (int64_t(1) << 24) || m >= (int64_t(1) << 24)) return {};
+    const float* sb = nullptr;
+    int sb_stride = 0, b_stride = (int)k;
+    if (packed) {
+        if (n < 1 || n >= (int64_t(1) << 24) || !weight.is_contiguous()) return {};
+        const size_t plain = hfrk_packed_weight_bytes((int)n, (int)k), scaled = hfrk_packed_weight_bytes_scaled((int)n, (int)k);
+        const size_t have = (size_t)weight.numel();
+        if (plain == 0 || (have != plain && have != scaled)) return {};
+        if (!weight_scale.has_value()) {  // the per-channel scales stored behind the packed bytes
+            if (have == plain) return {};
+            sb = reinterpret_cast<const float*>(static_cast<const uint8_t*>(weight.data_ptr()) + plain);
+            sb_stride = 1;
+        }
+    } else {
+        if (weight.dim() != 2 || weight.size(1) != k || weight.stride(1) != 1 || !weight_scale.has_value()) return {};
+        n = weight.size(0);
+        if (n < 1 || n >= (int64_t(1) << 24) || weight.stride(0) < k || weight.stride(0) >= (int64_t(1) << 30)) return {};
+        b_stride = (int)weight.stride(0);
+    }
+    if (weight_scale.has_value()) {
+        if (!float_vector(*weight_scale, n, input)) return {};
+        sb = weight_scale->data_ptr<float>();
+        sb_stride = weight_scale->numel() == 1 ? 0 : 1;
+    }
+    if (quantised && !input_scale.has_value()) return {};
+    if (input_scale.has_value() && !(quantised ? float_vector(*input_scale, m, input) : one_float(*input_scale, input))) return {};
+    if (!quantised && (k % 8 != 0 || k > 32768)) return {};
+    const at::ScalarType dtype = out_dtype.value_or(quantised ? at::kBFloat16 : input.scalar_type());
+    if (!is_16bit(dtype) || (bias.has_value() && residual.has_value())) return {};
+    const bool tiled = m > HFRK_GEMM_MAX_M;
+    at::Tensor base;
+    int base_stride = (int)n;
+    if (residual.has_value()) {
+        if (residual->numel() != m * n || !residual->is_contiguous() || residual->scalar_type() != dtype) return {};
+        base = *residual;
+    } else if (bias.has_value()) {
+        if (bias->dim() != 1 || bias->size(0) != n || !bias->is_contiguous() || bias->scalar_type() != dtype) return {};
+        base = *bias;
+        base_stride = 0;
+    }
+    if (base.defined() && base.device() != input.device()) return {};
+
+    DeviceScope scope(input);
+    void* const stream = current_stream(input);
+    if (base.defined() && base_stride == 0 && !tiled) base = base.expand({m, n}).contiguous();
+    at::DimVector sizes(input.sizes());
+    sizes.back() = n;
+    at::Tensor out = at::empty(sizes, input.options().dtype(dtype));
+    const void* a = input.data_ptr();
+    const float* sa = nullptr;
+    int sa_stride = 0;
+    at::Tensor scratch;  // the quantised rows, then their scales
+    if (input_scale.has_value()) {
+        sa = input_scale->data_ptr<float>();
+        sa_stride = input_scale->numel() == 1 ? 0 : 1;
+    }
+    if (!quantised) {
+        const int64_t bytes = (m * k + 15) / 16 * 16;
+        scratch = at::empty({bytes + (sa ? 0 : 4 * m)}, input.options().dtype(at::kByte));
+        uint8_t* const q = static_cast<uint8_t*>(scratch.data_ptr());
+        float* const row_scales = reinterpret_cast<float*>(q + bytes);
+        if (hfrk_quantize_fp8(a, sa, q, sa ? nullptr : row_scales, (int)m, (int)k, input.scalar_type() == at::kBFloat16 ? HFRK_BF16 : HFRK_F16,
+                              stream) != HFRK_SUCCESS)
+            return {};
+        a = q;
+        if (!sa) {
+            sa = row_scales;
+            sa_stride = 1;
+        }
+    }
+    const void* const base_ptr = base.defined() ? base.data_ptr() : nullptr;
+    const int d_dtype = dtype == at::kBFloat16 ? HFRK_BF16 : HFRK_F16;
+    int status;
+    if (tiled)
+        status = hfrk_tiled_gemm(a, weight.data_ptr(), packed ? 1 : 0, out.data_ptr(), base_ptr, base_stride, sa, sa_stride, sb, sb_stride,
+                                 (int)m, (int)n, (int)k, b_stride, d_dtype, nullptr, stream);
+    else if (packed)
+        status = hfrk_skinny_gemm_packed(a, weight.data_ptr(), out.data_ptr(), base_ptr, sa, sa_stride, sb, sb_stride, nullptr, (int)m,
+                                         (int)n, (int)k, d_dtype, HFRK_EPILOGUE_NONE, nullptr, stream);
+    else
+        status = hfrk_skinny_gemm_fused(a, weight.data_ptr(), out.data_ptr(), base_ptr, sa, sa_stride, sb, sb_stride, nullptr, (int)m,
+                                        (int)n, (int)k, b_stride, d_dtype, HFRK_EPILOGUE_NONE, nullptr, stream);
+    return status == HFRK_SUCCESS ? out : at::Tensor();
+}
+
+// The operands `skinny_gemm` takes with nothing to convert or report: a row-major weight whose rows are whole 256-byte chunks.
+bool plain_gemm_operands(const at::Tensor& A, const at::Tensor& B, const at::Tensor& scale) {
+    return A.is_cuda() && A.dim() == 2 && B.dim() == 2 && A.scalar_type() == at::kFloat8_e4m3fn && B.scalar_type() == at::kFloat8_e4m3fn &&
+           A.is_contiguous() && B.size(0) == A.size(1) && B.stride(0) == 1 && A.size(0) >= 1 && A.size(0) <= HFRK_GEMM_MAX_M &&
+           A.size(1) >= 256 && A.size(1) % 256 == 0 && A.size(1) < (int64_t(1) << 24) && B.size(1) >= 2 && B.size(1) % 2 == 0 &&
+           B.size(1) < (int64_t(1) << 24) && B.stride(1) >= A.size(1) && B.stride(1) < (int64_t(1) << 30) && B.device() == A.device() &&
+           one_float(scale, A);
+}
+
+int plain_gemm(const at::Tensor& A, const at::Tensor& B, const at::Tensor& scale, const at::Tensor& D, bool accumulate) {
+    return hfrk_skinny_gemm_ex(A.data_ptr(), B.data_ptr(), D.data_ptr(), scale.data_ptr<float>(), 0, nullptr, 0, (int)A.size(0),
+                               (int)B.size(1), (int)A.size(1), (int)B.stride(1), dtype16(D, "D"), accumulate ? 1 : 0, nullptr,
+                               current_stream(A));
+}
+
+// A new float16 tensor: written whole, where the reference's wrapper clears one and accumulates into it (wrapped.py:119).
+at::Tensor skinny_gemm_new(const at::Tensor& A, const at::Tensor& B, const at::Tensor& scale) {
+    if (!plain_gemm_operands(A, B, scale)) return {};
+    DeviceScope scope(A);
+    at::Tensor D = at::empty({A.size(0), B.size(1)}, A.options().dtype(at::kHalf));
+    return plain_gemm(A, B, scale, D, false) == HFRK_SUCCESS ? D : at::Tensor();
+}
+
+bool skinny_gemm_into(const at::Tensor& A, const at::Tensor& B, const at::Tensor& scale, at::Tensor& D) {
+    if (!plain_gemm_operands(A, B, scale) || D.dim() != 2 || D.size(0) != A.size(0) || D.size(1) != B.size(1) || !D.is_contiguous() ||
+        !is_16bit(D.scalar_type()) || D.device() != A.device())
+        return false;
+    DeviceScope scope(A);
+    return plain_gemm(A, B, scale, D, true) == HFRK_SUCCESS;
+}
+
 bool is_byte_tensor(const at::Tensor& t) {
     return t.scalar_type() == at::kByte || t.scalar_type() == at::kFloat8_e4m3fn || t.scalar_type() == at::kFloat8_e4m3fnuz;
 }
@@ -583,6 +726,18 @@ TORCH_LIBRARY(_HFRK_C, ops) {
 
     ops.def("swiglu_dynamic(Tensor gate_up, Tensor! output, Tensor! scales, Tensor! next_buffer) -> ()");
     ops.impl("swiglu_dynamic", c10::kCUDA, &swiglu_dynamic);
+
+    // Outputs carry no autograd history, as those of the operators that write into a tensor of the caller's.
+    ops.def(
+        "fp8_linear(Tensor input, Tensor weight, int n, Tensor? weight_scale, Tensor? input_scale, Tensor? bias, Tensor? residual, "
+        "ScalarType? out_dtype) -> Tensor");
+    ops.impl("fp8_linear", c10::kCUDA, &fp8_linear);
+    ops.impl("fp8_linear", torch::dispatch(c10::DispatchKey::Autograd, torch::CppFunction::makeFallthrough()));
+    ops.def("skinny_gemm_new(Tensor A, Tensor B, Tensor scale) -> Tensor");
+    ops.impl("skinny_gemm_new", c10::kCUDA, &skinny_gemm_new);
+    ops.impl("skinny_gemm_new", torch::dispatch(c10::DispatchKey::Autograd, torch::CppFunction::makeFallthrough()));
+    ops.def("skinny_gemm_into(Tensor A, Tensor B, Tensor scale, Tensor! D) -> bool");
+    ops.impl("skinny_gemm_into", c10::kCUDA, &skinny_gemm_into);
 
     ops.def("quantize_fp8(Tensor input, Tensor? scale_tensor, Tensor! output, Tensor! scales) -> ()");
     ops.impl("quantize_fp8", c10::kCUDA, &quantize_fp8);

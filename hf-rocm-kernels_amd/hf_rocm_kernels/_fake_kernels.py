@@ -16,7 +16,9 @@ import hf_rocm_kernels._HFRK_C  # noqa: F401  (registers torch.ops._HFRK_C)
 
 _RETURNS_NOTHING = ("increment", "residual_rms", "swiglu", "pack_weight", "pack_weight_scaled", "unpack_weight", "reencode_fnuz",
                     "residual_rms_dynamic", "swiglu_dynamic", "quantize_fp8", "skinny_gemm_checked", "tiled_gemm")
-_RETURNS_STATUS = ("skinny_gemm_tb", "skinny_gemm_scaled", "skinny_gemm_fused", "skinny_gemm_packed", "skinny_gemm_rms_fused")
+_RETURNS_STATUS = ("skinny_gemm_tb", "skinny_gemm_scaled", "skinny_gemm_fused", "skinny_gemm_packed", "skinny_gemm_rms_fused",
+                   # a new tensor, or whether the call was one they take: _OTHER_RESULT
+                   "fp8_linear", "skinny_gemm_new", "skinny_gemm_into")
 
 
 def _nothing(*args, **kwargs) -> None:
@@ -27,11 +29,23 @@ def _success(*args, **kwargs) -> int:
     return 0
 
 
+def _fp8_linear(input, weight, n, weight_scale, input_scale, bias, residual, out_dtype):
+    dtype = out_dtype or (torch.bfloat16 if input.dtype == torch.float8_e4m3fn else input.dtype)
+    return input.new_empty((*input.shape[:-1], n if n >= 0 else weight.shape[0]), dtype=dtype)
+
+
+def _skinny_gemm_new(A, B, scale):
+    return A.new_empty((A.shape[0], B.shape[1]), dtype=torch.float16)
+
+
+_OTHER_RESULT = {"fp8_linear": _fp8_linear, "skinny_gemm_new": _skinny_gemm_new, "skinny_gemm_into": lambda A, B, scale, D: True}
+
+
 def register() -> None:
     for name in _RETURNS_NOTHING:
         torch.library.register_fake(f"_HFRK_C::{name}", _nothing)
     for name in _RETURNS_STATUS:
-        torch.library.register_fake(f"_HFRK_C::{name}", _success)
+        torch.library.register_fake(f"_HFRK_C::{name}", _OTHER_RESULT.get(name, _success))
 
 
 register()

@@ -21,6 +21,7 @@ from ..utils.fp8 import amax_scale, fp8_quantize
 from ..utils.weight_format import PackedWeight, pack_weight
 
 Weight = Union[Tensor, PackedWeight]
+_fp8_linear = torch.ops._HFRK_C.fp8_linear.default
 
 
 def _weight_view(weight: Weight) -> Weight:
@@ -48,6 +49,12 @@ def apply_fp8_linear(
       with the product, one rounding).  Given both, the bias is added to the residual first (one 16-bit add).
     - out_dtype: float16/bfloat16; defaults to the input's (bfloat16 for an fp8 input)
     """
+    if input.is_cuda and not torch.compiler.is_compiling():  # usual calls run as one native operator; None: not one of those
+        packed = isinstance(weight, PackedWeight)
+        out = _fp8_linear(input, weight.data if packed else weight, weight.n if packed else -1, weight_scale, input_scale, bias, residual,
+                          out_dtype)
+        if out is not None:
+            return out
     k = input.shape[-1]
     lead = input.shape[:-1]
     x = input.reshape(-1, k)

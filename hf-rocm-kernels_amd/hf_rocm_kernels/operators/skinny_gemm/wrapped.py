@@ -8,6 +8,8 @@ from ...utils.weight_format import PackedWeight
 from .binding import _skinny_gemm, _skinny_gemm_checked, _skinny_gemm_fused, _skinny_gemm_packed, _skinny_gemm_scaled
 
 _OUT_DTYPES = (torch.bfloat16, torch.float16)
+_skinny_gemm_new = torch.ops._HFRK_C.skinny_gemm_new.default
+_skinny_gemm_into = torch.ops._HFRK_C.skinny_gemm_into.default
 
 
 def skinny_gemm_checks(
@@ -117,6 +119,14 @@ def skinny_gemm(
         the (m, n) output tensor.
     Unlike the reference, a launcher status other than 0 raises instead of leaving the output untouched.
     """
+    if skinny_a.is_cuda and not isinstance(b, PackedWeight) and not torch.compiler.is_compiling():
+        # the usual call as one native operator, which takes only what needs no check below (None / False: not one of those)
+        if output is None:
+            result = _skinny_gemm_new(skinny_a, b, scale_tensor)
+            if result is not None:
+                return result
+        elif _skinny_gemm_into(skinny_a, b, scale_tensor, output):
+            return output
     if output is None:
         output = torch.zeros(size=(skinny_a.size(0), b.size(1)), dtype=torch.float16, device=skinny_a.device)
     skinny_gemm_checks(skinny_a, b, scale_tensor, output)

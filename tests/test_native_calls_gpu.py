@@ -1,0 +1,88 @@
+"""`Fp8Linear` / `apply_fp8_linear` and `skinny_gemm` as one native operator against the operator-by-operator path they replace
+(same kernels: same bits), and the calls the operator leaves to that path."""
+import itertools
+
+import pytest
+import torch
+
+import hf_rocm_kernels
+from hf_rocm_kernels.layers import Fp8Linear, apply_fp8_linear, fp8_linear
+from hf_rocm_kernels.operators.skinny_gemm import wrapped
+from hf_rocm_kernels.utils.fp8 import amax_scale, fp8_quantize
+from hf_rocm_kernels.utils.weight_format import pack_weight
+
+pytestmark = pytest.mark.gpu
+
+
+def _general(monkeypatch):
+    monkeypatch.setattr(fp8_linear, "_fp8_linear", lambda *args: None)
+    monkeypatch.setattr(wrapped, "_skinny_gemm_new", lambda *args: None)
+    monkeypatch.setattr(wrapped, "_skinny_gemm_into", lambda *args: False)
+
+
+def _bits(t):
+    return t.contiguous().view(torch.uint8)
+
+
+@pytest.mark.parametrize("rows", [1, 5, 17, 64, 65, 130])
+@pytest.mark.parametrize("n,k", [(1024, 512), (515, 1024), (2304, 4096)])
+def test_linear_same_bits_as_the_general_path(rows, n, k, monkeypatch):
+    torch.manual_seed(rows * 1000 + n)
+    w = torch.randn(n, k, device="cuda") * 0.02
+    sw = amax_scale(w, dim=1)
+    q = fp8_quantize(w, sw)[0]
+    sw = sw.reshape(-1).contiguous()
+    wide = torch.zeros(n, k + 256, device="cuda").to(q.dtype)
+    wide[:, :k].copy_(q)  # rows further apart than k
+    weights = [(q, sw), (q, sw[:1].clone()), (pack_weight(q), sw), (pack_weight(q, sw), None), (wide[:, :k], sw)]
+    for dtype, (weight, scale) in itertools.product((torch.bfloat16, torch.float16), weights):
+        x = torch.randn(rows, k, device="cuda").to(dtype)
+        x8, sx = hf_rocm_kernels.quantize_fp8(x)
+        static = (x.abs().amax().float() / 448).reshape(1)
+        bias, residual = torch.randn(n, device="cuda").to(dtype), torch.randn(rows, n, device="cuda").to(dtype)
+        calls = [dict(input=x), dict(input=x.view(1, rows, k), input_scale=static), dict(input=x, bias=bias), dict(input=x, residual=residual),
+                 dict(input=x8, input_scale=sx, out_dtype=dtype), dict(input=x8, input_scale=static, residual=residual, out_dtype=dtype),
+                 dict(input=x, bias=bias, residual=residual), dict(input=x.t().contiguous().t(), bias=bias)]
+        got = [apply_fp8_linear(weight=weight, weight_scale=scale, **c) for c in calls]
+        with monkeypatch.context() as patch:
+            _general(patch)
+            want = [apply_fp8_linear(weight=weight, weight_scale=scale, **c) for c in calls]
+        for g, w_ in zip(got, want):
+            assert g.shape == w_.shape and g.dtype == w_.dtype and torch.equal(_bits(g), _bits(w_))
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 4096, 4096), (7, 514, 512), (33, 1024, 2304), (64, 130, 256), (3, 512, 384)])
+def test_skinny_gemm_same_bits_as_the_general_path(m, n, k, monkeypatch):
+    torch.manual_seed(m)
+    a = torch.randn(m, k, device="cuda").to(torch.float8_e4m3fn)
+    b = torch.randn(n, k, device="cuda").to(torch.float8_e4m3fn).t()
+    scale = torch.tensor([0.013], device="cuda")
+    base = torch.randn(m, n, device="cuda").to(torch.bfloat16)
+    got = hf_rocm_kernels.skinny_gemm(a, b, scale), hf_rocm_kernels.skinny_gemm(a, b, scale, base.clone())
+    _general(monkeypatch)
+    want = hf_rocm_kernels.skinny_gemm(a, b, scale), hf_rocm_kernels.skinny_gemm(a, b, scale, base.clone())
+    for g, w in zip(got, want):
+        assert g.dtype == w.dtype and torch.equal(g, w)
+
+
+def test_refused_calls_are_refused_as_before():
+    a = torch.zeros(4, 512, device="cuda").to(torch.float8_e4m3fn)
+    b = torch.zeros(64, 512, device="cuda").to(torch.float8_e4m3fn)
+    one = torch.ones(1, device="cuda")
+    for bad in (lambda: hf_rocm_kernels.skinny_gemm(a, b, one), lambda: hf_rocm_kernels.skinny_gemm(a, b.t(), one.double()),
+                lambda: hf_rocm_kernels.skinny_gemm(a, b.t(), one, torch.zeros(4, 63, device="cuda", dtype=torch.float16)),
+                lambda: hf_rocm_kernels.skinny_gemm(a, b.t(), one.cpu()), lambda: apply_fp8_linear(a, b, one),
+                lambda: apply_fp8_linear(torch.zeros(4, 512, device="cuda"), b, one),
+                lambda: apply_fp8_linear(torch.zeros(4, 512, device="cuda").half(), b, None)):
+        with pytest.raises(AssertionError):
+            bad()
+    with pytest.raises(RuntimeError):
+        hf_rocm_kernels.skinny_gemm(a, b[:63].t(), one)  # an odd number of columns
+
+
+def test_linear_outputs_carry_no_autograd_history_and_keep_leading_dimensions():
+    layer = Fp8Linear.from_float(torch.nn.Linear(512, 256, device="cuda", dtype=torch.float16))
+    x = torch.randn(2, 3, 512, device="cuda", dtype=torch.float16, requires_grad=True)
+    y = layer(x)
+    assert y.shape == (2, 3, 256) and not y.requires_grad
+    assert layer(x[:0]).shape == (0, 3, 256)
