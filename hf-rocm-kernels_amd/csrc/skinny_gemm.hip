@@ -117,7 +117,7 @@ __global__ void __launch_bounds__(kGemmThreads) skinny_gemm_kernel(const GemmArg
                 dd[rt * MT + mt] = make_uint2(0u, 0u);
                 const int mrow = mt * 16 + li;
                 if (accumulate && mrow < a.m) {
-                    const uint16_t* const drow = Dbase + (long)mrow * a.n;
+                    const uint16_t* const drow = Dbase + (long)mrow * a.base_stride;
                     if (n_vec && n0 + 3 < a.n) {
                         dd[rt * MT + mt] = *reinterpret_cast<const uint2*>(drow + n0);
                     } else {
@@ -645,6 +645,7 @@ static int choose_plan(int m, int n, int k, bool packed, hfrk_gemm_plan* plan) {
 
 // D = (base ? base : 0) + scale_a x scale_b x A.B   (epilogue 0), or the fused SwiGLU form (epilogue 1).
 // use_static: partial sums and counters go to this device's `scratch` array instead of the stream's workspace.
+// base_row: base is one row of n values, added to every row.
 // rms: the activations are not read from A but built by the kernel's RMSNorm prologue from these 16-bit tensors.
 struct RmsPrologue {
     const void* input;
@@ -658,7 +659,7 @@ struct RmsPrologue {
 static int gemm_launch(const void* A, const void* B, void* D, const void* base, const float* scale_a, int sa_stride,
                        const float* scale_b, int sb_stride, const float* out_scale, int m, int n, int k, int b_stride,
                        int d_dtype, int epilogue, const hfrk_gemm_plan* user_plan, hipStream_t stream, bool packed = false,
-                       bool use_static = false, const RmsPrologue* rms = nullptr) {
+                       bool use_static = false, const RmsPrologue* rms = nullptr, bool base_row = false) {
     if (packed) b_stride = k;
     if (m < 1 || m > HFRK_GEMM_MAX_M || n < 1 || k < 1 || b_stride < k) return HFRK_BAD_SHAPE;
     if (k % 16 != 0 || (packed && k % 256 != 0)) return HFRK_K_NOT_DIVISIBLE_BY_WARPTILE_K;
@@ -700,12 +701,12 @@ static int gemm_launch(const void* A, const void* B, void* D, const void* base, 
         const int first = kStreamMaxM;
         const size_t row_bytes = (size_t)n * 2;
         int rc = gemm_launch(A, B, D, base, scale_a, sa_stride, scale_b, sb_stride, out_scale, first, n, k, b_stride, d_dtype,
-                             epilogue, nullptr, stream, packed, use_static);
+                             epilogue, nullptr, stream, packed, use_static, nullptr, base_row);
         if (rc != HFRK_SUCCESS) return rc;
         return gemm_launch(static_cast<const uint8_t*>(A) + (size_t)first * k, B, static_cast<uint8_t*>(D) + first * row_bytes,
-                           base ? static_cast<const uint8_t*>(base) + first * row_bytes : nullptr, scale_a + (size_t)first * sa_stride,
+                           base && !base_row ? static_cast<const uint8_t*>(base) + first * row_bytes : base, scale_a + (size_t)first * sa_stride,
                            sa_stride, scale_b, sb_stride, out_scale, m - first, n, k, b_stride, d_dtype, epilogue, nullptr, stream,
-                           packed, use_static);
+                           packed, use_static, nullptr, base_row);
     }
     hfrk_gemm_plan p;
     if (user_plan) {
@@ -775,6 +776,7 @@ static int gemm_launch(const void* A, const void* B, void* D, const void* base, 
     args.B = static_cast<const uint8_t*>(B);
     args.D = D;
     args.base = base;
+    args.base_stride = base_row ? 0 : n;
     args.out_scale = out_scale;
     args.scale_a = scale_a;
     args.scale_b = scale_b;
@@ -993,6 +995,15 @@ int hfrk_skinny_gemm_fused(const void* A, const void* B, void* D, const void* ba
                            int b_stride, int d_dtype, int epilogue, const hfrk_gemm_plan* plan, void* stream) {
     return hfrk::gemm_launch(A, B, D, base, scale_a, sa_stride, scale_b, sb_stride, out_scale, m, n, k, b_stride, d_dtype,
                              epilogue, plan, static_cast<hipStream_t>(stream));
+}
+
+int hfrk_linear_gemm(const void* A, const void* B, int packed, void* D, const void* base, int base_stride, const float* scale_a,
+                     int sa_stride, const float* scale_b, int sb_stride, int m, int n, int k, int b_stride, int d_dtype, void* stream) {
+    if (m > HFRK_GEMM_MAX_M)
+        return hfrk_tiled_gemm(A, B, packed, D, base, base_stride, scale_a, sa_stride, scale_b, sb_stride, m, n, k, b_stride, d_dtype, nullptr, stream);
+    if (base && base_stride != 0 && base_stride != n) return HFRK_BAD_SHAPE;
+    return hfrk::gemm_launch(A, B, D, base, scale_a, sa_stride, scale_b, sb_stride, nullptr, m, n, k, b_stride, d_dtype, HFRK_EPILOGUE_NONE,
+                             nullptr, static_cast<hipStream_t>(stream), packed != 0, false, nullptr, base && base_stride == 0);
 }
 
 int hfrk_skinny_gemm_rms_plan(int m, int n, int k, int epilogue, hfrk_gemm_plan* plan) {

@@ -67,7 +67,7 @@ __global__ void __launch_bounds__(kGemmThreads) skinny_gemm_ksplit_kernel(const 
     const __amdgpu_buffer_rsrc_t ws_rsrc = make_rsrc(a.ws, a.ws_bytes);
     const int n_out = SWIGLU ? (a.n >> 1) : a.n;  // columns of D
     const __amdgpu_buffer_rsrc_t d_rsrc = make_rsrc(a.D, (uint32_t)a.m * (uint32_t)n_out * (SWIGLU ? 1u : 2u));
-    const __amdgpu_buffer_rsrc_t base_rsrc = make_rsrc(a.base, a.base ? (uint32_t)a.m * (uint32_t)a.n * 2u : 0u);
+    const __amdgpu_buffer_rsrc_t base_rsrc = make_rsrc(a.base, a.base ? ((uint32_t)(a.m - 1) * (uint32_t)a.base_stride + (uint32_t)a.n) * 2u : 0u);
     const __amdgpu_buffer_rsrc_t sb_rsrc = make_rsrc(a.scale_b, a.scale_b ? (uint32_t)a.n * 4u : 0u);
     const bool accumulate = !SWIGLU && a.base != nullptr;
     const bool per_channel = a.scale_b && a.sb_stride;
@@ -156,18 +156,19 @@ __global__ void __launch_bounds__(kGemmThreads) skinny_gemm_ksplit_kernel(const 
         const int mrow = mt * 16 + li;
         const bool live = mrow < a.m && n0 < a.n;
         const uint32_t d_off = ((uint32_t)mrow * (uint32_t)a.n + (uint32_t)n0) * 2u;
+        const uint32_t base_off = ((uint32_t)mrow * (uint32_t)a.base_stride + (uint32_t)n0) * 2u;
         uint32_t old[4], off[4];
         v4f sb;
         if (vec) {
             sb = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(sb_rsrc, (live && per_channel) ? n0 * 4 : (int)kOutOfRange, 0, 0));
-            const v2i d = __builtin_amdgcn_raw_buffer_load_b64(base_rsrc, (live && accumulate) ? (int)d_off : (int)kOutOfRange, 0, 0);
+            const v2i d = __builtin_amdgcn_raw_buffer_load_b64(base_rsrc, (live && accumulate) ? (int)base_off : (int)kOutOfRange, 0, 0);
             old[0] = (uint32_t)d[0] & 0xffffu; old[1] = (uint32_t)d[0] >> 16;
             old[2] = (uint32_t)d[1] & 0xffffu; old[3] = (uint32_t)d[1] >> 16;
         } else {
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 off[v] = (live && n0 + v < a.n) ? d_off + 2u * v : kOutOfRange;
-                old[v] = accumulate ? (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(base_rsrc, (int)off[v], 0, 0) : 0u;
+                old[v] = accumulate ? (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(base_rsrc, off[v] == kOutOfRange ? (int)kOutOfRange : (int)(base_off + 2u * v), 0, 0) : 0u;
                 sb[v] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sb_rsrc, (live && per_channel && n0 + v < a.n) ? (n0 + v) * 4 : (int)kOutOfRange, 0, 0));
             }
         }

@@ -37,7 +37,7 @@ struct RowsEpilogue {
     __device__ __forceinline__ RowsEpilogue(const GemmArgs& args, int lane) : a(args), li(lane & 15), lg(lane >> 4) {
         n_out = SWIGLU ? (a.n >> 1) : a.n;
         d_rsrc = make_rsrc(a.D, (uint32_t)a.m * (uint32_t)n_out * (SWIGLU ? 1u : 2u));
-        base_rsrc = make_rsrc(a.base, a.base ? (uint32_t)a.m * (uint32_t)a.n * 2u : 0u);
+        base_rsrc = make_rsrc(a.base, a.base ? ((uint32_t)(a.m - 1) * (uint32_t)a.base_stride + (uint32_t)a.n) * 2u : 0u);
         sb_rsrc = make_rsrc(a.scale_b, a.scale_b ? (uint32_t)a.n * 4u : 0u);
         accumulate = !SWIGLU && a.base != nullptr;
         vec = SWIGLU || (a.n & 3) == 0;  // then a lane's four outputs are all inside n and aligned
@@ -71,7 +71,7 @@ struct RowsEpilogue {
                 p.sb[rt] = __builtin_amdgcn_raw_buffer_load_b128(sb_rsrc, (per_channel && ok) ? n0 * 4 : (int)kOutOfRange, 0, 0);
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt)
-                    p.d[mt * RT + rt] = __builtin_amdgcn_raw_buffer_load_b64(base_rsrc, (accumulate && ok && 16 * mt + li < a.m) ? (int)(((uint32_t)(16 * mt + li) * (uint32_t)a.n + (uint32_t)n0) * 2u) : (int)kOutOfRange, 0, 0);
+                    p.d[mt * RT + rt] = __builtin_amdgcn_raw_buffer_load_b64(base_rsrc, (accumulate && ok && 16 * mt + li < a.m) ? (int)(((uint32_t)(16 * mt + li) * (uint32_t)a.base_stride + (uint32_t)n0) * 2u) : (int)kOutOfRange, 0, 0);
             }
         }
         return p;
@@ -135,7 +135,8 @@ struct RowsEpilogue {
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
                     const uint32_t off = (live && n0 + v < a.n) ? d_off + 2u * v : kOutOfRange;
-                    const uint32_t old = accumulate ? (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(base_rsrc, (int)off, 0, 0) : 0u;
+                    const uint32_t base_off = off == kOutOfRange ? off : ((uint32_t)arow * (uint32_t)a.base_stride + (uint32_t)(n0 + v)) * 2u;
+                    const uint32_t old = accumulate ? (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(base_rsrc, (int)base_off, 0, 0) : 0u;
                     const float sbv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sb_rsrc, (live && per_channel && n0 + v < a.n) ? (n0 + v) * 4 : (int)kOutOfRange, 0, 0));
                     float r = acc[u][v] * (per_channel ? sa * sbv : sa);
                     if (accumulate) r += bf16 ? bf16_bits_to_float((uint16_t)old) : f16_bits_to_float((uint16_t)old);

@@ -121,7 +121,7 @@ __global__ void __launch_bounds__(kGemmThreads) skinny_gemm_stream_kernel(const 
     const __amdgpu_buffer_rsrc_t ws_rsrc = make_rsrc(a.ws, a.ws_bytes);
     const int n_out = SWIGLU ? (a.n >> 1) : a.n;  // columns of D
     const __amdgpu_buffer_rsrc_t d_rsrc = make_rsrc(a.D, (uint32_t)a.m * (uint32_t)n_out * (SWIGLU ? 1u : 2u));
-    const __amdgpu_buffer_rsrc_t base_rsrc = make_rsrc(a.base, a.base ? (uint32_t)a.m * (uint32_t)a.n * 2u : 0u);
+    const __amdgpu_buffer_rsrc_t base_rsrc = make_rsrc(a.base, a.base ? ((uint32_t)(a.m - 1) * (uint32_t)a.base_stride + (uint32_t)a.n) * 2u : 0u);
     const bool accumulate = !SWIGLU && a.base != nullptr;
     const __amdgpu_buffer_rsrc_t sb_rsrc = make_rsrc(a.scale_b, a.scale_b ? (uint32_t)a.n * 4u : 0u);
     const bool vec = SWIGLU || ((a.n & 3) == 0);  // then a lane's four outputs n0 .. n0+3 are all inside n and aligned
@@ -173,7 +173,7 @@ __global__ void __launch_bounds__(kGemmThreads) skinny_gemm_stream_kernel(const 
                 for (int mt = 0; mt < MT; ++mt) {
                     const int mrow = mt * 16 + li;
                     const bool ok = accumulate && mrow < a.m && n0 < a.n;
-                    p.d[rt * MT + mt] = __builtin_amdgcn_raw_buffer_load_b64(base_rsrc, ok ? (int)(((uint32_t)mrow * (uint32_t)a.n + (uint32_t)n0) * 2u) : (int)kOutOfRange, 0, 0);
+                    p.d[rt * MT + mt] = __builtin_amdgcn_raw_buffer_load_b64(base_rsrc, ok ? (int)(((uint32_t)mrow * (uint32_t)a.base_stride + (uint32_t)n0) * 2u) : (int)kOutOfRange, 0, 0);
                 }
             }
         }
@@ -228,7 +228,8 @@ __global__ void __launch_bounds__(kGemmThreads) skinny_gemm_stream_kernel(const 
 #pragma unroll
                     for (int v = 0; v < 4; ++v) {
                         off[v] = (live && n0 + v < a.n) ? d_off + 2u * v : kOutOfRange;
-                        old[v] = accumulate ? (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(base_rsrc, (int)off[v], 0, 0) : 0u;
+                        const uint32_t base_off = off[v] == kOutOfRange ? off[v] : ((uint32_t)mrow * (uint32_t)a.base_stride + (uint32_t)(n0 + v)) * 2u;
+                        old[v] = accumulate ? (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(base_rsrc, (int)base_off, 0, 0) : 0u;
                         sb[v] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sb_rsrc, (live && per_channel && n0 + v < a.n) ? (n0 + v) * 4 : (int)kOutOfRange, 0, 0));
                     }
                 }

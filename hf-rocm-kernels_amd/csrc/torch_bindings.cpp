@@ -512,7 +512,6 @@ at::Tensor fp8_linear(const at::Tensor& input, const at::Tensor& weight, int64_t
     if (!quantised && (k % 8 != 0 || k > 32768)) return {};
     const at::ScalarType dtype = out_dtype.value_or(quantised ? at::kBFloat16 : input.scalar_type());
     if (!is_16bit(dtype) || (bias.has_value() && residual.has_value())) return {};
-    const bool tiled = m > HFRK_GEMM_MAX_M;
     at::Tensor base;
     int base_stride = (int)n;
     if (residual.has_value()) {
@@ -527,7 +526,6 @@ at::Tensor fp8_linear(const at::Tensor& input, const at::Tensor& weight, int64_t
 
     DeviceScope scope(input);
     void* const stream = current_stream(input);
-    if (base.defined() && base_stride == 0 && !tiled) base = base.expand({m, n}).contiguous();
     at::DimVector sizes(input.sizes());
     sizes.back() = n;
     at::Tensor out = at::empty(sizes, input.options().dtype(dtype));
@@ -555,16 +553,8 @@ at::Tensor fp8_linear(const at::Tensor& input, const at::Tensor& weight, int64_t
     }
     const void* const base_ptr = base.defined() ? base.data_ptr() : nullptr;
     const int d_dtype = dtype == at::kBFloat16 ? HFRK_BF16 : HFRK_F16;
-    int status;
-    if (tiled)
-        status = hfrk_tiled_gemm(a, weight.data_ptr(), packed ? 1 : 0, out.data_ptr(), base_ptr, base_stride, sa, sa_stride, sb, sb_stride,
-                                 (int)m, (int)n, (int)k, b_stride, d_dtype, nullptr, stream);
-    else if (packed)
-        status = hfrk_skinny_gemm_packed(a, weight.data_ptr(), out.data_ptr(), base_ptr, sa, sa_stride, sb, sb_stride, nullptr, (int)m,
-                                         (int)n, (int)k, d_dtype, HFRK_EPILOGUE_NONE, nullptr, stream);
-    else
-        status = hfrk_skinny_gemm_fused(a, weight.data_ptr(), out.data_ptr(), base_ptr, sa, sa_stride, sb, sb_stride, nullptr, (int)m,
-                                        (int)n, (int)k, b_stride, d_dtype, HFRK_EPILOGUE_NONE, nullptr, stream);
+    const int status = hfrk_linear_gemm(a, weight.data_ptr(), packed ? 1 : 0, out.data_ptr(), base_ptr, base_stride, sa, sa_stride, sb,
+                                        sb_stride, (int)m, (int)n, (int)k, b_stride, d_dtype, stream);
     return status == HFRK_SUCCESS ? out : at::Tensor();
 }
 

@@ -268,6 +268,11 @@ int hfrk_skinny_gemm_packed(const void* A, const void* B_packed, void* D, const 
                             int sa_stride, const float* scale_b, int sb_stride, const float* out_scale, int m, int n,
                             int k, int d_dtype, int epilogue, const hfrk_gemm_plan* plan, void* stream);
 
+/* The linear layer's GEMM for any number of rows, under the library's own plan: a skinny GEMM up to 64 rows, hfrk_tiled_gemm (below,
+ * same arguments) above.  base_stride is 0 (one row of n values added to every row of D: a bias) or, up to 64 rows, n. */
+int hfrk_linear_gemm(const void* A, const void* B, int packed, void* D, const void* base, int base_stride, const float* scale_a,
+                     int sa_stride, const float* scale_b, int sb_stride, int m, int n, int k, int b_stride, int d_dtype, void* stream);
+
 /* How one tiled GEMM call is decomposed: an index into the library's tile shapes (0: 256 x 256, 1: 256 x 128, 2: 128 x 128,
  * 3: 128 x 64, 4: 64 x 64 rows x columns of D per workgroup), how many workgroups share a tile's k, and how many rows of tiles
  * the workgroups walk side by side. */
