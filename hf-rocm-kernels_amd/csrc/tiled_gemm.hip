@@ -59,8 +59,9 @@ static void make_tiled_plan(int m, int n, int k, hfrk_tiled_plan* plan) {
         const int tiles_m = div_up(m, s.bm);
         const long tiles = (long)tiles_m * div_up(n, s.bn);
         for (int splits = 1; splits <= 8 && splits <= stages; ++splits) {
-            // a split keeps at least two stages and the launch at most two workgroups per compute unit
-            if (splits > 1 && (tiles * splits > 2 * kNumCU || stages < 2 * splits)) break;
+            // a split keeps at least two stages, the launch at most two workgroups per compute unit, and the partial tiles fit the
+            // stream's workspace (256 x 256 tiles: 256 of them)
+            if (splits > 1 && (tiles * splits > 2 * kNumCU || stages < 2 * splits || tiled_ws_bytes(s, m, n, splits) > kWsFloats * sizeof(float))) break;
             const float t = tiled_cost(m, n, k, shape, splits);
             if (t < best) {
                 best = t;
