@@ -17,6 +17,7 @@ from .. import _capi
 from ..operators.quantize import quantize_fp8
 from ..operators.skinny_gemm import skinny_gemm_add, skinny_gemm_scaled
 from ..operators.skinny_gemm.wrapped import skinny_gemm_checks
+from ..utils.dispatch import runs_now
 from ..utils.fp8 import amax_scale, fp8_quantize
 from ..utils.weight_format import PackedWeight, pack_weight
 
@@ -49,7 +50,7 @@ def apply_fp8_linear(
       with the product, one rounding).  Given both, the bias is added to the residual first (one 16-bit add).
     - out_dtype: float16/bfloat16; defaults to the input's (bfloat16 for an fp8 input)
     """
-    if input.is_cuda and not torch.compiler.is_compiling():  # usual calls run as one native operator; None: not one of those
+    if runs_now(input):  # usual calls run as one native operator; None: not one of those
         packed = isinstance(weight, PackedWeight)
         out = _fp8_linear(input, weight.data if packed else weight, weight.n if packed else -1, weight_scale, input_scale, bias, residual,
                           out_dtype)

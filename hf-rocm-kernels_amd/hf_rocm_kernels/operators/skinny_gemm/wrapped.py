@@ -4,6 +4,7 @@ import torch
 from torch import Tensor
 
 from ... import _capi
+from ...utils.dispatch import runs_now
 from ...utils.weight_format import PackedWeight
 from .binding import _skinny_gemm, _skinny_gemm_checked, _skinny_gemm_fused, _skinny_gemm_packed, _skinny_gemm_scaled
 
@@ -119,7 +120,7 @@ def skinny_gemm(
         the (m, n) output tensor.
     Unlike the reference, a launcher status other than 0 raises instead of leaving the output untouched.
     """
-    if skinny_a.is_cuda and not isinstance(b, PackedWeight) and not torch.compiler.is_compiling():
+    if not isinstance(b, PackedWeight) and runs_now(skinny_a):
         # the usual call as one native operator, which takes only what needs no check below (None / False: not one of those)
         if output is None:
             result = _skinny_gemm_new(skinny_a, b, scale_tensor)

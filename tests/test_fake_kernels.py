@@ -108,3 +108,17 @@ def test_convert_linear_layers_and_state_dict_round_trip_on_the_cpu():
         assert torch.equal(a.weight_data.view(torch.uint8), b.weight_data.view(torch.uint8)) and torch.equal(a.weight_scale, b.weight_scale)
         assert b.weight is b.weight_data and not b.packed
     assert "weight=row-major" in repr(other.down)
+
+
+def test_a_traced_call_records_operators_that_check_their_arguments():
+    """The whole-call operators return nothing for a call they do not take, so a trace must not hold one, and a call that is
+    refused on tensors is refused on fake ones."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    with FakeTensorMode():
+        x, w, sw = torch.empty(8, 512, device="cuda", dtype=torch.bfloat16), _fp8(256, 512), torch.empty(256, device="cuda")
+        graph = make_fx(lambda a: apply_fp8_linear(a, w, sw))(x)
+        assert not any("fp8_linear" in str(node.target) for node in graph.graph.nodes)
+        with pytest.raises(AssertionError):
+            apply_fp8_linear(x, _fp8(256, 768), sw)
+        with pytest.raises(AssertionError):
+            hf_rocm_kernels.skinny_gemm(_fp8(8, 512), _fp8(256, 768).t(), torch.empty(1, device="cuda"))
