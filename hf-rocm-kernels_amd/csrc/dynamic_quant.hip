@@ -20,39 +20,6 @@ namespace hfrk {
 constexpr int kDynMaxThreads = 1024;
 constexpr int kDynMaxIters = 4;
 
-__device__ __forceinline__ float dyn_wave_sum(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
-__device__ __forceinline__ float dyn_wave_max(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-    return v;
-}
-
-// Sum / max over the workgroup; every thread returns the same bits.  `red` holds 16 floats and is not reused.
-__device__ __forceinline__ float dyn_block_sum(float v, float* red) {
-    v = dyn_wave_sum(v);
-    const int wave = threadIdx.x >> 6, nwaves = (blockDim.x + 63) >> 6;
-    if ((threadIdx.x & 63) == 0) red[wave] = v;
-    __syncthreads();
-    float total = 0.f;
-    for (int w = 0; w < nwaves; ++w) total += red[w];
-    return total;
-}
-
-__device__ __forceinline__ float dyn_block_max(float v, float* red) {
-    v = dyn_wave_max(v);
-    const int wave = threadIdx.x >> 6, nwaves = (blockDim.x + 63) >> 6;
-    if ((threadIdx.x & 63) == 0) red[wave] = v;
-    __syncthreads();
-    float m = 0.f;
-    for (int w = 0; w < nwaves; ++w) m = fmaxf(m, red[w]);
-    return m;
-}
-
 __device__ __forceinline__ void dyn_zero_row(uint16_t* next_buffer, int buffer_cols) {
     if (buffer_cols <= 0) return;
     uint16_t* const row = next_buffer + (long)blockIdx.x * buffer_cols;
@@ -68,22 +35,23 @@ __device__ __forceinline__ void dyn_zero_row(uint16_t* next_buffer, int buffer_c
 
 // Quantise the cached row: scale from the row maximum, 8 values per 8-byte store.
 template <int ITERS>
-__device__ __forceinline__ void dyn_quantise_row(const float (&y)[ITERS][8], float amax, uint8_t* out_row, float* scales,
-                                                 int nvec) {
+__device__ __forceinline__ void dyn_store_row(const float (&y)[ITERS][8], float inv, __amdgpu_buffer_rsrc_t out_row) {
+#pragma unroll
+    for (int it = 0; it < ITERS; ++it) {
+        uint32_t p0 = cvt_pk_fp8(y[it][0] * inv, y[it][1] * inv, 0u, false);
+        p0 = cvt_pk_fp8(y[it][2] * inv, y[it][3] * inv, p0, true);
+        uint32_t p1 = cvt_pk_fp8(y[it][4] * inv, y[it][5] * inv, 0u, false);
+        p1 = cvt_pk_fp8(y[it][6] * inv, y[it][7] * inv, p1, true);
+        store_fp8_piece(out_row, threadIdx.x + it * blockDim.x, make_uint2(p0, p1));
+    }
+}
+
+template <int ITERS>
+__device__ __forceinline__ void dyn_quantise_row(const float (&y)[ITERS][8], float amax, __amdgpu_buffer_rsrc_t out_row, float* scales) {
     const float scale = fmaxf(amax / 448.0f, FLT_MIN);
     const float inv = 1.0f / scale;
     if (threadIdx.x == 0) scales[blockIdx.x] = scale;
-#pragma unroll
-    for (int it = 0; it < ITERS; ++it) {
-        const int v = threadIdx.x + it * blockDim.x;
-        if (v < nvec) {
-            uint32_t p0 = cvt_pk_fp8(y[it][0] * inv, y[it][1] * inv, 0u, false);
-            p0 = cvt_pk_fp8(y[it][2] * inv, y[it][3] * inv, p0, true);
-            uint32_t p1 = cvt_pk_fp8(y[it][4] * inv, y[it][5] * inv, 0u, false);
-            p1 = cvt_pk_fp8(y[it][6] * inv, y[it][7] * inv, p1, true);
-            reinterpret_cast<uint2*>(out_row)[v] = make_uint2(p0, p1);
-        }
-    }
+    dyn_store_row<ITERS>(y, inv, out_row);
 }
 
 template <int DT, int ITERS>
@@ -91,42 +59,39 @@ __global__ void __launch_bounds__(kDynMaxThreads) residual_rms_dynamic_kernel(
     const uint16_t* __restrict__ input, uint16_t* __restrict__ residual, const uint16_t* __restrict__ weight,
     uint8_t* __restrict__ output, float* __restrict__ scales, uint16_t* __restrict__ next_buffer, float epsilon, int cols,
     int buffer_cols) {
-    __shared__ float red_sum[16], red_max[16];
+    __shared__ __align__(16) float red_sum[16], red_max[16];
     const long row_off = (long)blockIdx.x * cols;
-    const int nvec = cols >> 3;
-    uint4 wreg[ITERS];
+    const uint32_t row_bytes = (uint32_t)cols * 2u;
+    const __amdgpu_buffer_rsrc_t rin = make_rsrc(input + row_off, row_bytes), rres = make_rsrc(residual + row_off, row_bytes),
+                                 rweight = make_rsrc(weight, row_bytes);
+    uint4 areg[ITERS], rreg[ITERS], wreg[ITERS];
     float y[ITERS][8];
     float ssq = 0.f;
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
         const int v = threadIdx.x + it * blockDim.x;
-        wreg[it] = make_uint4(0, 0, 0, 0);
-        if (v < nvec) wreg[it] = reinterpret_cast<const uint4*>(weight)[v];
+        areg[it] = load_piece(rin, v);
+        rreg[it] = load_piece(rres, v);
     }
+#pragma unroll
+    for (int it = 0; it < ITERS; ++it) wreg[it] = load_piece(rweight, threadIdx.x + it * blockDim.x);
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
-        const int v = threadIdx.x + it * blockDim.x;
+        const uint32_t aw[4] = {areg[it].x, areg[it].y, areg[it].z, areg[it].w}, rw[4] = {rreg[it].x, rreg[it].y, rreg[it].z, rreg[it].w};
+        uint32_t zw[4];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) y[it][j] = 0.f;
-        if (v < nvec) {
-            const uint4 a = reinterpret_cast<const uint4*>(input + row_off)[v];
-            const uint4 r = reinterpret_cast<const uint4*>(residual + row_off)[v];
-            const uint32_t aw[4] = {a.x, a.y, a.z, a.w}, rw[4] = {r.x, r.y, r.z, r.w};
-            uint32_t zw[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const uint16_t lo = store16<DT>(load16<DT>((uint16_t)(aw[j] & 0xffff)) + load16<DT>((uint16_t)(rw[j] & 0xffff)));
-                const uint16_t hi = store16<DT>(load16<DT>((uint16_t)(aw[j] >> 16)) + load16<DT>((uint16_t)(rw[j] >> 16)));
-                y[it][2 * j] = load16<DT>(lo);
-                y[it][2 * j + 1] = load16<DT>(hi);
-                ssq += y[it][2 * j] * y[it][2 * j];
-                ssq += y[it][2 * j + 1] * y[it][2 * j + 1];
-                zw[j] = (uint32_t)lo | ((uint32_t)hi << 16);
-            }
-            reinterpret_cast<uint4*>(residual + row_off)[v] = make_uint4(zw[0], zw[1], zw[2], zw[3]);
+        for (int j = 0; j < 4; ++j) {
+            const uint16_t lo = store16<DT>(load16<DT>((uint16_t)(aw[j] & 0xffff)) + load16<DT>((uint16_t)(rw[j] & 0xffff)));
+            const uint16_t hi = store16<DT>(load16<DT>((uint16_t)(aw[j] >> 16)) + load16<DT>((uint16_t)(rw[j] >> 16)));
+            y[it][2 * j] = load16<DT>(lo);
+            y[it][2 * j + 1] = load16<DT>(hi);
+            ssq += y[it][2 * j] * y[it][2 * j];
+            ssq += y[it][2 * j + 1] * y[it][2 * j + 1];
+            zw[j] = (uint32_t)lo | ((uint32_t)hi << 16);
         }
+        store_piece(rres, threadIdx.x + it * blockDim.x, make_uint4(zw[0], zw[1], zw[2], zw[3]));
     }
-    const float norm = rsqrtf(dyn_block_sum(ssq, red_sum) / (float)cols + epsilon);
+    const float norm = rsqrtf(block_sum(ssq, red_sum) / (float)cols + epsilon);
     float amax = 0.f;
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
@@ -138,8 +103,8 @@ __global__ void __launch_bounds__(kDynMaxThreads) residual_rms_dynamic_kernel(
             amax = fmaxf(amax, fmaxf(fabsf(y[it][2 * j]), fabsf(y[it][2 * j + 1])));
         }
     }
-    amax = dyn_block_max(amax, red_max);
-    dyn_quantise_row<ITERS>(y, amax, output + row_off, scales, nvec);
+    amax = block_max(amax, red_max);
+    dyn_quantise_row<ITERS>(y, amax, make_rsrc(output + row_off, (uint32_t)cols), scales);
     dyn_zero_row(next_buffer, buffer_cols);
 }
 
@@ -147,31 +112,30 @@ template <int DT, int ITERS>
 __global__ void __launch_bounds__(kDynMaxThreads) swiglu_dynamic_kernel(
     const uint16_t* __restrict__ gate_up, uint8_t* __restrict__ output, float* __restrict__ scales,
     uint16_t* __restrict__ next_buffer, int cols, int buffer_cols) {
-    __shared__ float red_max[16];
+    __shared__ __align__(16) float red_max[16];
     const uint16_t* const grow = gate_up + (long)blockIdx.x * 2 * cols;
-    const int nvec = cols >> 3;
+    const __amdgpu_buffer_rsrc_t rgate = make_rsrc(grow, (uint32_t)cols * 2u), rup = make_rsrc(grow + cols, (uint32_t)cols * 2u);
+    uint4 g[ITERS], u[ITERS];
     float y[ITERS][8];
     float amax = 0.f;
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
         const int v = threadIdx.x + it * blockDim.x;
+        g[it] = load_piece<true>(rgate, v);
+        u[it] = load_piece<true>(rup, v);
+    }
 #pragma unroll
-        for (int j = 0; j < 8; ++j) y[it][j] = 0.f;
-        if (v < nvec) {
-            const v4i g = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(grow) + v);
-            const v4i u = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(grow + cols) + v);
-            const uint32_t gw[4] = {(uint32_t)g[0], (uint32_t)g[1], (uint32_t)g[2], (uint32_t)g[3]};
-            const uint32_t uw[4] = {(uint32_t)u[0], (uint32_t)u[1], (uint32_t)u[2], (uint32_t)u[3]};
+    for (int it = 0; it < ITERS; ++it) {
+        const uint32_t gw[4] = {g[it].x, g[it].y, g[it].z, g[it].w}, uw[4] = {u[it].x, u[it].y, u[it].z, u[it].w};
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                y[it][2 * j] = silu_mul(load16<DT>((uint16_t)(gw[j] & 0xffff)), load16<DT>((uint16_t)(uw[j] & 0xffff)), 1.0f);
-                y[it][2 * j + 1] = silu_mul(load16<DT>((uint16_t)(gw[j] >> 16)), load16<DT>((uint16_t)(uw[j] >> 16)), 1.0f);
-                amax = fmaxf(amax, fmaxf(fabsf(y[it][2 * j]), fabsf(y[it][2 * j + 1])));
-            }
+        for (int j = 0; j < 4; ++j) {
+            y[it][2 * j] = silu_mul(load16<DT>((uint16_t)(gw[j] & 0xffff)), load16<DT>((uint16_t)(uw[j] & 0xffff)), 1.0f);
+            y[it][2 * j + 1] = silu_mul(load16<DT>((uint16_t)(gw[j] >> 16)), load16<DT>((uint16_t)(uw[j] >> 16)), 1.0f);
+            amax = fmaxf(amax, fmaxf(fabsf(y[it][2 * j]), fabsf(y[it][2 * j + 1])));
         }
     }
-    amax = dyn_block_max(amax, red_max);
-    dyn_quantise_row<ITERS>(y, amax, output + (long)blockIdx.x * cols, scales, nvec);
+    amax = block_max(amax, red_max);
+    dyn_quantise_row<ITERS>(y, amax, make_rsrc(output + (long)blockIdx.x * cols, (uint32_t)cols), scales);
     dyn_zero_row(next_buffer, buffer_cols);
 }
 
@@ -182,44 +146,30 @@ template <int DT, int ITERS>
 __global__ void __launch_bounds__(kDynMaxThreads) quantize_rows_kernel(
     const uint16_t* __restrict__ input, const float* __restrict__ static_scale, uint8_t* __restrict__ output,
     float* __restrict__ scales, int cols) {
-    __shared__ float red_max[16];
-    const uint16_t* const row = input + (long)blockIdx.x * cols;
-    const int nvec = cols >> 3;
+    __shared__ __align__(16) float red_max[16];
+    const __amdgpu_buffer_rsrc_t rin = make_rsrc(input + (long)blockIdx.x * cols, (uint32_t)cols * 2u),
+                                 rout = make_rsrc(output + (long)blockIdx.x * cols, (uint32_t)cols);
+    uint4 x[ITERS];
     float y[ITERS][8];
     float amax = 0.f;
 #pragma unroll
+    for (int it = 0; it < ITERS; ++it) x[it] = load_piece<true>(rin, threadIdx.x + it * blockDim.x);
+#pragma unroll
     for (int it = 0; it < ITERS; ++it) {
-        const int v = threadIdx.x + it * blockDim.x;
+        const uint32_t xw[4] = {x[it].x, x[it].y, x[it].z, x[it].w};
 #pragma unroll
-        for (int j = 0; j < 8; ++j) y[it][j] = 0.f;
-        if (v < nvec) {
-            const v4i x = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(row) + v);
-            const uint32_t xw[4] = {(uint32_t)x[0], (uint32_t)x[1], (uint32_t)x[2], (uint32_t)x[3]};
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                y[it][2 * j] = load16<DT>((uint16_t)(xw[j] & 0xffff));
-                y[it][2 * j + 1] = load16<DT>((uint16_t)(xw[j] >> 16));
-                amax = fmaxf(amax, fmaxf(fabsf(y[it][2 * j]), fabsf(y[it][2 * j + 1])));
-            }
+        for (int j = 0; j < 4; ++j) {
+            y[it][2 * j] = load16<DT>((uint16_t)(xw[j] & 0xffff));
+            y[it][2 * j + 1] = load16<DT>((uint16_t)(xw[j] >> 16));
+            amax = fmaxf(amax, fmaxf(fabsf(y[it][2 * j]), fabsf(y[it][2 * j + 1])));
         }
     }
     if (static_scale) {
-        const float inv = 1.0f / static_scale[0];
-#pragma unroll
-        for (int it = 0; it < ITERS; ++it) {
-            const int v = threadIdx.x + it * blockDim.x;
-            if (v < nvec) {
-                uint32_t p0 = cvt_pk_fp8(y[it][0] * inv, y[it][1] * inv, 0u, false);
-                p0 = cvt_pk_fp8(y[it][2] * inv, y[it][3] * inv, p0, true);
-                uint32_t p1 = cvt_pk_fp8(y[it][4] * inv, y[it][5] * inv, 0u, false);
-                p1 = cvt_pk_fp8(y[it][6] * inv, y[it][7] * inv, p1, true);
-                reinterpret_cast<uint2*>(output + (long)blockIdx.x * cols)[v] = make_uint2(p0, p1);
-            }
-        }
+        dyn_store_row<ITERS>(y, 1.0f / static_scale[0], rout);
         return;
     }
-    amax = dyn_block_max(amax, red_max);
-    dyn_quantise_row<ITERS>(y, amax, output + (long)blockIdx.x * cols, scales, nvec);
+    amax = block_max(amax, red_max);
+    dyn_quantise_row<ITERS>(y, amax, rout, scales);
 }
 
 static bool dyn_aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }

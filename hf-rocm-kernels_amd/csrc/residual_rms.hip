@@ -3,7 +3,7 @@
 // Replaces csrc/op_src/residual_rms/residual_rms_dispatch.cu:8-63 and its two kernels
 // (residual_rms_scalar.cu:11-74, residual_rms_vectorized.cu:13-172).  One workgroup per row.  The summed row is
 // kept in registers between the two passes (the reference parks it in a 32 KB LDS array), the sum of squares is
-// reduced with cross-lane shuffles inside each wavefront and one LDS exchange of <= 16 floats between wavefronts,
+// reduced in registers inside each wavefront and by one LDS exchange of <= 16 floats between wavefronts,
 // and every thread adds those partials in the same order, so the normaliser is identical for the whole row.
 //
 // Arithmetic (same points of rounding as the reference's torch functions, operators/residual_rms/reference.py:7-36):
@@ -17,17 +17,6 @@
 namespace hfrk {
 
 constexpr int kRmsMaxThreads = 1024;
-
-// Sum over the workgroup; every thread returns the same bits.
-__device__ __forceinline__ float block_sum(float v, float* red) {
-    v = wave_sum(v);
-    const int wave = threadIdx.x >> 6, nwaves = (blockDim.x + 63) >> 6;
-    if ((threadIdx.x & 63) == 0) red[wave] = v;
-    __syncthreads();
-    float total = 0.f;
-    for (int w = 0; w < nwaves; ++w) total += red[w];
-    return total;
-}
 
 __device__ __forceinline__ void zero_next_buffer_row(uint16_t* next_buffer, int buffer_cols) {
     if (buffer_cols <= 0) return;
@@ -49,29 +38,31 @@ __global__ void __launch_bounds__(kRmsMaxThreads) residual_rms_vec_kernel(
     const uint16_t* __restrict__ input, uint16_t* __restrict__ residual, const uint16_t* __restrict__ weight,
     const float* __restrict__ scale_tensor, void* __restrict__ output, uint16_t* __restrict__ next_buffer,
     float epsilon, int cols, int buffer_cols) {
-    __shared__ float red[16];
+    __shared__ __align__(16) float red[16];
     const long row_off = (long)blockIdx.x * cols;
-    const int nvec = cols >> 3;
-    uint4 z[ITERS], wreg[ITERS];
+    const uint32_t row_bytes = (uint32_t)cols * 2u;
+    const __amdgpu_buffer_rsrc_t rin = make_rsrc(input + row_off, row_bytes), rres = make_rsrc(residual + row_off, row_bytes),
+                                 rweight = make_rsrc(weight, row_bytes);
+    const __amdgpu_buffer_rsrc_t rout = FP8_OUT ? make_rsrc(static_cast<uint8_t*>(output) + row_off, (uint32_t)cols)
+                                                : make_rsrc(static_cast<uint16_t*>(output) + row_off, row_bytes);
+    uint4 a[ITERS], z[ITERS], wreg[ITERS];
     float ssq = 0.f;
-    // Everything the second pass needs is requested now, so that the kernel pays one memory latency, not two.
+    // Everything both passes need is requested now, so that the kernel pays one memory latency.  The input is read past the caches:
+    // nobody reads it again, and the residual and the weight keep their place (2048 x 16384 fp16: 41.5 -> 37 us, 6.3 TB/s).
     float scale = 1.f;
     if constexpr (FP8_OUT) scale = scale_tensor[0];
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
         const int v = threadIdx.x + it * blockDim.x;
-        wreg[it] = make_uint4(0, 0, 0, 0);
-        if (v < nvec) wreg[it] = reinterpret_cast<const uint4*>(weight)[v];
+        a[it] = load_piece<true>(rin, v);
+        z[it] = load_piece(rres, v);
     }
 #pragma unroll
+    for (int it = 0; it < ITERS; ++it) wreg[it] = load_piece(rweight, threadIdx.x + it * blockDim.x);
+#pragma unroll
     for (int it = 0; it < ITERS; ++it) {
-        const int v = threadIdx.x + it * blockDim.x;
-        if (v < nvec) {
-            const uint4 a = reinterpret_cast<const uint4*>(input + row_off)[v];
-            const uint4 r = reinterpret_cast<const uint4*>(residual + row_off)[v];
-            z[it] = rms_add_square<DT>(a, r, ssq);
-            reinterpret_cast<uint4*>(residual + row_off)[v] = z[it];
-        }
+        z[it] = rms_add_square<DT>(a[it], z[it], ssq);
+        store_piece(rres, threadIdx.x + it * blockDim.x, z[it]);
     }
     const float total = block_sum(ssq, red);
     const float norm = rsqrtf(total / (float)cols + epsilon);
@@ -80,23 +71,21 @@ __global__ void __launch_bounds__(kRmsMaxThreads) residual_rms_vec_kernel(
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
         const int v = threadIdx.x + it * blockDim.x;
-        if (v < nvec) {
-            const uint4 w = wreg[it];
-            const uint32_t zw[4] = {z[it].x, z[it].y, z[it].z, z[it].w}, ww[4] = {w.x, w.y, w.z, w.w};
-            if constexpr (FP8_OUT) {
-                reinterpret_cast<uint2*>(static_cast<uint8_t*>(output) + row_off)[v] = rms_scale_to_fp8<DT>(z[it], w, norm, inv_scale);
-            } else {
-                uint32_t ow[4];
+        const uint4 w = wreg[it];
+        const uint32_t zw[4] = {z[it].x, z[it].y, z[it].z, z[it].w}, ww[4] = {w.x, w.y, w.z, w.w};
+        if constexpr (FP8_OUT) {
+            store_fp8_piece(rout, v, rms_scale_to_fp8<DT>(z[it], w, norm, inv_scale));
+        } else {
+            uint32_t ow[4];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const uint16_t nl = store16<DT>(load16<DT>((uint16_t)(zw[j] & 0xffff)) * norm);
-                    const uint16_t nh = store16<DT>(load16<DT>((uint16_t)(zw[j] >> 16)) * norm);
-                    const uint16_t ol = store16<DT>(load16<DT>(nl) * load16<DT>((uint16_t)(ww[j] & 0xffff)));
-                    const uint16_t oh = store16<DT>(load16<DT>(nh) * load16<DT>((uint16_t)(ww[j] >> 16)));
-                    ow[j] = (uint32_t)ol | ((uint32_t)oh << 16);
-                }
-                reinterpret_cast<uint4*>(static_cast<uint16_t*>(output) + row_off)[v] = make_uint4(ow[0], ow[1], ow[2], ow[3]);
+            for (int j = 0; j < 4; ++j) {
+                const uint16_t nl = store16<DT>(load16<DT>((uint16_t)(zw[j] & 0xffff)) * norm);
+                const uint16_t nh = store16<DT>(load16<DT>((uint16_t)(zw[j] >> 16)) * norm);
+                const uint16_t ol = store16<DT>(load16<DT>(nl) * load16<DT>((uint16_t)(ww[j] & 0xffff)));
+                const uint16_t oh = store16<DT>(load16<DT>(nh) * load16<DT>((uint16_t)(ww[j] >> 16)));
+                ow[j] = (uint32_t)ol | ((uint32_t)oh << 16);
             }
+            store_piece(rout, v, make_uint4(ow[0], ow[1], ow[2], ow[3]));
         }
     }
     zero_next_buffer_row(next_buffer, buffer_cols);
@@ -109,7 +98,7 @@ __global__ void __launch_bounds__(kRmsMaxThreads) residual_rms_scalar_kernel(
     const uint16_t* __restrict__ input, uint16_t* __restrict__ residual, const uint16_t* __restrict__ weight,
     const float* __restrict__ scale_tensor, void* __restrict__ output, uint16_t* __restrict__ next_buffer,
     float epsilon, int cols, int buffer_cols) {
-    __shared__ float red[16];
+    __shared__ __align__(16) float red[16];
     const long row_off = (long)blockIdx.x * cols;
     float ssq = 0.f;
     for (int i = threadIdx.x; i < cols; i += blockDim.x) {
