@@ -24,47 +24,56 @@ __device__ __forceinline__ void zero_next_buffer(uint16_t* next_buffer, long tot
     for (long i = head + body * 8 + tid; i < total; i += nthreads) next_buffer[i] = 0;
 }
 
-template <int DT>
+constexpr int kSwigluPieces = 2;
+
+// Bound by memory.  A thread requests all its pieces before it works on the first, and each further set behind them.  INDEX is
+// 32 bits wide wherever the pieces can be counted in it: the division by the row length is per piece, and in 64 bits it was most
+// of the kernel's instructions.  2048 x 6656 fp16: 14.1 -> 11.9 us.
+template <int DT, typename INDEX>
 __global__ void __launch_bounds__(1024) swiglu_vec_kernel(const uint16_t* __restrict__ gate_up,
                                                           const float* __restrict__ scale_tensor,
                                                           uint8_t* __restrict__ output, uint16_t* __restrict__ next_buffer,
                                                           int rows, int cols, int buffer_cols) {
-    const int vpr = cols >> 3;  // 8-element pieces per output row
-    const long nvec = (long)rows * vpr;
-    const long stride = (long)gridDim.x * blockDim.x;
-    long v = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    v4i g = {0, 0, 0, 0}, u = {0, 0, 0, 0};
-    auto fetch = [&](long idx) __attribute__((always_inline)) {
-        const long r = idx / vpr;
-        const int c = (int)(idx - r * vpr);
-        const uint16_t* const grow = gate_up + r * 2 * cols;
-        g = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(grow) + c);
-        u = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(grow + cols) + c);
+    const INDEX vpr = (INDEX)(cols >> 3);  // 8-element pieces per output row
+    const INDEX nvec = (INDEX)rows * vpr;
+    const INDEX stride = (INDEX)gridDim.x * blockDim.x;
+    const INDEX first = (INDEX)blockIdx.x * blockDim.x + threadIdx.x;
+    v4i g[kSwigluPieces], u[kSwigluPieces];
+    auto fetch = [&](INDEX at) __attribute__((always_inline)) {
+#pragma unroll
+        for (int p = 0; p < kSwigluPieces; ++p) {
+            const INDEX v = at + p * stride;
+            if (v < nvec) {
+                const INDEX r = v / vpr;
+                const uint16_t* const grow = gate_up + (long)r * 2 * cols;
+                g[p] = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(grow) + (v - r * vpr));
+                u[p] = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(grow + cols) + (v - r * vpr));
+            }
+        }
     };
-    // The first piece is requested before the scale, and each next piece before the current one is processed: the
-    // kernel is a few microseconds long and pays every dependent memory latency in full.
-    if (v < nvec) fetch(v);
+    fetch(first);
     const float s = scale_tensor[0];
     const float inv_scale = (s != 0.f) ? 1.f / s : 1.f;
-    while (v < nvec) {
-        const uint32_t gw[4] = {(uint32_t)g[0], (uint32_t)g[1], (uint32_t)g[2], (uint32_t)g[3]};
-        const uint32_t uw[4] = {(uint32_t)u[0], (uint32_t)u[1], (uint32_t)u[2], (uint32_t)u[3]};
-        const long cur = v;
-        v += stride;
-        if (v < nvec) fetch(v);
-        float y[8];
+    for (INDEX at = first; at < nvec; at += kSwigluPieces * stride) {
+        if (at != first) fetch(at);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            y[2 * j] = silu_mul(load16<DT>((uint16_t)(gw[j] & 0xffff)), load16<DT>((uint16_t)(uw[j] & 0xffff)), inv_scale);
-            y[2 * j + 1] = silu_mul(load16<DT>((uint16_t)(gw[j] >> 16)), load16<DT>((uint16_t)(uw[j] >> 16)), inv_scale);
+        for (int p = 0; p < kSwigluPieces; ++p) {
+            const INDEX v = at + p * stride;
+            if (v >= nvec) break;
+            float y[8];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t gw = (uint32_t)g[p][j], uw = (uint32_t)u[p][j];
+                y[2 * j] = silu_mul(load16<DT>((uint16_t)(gw & 0xffff)), load16<DT>((uint16_t)(uw & 0xffff)), inv_scale);
+                y[2 * j + 1] = silu_mul(load16<DT>((uint16_t)(gw >> 16)), load16<DT>((uint16_t)(uw >> 16)), inv_scale);
+            }
+            uint32_t p0 = cvt_pk_fp8(y[0], y[1], 0u, false);
+            p0 = cvt_pk_fp8(y[2], y[3], p0, true);
+            uint32_t p1 = cvt_pk_fp8(y[4], y[5], 0u, false);
+            p1 = cvt_pk_fp8(y[6], y[7], p1, true);
+            // rows of the output follow one another: piece v lies at 8 v
+            reinterpret_cast<uint2*>(output)[v] = make_uint2(p0, p1);
         }
-        uint32_t p0 = cvt_pk_fp8(y[0], y[1], 0u, false);
-        p0 = cvt_pk_fp8(y[2], y[3], p0, true);
-        uint32_t p1 = cvt_pk_fp8(y[4], y[5], 0u, false);
-        p1 = cvt_pk_fp8(y[6], y[7], p1, true);
-        const long r = cur / vpr;
-        const int c = (int)(cur - r * vpr);
-        reinterpret_cast<uint2*>(output + r * cols)[c] = make_uint2(p0, p1);
     }
     zero_next_buffer(next_buffer, (long)rows * buffer_cols);
 }
@@ -107,17 +116,26 @@ extern "C" int hfrk_swiglu(const void* gate_up, const float* scale_tensor, void*
     int threads = num_threads > 0 ? num_threads : 256;
     const long work = vec ? (long)rows * (cols / 8) : (long)rows * cols;
     long blocks = (work + threads - 1) / threads;
-    // enough workgroups to cover the chip a few times over; the loop in the kernel strides over the rest
-    const long cap = (long)kNumCU * 16;
+    // one piece per thread until the chip is full of threads (2048 per compute unit), then kSwigluPieces; the loop in the kernel
+    // strides over what a launch of 64 workgroups per compute unit leaves
+    if (vec && work > (long)kNumCU * 2048) blocks = (work + (long)threads * kSwigluPieces - 1) / ((long)threads * kSwigluPieces);
+    const long cap = vec ? (long)kNumCU * 64 : (long)kNumCU * 16;
     if (blocks > cap) blocks = cap;
     if (blocks < 1) blocks = 1;
+    // no index of a thread, the first one past the end among them, leaves 32 bits
+    const bool narrow = work + 2L * kSwigluPieces * blocks * threads < (1L << 32);
+#define HFRK_SWIGLU(KERNEL) \
+    hipLaunchKernelGGL((KERNEL), dim3((unsigned)blocks), dim3(threads), 0, s, in, scale_tensor, out, nb, rows, cols, buffer_cols)
     if (io_dtype == HFRK_F16) {
-        if (vec) hipLaunchKernelGGL((swiglu_vec_kernel<HFRK_F16>), dim3((unsigned)blocks), dim3(threads), 0, s, in, scale_tensor, out, nb, rows, cols, buffer_cols);
-        else hipLaunchKernelGGL((swiglu_scalar_kernel<HFRK_F16>), dim3((unsigned)blocks), dim3(threads), 0, s, in, scale_tensor, out, nb, rows, cols, buffer_cols);
+        if (!vec) HFRK_SWIGLU(swiglu_scalar_kernel<HFRK_F16>);
+        else if (narrow) HFRK_SWIGLU((swiglu_vec_kernel<HFRK_F16, uint32_t>));
+        else HFRK_SWIGLU((swiglu_vec_kernel<HFRK_F16, uint64_t>));
     } else {
-        if (vec) hipLaunchKernelGGL((swiglu_vec_kernel<HFRK_BF16>), dim3((unsigned)blocks), dim3(threads), 0, s, in, scale_tensor, out, nb, rows, cols, buffer_cols);
-        else hipLaunchKernelGGL((swiglu_scalar_kernel<HFRK_BF16>), dim3((unsigned)blocks), dim3(threads), 0, s, in, scale_tensor, out, nb, rows, cols, buffer_cols);
+        if (!vec) HFRK_SWIGLU(swiglu_scalar_kernel<HFRK_BF16>);
+        else if (narrow) HFRK_SWIGLU((swiglu_vec_kernel<HFRK_BF16, uint32_t>));
+        else HFRK_SWIGLU((swiglu_vec_kernel<HFRK_BF16, uint64_t>));
     }
+#undef HFRK_SWIGLU
     HFRK_HIP_TRY(hipGetLastError());
     return HFRK_SUCCESS;
 }
