@@ -36,6 +36,7 @@
 
 #include "skinny_gemm_args.h"
 #include "skinny_gemm_plan.h"
+#include "tiled_gemm.h"
 
 namespace hfrk {
 
@@ -999,9 +1000,20 @@ int hfrk_skinny_gemm_fused(const void* A, const void* B, void* D, const void* ba
 
 int hfrk_linear_gemm(const void* A, const void* B, int packed, void* D, const void* base, int base_stride, const float* scale_a,
                      int sa_stride, const float* scale_b, int sb_stride, int m, int n, int k, int b_stride, int d_dtype, void* stream) {
-    if (m > HFRK_GEMM_MAX_M)
+    if (m > HFRK_GEMM_MAX_M && hfrk::tiled_size_ok(m, n, k) && (packed || b_stride <= (1 << 21)))
         return hfrk_tiled_gemm(A, B, packed, D, base, base_stride, scale_a, sa_stride, scale_b, sb_stride, m, n, k, b_stride, d_dtype, nullptr, stream);
     if (base && base_stride != 0 && base_stride != n) return HFRK_BAD_SHAPE;
+    if (m > HFRK_GEMM_MAX_M) {  // beyond the tiled kernel's 32-bit offsets: one skinny GEMM per 64 rows
+        for (int r0 = 0; r0 < m; r0 += HFRK_GEMM_MAX_M) {
+            const int rows = m - r0 < HFRK_GEMM_MAX_M ? m - r0 : HFRK_GEMM_MAX_M;
+            const size_t d0 = (size_t)r0 * n * 2;
+            const int rc = hfrk_linear_gemm(static_cast<const uint8_t*>(A) + (size_t)r0 * k, B, packed, static_cast<uint8_t*>(D) + d0,
+                                            base && base_stride ? static_cast<const uint8_t*>(base) + d0 : base, base_stride,
+                                            scale_a + (size_t)r0 * sa_stride, sa_stride, scale_b, sb_stride, rows, n, k, b_stride, d_dtype, stream);
+            if (rc != HFRK_SUCCESS) return rc;
+        }
+        return HFRK_SUCCESS;
+    }
     return hfrk::gemm_launch(A, B, D, base, scale_a, sa_stride, scale_b, sb_stride, nullptr, m, n, k, b_stride, d_dtype, HFRK_EPILOGUE_NONE,
                              nullptr, static_cast<hipStream_t>(stream), packed != 0, false, nullptr, base && base_stride == 0);
 }

@@ -48,6 +48,7 @@ constexpr TiledShape kTiledShapes[] = {HFRK_TILED_SHAPES(HFRK_TILED_ROW)};
 constexpr int kTiledShapeCount = sizeof(kTiledShapes) / sizeof(kTiledShapes[0]);
 constexpr int tiled_lds_bytes(const TiledShape& s) { return (s.bm + s.bn) * kTiledStage * s.stages; }
 
+bool tiled_size_ok(int m, int n, int k);  // tiled_gemm.hip
 int launch_tiled_rowmajor(const TiledGemmArgs& args, int shape, hipStream_t stream);  // tiled_gemm_rowmajor.hip
 int launch_tiled_packed(const TiledGemmArgs& args, int shape, hipStream_t stream);    // tiled_gemm_packed.hip
 

@@ -7,7 +7,7 @@ namespace hfrk {
 
 static int div_up(long a, long b) { return (int)((a + b - 1) / b); }
 
-static bool tiled_size_ok(int m, int n, int k) {
+bool tiled_size_ok(int m, int n, int k) {
     // every offset the kernel forms inside one tile's buffers stays below 2^31, every tile count and workspace index in 32 bits
     constexpr int kMost = 1 << 21;
     return m >= 1 && n >= 1 && k >= 1 && m <= (1 << 24) && n <= kMost && k <= kMost &&
@@ -51,14 +51,16 @@ static float tiled_cost(int m, int n, int k, int shape, int splits) {
     return t;
 }
 
-static void make_tiled_plan(int m, int n, int k, hfrk_tiled_plan* plan) {
+constexpr int kTiledMaxSplits = 8;
+
+static void make_tiled_plan(int m, int n, int k, int max_splits, hfrk_tiled_plan* plan) {
     float best = INFINITY;
     const int stages = div_up(k, kTiledStage);
     for (int shape = 0; shape < kTiledShapeCount; ++shape) {
         const TiledShape& s = kTiledShapes[shape];
         const int tiles_m = div_up(m, s.bm);
         const long tiles = (long)tiles_m * div_up(n, s.bn);
-        for (int splits = 1; splits <= 8 && splits <= stages; ++splits) {
+        for (int splits = 1; splits <= max_splits && splits <= stages; ++splits) {
             // a split keeps at least two stages, the launch at most two workgroups per compute unit, and the partial tiles fit the
             // stream's workspace (256 x 256 tiles: 256 of them)
             if (splits > 1 && (tiles * splits > 2 * kNumCU || stages < 2 * splits || tiled_ws_bytes(s, m, n, splits) > kWsFloats * sizeof(float))) break;
@@ -82,7 +84,7 @@ extern "C" {
 int hfrk_tiled_gemm_plan(int m, int n, int k, hfrk_tiled_plan* plan) {
     if (!plan || !hfrk::tiled_size_ok(m, n, k)) return HFRK_BAD_SHAPE;
     if (k % 16 != 0) return HFRK_K_NOT_DIVISIBLE_BY_WARPTILE_K;
-    hfrk::make_tiled_plan(m, n, k, plan);
+    hfrk::make_tiled_plan(m, n, k, hfrk::kTiledMaxSplits, plan);
     return HFRK_SUCCESS;
 }
 
@@ -105,10 +107,18 @@ int hfrk_tiled_gemm(const void* A, const void* B, int packed, void* D, const voi
         const int rc = check_tiled_plan(m, n, k, p);
         if (rc != HFRK_SUCCESS) return rc;
     } else {
-        make_tiled_plan(m, n, k, &p);
+        make_tiled_plan(m, n, k, kTiledMaxSplits, &p);
+    }
+    TiledGemmArgs args{};
+    if (p.splits > 1) {
+        size_t bytes = 0;
+        const int rc = stream_workspace(static_cast<hipStream_t>(stream), &args.ws, &bytes, &args.counters);
+        if (rc == HFRK_SUCCESS) args.ws_bytes = (uint32_t)bytes;
+        // no workspace left, or none before a capture began: a call that names no plan runs without splitting k
+        else if (!plan && (rc == HFRK_NO_WORKSPACE || rc == HFRK_NOT_INITIALISED)) make_tiled_plan(m, n, k, 1, &p);
+        else return rc;
     }
     const TiledShape& s = kTiledShapes[p.shape];
-    TiledGemmArgs args{};
     args.A = static_cast<const uint8_t*>(A);
     args.B = static_cast<const uint8_t*>(B);
     args.D = D;
@@ -131,12 +141,6 @@ int hfrk_tiled_gemm(const void* A, const void* B, int packed, void* D, const voi
     args.splits = p.splits;
     args.stages_q = stages / p.splits;
     args.stages_r = stages % p.splits;
-    if (p.splits > 1) {
-        size_t bytes = 0;
-        const int rc = stream_workspace(static_cast<hipStream_t>(stream), &args.ws, &bytes, &args.counters);
-        if (rc != HFRK_SUCCESS) return rc;
-        args.ws_bytes = (uint32_t)bytes;
-    }
     return packed ? launch_tiled_packed(args, p.shape, static_cast<hipStream_t>(stream))
                   : launch_tiled_rowmajor(args, p.shape, static_cast<hipStream_t>(stream));
 }

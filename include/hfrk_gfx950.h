@@ -269,7 +269,8 @@ int hfrk_skinny_gemm_packed(const void* A, const void* B_packed, void* D, const 
                             int k, int d_dtype, int epilogue, const hfrk_gemm_plan* plan, void* stream);
 
 /* The linear layer's GEMM for any number of rows, under the library's own plan: a skinny GEMM up to 64 rows, hfrk_tiled_gemm (below,
- * same arguments) above.  base_stride is 0 (one row of n values added to every row of D: a bias) or, up to 64 rows, n. */
+ * same arguments) above, or one skinny GEMM per 64 rows where a size is beyond the tiled kernel's.  base_stride is 0 (one row of n
+ * values added to every row of D: a bias) or, where a skinny GEMM runs, n. */
 int hfrk_linear_gemm(const void* A, const void* B, int packed, void* D, const void* base, int base_stride, const float* scale_a,
                      int sa_stride, const float* scale_b, int sb_stride, int m, int n, int k, int b_stride, int d_dtype, void* stream);
 
@@ -293,7 +294,8 @@ int hfrk_tiled_gemm_plan(int m, int n, int k, hfrk_tiled_plan* plan);
  *   base  16-bit addend of D's type or NULL; base_stride elements between its rows, 0: one row for all (a bias)
  * fp32 accumulation, one rounding, bit-reproducible.  k % 16 == 0 (256 for a packed weight); n, k and the strides at most 2^21.
  * A and B 16-byte aligned, b_stride a multiple of 16; D and base may have any alignment, 16 bytes with n % 8 == 0 is the fast one.
- * A plan whose k is split needs the stream's workspace like the skinny GEMMs (see hfrk_init). */
+ * A plan whose k is split needs the stream's workspace like the skinny GEMMs (see hfrk_init); without a plan and without a
+ * workspace k is not split. */
 int hfrk_tiled_gemm(const void* A, const void* B, int packed, void* D, const void* base, int base_stride, const float* scale_a,
                     int sa_stride, const float* scale_b, int sb_stride, int m, int n, int k, int b_stride, int d_dtype,
                     const hfrk_tiled_plan* plan, void* stream);

@@ -2,6 +2,9 @@
 kernels: one output ulp plus 2^-16 of the sum of absolute products.  Every tile shape in both weight layouts, at sizes around
 the edges of tiles, stages and splits."""
 import ctypes
+import os
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -88,3 +91,53 @@ def test_argument_errors_and_plans():
     assert call(a=p + 8) == _capi.BAD_ALIGNMENT
     for bad in ((5, 1, 1), (-1, 1, 1), (0, 2, 1), (0, 1, 2), (4, 0, 1)):
         assert call(plan=ctypes.byref(_capi.TiledPlan(*bad))) == _capi.INVALID_CONFIG, bad
+
+
+def test_weights_beyond_the_tiled_kernels_sizes_run_in_pieces():
+    from hf_rocm_kernels.layers import apply_fp8_linear
+    m, n, k = 66, (1 << 21) + 16, 256
+    g = torch.Generator(device="cuda").manual_seed(1)
+    a = torch.randint(0, 0x70, (m, k), dtype=torch.uint8, device="cuda", generator=g).view(torch.float8_e4m3fn)
+    w = torch.randint(0, 0x70, (n, k), dtype=torch.uint8, device="cuda", generator=g).view(torch.float8_e4m3fn)
+    sa, sw = torch.rand(m, device="cuda", generator=g) * 1e-4, torch.full((1,), 1e-2, device="cuda")
+    bias = torch.randn(n, device="cuda", generator=g).to(torch.bfloat16)
+    whole = apply_fp8_linear(a, w, sw, sa, bias=bias)
+    for r0, r1 in ((0, 64), (64, m)):
+        assert torch.equal(whole[r0:r1], apply_fp8_linear(a[r0:r1], w, sw, sa[r0:r1], bias=bias))
+
+
+# A process of its own: it takes every workspace there is.
+_NO_WORKSPACE = """
+import ctypes, torch
+from hf_rocm_kernels import _capi
+lib = _capi.load()
+torch.zeros(1, device="cuda")
+hip = ctypes.CDLL(next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line))
+m, n, k = 65, 64, 4096
+a, w = (torch.randn(r, k, device="cuda").to(torch.float8_e4m3fn) for r in (m, n))
+one = torch.ones(1, device="cuda")
+
+def call(stream, splits):
+    out = torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
+    plan = ctypes.byref(_capi.TiledPlan(4, splits, 1)) if splits else None
+    status = lib.hfrk_tiled_gemm(a.data_ptr(), w.data_ptr(), 0, out.data_ptr(), None, 0, one.data_ptr(), 0, None, 0, m, n, k, k, _capi.BF16, plan, stream)
+    torch.cuda.synchronize()
+    return status, out
+
+chosen = _capi.TiledPlan()
+assert lib.hfrk_tiled_gemm_plan(m, n, k, ctypes.byref(chosen)) == _capi.SUCCESS and chosen.splits > 1
+for i in range(64):
+    stream = ctypes.c_void_p()
+    assert hip.hipStreamCreate(ctypes.byref(stream)) == 0
+    assert call(stream, 2)[0] == _capi.SUCCESS, i
+assert hip.hipStreamCreate(ctypes.byref(stream)) == 0
+assert call(stream, 2)[0] == _capi.NO_WORKSPACE
+status, out = call(stream, 0)
+want = call(stream, 1)
+assert status == want[0] == _capi.SUCCESS and torch.equal(out, want[1])
+"""
+
+
+def test_a_stream_without_a_workspace_does_not_split_k():
+    env = dict(os.environ, PYTHONPATH=os.pathsep.join(p for p in sys.path if p))
+    subprocess.run([sys.executable, "-c", _NO_WORKSPACE], check=True, timeout=100, env=env)
