@@ -1000,7 +1000,10 @@ int hfrk_skinny_gemm_fused(const void* A, const void* B, void* D, const void* ba
 
 int hfrk_linear_gemm(const void* A, const void* B, int packed, void* D, const void* base, int base_stride, const float* scale_a,
                      int sa_stride, const float* scale_b, int sb_stride, int m, int n, int k, int b_stride, int d_dtype, void* stream) {
-    if (m > HFRK_GEMM_MAX_M && hfrk::tiled_size_ok(m, n, k) && (packed || b_stride <= (1 << 21)))
+    // A k that ends inside a 256-byte chunk is handled by the skinny kernels for up to 32 rows; 33..64 rows were two launches over the
+    // same weight.  Measured, skinny / tiled: 4104 x 1936 at 33 rows 13.7 / 9.4 us, at 64 rows 15.9 / 10.3.  With whole chunks the
+    // skinny kernels stay, as on few columns of a very long k (1024 x 28656 at 33 rows 24.3 / 26.6; 2056 x 16400 28.2 / 19.0): one launch, and 4096 x 4096 at 64 rows 8.5 / 10.7, 28672 x 4096 25.0 / 31.8.
+    if ((m > HFRK_GEMM_MAX_M || (m > hfrk::kStreamMaxM && k % 256 != 0 && k <= 16L * n)) && hfrk::tiled_size_ok(m, n, k) && (packed || b_stride <= (1 << 21)))
         return hfrk_tiled_gemm(A, B, packed, D, base, base_stride, scale_a, sa_stride, scale_b, sb_stride, m, n, k, b_stride, d_dtype, nullptr, stream);
     if (base && base_stride != 0 && base_stride != n) return HFRK_BAD_SHAPE;
     if (m > HFRK_GEMM_MAX_M) {  // beyond the tiled kernel's 32-bit offsets: one skinny GEMM per 64 rows

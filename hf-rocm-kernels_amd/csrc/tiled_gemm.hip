@@ -56,6 +56,17 @@ constexpr int kTiledMaxSplits = 8;
 static void make_tiled_plan(int m, int n, int k, int max_splits, hfrk_tiled_plan* plan) {
     float best = INFINITY;
     const int stages = div_up(k, kTiledStage);
+    if (m <= 64) {
+        // One row of tiles streams the weight: the deepest pipeline (64 x 64), k split up to one workgroup per compute unit but
+        // at most 4 ways and not below 8 stages.  The fit below starts at 65 rows and splits too little here: 4096 x 14336 at 64 rows
+        // 24.4 -> 18.1 us, 8192 x 28672 at 33 rows 67 -> 45, 4104 x 1936 at 64 rows 11.8 -> 10.3.
+        int splits = kNumCU / div_up(n, 64);
+        splits = splits < stages / 8 ? splits : stages / 8;
+        splits = splits < 4 ? splits : 4;
+        splits = splits < max_splits ? splits : max_splits;
+        *plan = {4, splits < 1 ? 1 : splits, 1};
+        return;
+    }
     for (int shape = 0; shape < kTiledShapeCount; ++shape) {
         const TiledShape& s = kTiledShapes[shape];
         const int tiles_m = div_up(m, s.bm);

@@ -452,11 +452,8 @@ void tiled_gemm(at::Tensor& A, at::Tensor& B, bool packed, int64_t n, at::Tensor
     DeviceScope scope(A);
     const int sa_stride = scale_a.numel() == 1 ? 0 : 1, b_stride = packed ? (int)k : (int)B.stride(1);
     const float* const sa = scale_a.data_ptr<float>();
-    raise_on(m > HFRK_GEMM_MAX_M
-                 ? hfrk_linear_gemm(A.data_ptr(), B.data_ptr(), packed ? 1 : 0, D.data_ptr(), base_ptr, base_stride, sa, sa_stride, scale_b_ptr,
-                                    sb_stride, (int)m, (int)n, (int)k, b_stride, d_dtype, current_stream(A))
-                 : hfrk_tiled_gemm(A.data_ptr(), B.data_ptr(), packed ? 1 : 0, D.data_ptr(), base_ptr, base_stride, sa, sa_stride, scale_b_ptr,
-                                   sb_stride, (int)m, (int)n, (int)k, b_stride, d_dtype, nullptr, current_stream(A)),
+    raise_on(hfrk_linear_gemm(A.data_ptr(), B.data_ptr(), packed ? 1 : 0, D.data_ptr(), base_ptr, base_stride, sa, sa_stride, scale_b_ptr,
+                              sb_stride, (int)m, (int)n, (int)k, b_stride, d_dtype, current_stream(A)),
              "tiled_gemm");
 }
 

@@ -6,7 +6,8 @@ usual (input, weight, weight_scale, input_scale, bias) signature, and an nn.Modu
 
 A call runs as one quantisation kernel (skipped when the caller already holds fp8 activations and their scales, e.g. from
 `residual_rms_dynamic` / `swiglu_dynamic`) and one GEMM with the scales, the bias or residual folded into its epilogue: a
-skinny GEMM for decode batches (up to 64 tokens), the tiled GEMM for everything larger, up to whole prompts.
+skinny GEMM for decode batches (up to 64 tokens; 32 where k ends inside a 256-byte chunk), the tiled GEMM for everything larger,
+up to whole prompts.
 """
 from typing import Optional, Sequence, Tuple, Union
 
@@ -75,7 +76,7 @@ def apply_fp8_linear(
     else:
         sb = weight_scale.reshape(-1)
     m = q.size(0)
-    tiled = m > _capi.GEMM_MAX_M
+    tiled = m > _capi.GEMM_MAX_M or (m > 32 and k % 256 != 0 and k <= 16 * n)  # as hfrk_linear_gemm has it
     base = None
     if residual is not None:
         base = residual.reshape(m, n)

@@ -268,8 +268,8 @@ int hfrk_skinny_gemm_packed(const void* A, const void* B_packed, void* D, const 
                             int sa_stride, const float* scale_b, int sb_stride, const float* out_scale, int m, int n,
                             int k, int d_dtype, int epilogue, const hfrk_gemm_plan* plan, void* stream);
 
-/* The linear layer's GEMM for any number of rows, under the library's own plan: a skinny GEMM up to 64 rows, hfrk_tiled_gemm (below,
- * same arguments) above, or one skinny GEMM per 64 rows where a size is beyond the tiled kernel's.  base_stride is 0 (one row of n
+/* The linear layer's GEMM for any number of rows, under the library's own plan: a skinny GEMM up to 64 rows (32 where k % 256 != 0),
+ * hfrk_tiled_gemm (below, same arguments) above, or one skinny GEMM per 64 rows where a size is beyond the tiled kernel's.  base_stride is 0 (one row of n
  * values added to every row of D: a bias) or, where a skinny GEMM runs, n. */
 int hfrk_linear_gemm(const void* A, const void* B, int packed, void* D, const void* base, int base_stride, const float* scale_a,
                      int sa_stride, const float* scale_b, int sb_stride, int m, int n, int k, int b_stride, int d_dtype, void* stream);

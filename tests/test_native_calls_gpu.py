@@ -10,6 +10,7 @@ from hf_rocm_kernels.layers import Fp8Linear, apply_fp8_linear, fp8_linear
 from hf_rocm_kernels.operators.skinny_gemm import wrapped
 from hf_rocm_kernels.utils.fp8 import amax_scale, fp8_quantize
 from hf_rocm_kernels.utils.weight_format import pack_weight
+from test_gemm_gpu import oracle_checker
 
 pytestmark = pytest.mark.gpu
 
@@ -49,6 +50,24 @@ def test_linear_same_bits_as_the_general_path(rows, n, k, monkeypatch):
             want = [apply_fp8_linear(weight=weight, weight_scale=scale, **c) for c in calls]
         for g, w_ in zip(got, want):
             assert g.shape == w_.shape and g.dtype == w_.dtype and torch.equal(_bits(g), _bits(w_))
+
+
+@pytest.mark.parametrize("m", [32, 33, 48, 64])
+@pytest.mark.parametrize("n,k", [(64, 272), (515, 1040), (4104, 1936), (1000, 4112)])
+def test_rows_33_to_64_with_a_cut_last_chunk_match_the_oracle(m, n, k, monkeypatch):
+    g = torch.Generator().manual_seed(m + n)
+    a, w = torch.randn(m, k, generator=g), torch.randn(n, k, generator=g) * 0.02
+    sa, sw = amax_scale(a, dim=1), amax_scale(w, dim=1)
+    a, w, sa, sw = fp8_quantize(a, sa)[0], fp8_quantize(w, sw)[0], sa.reshape(-1), sw.reshape(-1)
+    bias = torch.randn(n, generator=g).to(torch.bfloat16)
+    for b in (None, bias):
+        check = oracle_checker(a, w.t(), sa, sw, torch.bfloat16, base=None if b is None else b.expand(m, n).contiguous())
+        args = a.cuda(), w.cuda(), sw.cuda(), sa.cuda(), None if b is None else b.cuda()
+        native = apply_fp8_linear(*args)
+        check(native)
+        with monkeypatch.context() as patch:
+            _general(patch)
+            assert torch.equal(native, apply_fp8_linear(*args))
 
 
 @pytest.mark.parametrize("m,n,k", [(1, 4096, 4096), (7, 514, 512), (33, 1024, 2304), (64, 130, 256), (3, 512, 384)])
