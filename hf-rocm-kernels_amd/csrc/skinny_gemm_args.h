@@ -62,6 +62,12 @@ struct GemmArgs {
     int* counters;           // arrival counters, zero between launches
 };
 
+// Loads requested so far stay in front of what follows.  The compiler sinks a load behind whatever writes no memory, and how far depends on
+// the size of what it is sunk past: when the SwiGLU epilogue became shorter, the row-split kernel's next chunk was requested 130
+// instructions and nine branches later than written, and the activation scales 250 (28672 x 4096 with SwiGLU at 1 row, float16 / bfloat16:
+// 19.6 / 20.0 us with the long epilogue, 20.1 / 20.25 with the short one, 19.6 / 19.8 with the requests held in place).
+__device__ __forceinline__ void requests_end() { asm volatile("" ::: "memory"); }
+
 // The split-K workspace of `stream` on the current device: fp32 partial sums (kWsFloats) and kMaxPanels arrival counters, zero
 // between launches (skinny_gemm.hip).
 int stream_workspace(hipStream_t stream, float** ws, size_t* ws_bytes, int** counters);

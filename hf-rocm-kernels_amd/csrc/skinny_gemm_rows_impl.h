@@ -176,6 +176,7 @@ __global__ void __launch_bounds__(kGemmThreads) skinny_gemm_rows_kernel(const Ge
     // everything the end of the kernel needs to turn a sum into output: buffer resources, scales, dtype (skinny_gemm_rows_epilogue.h)
     const RowsEpilogue<MT, RT, SWIGLU> epi(a, lane);
     using Pre = typename RowsEpilogue<MT, RT, SWIGLU>::Pre;
+    requests_end();
 
     uint8_t* const tw = lds + wv * kWaveLds;  // this wave's RT weight tiles, then its activation tile(s)
     uint8_t* const ta = tw + RT * kTileBytes;
@@ -323,6 +324,7 @@ __global__ void __launch_bounds__(kGemmThreads) skinny_gemm_rows_kernel(const Ge
         pre_cur = pre_next;
         if (i + 1 < count) {  // registers are free again: request the next chunk before the LDS reads and MFMAs
             issue_chunk();
+            requests_end();
             // the chunk that ends a tile this wave finishes in the loop brings the tile's D along
             pre_next = prefetch(irow0, iunits, ikc == KC - 1 && !(itile == tile_h && kb0 != 0));
             if (i + 2 == count && finisher && late_pre) pre_l = prefetch(row0_l, units_l, true);
@@ -411,6 +413,7 @@ __global__ void __launch_bounds__(kGemmThreads) skinny_gemm_rows_kernel(const Ge
         for (int j = 1; j < kGemmWaves; ++j)
 #pragma unroll
             for (int u = 0; u < RT; ++u) other[j][u] = slots[j * kSlotStride + (mt * RT + u) * 64 + lane];
+        requests_end();
 #pragma unroll
         for (int j = 1; j < kGemmWaves; ++j) {
             const float f = (addmask >> j) & 1u ? 1.0f : 0.0f;
