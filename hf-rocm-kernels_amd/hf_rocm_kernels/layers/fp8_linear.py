@@ -84,7 +84,10 @@ def apply_fp8_linear(
             base = base + bias
         base = base.contiguous()
     elif bias is not None:
-        base = bias.to(out_dtype).contiguous() if tiled else bias.to(out_dtype).expand(m, n).contiguous()
+        base = bias.to(out_dtype)
+        if not tiled or base.shape != (n,):  # the tiled kernel reads a row of n values as it is; other forms are spread over the rows
+            base = base.expand(m, n)
+        base = base.contiguous()
     out = torch.empty((m, n), dtype=out_dtype, device=q.device)
     if tiled:
         skinny_gemm_checks(q, w, sa[:1], out)

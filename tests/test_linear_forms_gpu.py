@@ -1,0 +1,38 @@
+"""`apply_fp8_linear` takes the same forms of its arguments, and refuses the same ones, at every row count: one skinny GEMM (5, 40),
+two of them or one tiled GEMM (40 with k = 528), one tiled GEMM (65, 130)."""
+import pytest
+import torch
+
+import hf_rocm_kernels
+from hf_rocm_kernels.layers import apply_fp8_linear
+from hf_rocm_kernels.utils.fp8 import amax_scale, fp8_quantize
+
+pytestmark = pytest.mark.gpu
+N = 264
+SIZES = [(5, 512), (40, 512), (40, 528), (65, 512), (130, 528)]
+
+
+def _operands(m, k):
+    torch.manual_seed(m + k)
+    w = torch.randn(N, k, device="cuda") * 0.02
+    sw = amax_scale(w, dim=1)
+    return torch.randn(m, k, device="cuda").to(torch.bfloat16), fp8_quantize(w, sw)[0], sw.reshape(-1).contiguous()
+
+
+@pytest.mark.parametrize("m,k", SIZES)
+@pytest.mark.parametrize("shape", [(N,), (1, N), (1,), (), "rows", "column"])
+def test_a_bias_of_any_shape_that_broadcasts(m, k, shape):
+    x, w, sw = _operands(m, k)
+    shape = {"rows": (m, N), "column": (m, 1)}.get(shape, shape)
+    bias = torch.randn(shape, device="cuda").to(torch.bfloat16)
+    want = apply_fp8_linear(x, w, sw, residual=bias.expand(m, N).contiguous())  # one addend per value, added and rounded the same way
+    assert torch.equal(apply_fp8_linear(x, w, sw, bias=bias), want)
+    assert torch.equal(apply_fp8_linear(x, w, sw, bias=bias.float()), want)
+
+
+@pytest.mark.parametrize("m,k", SIZES)
+def test_a_bias_that_does_not_broadcast_is_refused(m, k):
+    x, w, sw = _operands(m, k)
+    for shape in ((N - 1,), (N, 1), (m + 1, N)):
+        with pytest.raises(RuntimeError):
+            apply_fp8_linear(x, w, sw, bias=torch.zeros(shape, device="cuda", dtype=torch.bfloat16))
