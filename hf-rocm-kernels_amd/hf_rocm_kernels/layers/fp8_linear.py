@@ -76,6 +76,8 @@ def apply_fp8_linear(
     else:
         sb = weight_scale.reshape(-1)
     m = q.size(0)
+    if sa.numel() != 1:
+        sa = sa[:m]  # a buffer of scales may be longer than the batch
     tiled = m > _capi.GEMM_MAX_M or (m > 32 and k % 256 != 0 and k <= 16 * n)  # as hfrk_linear_gemm has it
     base = None
     if residual is not None:

@@ -36,3 +36,12 @@ def test_a_bias_that_does_not_broadcast_is_refused(m, k):
     for shape in ((N - 1,), (N, 1), (m + 1, N)):
         with pytest.raises(RuntimeError):
             apply_fp8_linear(x, w, sw, bias=torch.zeros(shape, device="cuda", dtype=torch.bfloat16))
+
+
+@pytest.mark.parametrize("m,k", SIZES)
+def test_scales_of_a_longer_batch(m, k):
+    """A buffer of scales for more rows than the call has (a batch that shrank): the first m belong to it."""
+    x, w, sw = _operands(m, k)
+    q, sx = hf_rocm_kernels.quantize_fp8(x)
+    longer = torch.cat([sx, torch.full((3,), float("nan"), device="cuda")])
+    assert torch.equal(apply_fp8_linear(q, w, sw, longer), apply_fp8_linear(q, w, sw, sx))
