@@ -17,7 +17,7 @@ from torch import Tensor
 from .. import _capi
 from ..operators.quantize import quantize_fp8
 from ..operators.skinny_gemm import skinny_gemm_add, skinny_gemm_scaled
-from ..operators.skinny_gemm.wrapped import skinny_gemm_checks
+from ..operators.skinny_gemm.wrapped import scale_vectors, skinny_gemm_checks
 from ..utils.dispatch import runs_now
 from ..utils.fp8 import amax_scale, fp8_quantize
 from ..utils.weight_format import PackedWeight, pack_weight
@@ -93,8 +93,10 @@ def apply_fp8_linear(
     out = torch.empty((m, n), dtype=out_dtype, device=q.device)
     if tiled:
         skinny_gemm_checks(q, w, sa[:1], out)
+        assert base is None or base.dtype == out_dtype, f"Expected {base.dtype = } to be {out_dtype = }"
+        sa, sb = scale_vectors(q, w, sa, sb)
         packed = isinstance(w, PackedWeight)
-        torch.ops._HFRK_C.tiled_gemm(q, w.data if packed else w, packed, n, out, base, sa.contiguous(), sb.contiguous())
+        torch.ops._HFRK_C.tiled_gemm(q, w.data if packed else w, packed, n, out, base, sa, sb)
     elif m == 0:
         pass
     elif base is None:

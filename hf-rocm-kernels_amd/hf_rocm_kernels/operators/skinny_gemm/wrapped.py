@@ -187,7 +187,7 @@ class _ShapeOnly:
         return (self.shape[1], 1)
 
 
-def _scale_vectors(skinny_a: Tensor, b: Tensor, scale_a: Tensor, scale_b: Optional[Tensor]) -> Tuple[Tensor, Optional[Tensor]]:
+def scale_vectors(skinny_a: Tensor, b: Tensor, scale_a: Tensor, scale_b: Optional[Tensor]) -> Tuple[Tensor, Optional[Tensor]]:
     m, n = skinny_a.size(0), b.size(1)
     assert scale_a.numel() in (1, m) and scale_a.dtype == torch.float32, f"Expected 1 or {m} float32 in scale_a"
     if scale_b is None:  # one combined scale in scale_a: the weight's side of it is 1, whatever the weight's layout
@@ -214,7 +214,7 @@ def skinny_gemm_add(
     skinny_gemm_checks(skinny_a, b, scale_a.reshape(-1)[:1], output)
     assert base.shape == output.shape and base.dtype == output.dtype and base.is_contiguous(), (
         f"Expected base to be contiguous with {output.shape = } and {output.dtype = }")
-    sa, sb = _scale_vectors(skinny_a, b, scale_a, scale_b)
+    sa, sb = scale_vectors(skinny_a, b, scale_a, scale_b)
     _fused(skinny_a, b, output, base, sa, sb, None, _capi.EPILOGUE_NONE, 0)
     return output
 
@@ -266,7 +266,7 @@ def skinny_gemm_swiglu(
         f"Expected a contiguous float8_e4m3fn output of shape {(m, n // 2)}")
     skinny_gemm_checks(skinny_a, gate_up_weight, scale_a.reshape(-1)[:1],
                        _ShapeOnly(m, n, intermediate_dtype, skinny_a.device))
-    sa, sb = _scale_vectors(skinny_a, gate_up_weight, scale_a, scale_b)
+    sa, sb = scale_vectors(skinny_a, gate_up_weight, scale_a, scale_b)
     dtype_tag = _capi.BF16 if intermediate_dtype == torch.bfloat16 else _capi.F16
     if maybe:
         status = _skinny_gemm_fused(skinny_a, gate_up_weight, output, None, sa, sb, out_scale, _capi.EPILOGUE_SWIGLU, dtype_tag)

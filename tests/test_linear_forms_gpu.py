@@ -45,3 +45,13 @@ def test_scales_of_a_longer_batch(m, k):
     q, sx = hf_rocm_kernels.quantize_fp8(x)
     longer = torch.cat([sx, torch.full((3,), float("nan"), device="cuda")])
     assert torch.equal(apply_fp8_linear(q, w, sw, longer), apply_fp8_linear(q, w, sw, sx))
+
+
+@pytest.mark.parametrize("m,k", SIZES)
+def test_operands_that_do_not_fit_are_refused_alike(m, k):
+    x, w, sw = _operands(m, k)
+    q, sx = hf_rocm_kernels.quantize_fp8(x)
+    for bad in (dict(weight_scale=sw[:-1]), dict(weight_scale=sw.double()), dict(input_scale=sx[:3]), dict(input_scale=sx.double()),
+                dict(residual=torch.zeros(m, N, device="cuda", dtype=torch.float16)), dict(out_dtype=torch.float32), dict(weight=w[:, :256])):
+        with pytest.raises(AssertionError):
+            apply_fp8_linear(**{**dict(input=q, weight=w, weight_scale=sw, input_scale=sx), **bad})
