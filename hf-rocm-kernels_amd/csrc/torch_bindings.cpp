@@ -4,6 +4,7 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/library.h>
@@ -734,8 +735,17 @@ TORCH_LIBRARY(_HFRK_C, ops) {
     ops.impl("quantize_fp8", c10::kCUDA, &quantize_fp8);
 }
 
+// nothing_intercepts() -> bool: whether an operator called now, on plain tensors, runs its kernel and is seen by nobody else.  Whatever
+// records, batches or replaces calls (torch.jit.trace, functorch's transforms, dispatch modes and fake tensors, pre-dispatch tracing,
+// functionalisation) does so by a dispatch key that it includes for the thread.
+static PyObject* nothing_intercepts(PyObject*, PyObject*) {
+    const bool none = (c10::impl::tls_local_dispatch_key_set().included_ - c10::default_included_set).empty();
+    return PyBool_FromLong(none);
+}
+
 // `import hf_rocm_kernels._HFRK_C` loads this library and thereby runs the registration above.
 PyMODINIT_FUNC PyInit__HFRK_C(void) {
-    static struct PyModuleDef module = {PyModuleDef_HEAD_INIT, "_HFRK_C", nullptr, 0, nullptr};
+    static PyMethodDef methods[] = {{"nothing_intercepts", nothing_intercepts, METH_NOARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
+    static struct PyModuleDef module = {PyModuleDef_HEAD_INIT, "_HFRK_C", nullptr, 0, methods};
     return PyModule_Create(&module);
 }

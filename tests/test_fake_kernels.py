@@ -122,3 +122,53 @@ def test_a_traced_call_records_operators_that_check_their_arguments():
             apply_fp8_linear(x, _fp8(256, 768), sw)
         with pytest.raises(AssertionError):
             hf_rocm_kernels.skinny_gemm(_fp8(8, 512), _fp8(256, 768).t(), torch.empty(1, device="cuda"))
+
+
+def _interceptors():
+    """Ways a call is recorded, batched or replaced: each runs its argument with a tensor."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Passing(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    def inside(mode, f):
+        with mode:
+            return f(torch.ones(2, 2))
+
+    ones = torch.ones(2, 2)
+    return {
+        "jit.trace": lambda f: torch.jit.trace(f, ones, check_trace=False),
+        "make_fx": lambda f: make_fx(f)(ones),
+        "make_fx before dispatch": lambda f: make_fx(f, pre_dispatch=True)(ones),
+        "vmap": lambda f: torch.vmap(f)(ones),
+        "jvp": lambda f: torch.func.jvp(f, (ones,), (ones,)),
+        "grad": lambda f: torch.func.grad(lambda x: f(x).sum())(ones),
+        "functionalize": lambda f: torch.func.functionalize(f)(ones),
+        "fake": lambda f: inside(FakeTensorMode(), f),
+        "dispatch mode": lambda f: inside(Passing(), f),
+    }
+
+
+@pytest.mark.parametrize("way", sorted(_interceptors()))
+def test_whole_call_operators_stay_out_of_calls_that_something_intercepts(way):
+    from hf_rocm_kernels._HFRK_C import nothing_intercepts
+    seen = []
+
+    def call(x):
+        seen.append(nothing_intercepts())
+        return x * 2
+
+    assert nothing_intercepts()
+    _interceptors()[way](call)
+    assert seen and not any(seen)
+    assert nothing_intercepts()
+
+
+def test_settings_that_change_no_call_are_no_interception():
+    from hf_rocm_kernels._HFRK_C import nothing_intercepts
+    for setting in (torch.no_grad(), torch.inference_mode(), torch.autocast("cpu", dtype=torch.bfloat16), torch.device("cpu"),
+                    torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t)):
+        with setting:
+            assert nothing_intercepts()

@@ -105,3 +105,20 @@ def test_linear_outputs_carry_no_autograd_history_and_keep_leading_dimensions():
     y = layer(x)
     assert y.shape == (2, 3, 256) and not y.requires_grad
     assert layer(x[:0]).shape == (0, 3, 256)
+
+
+@pytest.mark.parametrize("rows", [4, 80])
+def test_recorded_and_batched_calls_go_the_general_way(rows):
+    """A trace that held a whole-call operator would replay it on inputs it does not take, and get nothing back."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    layer = Fp8Linear.from_float(torch.nn.Linear(512, 256, device="cuda", dtype=torch.float16))
+    x = torch.randn(rows, 512, device="cuda", dtype=torch.float16)
+    for pre_dispatch in (False, True):
+        graph = make_fx(lambda a: layer(a), pre_dispatch=pre_dispatch)(x)
+        names = [str(node.target) for node in graph.graph.nodes]
+        assert any("quantize_fp8" in name for name in names) and not any("fp8_linear" in name for name in names)
+        assert torch.equal(graph(x), layer(x))
+    with pytest.raises(RuntimeError):
+        torch.jit.trace(layer, x, check_trace=False)
+    with pytest.raises(RuntimeError):
+        torch.vmap(layer)(x.view(2, rows // 2, 512))
