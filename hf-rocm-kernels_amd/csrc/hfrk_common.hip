@@ -5,7 +5,11 @@ namespace hfrk {
 
 static thread_local int g_last_hip_error = 0;
 
-void set_last_hip_error(hipError_t e) { g_last_hip_error = static_cast<int>(e); }
+// The runtime keeps a failed call's error too, and the check behind the next launch would take it for that launch's.
+void set_last_hip_error(hipError_t e) {
+    g_last_hip_error = static_cast<int>(e);
+    (void)hipGetLastError();
+}
 
 }  // namespace hfrk
 

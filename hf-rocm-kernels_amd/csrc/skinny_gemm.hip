@@ -532,7 +532,10 @@ static int workspace_for(int dev, hipStream_t stream, Workspace* out) {
         if ((int)d.pool.size() >= kMaxWorkspaces) return HFRK_NO_WORKSPACE;
         do {  // the first launch on a device does what hfrk_init does
             const int rc = grow_pool(d);
-            if (rc != HFRK_SUCCESS) return rc;
+            if (rc != HFRK_SUCCESS) {
+                if (d.unassigned.empty()) return rc;
+                break;  // memory for this stream's, not for those behind it
+            }
         } while ((int)d.pool.size() < kInitialWorkspaces);
     }
     const int idx = d.unassigned.back();

@@ -125,8 +125,10 @@ int hfrk_tiled_gemm(const void* A, const void* B, int packed, void* D, const voi
         size_t bytes = 0;
         const int rc = stream_workspace(static_cast<hipStream_t>(stream), &args.ws, &bytes, &args.counters);
         if (rc == HFRK_SUCCESS) args.ws_bytes = (uint32_t)bytes;
-        // no workspace left, or none before a capture began: a call that names no plan runs without splitting k
-        else if (!plan && (rc == HFRK_NO_WORKSPACE || rc == HFRK_NOT_INITIALISED)) make_tiled_plan(m, n, k, 1, &p);
+        // no workspace left, no memory for one (a caching allocator may hold it all), or none before a capture began: a call that names
+        // no plan runs without splitting k
+        else if (!plan && (rc == HFRK_NO_WORKSPACE || rc == HFRK_NOT_INITIALISED ||
+                           (rc == HFRK_HIP_ERROR && hfrk_last_hip_error() == (int)hipErrorOutOfMemory))) make_tiled_plan(m, n, k, 1, &p);
         else return rc;
     }
     const TiledShape& s = kTiledShapes[p.shape];

@@ -1,0 +1,107 @@
+"""What a launch does when the split-K workspace is not to be had, on the CPU: the library runs over a stand-in for the HIP runtime that
+hands out a given number of allocations, can claim that a stream is capturing, keeps the last error as the runtime does, and notes the
+grid of every launch instead of running it."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+_STAND_IN = r"""
+#include <stddef.h>
+#include <stdint.h>
+typedef struct { uint32_t x, y, z; } dim3_;
+static int allocations, capturing, last_error;
+static uint32_t grid;
+static uintptr_t next_block = 1 << 20;
+void stand_in(int allocs, int capture) { allocations = allocs; capturing = capture; grid = 0; }
+uint32_t stand_in_grid(void) { return grid; }
+static int fail(int e) { return last_error = e; }
+int hipGetDevice(int* d) { *d = 0; return 0; }
+int hipMalloc(void** p, size_t n) { if (allocations-- <= 0) return fail(2); *p = (void*)next_block; next_block += (n + 4095) & ~(size_t)4095; return 0; }
+int hipFree(void* p) { return 0; }
+int hipMemset(void* p, int v, size_t n) { return 0; }
+int hipStreamIsCapturing(void* s, int* state) { *state = capturing; return 0; }
+int hipFuncSetAttribute(const void* f, int a, int v) { return 0; }
+int hipGetLastError(void) { int e = last_error; last_error = 0; return e; }
+static dim3_ g, b; static size_t l; static void* s;
+int __hipPushCallConfiguration(dim3_ grid_, dim3_ block_, size_t lds, void* stream) { g = grid_; b = block_; l = lds; s = stream; return 0; }
+int __hipPopCallConfiguration(dim3_* grid_, dim3_* block_, size_t* lds, void** stream) { *grid_ = g; *block_ = b; *lds = l; *stream = s; return 0; }
+int hipLaunchKernel(const void* f, dim3_ grid_, dim3_ block_, void** args, size_t lds, void* stream) { grid = grid_.x; return 0; }
+"""
+
+# m = 65: one row of 64 x 64 tiles more than the skinny kernels take, k long enough to be split
+_PRELUDE = """
+import ctypes, sys
+sys.path.insert(0, {package!r})
+import _capi
+lib, stand_in = _capi.load(), ctypes.CDLL({stand_in!r})
+m, n, k = 65, 64, 4096
+
+def tiled(stream, plan=None):
+    plan = plan and ctypes.byref(_capi.TiledPlan(*plan))
+    return lib.hfrk_tiled_gemm(4096, 8192, 0, 16384, None, 0, 64, 0, None, 0, m, n, k, k, _capi.BF16, plan, stream)
+
+def skinny(stream, plan=None):  # (64 rows of a narrow weight: k is split between workgroups)
+    return lib.hfrk_skinny_gemm_fused(4096, 8192, 16384, None, 64, 0, None, 0, None, 64, 64, 16384, 16384, _capi.BF16, 0, plan, stream)
+
+chosen = _capi.TiledPlan()
+assert lib.hfrk_tiled_gemm_plan(m, n, k, ctypes.byref(chosen)) == _capi.SUCCESS and chosen.splits > 1
+rows, columns = [(256, 256), (256, 128), (128, 128), (128, 64), (64, 64)][chosen.shape]
+split_grid = -(-m // rows) * -(-n // columns) * chosen.splits
+"""
+
+_CASES = {
+    "no memory": """
+stand_in.stand_in(0, 0)
+assert tiled(1) == _capi.SUCCESS and 0 < stand_in.stand_in_grid() < split_grid and stand_in.stand_in_grid() <= 2
+assert stand_in.hipGetLastError() == 0
+assert tiled(1, (4, 1, 1)) == _capi.SUCCESS  # and no later launch is taken for the one that failed
+stand_in.stand_in(1, 0)  # the sums, but not the counters
+assert tiled(1) == _capi.SUCCESS and 0 < stand_in.stand_in_grid() <= 2
+""",
+    "memory for one": """
+stand_in.stand_in(2, 0)
+assert tiled(1) == _capi.SUCCESS and stand_in.stand_in_grid() == split_grid
+assert tiled(1) == _capi.SUCCESS and stand_in.stand_in_grid() == split_grid
+assert tiled(2) == _capi.SUCCESS and 0 < stand_in.stand_in_grid() <= 2
+assert tiled(1) == _capi.SUCCESS and stand_in.stand_in_grid() == split_grid
+""",
+    "capturing": """
+stand_in.stand_in(100, 1)
+assert tiled(1) == _capi.SUCCESS and 0 < stand_in.stand_in_grid() <= 2
+stand_in.stand_in(100, 0)
+assert tiled(1) == _capi.SUCCESS and stand_in.stand_in_grid() == split_grid
+stand_in.stand_in(0, 1)
+for stream in (2, 3, 4):  # three more workspaces came with the first
+    assert tiled(stream) == _capi.SUCCESS and stand_in.stand_in_grid() == split_grid
+assert tiled(5) == _capi.SUCCESS and 0 < stand_in.stand_in_grid() <= 2
+""",
+    "a split that was asked for": """
+stand_in.stand_in(0, 0)
+assert tiled(1, (4, 2, 1)) == _capi.HIP_ERROR and lib.hfrk_last_hip_error() == 2 and stand_in.hipGetLastError() == 0
+assert skinny(1) == _capi.HIP_ERROR and lib.hfrk_last_hip_error() == 2 and stand_in.hipGetLastError() == 0
+stand_in.stand_in(100, 1)
+assert tiled(1, (4, 2, 1)) == skinny(1) == _capi.NOT_INITIALISED
+stand_in.stand_in(2, 0)
+assert skinny(1) == _capi.SUCCESS
+""",
+}
+
+
+@pytest.fixture(scope="module")
+def stand_in(tmp_path_factory):
+    directory = tmp_path_factory.mktemp("stand_in")
+    source, library = os.path.join(directory, "stand_in.c"), os.path.join(directory, "libstand_in.so")
+    with open(source, "w") as f:
+        f.write(_STAND_IN)
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", source, "-o", library], check=True)
+    return library
+
+
+@pytest.mark.parametrize("case", sorted(_CASES))
+def test_launches_without_a_workspace(case, stand_in):
+    from hf_rocm_kernels import _capi
+    preload = ":".join(p for p in (stand_in, os.environ.get("LD_PRELOAD")) if p)
+    code = _PRELUDE.format(package=os.path.dirname(_capi.__file__), stand_in=stand_in) + _CASES[case]
+    subprocess.run([sys.executable, "-c", code], check=True, timeout=100, env=dict(os.environ, LD_PRELOAD=preload))
