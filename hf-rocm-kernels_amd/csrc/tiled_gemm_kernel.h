@@ -34,7 +34,8 @@ namespace hfrk {
 typedef float v16f __attribute__((ext_vector_type(16)));
 
 // One 16-byte-per-lane load from memory straight into LDS: lane l's piece lands at lds_base + 16 l.  As inline assembly because the
-// compiler, when it knows of such a load, waits for it before every LDS read that follows; the waits are placed by hand here.
+// compiler, when it knows of such a load, waits for it before every LDS read that follows; the waits are placed by hand here.  m0 is
+// reserved: the compiler sets it in front of each use of its own, and a clobber list may not name it.
 __device__ __forceinline__ void load_to_lds(const v4i& rsrc, int voffset, uint32_t lds_base) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds_base), "v"(voffset), "s"(rsrc) : "memory");
 }
@@ -233,7 +234,9 @@ __global__ void __launch_bounds__(kTiledThreads, WGS) tiled_gemm_kernel(const Ti
     };
 
     // ---- main loop ---------------------------------------------------------------------------------------------------
-    asm volatile("s_nop 4" ::: "memory");  // scalars a vector instruction wrote are not read by a load at once
+    // A load may read a scalar that a vector instruction wrote (v_readfirstlane) only five cycles later, and nobody looks after that
+    // for a load in inline assembly: both buffers pass through the wait.  From here on scalar instructions move them.
+    asm volatile("s_nop 4" : "+s"(ra), "+s"(rb) : : "memory");
 #pragma unroll 1
     for (int s = 0; s < NST; ++s) {
         issue_begin();

@@ -1,5 +1,4 @@
-"""The order of the row-split kernel's memory requests, read from the assembly the build's own command line gives: a decode GEMM lives
-10-20 us, and a request that the compiler moves behind a hundred instructions costs 1-3 % of it while every result stays the same."""
+"""What the compiler makes of orders that the sources rely on, read from the assembly the build's own command line gives."""
 import importlib.util
 import os
 import re
@@ -11,20 +10,20 @@ import pytest
 _PACKAGE = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "hf-rocm-kernels_amd")
 
 
-def _instances(tmp_path):
-    """(template arguments, instructions and labels) of every instance of the kernel on row-major weights in 4-row units."""
+def _instances(source, kernel, tmp_path):
+    """Template arguments -> instructions and labels, for every instance of `kernel` that `source` compiles."""
     spec = importlib.util.spec_from_file_location("hfrk_build", os.path.join(_PACKAGE, "build.py"))
     build = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(build)
     hipcc = shutil.which("hipcc") or os.path.join(build.ROCM, "bin", "hipcc")
     if not os.path.exists(hipcc):
         pytest.skip("no hipcc here")
-    out = os.path.join(tmp_path, "rows.s")
-    subprocess.run([hipcc] + build.HIPCC_FLAGS + ["--offload-device-only", "-S", os.path.join(build.CSRC, "skinny_gemm_rows.hip"), "-o", out],
+    out = os.path.join(tmp_path, "kernels.s")
+    subprocess.run([hipcc] + build.HIPCC_FLAGS + ["--offload-device-only", "-S", os.path.join(build.CSRC, source), "-o", out],
                    check=True, capture_output=True)
     found, body = {}, None
     for line in open(out):
-        start = re.match(r"_ZN4hfrk\d+skinny_gemm_rows_kernelI(\S+?)EEEv", line)
+        start = re.match(r"_ZN4hfrk\d+%sI(\S+?)EEEv" % kernel, line)
         if start:
             body = found.setdefault(start[1], [])
         elif line.startswith(".Lfunc_end"):
@@ -36,8 +35,10 @@ def _instances(tmp_path):
     return found
 
 
-def test_requests_stay_where_the_kernel_makes_them(tmp_path):
-    instances = _instances(tmp_path)
+def test_row_split_requests_stay_where_the_kernel_makes_them(tmp_path):
+    """A decode GEMM lives 10-20 us: a request that the compiler moves behind a hundred instructions costs 1-3 % of it, while every result
+    stays the same."""
+    instances = _instances("skinny_gemm_rows.hip", "skinny_gemm_rows_kernel", tmp_path)
     assert len(instances) == 20
     for name, body in instances.items():
         first = next(i for i, x in enumerate(body) if x.startswith("buffer_load_dwordx4") and " nt" in x)
@@ -50,3 +51,17 @@ def test_requests_stay_where_the_kernel_makes_them(tmp_path):
         copied = max(i for i, x in enumerate(turn[:request]) if x.startswith("ds_write_b128"))
         branches = sum(x.startswith(("s_cbranch", "s_branch")) for x in turn[copied:request])
         assert branches <= 1 and request - copied < 30, (name, "the next chunk is requested behind the copy of this one", branches, request - copied)
+
+
+@pytest.mark.parametrize("layout", ["rowmajor", "packed"])
+def test_tiled_loads_read_no_scalar_that_a_vector_instruction_has_just_written(layout, tmp_path):
+    """The compiler puts no wait states in front of a load in inline assembly: the kernel's own stand between the last
+    v_readfirstlane that makes a buffer and the first load, and nothing makes one afterwards."""
+    instances = _instances(f"tiled_gemm_{layout}.hip", "tiled_gemm_kernel", tmp_path)
+    assert len(instances) == 5
+    for name, body in instances.items():
+        loads = [i for i, x in enumerate(body) if x.endswith(" lds")]
+        waits = [i for i, x in enumerate(body) if x == "s_nop 4"]
+        written = [i for i, x in enumerate(body) if x.startswith(("v_readfirstlane", "v_readlane"))]
+        assert loads and len(waits) == 1 and waits[0] < loads[0], name
+        assert not [i for i in written if waits[0] < i < loads[-1]], name
