@@ -320,8 +320,9 @@ __global__ void __launch_bounds__(kTiledThreads, WGS) tiled_gemm_kernel(const Ti
     static_assert(4 * 32 * RS * 4 <= NST * STAGE, "the staging fits in the operands' LDS");
     float* const stage = reinterpret_cast<float*>(lds) + wave * (32 * RS);
     const int row0 = wm * TM * 32, col = wn * TN * 32 + (lane % LPR) * 8;
-    // buffers over the tile's rows: what lies outside reads as zero and is not stored
-    const int outside = n0 + col < a.n ? 0 : kOutside;
+    // buffers over the tile's rows: what lies outside reads as zero and is not stored.  A column past n is marked by bits that no row
+    // step clears: a tile's rows reach over less than 2^30 bytes, so the sums stay above every range and below 2^32.
+    const uint32_t outside = n0 + col < a.n ? 0u : (uint32_t)kOutside;
     const __amdgpu_buffer_rsrc_t rd = make_rsrc(static_cast<uint16_t*>(a.D) + (long)m0 * a.n, (uint32_t)rows_a * (uint32_t)a.n * 2u);
     const __amdgpu_buffer_rsrc_t rbase = make_rsrc(static_cast<const uint16_t*>(a.base) + (long)m0 * a.base_stride,
                                                    a.base ? (uint32_t)((rows_a - 1) * a.base_stride + a.n) * 2u : 0u);
@@ -335,15 +336,17 @@ __global__ void __launch_bounds__(kTiledThreads, WGS) tiled_gemm_kernel(const Ti
         // are requested before the stores of the 32 rows in front.
         v4i add[2][PASSES];
         float sa[2][PASSES];
-        const int base_off = ((row0 + lane / LPR) * a.base_stride + n0 + col) * 2 | outside, base_step = RPI * a.base_stride * 2;
+        const uint32_t base_off = ((uint32_t)(row0 + lane / LPR) * (uint32_t)a.base_stride + (uint32_t)(n0 + col)) * 2u | outside;
+        const uint32_t base_step = (uint32_t)(RPI * 2) * (uint32_t)a.base_stride;
         auto fetch = [&](int i) __attribute__((always_inline)) {
 #pragma unroll
             for (int r = 0; r < PASSES; ++r) {
                 sa[i & 1][r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsa, (row0 + i * 32 + r * RPI + lane / LPR) * a.sa_stride * 4, 0, 0));
-                add[i & 1][r] = __builtin_amdgcn_raw_buffer_load_b128(rbase, base_off + (i * PASSES + r) * base_step, 0, 0);
+                add[i & 1][r] = __builtin_amdgcn_raw_buffer_load_b128(rbase, (int)(base_off + (uint32_t)(i * PASSES + r) * base_step), 0, 0);
             }
         };
-        const int d_off = ((row0 + lane / LPR) * a.n + n0 + col) * 2 | outside, d_step = RPI * a.n * 2;
+        const uint32_t d_off = ((uint32_t)(row0 + lane / LPR) * (uint32_t)a.n + (uint32_t)(n0 + col)) * 2u | outside;
+        const uint32_t d_step = (uint32_t)(RPI * 2) * (uint32_t)a.n;
         if (a.vec) fetch(0);
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
@@ -370,7 +373,7 @@ __global__ void __launch_bounds__(kTiledThreads, WGS) tiled_gemm_kernel(const Ti
                         o[v] = (int)pack_pair<DT>(load16<DT>((uint16_t)(b & 0xffff)) + x[2 * v] * (sa[i & 1][r] * sb[2 * v]),
                                                load16<DT>((uint16_t)(b >> 16)) + x[2 * v + 1] * (sa[i & 1][r] * sb[2 * v + 1]));
                     }
-                    __builtin_amdgcn_raw_buffer_store_b128(o, rd, d_off + (i * PASSES + r) * d_step, 0, 0);
+                    __builtin_amdgcn_raw_buffer_store_b128(o, rd, (int)(d_off + (uint32_t)(i * PASSES + r) * d_step), 0, 0);
                 }
             } else {  // rows of D or base that are not 16-byte aligned: one element per lane
 #pragma unroll 1
