@@ -126,6 +126,12 @@ void swiglu(at::Tensor& gate_up, at::Tensor& scale_tensor, at::Tensor& output, a
              "swiglu");
 }
 
+// Elements between the weight's rows, which the C ABI takes as an int: cut to one, a larger stride would name other rows.
+int row_stride(const at::Tensor& B) {
+    TORCH_CHECK(B.size(1) <= 1 || B.stride(1) < (int64_t(1) << 31), "the weight's rows must be less than 2^31 elements apart, got ", B.stride(1));
+    return (int)B.stride(1);
+}
+
 void check_gemm_operands(const at::Tensor& A, const at::Tensor& B, const at::Tensor& D) {
     TORCH_CHECK(A.dim() == 2 && A.is_contiguous(), "A must be a contiguous [m, k] tensor");
     TORCH_CHECK(B.dim() == 2 && B.size(0) == A.size(1) && B.stride(0) == 1, "B must be [k, n] with unit stride along k");
@@ -148,7 +154,7 @@ int64_t skinny_gemm_tb(at::Tensor& A, at::Tensor& B, at::Tensor& D, at::Tensor& 
     const int d_dtype = dtype16(D, "D");
     DeviceScope scope(A);  // before the stream is looked up
     return hfrk_skinny_gemm(A.data_ptr(), B.data_ptr(), D.data_ptr(), scale_tensor.data_ptr<float>(), (int)A.size(0),
-                            (int)B.size(1), (int)A.size(1), (int)B.stride(1), (int)split_k, (int)A_producers,
+                            (int)B.size(1), (int)A.size(1), row_stride(B), (int)split_k, (int)A_producers,
                             (int)B_producers, (int)consumers, (int)a_lanes, (int)b_lanes, (int)qsize, (int)op_m, (int)ops,
                             d_dtype, current_stream(A));
 }
@@ -168,7 +174,7 @@ int64_t skinny_gemm_scaled(at::Tensor& A, at::Tensor& B, at::Tensor& D, at::Tens
     DeviceScope scope(A);
     return hfrk_skinny_gemm_ex(A.data_ptr(), B.data_ptr(), D.data_ptr(), scale_a.data_ptr<float>(),
                                scale_a.numel() == 1 ? 0 : 1, scale_b.data_ptr<float>(), scale_b.numel() == 1 ? 0 : 1, (int)m,
-                               (int)n, (int)A.size(1), (int)B.stride(1), d_dtype, accumulate ? 1 : 0, nullptr,
+                               (int)n, (int)A.size(1), row_stride(B), d_dtype, accumulate ? 1 : 0, nullptr,
                                current_stream(A));
 }
 
@@ -328,7 +334,7 @@ int64_t gemm_fused_common(at::Tensor& A, at::Tensor& B, bool packed, int64_t n, 
                                        scale_a.numel() == 1 ? 0 : 1, scale_b_ptr, sb_stride, out_scale_ptr, (int)m, (int)n,
                                        (int)A.size(1), d_dtype, (int)epilogue, nullptr, current_stream(A));
     return hfrk_skinny_gemm_fused(A.data_ptr(), B.data_ptr(), D.data_ptr(), base_ptr, scale_a.data_ptr<float>(),
-                                  scale_a.numel() == 1 ? 0 : 1, scale_b_ptr, sb_stride, out_scale_ptr, (int)m, (int)n, (int)A.size(1), (int)B.stride(1), d_dtype, (int)epilogue,
+                                  scale_a.numel() == 1 ? 0 : 1, scale_b_ptr, sb_stride, out_scale_ptr, (int)m, (int)n, (int)A.size(1), row_stride(B), d_dtype, (int)epilogue,
                                   nullptr, current_stream(A));
 }
 
@@ -396,7 +402,7 @@ int64_t skinny_gemm_rms_fused(at::Tensor& input, at::Tensor& residual, at::Tenso
     DeviceScope scope(input);
     return hfrk_skinny_gemm_rms_fused(input.data_ptr(), residual.data_ptr(), residual_out.data_ptr(), rms_weight.data_ptr(), (float)epsilon,
                                       act_scale.data_ptr<float>(), io, B.data_ptr(), D.data_ptr(), base_ptr, scale_a.data_ptr<float>(),
-                                      scale_b_ptr, sb_stride, out_scale_ptr, (int)m, (int)n, (int)k, (int)B.stride(1), d_dtype,
+                                      scale_b_ptr, sb_stride, out_scale_ptr, (int)m, (int)n, (int)k, row_stride(B), d_dtype,
                                       (int)epilogue, nullptr, current_stream(input));
 }
 
@@ -451,7 +457,7 @@ void tiled_gemm(at::Tensor& A, at::Tensor& B, bool packed, int64_t n, at::Tensor
     }
     if (m == 0) return;
     DeviceScope scope(A);
-    const int sa_stride = scale_a.numel() == 1 ? 0 : 1, b_stride = packed ? (int)k : (int)B.stride(1);
+    const int sa_stride = scale_a.numel() == 1 ? 0 : 1, b_stride = packed ? (int)k : row_stride(B);
     const float* const sa = scale_a.data_ptr<float>();
     raise_on(hfrk_linear_gemm(A.data_ptr(), B.data_ptr(), packed ? 1 : 0, D.data_ptr(), base_ptr, base_stride, sa, sa_stride, scale_b_ptr,
                               sb_stride, (int)m, (int)n, (int)k, b_stride, d_dtype, current_stream(A)),

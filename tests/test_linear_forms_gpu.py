@@ -55,3 +55,16 @@ def test_operands_that_do_not_fit_are_refused_alike(m, k):
                 dict(residual=torch.zeros(m, N, device="cuda", dtype=torch.float16)), dict(out_dtype=torch.float32), dict(weight=w[:, :256])):
         with pytest.raises(AssertionError):
             apply_fp8_linear(**{**dict(input=q, weight=w, weight_scale=sw, input_scale=sx), **bad})
+
+
+@pytest.mark.parametrize("m", [5, 65])
+def test_rows_further_apart_than_an_int_counts_are_refused(m):
+    k, stride = 512, (1 << 32) + 512  # as an int: 512, the stride of other rows
+    x = torch.randn(m, k, device="cuda").to(torch.bfloat16)
+    storage = torch.zeros(stride + k, dtype=torch.uint8, device="cuda").view(torch.float8_e4m3fn)
+    w, sw = storage.as_strided((2, k), (stride, 1)), torch.ones(2, device="cuda")
+    q, sx = hf_rocm_kernels.quantize_fp8(x)
+    for call in (lambda: apply_fp8_linear(x, w, sw), lambda: hf_rocm_kernels.skinny_gemm_scaled(q, w.t(), sx, sw),
+                 lambda: hf_rocm_kernels.skinny_gemm(q, w.t(), sw[:1])):
+        with pytest.raises(RuntimeError):
+            call()
