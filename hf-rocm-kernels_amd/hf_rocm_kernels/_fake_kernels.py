@@ -17,7 +17,8 @@ import hf_rocm_kernels._HFRK_C  # noqa: F401  (registers torch.ops._HFRK_C)
 _RETURNS_NOTHING = ("increment", "residual_rms", "swiglu", "pack_weight", "pack_weight_scaled", "unpack_weight", "reencode_fnuz",
                     "residual_rms_dynamic", "swiglu_dynamic", "quantize_fp8", "skinny_gemm_checked", "tiled_gemm")
 _RETURNS_STATUS = ("skinny_gemm_tb", "skinny_gemm_scaled", "skinny_gemm_fused", "skinny_gemm_packed", "skinny_gemm_rms_fused",
-                   # a new tensor, or whether the call was one they take: _OTHER_RESULT
+                   # a result of their own, _OTHER_RESULT; the wrappers keep fake calls away from these (utils/dispatch.py), a caller of
+                   # torch.ops need not
                    "fp8_linear", "skinny_gemm_new", "skinny_gemm_into")
 
 
