@@ -141,3 +141,149 @@ assert status == want[0] == _capi.SUCCESS and torch.equal(out, want[1])
 def test_a_stream_without_a_workspace_does_not_split_k():
     env = dict(os.environ, PYTHONPATH=os.pathsep.join(p for p in sys.path if p))
     subprocess.run([sys.executable, "-c", _NO_WORKSPACE], check=True, timeout=100, env=env)
+
+
+def _call(lib, dev, weight, packed, out, base, base_stride, m, n, k, dtype, plan, stream=None):
+    from hf_rocm_kernels import _capi
+    return lib.hfrk_tiled_gemm(dev[0].data_ptr(), weight.data_ptr(), packed, out.data_ptr(), None if base is None else base.data_ptr(),
+                               base_stride, dev[2].data_ptr(), 1, dev[3].data_ptr(), 1, m, n, k, k,
+                               _capi.F16 if dtype == torch.float16 else _capi.BF16, ctypes.byref(plan),
+                               torch.cuda.current_stream().cuda_stream if stream is None else stream)
+
+
+# stages of 128 bytes over the splits: 11 -> 6 5; 15 -> 4 4 4 3; 21 -> 3 3 3 3 3 2 2 2 (the last stage of each cut to 16 bytes);
+# 22 -> 3 3 3 3 3 3 2 2 in both layouts; 13 -> 3 3 3 2 2
+@pytest.mark.parametrize("m,n,k,splits", [(130, 136, 1296, 2), (65, 200, 1808, 4), (70, 136, 2576, 8), (257, 264, 2816, 8), (40, 72, 1664, 5)])
+def test_uneven_splits_match_the_oracle(m, n, k, splits):
+    from hf_rocm_kernels import _capi
+    from hf_rocm_kernels.utils.weight_format import pack_weight
+    lib = _capi.load()
+    a, w, sa, sw = _operands(m, n, k, seed=m + n + k)
+    base = torch.randn(m, n, generator=torch.Generator().manual_seed(5)).to(torch.bfloat16)
+    check = oracle_checker(a, w.t(), sa, sw, torch.bfloat16, base=base)
+    dev, dev_base = [t.cuda() for t in (a, w, sa, sw)], base.cuda()
+    layouts = [(0, dev[1])] + ([(1, pack_weight(dev[1]).data)] if k % 256 == 0 else [])
+    for shape in range(5):
+        first = None
+        for packed, weight in layouts:
+            out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+            _capi.check(_call(lib, dev, weight, packed, out, dev_base, n, m, n, k, torch.bfloat16, _capi.TiledPlan(shape, splits, 1)), "tiled")
+            if first is None:
+                check(out)
+                first = out
+            assert torch.equal(out, first), (shape, packed)
+
+
+@pytest.mark.parametrize("shape", range(5))
+def test_rows_that_are_not_16_byte_aligned(shape):
+    """n % 8 == 0, but D and the addend start one element past an aligned address: the element-wise epilogue."""
+    from hf_rocm_kernels import _capi
+    lib = _capi.load()
+    m, n, k = 70, 136, 256
+    a, w, sa, sw = _operands(m, n, k, seed=2)
+    dev = [t.cuda() for t in (a, w, sa, sw)]
+    for rows in (m, 1):
+        base = torch.randn(rows * n + 1, device="cuda").to(torch.float16)[1:].view(rows, n)
+        for d_off, b in ((1, None), (0, base), (1, base)):
+            store = torch.full((m * n + 2,), 7.0, dtype=torch.float16, device="cuda")
+            out = store[d_off:d_off + m * n].view(m, n)
+            stride = 0 if b is None or rows == 1 else n
+            _capi.check(_call(lib, dev, dev[1], 0, out, b, stride, m, n, k, torch.float16, _capi.TiledPlan(shape, 1, 1)), "tiled")
+            oracle_checker(a, w.t(), sa, sw, torch.float16, base=None if b is None else b.expand(m, n).contiguous())(out)
+            assert (store[:d_off] == 7).all() and (store[d_off + m * n:] == 7).all()
+
+
+def _split_problem(seed):
+    m, n, k = 130, 520, 4096
+    a, w, sa, sw = _operands(m, n, k, seed=seed)
+    return m, n, k, [t.cuda() for t in (a, w, sa, sw)]
+
+
+def test_two_streams_with_split_plans_at_once():
+    from hf_rocm_kernels import _capi
+    lib = _capi.load()
+    problems, streams = [_split_problem(s) for s in (1, 2)], [torch.cuda.Stream() for _ in range(2)]
+    plan = _capi.TiledPlan(4, 6, 1)
+    wants = []
+    for m, n, k, dev in problems:
+        want = torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
+        _capi.check(_call(lib, dev, dev[1], 0, want, None, 0, m, n, k, torch.bfloat16, plan), "tiled")
+        wants.append(want)
+    torch.cuda.synchronize()
+    outs = [[], []]
+    for _ in range(20):
+        for i, (m, n, k, dev) in enumerate(problems):
+            with torch.cuda.stream(streams[i]):
+                out = torch.zeros(m, n, dtype=torch.bfloat16, device="cuda")
+            _capi.check(_call(lib, dev, dev[1], 0, out, None, 0, m, n, k, torch.bfloat16, plan, streams[i].cuda_stream), "tiled")
+            outs[i].append(out)
+    torch.cuda.synchronize()
+    for want, got in zip(wants, outs):
+        assert all(torch.equal(g, want) for g in got)
+
+
+def test_a_captured_split_plan_replays_like_the_eager_call():
+    from hf_rocm_kernels import _capi
+    lib = _capi.load()
+    m, n, k, dev = _split_problem(3)
+    plan, stream = _capi.TiledPlan(4, 6, 1), torch.cuda.Stream()
+    out = torch.zeros(m, n, dtype=torch.bfloat16, device="cuda")
+    torch.cuda.synchronize()
+
+    def call():
+        _capi.check(_call(lib, dev, dev[1], 0, out, None, 0, m, n, k, torch.bfloat16, plan, stream.cuda_stream), "tiled")
+
+    with torch.cuda.stream(stream):
+        call()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            call()
+        for turn in range(5):
+            dev[0].copy_(dev[0].flip(0))  # other inputs for every replay
+            call()
+            torch.cuda.synchronize()
+            want = out.clone()
+            out.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want) and want.float().abs().sum() > 0, turn
+
+
+def test_nan_and_infinities_reach_their_rows_and_columns_only():
+    from hf_rocm_kernels import _capi
+    lib = _capi.load()
+    m, n, k = 130, 136, 656
+    a, w, sa, sw = _operands(m, n, k, seed=9)
+    base = torch.randn(m, n, generator=torch.Generator().manual_seed(5))
+    a.view(torch.uint8)[63, k - 1] = 0x7F  # NaN at the end of a row, and of the last, cut stage
+    w.view(torch.uint8)[n - 1, 0] = 0xFF
+    sa[5], sw[3] = float("inf"), float("nan")
+    base[64, 7], base[129, 135 - 1] = float("inf"), float("-inf")
+    base = base.to(torch.bfloat16)
+    scales = sa.double()[:, None] * sw.double()[None]
+    want = (a.double() @ w.double().t()) * scales + base.double()
+    slack = want.abs() * 2.0 ** -8 + (a.double().abs() @ w.double().abs().t()) * scales * 2.0 ** -16 + 2.0 ** -126
+    dev, dev_base = [t.cuda() for t in (a, w, sa, sw)], base.cuda()
+    for shape in range(5):
+        for splits in (1, 3):
+            out = torch.zeros(m, n, dtype=torch.bfloat16, device="cuda")
+            _capi.check(_call(lib, dev, dev[1], 0, out, dev_base, n, m, n, k, torch.bfloat16, _capi.TiledPlan(shape, splits, 1)), "tiled")
+            got = out.cpu().double()
+            assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf()), (shape, splits)
+            fine = want.isfinite()
+            assert torch.equal(got[want.isinf()], want[want.isinf()]) and ((got - want).abs() <= slack)[fine].all(), (shape, splits)
+
+
+@pytest.mark.parametrize("m,n,k", [(65, 264, 4096), (130, 4104, 2304), (201, 1032, 1040), (300, 520, 14336)])
+def test_linear_layers_under_the_librarys_plan_match_the_oracle(m, n, k):
+    from hf_rocm_kernels.layers import apply_fp8_linear
+    from hf_rocm_kernels.utils.weight_format import pack_weight
+    a, w, sa, sw = _operands(m, n, k, seed=m + n)
+    g = torch.Generator().manual_seed(1)
+    bias, residual = torch.randn(n, generator=g).to(torch.bfloat16), torch.randn(m, n, generator=g).to(torch.bfloat16)
+    dev = [t.cuda() for t in (a, w, sa, sw)]
+    for add, base in ((dict(), None), (dict(bias=bias.cuda()), bias.expand(m, n).contiguous()), (dict(residual=residual.cuda()), residual)):
+        check = oracle_checker(a, w.t(), sa, sw, torch.bfloat16, base=base)
+        for weight in [dev[1]] + ([pack_weight(dev[1])] if k % 256 == 0 else []):
+            check(apply_fp8_linear(dev[0], weight, dev[3], dev[2], **add))

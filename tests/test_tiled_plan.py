@@ -6,6 +6,7 @@ from hf_rocm_kernels import _capi
 
 TILES = [(256, 256), (256, 128), (128, 128), (128, 64), (64, 64)]  # by shape index
 WORKSPACE_BYTES = 64 << 20  # partial sums of one stream
+MAX_COUNTERS = 1 << 20
 
 
 def _sizes():
@@ -25,3 +26,19 @@ def test_partial_sums_fit_the_workspace():
         tiles = -(-m // bm) * -(-n // bn)
         assert plan.splits == 1 or tiles * plan.splits * bm * bn * 4 <= WORKSPACE_BYTES, (m, n, k, plan.shape, plan.splits)
         assert plan.splits <= -(-k // 128) and 1 <= plan.group_m <= -(-m // bm)
+
+
+def test_plans_of_few_rows_and_of_small_weights():
+    """One row of tiles has a rule of its own, and small sizes leave few stages to split."""
+    lib = _capi.load()
+    rng = random.Random(2)
+    sizes = [(m, n, k) for m in (1, 33, 64, 65) for n in (1, 8, 64, 65, 4104, 28672, 1 << 21) for k in (16, 128, 144, 1008, 1040, 4112, 28656)]
+    sizes += [(rng.randint(1, 64), int(28672 ** rng.random()), int(1792 ** rng.random()) * 16) for _ in range(10000)]
+    sizes += [(int(65 * 63 ** rng.random()), int(1024 ** rng.random()), int(64 ** rng.random()) * 16) for _ in range(10000)]
+    for m, n, k in sizes:
+        plan = _capi.TiledPlan()
+        assert lib.hfrk_tiled_gemm_plan(m, n, k, ctypes.byref(plan)) == _capi.SUCCESS
+        bm, bn = TILES[plan.shape]
+        tiles, stages = -(-m // bm) * -(-n // bn), -(-k // 128)
+        assert 1 <= plan.splits <= stages and 1 <= plan.group_m <= -(-m // bm), (m, n, k, plan.shape, plan.splits)
+        assert plan.splits == 1 or (tiles * plan.splits * bm * bn * 4 <= WORKSPACE_BYTES and tiles <= MAX_COUNTERS and stages >= 2 * plan.splits)
