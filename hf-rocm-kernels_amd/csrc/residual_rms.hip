@@ -18,6 +18,13 @@ namespace hfrk {
 
 constexpr int kRmsMaxThreads = 1024;
 
+// From this many values on the input is read past the caches, which leaves their room (256 MB behind the L2s) to the residual, the weight
+// and the output.  Measured with both reads on fp16, us, kept / past.  Buffers used again and again: 2048 x 4096 10.2 / 11.2,
+// 2048 x 8192 18.3 / 19.7, 1536 x 16384 30.4 / 28.6, 2048 x 16384 43.2 / 37.9, 4096 x 16384 83.2 / 80.3.  With a kernel in front that
+// has just written the input, both: 2048 x 8192 30.9 / 31.5, 1536 x 16384 44.6 / 44.8, 4096 x 8192 66.2 / 59.0, 4096 x 16384 128.5 / 125.0.
+// At decode sizes reading past them cost an eager MLP block of 1 to 16 rows of 4096 0.4 us of 32.
+constexpr long kReadOnceFrom = 20L << 20;
+
 __device__ __forceinline__ void zero_next_buffer_row(uint16_t* next_buffer, int buffer_cols) {
     if (buffer_cols <= 0) return;
     uint16_t* const row = next_buffer + (long)blockIdx.x * buffer_cols;
@@ -33,7 +40,8 @@ __device__ __forceinline__ void zero_next_buffer_row(uint16_t* next_buffer, int 
 }
 
 // 8 elements (16 bytes) per thread per iteration, ITERS iterations cached in registers: cols <= 8*blockDim*ITERS.
-template <int DT, bool FP8_OUT, int ITERS>
+// READ_ONCE: the input is read past the caches (kReadOnceFrom).
+template <int DT, bool FP8_OUT, int ITERS, bool READ_ONCE>
 __global__ void __launch_bounds__(kRmsMaxThreads) residual_rms_vec_kernel(
     const uint16_t* __restrict__ input, uint16_t* __restrict__ residual, const uint16_t* __restrict__ weight,
     const float* __restrict__ scale_tensor, void* __restrict__ output, uint16_t* __restrict__ next_buffer,
@@ -47,14 +55,13 @@ __global__ void __launch_bounds__(kRmsMaxThreads) residual_rms_vec_kernel(
                                                 : make_rsrc(static_cast<uint16_t*>(output) + row_off, row_bytes);
     uint4 a[ITERS], z[ITERS], wreg[ITERS];
     float ssq = 0.f;
-    // Everything both passes need is requested now, so that the kernel pays one memory latency.  The input is read past the caches:
-    // nobody reads it again, and the residual and the weight keep their place (2048 x 16384 fp16: 41.5 -> 37 us, 6.3 TB/s).
+    // Everything both passes need is requested now, so that the kernel pays one memory latency.
     float scale = 1.f;
     if constexpr (FP8_OUT) scale = scale_tensor[0];
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
         const int v = threadIdx.x + it * blockDim.x;
-        a[it] = load_piece<true>(rin, v);
+        a[it] = load_piece<READ_ONCE>(rin, v);
         z[it] = load_piece(rres, v);
     }
 #pragma unroll
@@ -150,12 +157,18 @@ static int launch_rms(const void* input, void* residual, const void* weight, con
         const int iters = (nvec + threads - 1) / threads;
         if (iters > 4) vec = false;  // would not fit the register cache: fall through to the strided kernel
         else {
-#define HFRK_RMS_LAUNCH(IT)                                                                                          \
-    hipLaunchKernelGGL((residual_rms_vec_kernel<DT, FP8_OUT, IT>), dim3(rows), dim3(threads), 0, stream, in, res, w, \
+#define HFRK_RMS_LAUNCH(IT, ONCE)                                                                                          \
+    hipLaunchKernelGGL((residual_rms_vec_kernel<DT, FP8_OUT, IT, ONCE>), dim3(rows), dim3(threads), 0, stream, in, res, w, \
                        scale_tensor, output, nb, epsilon, cols, buffer_cols)
-            if (iters <= 1) HFRK_RMS_LAUNCH(1);
-            else if (iters == 2) HFRK_RMS_LAUNCH(2);
-            else HFRK_RMS_LAUNCH(4);
+#define HFRK_RMS_ITERS(ONCE)                         \
+    do {                                             \
+        if (iters <= 1) HFRK_RMS_LAUNCH(1, ONCE);    \
+        else if (iters == 2) HFRK_RMS_LAUNCH(2, ONCE); \
+        else HFRK_RMS_LAUNCH(4, ONCE);               \
+    } while (0)
+            if ((long)rows * cols >= kReadOnceFrom) HFRK_RMS_ITERS(true);
+            else HFRK_RMS_ITERS(false);
+#undef HFRK_RMS_ITERS
 #undef HFRK_RMS_LAUNCH
         }
     }

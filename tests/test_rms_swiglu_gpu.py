@@ -433,3 +433,21 @@ def test_traced_mlp_block_equals_the_eager_block(fused):
         torch.cuda.synchronize()
         assert torch.equal(got, want) and torch.equal(got_res, want_res), step
         assert got.float().abs().sum() > 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("fp8", [True, False])
+@pytest.mark.parametrize("rows,cols", [(1280, 16384), (5120, 4096), (2561, 8192)])
+def test_large_inputs_give_the_bits_of_their_halves(rows, cols, fp8, dtype):
+    """From 20 Mi values on the input is read past the caches; its halves are not.  Rows are independent."""
+    from hf_rocm_kernels import residual_rms
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    x, res = (torch.randn(rows, cols, device="cuda", generator=g).to(dtype) for _ in range(2))
+    w = (1 + 0.1 * torch.randn(cols, device="cuda", generator=g)).to(dtype)
+    scale = torch.tensor([6.0 / 448], device="cuda") if fp8 else None
+    whole, sums = residual_rms(x, res.clone(), w, 1e-5, scale)
+    half = rows // 2
+    for part in (slice(0, half), slice(half, rows)):
+        out, sum_ = residual_rms(x[part], res[part].clone(), w, 1e-5, scale)
+        assert torch.equal(whole[part].view(torch.uint8), out.view(torch.uint8)) and torch.equal(sums[part], sum_)
