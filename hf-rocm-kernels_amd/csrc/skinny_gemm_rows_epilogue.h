@@ -37,7 +37,7 @@ struct RowsEpilogue {
     __device__ __forceinline__ RowsEpilogue(const GemmArgs& args, int lane) : a(args), li(lane & 15), lg(lane >> 4) {
         n_out = SWIGLU ? (a.n >> 1) : a.n;
         d_rsrc = make_rsrc(a.D, (uint32_t)a.m * (uint32_t)n_out * (SWIGLU ? 1u : 2u));
-        base_rsrc = make_rsrc(a.base, a.base_bytes);
+        base_rsrc = make_rsrc(a.base, a.base ? ((uint32_t)(a.m - 1) * (uint32_t)a.base_stride + (uint32_t)a.n) * 2u : 0u);
         sb_rsrc = make_rsrc(a.scale_b, a.scale_b ? (uint32_t)a.n * 4u : 0u);
         accumulate = !SWIGLU && a.base != nullptr;
         vec = SWIGLU || (a.n & 3) == 0;  // then a lane's four outputs are all inside n and aligned

@@ -121,7 +121,7 @@ __global__ void __launch_bounds__(kGemmThreads) skinny_gemm_stream_kernel(const 
     const __amdgpu_buffer_rsrc_t ws_rsrc = make_rsrc(a.ws, a.ws_bytes);
     const int n_out = SWIGLU ? (a.n >> 1) : a.n;  // columns of D
     const __amdgpu_buffer_rsrc_t d_rsrc = make_rsrc(a.D, (uint32_t)a.m * (uint32_t)n_out * (SWIGLU ? 1u : 2u));
-    const __amdgpu_buffer_rsrc_t base_rsrc = make_rsrc(a.base, a.base_bytes);
+    const __amdgpu_buffer_rsrc_t base_rsrc = make_rsrc(a.base, a.base ? ((uint32_t)(a.m - 1) * (uint32_t)a.base_stride + (uint32_t)a.n) * 2u : 0u);
     const bool accumulate = !SWIGLU && a.base != nullptr;
     const __amdgpu_buffer_rsrc_t sb_rsrc = make_rsrc(a.scale_b, a.scale_b ? (uint32_t)a.n * 4u : 0u);
     const bool vec = SWIGLU || ((a.n & 3) == 0);  // then a lane's four outputs n0 .. n0+3 are all inside n and aligned
