@@ -37,7 +37,7 @@ struct RowsEpilogue {
     __device__ __forceinline__ RowsEpilogue(const GemmArgs& args, int lane) : a(args), li(lane & 15), lg(lane >> 4) {
         n_out = SWIGLU ? (a.n >> 1) : a.n;
         d_rsrc = make_rsrc(a.D, (uint32_t)a.m * (uint32_t)n_out * (SWIGLU ? 1u : 2u));
-        base_rsrc = make_rsrc(a.base, a.base ? ((uint32_t)(a.m - 1) * (uint32_t)a.base_stride + (uint32_t)a.n) * 2u : 0u);
+        base_rsrc = make_rsrc(a.base, a.base ? ((((uint32_t)(a.m - 1) * (uint32_t)a.n) & a.base_rows) + (uint32_t)a.n) * 2u : 0u);
         sb_rsrc = make_rsrc(a.scale_b, a.scale_b ? (uint32_t)a.n * 4u : 0u);
         accumulate = !SWIGLU && a.base != nullptr;
         vec = SWIGLU || (a.n & 3) == 0;  // then a lane's four outputs are all inside n and aligned
@@ -54,6 +54,16 @@ struct RowsEpilogue {
         }
     }
 
+    // Offsets into the addend are D's with the row's part masked away where it is one row: one product per row for both.  A product with
+    // the addend's own stride took four more registers through the weight loop, and from 25 rows on the kernel has none left: it kept
+    // 20 bytes in scratch (bfloat16, 2440 x 4352 at 26 rows 8.7 us, 2584 x 5376 at 31 rows 9.2, 5376 x 7936 with a residual at 26 rows
+    // 13.1; now 8.1, 8.65 and 12.6).  The mask is opaque, or the masked product would be kept as well.
+    __device__ __forceinline__ uint32_t base_rows() const {
+        uint32_t mask = a.base_rows;
+        asm volatile("" : "+s"(mask));
+        return mask;
+    }
+
     // Old D values and per-channel scales of a tile whose first row is `row0` and that holds `units` 4-row units (aligned n
     // only; ragged n fetches in the epilogue).  Nothing is requested when nothing is wanted.
     __device__ __forceinline__ Pre prefetch(int row0, int units, bool wanted) const {
@@ -63,6 +73,7 @@ struct RowsEpilogue {
 #pragma unroll
         for (int u = 0; u < MT * RT; ++u) p.d[u] = v2i{0, 0};
         if (wanted && want_pre) {
+            const uint32_t rows = base_rows();
 #pragma unroll
             for (int rt = 0; rt < RT; ++rt) {
                 const int ul = SWIGLU ? lg : 4 * rt + lg;                        // this lane's unit of the tile
@@ -71,7 +82,7 @@ struct RowsEpilogue {
                 p.sb[rt] = __builtin_amdgcn_raw_buffer_load_b128(sb_rsrc, (per_channel && ok) ? n0 * 4 : (int)kOutOfRange, 0, 0);
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt)
-                    p.d[mt * RT + rt] = __builtin_amdgcn_raw_buffer_load_b64(base_rsrc, (accumulate && ok && 16 * mt + li < a.m) ? (int)(((uint32_t)(16 * mt + li) * (uint32_t)a.base_stride + (uint32_t)n0) * 2u) : (int)kOutOfRange, 0, 0);
+                    p.d[mt * RT + rt] = __builtin_amdgcn_raw_buffer_load_b64(base_rsrc, (accumulate && ok && 16 * mt + li < a.m) ? (int)(((((uint32_t)(16 * mt + li) * (uint32_t)a.n) & rows) + (uint32_t)n0) * 2u) : (int)kOutOfRange, 0, 0);
             }
         }
         return p;
@@ -131,11 +142,12 @@ struct RowsEpilogue {
                 const v2i packed = {(int)pack16(r[0], r[1], bf16), (int)pack16(r[2], r[3], bf16)};
                 __builtin_amdgcn_raw_buffer_store_b64(packed, d_rsrc, live ? (int)d_off : (int)kOutOfRange, 0, 0);
             } else {
+                const uint32_t rows = base_rows();
                 // ragged n: 2-byte accesses whose out-of-range offsets mask the columns beyond n
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
                     const uint32_t off = (live && n0 + v < a.n) ? d_off + 2u * v : kOutOfRange;
-                    const uint32_t base_off = off == kOutOfRange ? off : ((uint32_t)arow * (uint32_t)a.base_stride + (uint32_t)(n0 + v)) * 2u;
+                    const uint32_t base_off = off == kOutOfRange ? off : ((((uint32_t)arow * (uint32_t)a.n) & rows) + (uint32_t)(n0 + v)) * 2u;
                     const uint32_t old = accumulate ? (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(base_rsrc, (int)base_off, 0, 0) : 0u;
                     const float sbv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sb_rsrc, (live && per_channel && n0 + v < a.n) ? (n0 + v) * 4 : (int)kOutOfRange, 0, 0));
                     float r = acc[u][v] * (per_channel ? sa * sbv : sa);

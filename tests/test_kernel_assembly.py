@@ -10,8 +10,7 @@ import pytest
 _PACKAGE = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "hf-rocm-kernels_amd")
 
 
-def _instances(source, kernel, tmp_path):
-    """Template arguments -> instructions and labels, for every instance of `kernel` that `source` compiles."""
+def _assembly(source, tmp_path):
     spec = importlib.util.spec_from_file_location("hfrk_build", os.path.join(_PACKAGE, "build.py"))
     build = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(build)
@@ -21,8 +20,14 @@ def _instances(source, kernel, tmp_path):
     out = os.path.join(tmp_path, "kernels.s")
     subprocess.run([hipcc] + build.HIPCC_FLAGS + ["--offload-device-only", "-S", os.path.join(build.CSRC, source), "-o", out],
                    check=True, capture_output=True)
+    with open(out) as f:
+        return f.readlines()
+
+
+def _instances(source, kernel, tmp_path):
+    """Template arguments -> instructions and labels, for every instance of `kernel` that `source` compiles."""
     found, body = {}, None
-    for line in open(out):
+    for line in _assembly(source, tmp_path):
         start = re.match(r"_ZN4hfrk\d+%sI(\S+?)EEEv" % kernel, line)
         if start:
             body = found.setdefault(start[1], [])
@@ -65,3 +70,9 @@ def test_tiled_loads_read_no_scalar_that_a_vector_instruction_has_just_written(l
         written = [i for i, x in enumerate(body) if x.startswith(("v_readfirstlane", "v_readlane"))]
         assert loads and len(waits) == 1 and waits[0] < loads[0], name
         assert not [i for i in written if waits[0] < i < loads[-1]], name
+
+
+@pytest.mark.parametrize("source", ["skinny_gemm_rows.hip", "skinny_gemm_rows_tiled.hip"])
+def test_row_split_kernels_keep_nothing_in_scratch(source, tmp_path):
+    sizes = re.findall(r"\.private_segment_fixed_size: (\d+)", "".join(_assembly(source, tmp_path)))
+    assert len(sizes) >= 20 and set(sizes) == {"0"}
