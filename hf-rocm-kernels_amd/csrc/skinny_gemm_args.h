@@ -64,9 +64,10 @@ struct GemmArgs {
 };
 
 // Loads requested so far stay in front of what follows.  The compiler sinks a load behind whatever writes no memory, and how far depends on
-// the size of what it is sunk past: when the SwiGLU epilogue became shorter, the row-split kernel's next chunk was requested 130
-// instructions and nine branches later than written, and the activation scales 250 (28672 x 4096 with SwiGLU at 1 row, float16 / bfloat16:
-// 19.6 / 20.0 us with the long epilogue, 20.1 / 20.25 with the short one, 19.6 / 19.8 with the requests held in place).
+// the size of what it is sunk past: when the SwiGLU epilogue became shorter, the row-split kernel's activation scales were requested 250
+// instructions later than written, behind the whole set-up, which then waited for them (28672 x 4096 with SwiGLU at 1 row, float16 /
+// bfloat16: 19.6 / 20.0 us with the long epilogue, 20.1 / 20.25 with the short one, 19.6 / 19.8 with the request held in place).  Holding
+// the next chunk's request and the reads of the partial sums in place as well changed nothing beyond noise, on 260 to 480 drawn calls.
 __device__ __forceinline__ void requests_end() { asm volatile("" ::: "memory"); }
 
 // The split-K workspace of `stream` on the current device: fp32 partial sums (kWsFloats) and kMaxPanels arrival counters, zero

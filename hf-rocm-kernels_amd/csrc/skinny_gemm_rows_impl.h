@@ -324,7 +324,6 @@ __global__ void __launch_bounds__(kGemmThreads) skinny_gemm_rows_kernel(const Ge
         pre_cur = pre_next;
         if (i + 1 < count) {  // registers are free again: request the next chunk before the LDS reads and MFMAs
             issue_chunk();
-            requests_end();
             // the chunk that ends a tile this wave finishes in the loop brings the tile's D along
             pre_next = prefetch(irow0, iunits, ikc == KC - 1 && !(itile == tile_h && kb0 != 0));
             if (i + 2 == count && finisher && late_pre) pre_l = prefetch(row0_l, units_l, true);
@@ -413,7 +412,6 @@ __global__ void __launch_bounds__(kGemmThreads) skinny_gemm_rows_kernel(const Ge
         for (int j = 1; j < kGemmWaves; ++j)
 #pragma unroll
             for (int u = 0; u < RT; ++u) other[j][u] = slots[j * kSlotStride + (mt * RT + u) * 64 + lane];
-        requests_end();
 #pragma unroll
         for (int j = 1; j < kGemmWaves; ++j) {
             const float f = (addmask >> j) & 1u ? 1.0f : 0.0f;
