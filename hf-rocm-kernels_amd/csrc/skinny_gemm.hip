@@ -493,12 +493,26 @@ static uint64_t stream_key(hipStream_t stream) {
     return key;
 }
 
+// The counters are zero before any stream may launch on them.  hipMemset does not do: it returns while the null stream still works (83 ms
+// early behind an 84 ms kernel), and a launch on another stream then counted its arrivals on memory that was cleared under it.  That
+// call's output stayed unwritten, and the counts stayed wrong for every later split on the workspace.
+static hipError_t zero_and_wait(int* p, int count) {
+    hipStream_t s = nullptr;
+    hipError_t e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);  // its own: the null stream may have a queue of work
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(zero_ints_kernel, dim3((count + 255) / 256), dim3(256), 0, s, p, count);
+    e = hipGetLastError();
+    const hipError_t waited = hipStreamSynchronize(s);
+    (void)hipStreamDestroy(s);
+    return e != hipSuccess ? e : waited;
+}
+
 // caller holds g_mutex
 static int grow_pool(DeviceState& d) {
     Workspace w;
     HFRK_HIP_TRY(hipMalloc(&w.ws, kWsFloats * sizeof(float)));
     hipError_t e = hipMalloc(&w.counters, kMaxPanels * sizeof(int));
-    if (e == hipSuccess) e = hipMemset(w.counters, 0, kMaxPanels * sizeof(int));
+    if (e == hipSuccess) e = zero_and_wait(w.counters, kMaxPanels);
     if (e != hipSuccess) {
         (void)hipFree(w.ws);
         if (w.counters) (void)hipFree(w.counters);

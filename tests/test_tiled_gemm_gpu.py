@@ -287,3 +287,44 @@ def test_linear_layers_under_the_librarys_plan_match_the_oracle(m, n, k):
         check = oracle_checker(a, w.t(), sa, sw, torch.bfloat16, base=base)
         for weight in [dev[1]] + ([pack_weight(dev[1])] if k % 256 == 0 else []):
             check(apply_fp8_linear(dev[0], weight, dev[3], dev[2], **add))
+
+
+# A process of its own: every stream takes a workspace.
+_NEW_STREAMS = """
+import ctypes, torch
+from hf_rocm_kernels import _capi
+lib = _capi.load()
+torch.manual_seed(0)
+m, n, k = 130, 520, 4096
+a, w = (torch.randn(r, k, device="cuda").to(torch.float8_e4m3fn) for r in (m, n))
+one = torch.full((1,), 1e-2, device="cuda")
+hip = ctypes.CDLL(next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line))
+
+def tiled(out, stream):
+    plan = ctypes.byref(_capi.TiledPlan(4, 6, 1))
+    return lib.hfrk_tiled_gemm(a.data_ptr(), w.data_ptr(), 0, out.data_ptr(), None, 0, one.data_ptr(), 0, None, 0, m, n, k, k, _capi.BF16, plan, stream)
+
+def skinny(out, stream):  # 64 columns: k is split between workgroups
+    return lib.hfrk_skinny_gemm_fused(a.data_ptr(), w.data_ptr(), out.data_ptr(), None, one.data_ptr(), 0, None, 0, None, 64, 64, k, k, _capi.BF16, 0, None, stream)
+
+def outputs():
+    return [torch.full((m, n), 7.0, dtype=torch.bfloat16, device="cuda"), torch.full((64, 64), 7.0, dtype=torch.bfloat16, device="cuda")]
+
+want = outputs()
+assert tiled(want[0], None) == skinny(want[1], None) == _capi.SUCCESS
+for i in range(24):
+    stream, got = ctypes.c_void_p(), [outputs() for _ in range(20)]
+    assert hip.hipStreamCreateWithFlags(ctypes.byref(stream), 1) == 0  # 1: does not wait for the null stream
+    torch.cuda.synchronize()
+    torch.cuda._sleep(200000)  # the null stream is busy for about 0.1 ms when the workspace is made, so that clearing ends between launches
+    for pair in got:
+        assert tiled(pair[0], stream) == skinny(pair[1], stream) == _capi.SUCCESS
+    torch.cuda.synchronize()
+    for turn, pair in enumerate(got):
+        assert all(torch.equal(g, x) for g, x in zip(pair, want)), (i, turn)
+"""
+
+
+def test_the_first_calls_on_a_new_stream():
+    env = dict(os.environ, PYTHONPATH=os.pathsep.join(p for p in sys.path if p))
+    subprocess.run([sys.executable, "-c", _NEW_STREAMS], check=True, timeout=100, env=env)

@@ -12,6 +12,8 @@ _STAND_IN = r"""
 #include <stdint.h>
 typedef struct { uint32_t x, y, z; } dim3_;
 static int allocations, capturing, last_error;
+static int clearing, early;          // memory is being cleared by work that nobody has waited for; a launch met it so
+static char own_stream;
 static uint32_t grid;
 static uintptr_t next_block = 1 << 20;
 void stand_in(int allocs, int capture) { allocations = allocs; capturing = capture; grid = 0; }
@@ -20,14 +22,24 @@ static int fail(int e) { return last_error = e; }
 int hipGetDevice(int* d) { *d = 0; return 0; }
 int hipMalloc(void** p, size_t n) { if (allocations-- <= 0) return fail(2); *p = (void*)next_block; next_block += (n + 4095) & ~(size_t)4095; return 0; }
 int hipFree(void* p) { return 0; }
-int hipMemset(void* p, int v, size_t n) { return 0; }
+int hipMemset(void* p, int v, size_t n) { clearing = 1; return 0; }  /* does not wait for the device */
+int hipStreamCreateWithFlags(void** s, unsigned flags) { *s = &own_stream; return 0; }
+int hipStreamDestroy(void* s) { return 0; }
+int hipStreamSynchronize(void* s) { clearing = 0; return 0; }
+int hipDeviceSynchronize(void) { clearing = 0; return 0; }
+int stand_in_early(void) { return early; }
 int hipStreamIsCapturing(void* s, int* state) { *state = capturing; return 0; }
 int hipFuncSetAttribute(const void* f, int a, int v) { return 0; }
 int hipGetLastError(void) { int e = last_error; last_error = 0; return e; }
 static dim3_ g, b; static size_t l; static void* s;
 int __hipPushCallConfiguration(dim3_ grid_, dim3_ block_, size_t lds, void* stream) { g = grid_; b = block_; l = lds; s = stream; return 0; }
 int __hipPopCallConfiguration(dim3_* grid_, dim3_* block_, size_t* lds, void** stream) { *grid_ = g; *block_ = b; *lds = l; *stream = s; return 0; }
-int hipLaunchKernel(const void* f, dim3_ grid_, dim3_ block_, void** args, size_t lds, void* stream) { grid = grid_.x; return 0; }
+int hipLaunchKernel(const void* f, dim3_ grid_, dim3_ block_, void** args, size_t lds, void* stream) {
+    grid = grid_.x;
+    if (stream == &own_stream) clearing = 1;
+    else if (clearing) early = 1;
+    return 0;
+}
 """
 
 # m = 65: one row of 64 x 64 tiles more than the skinny kernels take, k long enough to be split
@@ -76,6 +88,12 @@ stand_in.stand_in(0, 1)
 for stream in (2, 3, 4):  # three more workspaces came with the first
     assert tiled(stream) == _capi.SUCCESS and stand_in.stand_in_grid() == split_grid
 assert tiled(5) == _capi.SUCCESS and 0 < stand_in.stand_in_grid() <= 2
+""",
+    "counters are clear before the first launch": """
+stand_in.stand_in(100, 0)
+for stream in range(1, 8):  # four workspaces at once, then one by one
+    assert tiled(stream) == skinny(stream) == _capi.SUCCESS and stand_in.stand_in_grid() > 0
+assert not stand_in.stand_in_early()
 """,
     "a split that was asked for": """
 stand_in.stand_in(0, 0)
