@@ -795,7 +795,6 @@ static int gemm_launch(const void* A, const void* B, void* D, const void* base, 
     args.D = D;
     args.base = base;
     args.base_stride = base_row ? 0 : n;
-    args.base_rows = base_row ? 0u : ~0u;
     args.out_scale = out_scale;
     args.scale_a = scale_a;
     args.scale_b = scale_b;

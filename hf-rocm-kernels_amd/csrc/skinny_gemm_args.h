@@ -26,7 +26,6 @@ struct GemmArgs {
     void* D;
     const void* base;        // accumulate mode: the 16-bit [m,n] tensor added to the product (may be D itself); else null
     int base_stride;         // elements between rows of base: n, or 0 for one row added to every row (a bias)
-    uint32_t base_rows;      // the same as a mask of what row i contributes to an offset, i * n: all ones, or 0
     const float* out_scale;  // SwiGLU epilogue: the fp8 output is divided by out_scale[0]
     const float* scale_a;
     const float* scale_b;

@@ -20,7 +20,8 @@ __device__ __forceinline__ uint32_t pack16(float lo, float hi, bool bf16) {
 }
 
 // MT = 16-row activation tiles, RT = 16-row weight tiles per chunk.
-template <int MT, int RT, bool SWIGLU>
+// BASE_ROW: the addend is one row of n values, added to every row (a bias).
+template <int MT, int RT, bool SWIGLU, bool BASE_ROW>
 struct RowsEpilogue {
     static constexpr uint32_t kOutOfRange = 0x80000000u;
     // Old D values (accumulate mode) and per-channel scales of one tile, requested ahead of the epilogue that uses them
@@ -37,7 +38,7 @@ struct RowsEpilogue {
     __device__ __forceinline__ RowsEpilogue(const GemmArgs& args, int lane) : a(args), li(lane & 15), lg(lane >> 4) {
         n_out = SWIGLU ? (a.n >> 1) : a.n;
         d_rsrc = make_rsrc(a.D, (uint32_t)a.m * (uint32_t)n_out * (SWIGLU ? 1u : 2u));
-        base_rsrc = make_rsrc(a.base, a.base ? ((((uint32_t)(a.m - 1) * (uint32_t)a.n) & a.base_rows) + (uint32_t)a.n) * 2u : 0u);
+        base_rsrc = make_rsrc(a.base, a.base ? (BASE_ROW ? 1u : (uint32_t)a.m) * (uint32_t)a.n * 2u : 0u);
         sb_rsrc = make_rsrc(a.scale_b, a.scale_b ? (uint32_t)a.n * 4u : 0u);
         accumulate = !SWIGLU && a.base != nullptr;
         vec = SWIGLU || (a.n & 3) == 0;  // then a lane's four outputs are all inside n and aligned
@@ -54,15 +55,11 @@ struct RowsEpilogue {
         }
     }
 
-    // Offsets into the addend are D's with the row's part masked away where it is one row: one product per row for both.  A product with
-    // the addend's own stride took four more registers through the weight loop, and from 25 rows on the kernel has none left: it kept
-    // 20 bytes in scratch (bfloat16, 2440 x 4352 at 26 rows 8.7 us, 2584 x 5376 at 31 rows 9.2, 5376 x 7936 with a residual at 26 rows
-    // 13.1; now 8.1, 8.65 and 12.6).  The mask is opaque, or the masked product would be kept as well.
-    __device__ __forceinline__ uint32_t base_rows() const {
-        uint32_t mask = a.base_rows;
-        asm volatile("" : "+s"(mask));
-        return mask;
-    }
+    // The row's part of an offset into the addend: D's own, or nothing.  Two instances, because offsets of the addend's own took up to eight
+    // more registers through the weight loop: from 25 rows on the kernel has none left and kept 20 bytes in scratch (bfloat16, 2440 x 4352 at
+    // 26 rows 8.35 -> 8.75 us, 2584 x 5376 at 31 rows 8.8 -> 9.2), and in one product with a mask on the row's part it was 2 % slower still
+    // on some weights (5392 x 6144 at 18 rows 9.8 -> 10.1, 11136 x 6144 packed at 16 rows 14.2 -> 14.45).
+    __device__ __forceinline__ uint32_t base_row(uint32_t row) const { return BASE_ROW ? 0u : row * (uint32_t)a.n; }
 
     // Old D values and per-channel scales of a tile whose first row is `row0` and that holds `units` 4-row units (aligned n
     // only; ragged n fetches in the epilogue).  Nothing is requested when nothing is wanted.
@@ -73,7 +70,6 @@ struct RowsEpilogue {
 #pragma unroll
         for (int u = 0; u < MT * RT; ++u) p.d[u] = v2i{0, 0};
         if (wanted && want_pre) {
-            const uint32_t rows = base_rows();
 #pragma unroll
             for (int rt = 0; rt < RT; ++rt) {
                 const int ul = SWIGLU ? lg : 4 * rt + lg;                        // this lane's unit of the tile
@@ -82,7 +78,7 @@ struct RowsEpilogue {
                 p.sb[rt] = __builtin_amdgcn_raw_buffer_load_b128(sb_rsrc, (per_channel && ok) ? n0 * 4 : (int)kOutOfRange, 0, 0);
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt)
-                    p.d[mt * RT + rt] = __builtin_amdgcn_raw_buffer_load_b64(base_rsrc, (accumulate && ok && 16 * mt + li < a.m) ? (int)(((((uint32_t)(16 * mt + li) * (uint32_t)a.n) & rows) + (uint32_t)n0) * 2u) : (int)kOutOfRange, 0, 0);
+                    p.d[mt * RT + rt] = __builtin_amdgcn_raw_buffer_load_b64(base_rsrc, (accumulate && ok && 16 * mt + li < a.m) ? (int)((base_row((uint32_t)(16 * mt + li)) + (uint32_t)n0) * 2u) : (int)kOutOfRange, 0, 0);
             }
         }
         return p;
@@ -142,12 +138,11 @@ struct RowsEpilogue {
                 const v2i packed = {(int)pack16(r[0], r[1], bf16), (int)pack16(r[2], r[3], bf16)};
                 __builtin_amdgcn_raw_buffer_store_b64(packed, d_rsrc, live ? (int)d_off : (int)kOutOfRange, 0, 0);
             } else {
-                const uint32_t rows = base_rows();
                 // ragged n: 2-byte accesses whose out-of-range offsets mask the columns beyond n
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
                     const uint32_t off = (live && n0 + v < a.n) ? d_off + 2u * v : kOutOfRange;
-                    const uint32_t base_off = off == kOutOfRange ? off : ((((uint32_t)arow * (uint32_t)a.n) & rows) + (uint32_t)(n0 + v)) * 2u;
+                    const uint32_t base_off = !BASE_ROW || off == kOutOfRange ? off : (uint32_t)(n0 + v) * 2u;
                     const uint32_t old = accumulate ? (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(base_rsrc, (int)base_off, 0, 0) : 0u;
                     const float sbv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sb_rsrc, (live && per_channel && n0 + v < a.n) ? (n0 + v) * 4 : (int)kOutOfRange, 0, 0));
                     float r = acc[u][v] * (per_channel ? sa * sbv : sa);

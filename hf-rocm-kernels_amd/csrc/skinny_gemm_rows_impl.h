@@ -53,6 +53,7 @@ namespace hfrk {
 // sums are added in the stand-alone kernel's order, and both use the same per-piece functions: the activations are
 // bit-identical to residual_rms's.  Workgroup r stores row r of the summed residual (to a buffer of its own: every
 // workgroup reads the old residual, so it cannot be updated in place).  k = 4096 or 8192, up to 8 rows.
+// BASE_ROW: the addend is one row for every row of D (a bias).
 // LAYOUT: how the weight rows are dealt out and read.
 //   kRowsUnits   row-major weights, bands of any number of 4-row units, cut into tiles of nearly equal height (above).
 //   kRowsTiles   row-major weights, bands of whole 16-row tiles: `rows_q` / `rows_r` count tiles, and a band is cut into
@@ -62,7 +63,7 @@ namespace hfrk {
 //                whose registers are the operands, no pass through LDS for the weights.  Chunk sequence, runs per wave,
 //                operands and order of every sum are those of kRowsTiles: the two give the same bits.
 enum { kRowsUnits = 0, kRowsTiles = 1, kRowsPacked = 2 };
-template <int MA, int RT, bool SWIGLU, bool RMS, int LAYOUT = kRowsUnits>
+template <int MA, int RT, bool SWIGLU, bool RMS, int LAYOUT, bool BASE_ROW>
 __global__ void __launch_bounds__(kGemmThreads) skinny_gemm_rows_kernel(const GemmArgs a) {
     constexpr bool TILED = LAYOUT != kRowsUnits, PACKED = LAYOUT == kRowsPacked;
     static_assert(!(TILED && RMS), "the RMSNorm prologue exists for row-major weights dealt out in 4-row units");
@@ -174,9 +175,9 @@ __global__ void __launch_bounds__(kGemmThreads) skinny_gemm_rows_kernel(const Ge
 
     // ---- the rest of the set-up, while the first chunk is on its way -------------------------------------------------
     // everything the end of the kernel needs to turn a sum into output: buffer resources, scales, dtype (skinny_gemm_rows_epilogue.h)
-    const RowsEpilogue<MT, RT, SWIGLU> epi(a, lane);
-    using Pre = typename RowsEpilogue<MT, RT, SWIGLU>::Pre;
-    requests_end();
+    const RowsEpilogue<MT, RT, SWIGLU, BASE_ROW> epi(a, lane);
+    using Pre = typename RowsEpilogue<MT, RT, SWIGLU, BASE_ROW>::Pre;
+    if constexpr (SWIGLU || BASE_ROW) requests_end();  // (in the other instances the loads stay by themselves)
 
     uint8_t* const tw = lds + wv * kWaveLds;  // this wave's RT weight tiles, then its activation tile(s)
     uint8_t* const ta = tw + RT * kTileBytes;
@@ -424,9 +425,9 @@ __global__ void __launch_bounds__(kGemmThreads) skinny_gemm_rows_kernel(const Ge
     epilogue(row0_l, units_l, acc, pre_l);
 }
 
-template <int MA, int RT, bool SWIGLU, bool RMS, int LAYOUT = kRowsUnits>
-static int launch_rows_one(const GemmArgs& args, int lds_bytes, hipStream_t stream) {
-    auto kern = skinny_gemm_rows_kernel<MA, RT, SWIGLU, RMS, LAYOUT>;
+template <int MA, int RT, bool SWIGLU, bool RMS, int LAYOUT, bool BASE_ROW>
+static int launch_rows_instance(const GemmArgs& args, int lds_bytes, hipStream_t stream) {
+    auto kern = skinny_gemm_rows_kernel<MA, RT, SWIGLU, RMS, LAYOUT, BASE_ROW>;
     static bool attr_done[kMaxDevices] = {};
     int dev = 0;
     HFRK_HIP_TRY(hipGetDevice(&dev));
@@ -437,6 +438,14 @@ static int launch_rows_one(const GemmArgs& args, int lds_bytes, hipStream_t stre
     hipLaunchKernelGGL(kern, dim3(args.grid), dim3(kGemmThreads), lds_bytes, stream, args);
     HFRK_HIP_TRY(hipGetLastError());
     return HFRK_SUCCESS;
+}
+
+template <int MA, int RT, bool SWIGLU, bool RMS, int LAYOUT = kRowsUnits>
+static int launch_rows_one(const GemmArgs& args, int lds_bytes, hipStream_t stream) {
+    if constexpr (!SWIGLU && !RMS) {
+        if (args.base && args.base_stride == 0) return launch_rows_instance<MA, RT, SWIGLU, RMS, LAYOUT, true>(args, lds_bytes, stream);
+    }
+    return launch_rows_instance<MA, RT, SWIGLU, RMS, LAYOUT, false>(args, lds_bytes, stream);
 }
 
 }  // namespace hfrk
