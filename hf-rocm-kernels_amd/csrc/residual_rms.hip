@@ -19,11 +19,12 @@ namespace hfrk {
 constexpr int kRmsMaxThreads = 1024;
 
 // From this many values on the input is read past the caches, which leaves their room (256 MB behind the L2s) to the residual, the weight
-// and the output.  Measured with both reads on fp16, us, kept / past.  Buffers used again and again: 2048 x 4096 10.2 / 11.2,
-// 2048 x 8192 18.3 / 19.7, 1536 x 16384 30.4 / 28.6, 2048 x 16384 43.2 / 37.9, 4096 x 16384 83.2 / 80.3.  With a kernel in front that
-// has just written the input, both: 2048 x 8192 30.9 / 31.5, 1536 x 16384 44.6 / 44.8, 4096 x 8192 66.2 / 59.0, 4096 x 16384 128.5 / 125.0.
-// At decode sizes reading past them cost an eager MLP block of 1 to 16 rows of 4096 0.4 us of 32.
-constexpr long kReadOnceFrom = 20L << 20;
+// and the output.  Measured with both reads on fp16, us, kept / past.  Calls on buffers that change: 2048 x 4096 10.2 / 11.2,
+// 2048 x 8192 18.3 / 19.7, 1536 x 16384 30.4 / 28.6, 1792 x 16384 36.9 / 33.4, 2048 x 16384 43.2 / 37.9, 4096 x 16384 83.2 / 80.3.  With a
+// kernel in front that has just written the input, both: 2048 x 8192 30.9 / 31.5, 1536 x 16384 44.6 / 44.8, 4096 x 8192 66.2 / 59.0,
+// 4096 x 16384 128.5 / 125.0.  One set of buffers again and again, nothing else between: 1965 x 11328 25.1 / 27.7, 2048 x 16384 35.5 / 38.5,
+// 4096 x 16384 72.1 / 72.4.  At decode sizes reading past them cost an eager MLP block of 1 to 16 rows of 4096 0.4 us of 32.
+constexpr long kReadOnceFrom = 28L << 20;
 
 __device__ __forceinline__ void zero_next_buffer_row(uint16_t* next_buffer, int buffer_cols) {
     if (buffer_cols <= 0) return;

@@ -438,9 +438,9 @@ def test_traced_mlp_block_equals_the_eager_block(fused):
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("fp8", [True, False])
-@pytest.mark.parametrize("rows,cols", [(1280, 16384), (5120, 4096), (2561, 8192)])
+@pytest.mark.parametrize("rows,cols", [(1792, 16384), (7168, 4096), (3585, 8192)])
 def test_large_inputs_give_the_bits_of_their_halves(rows, cols, fp8, dtype):
-    """From 20 Mi values on the input is read past the caches; its halves are not.  Rows are independent."""
+    """From 28 Mi values on the input is read past the caches; its halves are not.  Rows are independent."""
     from hf_rocm_kernels import residual_rms
     g = torch.Generator(device="cuda").manual_seed(rows)
     x, res = (torch.randn(rows, cols, device="cuda", generator=g).to(dtype) for _ in range(2))
