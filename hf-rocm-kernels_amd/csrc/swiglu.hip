@@ -28,16 +28,23 @@ constexpr int kSwigluPieces = 2;
 
 // Bound by memory.  A thread requests all its pieces before it works on the first, and each further set behind them.  INDEX is
 // 32 bits wide wherever the pieces can be counted in it: the division by the row length is per piece, and in 64 bits it was most
-// of the kernel's instructions.  2048 x 6656 fp16: 14.1 -> 11.9 us.
-template <int DT, typename INDEX>
+// of the kernel's instructions.  fp16, us, before both / now: 2048 x 6656 13.8 / 12.6, the same buffers again and again (136 MB, in the
+// caches) 12.3 / 11.05; 256 x 14336 4.9 / 4.6.
+// TOGETHER: a workgroup's pieces follow one another; otherwise a thread's are a whole launch apart.  Apart is faster up to about 3.5
+// million pieces (2048 x 6656 12.3 / 12.6 together, 1228 x 8384 9.25 / 9.55), together from 4 million on (kTogetherFrom: 4096 x 8192
+// 28.9 / 28.5, 3408 x 14520 40.6 / 39.7, and 4007 x 8272, where the two halves fall on the same channels, 31.7 / 29.5).
+constexpr long kTogetherFrom = 4000000;
+
+template <int DT, typename INDEX, bool TOGETHER>
 __global__ void __launch_bounds__(1024) swiglu_vec_kernel(const uint16_t* __restrict__ gate_up,
                                                           const float* __restrict__ scale_tensor,
                                                           uint8_t* __restrict__ output, uint16_t* __restrict__ next_buffer,
                                                           int rows, int cols, int buffer_cols) {
     const INDEX vpr = (INDEX)(cols >> 3);  // 8-element pieces per output row
     const INDEX nvec = (INDEX)rows * vpr;
-    const INDEX stride = (INDEX)gridDim.x * blockDim.x;
-    const INDEX first = (INDEX)blockIdx.x * blockDim.x + threadIdx.x;
+    const INDEX launch = (INDEX)gridDim.x * blockDim.x;
+    const INDEX stride = TOGETHER ? (INDEX)blockDim.x : launch;  // between a thread's pieces
+    const INDEX first = (INDEX)blockIdx.x * (TOGETHER ? kSwigluPieces : 1) * blockDim.x + threadIdx.x;
     v4i g[kSwigluPieces], u[kSwigluPieces];
     auto fetch = [&](INDEX at) __attribute__((always_inline)) {
 #pragma unroll
@@ -54,7 +61,7 @@ __global__ void __launch_bounds__(1024) swiglu_vec_kernel(const uint16_t* __rest
     fetch(first);
     const float s = scale_tensor[0];
     const float inv_scale = (s != 0.f) ? 1.f / s : 1.f;
-    for (INDEX at = first; at < nvec; at += kSwigluPieces * stride) {
+    for (INDEX at = first; at < nvec; at += kSwigluPieces * launch) {
         if (at != first) fetch(at);
 #pragma unroll
         for (int p = 0; p < kSwigluPieces; ++p) {
@@ -126,15 +133,20 @@ extern "C" int hfrk_swiglu(const void* gate_up, const float* scale_tensor, void*
     const bool narrow = work + 2L * kSwigluPieces * blocks * threads < (1L << 32);
 #define HFRK_SWIGLU(KERNEL) \
     hipLaunchKernelGGL((KERNEL), dim3((unsigned)blocks), dim3(threads), 0, s, in, scale_tensor, out, nb, rows, cols, buffer_cols)
+#define HFRK_SWIGLU_VEC(DT_)                                                        \
+    do {                                                                            \
+        if (!narrow) HFRK_SWIGLU((swiglu_vec_kernel<DT_, uint64_t, true>));         \
+        else if (work >= kTogetherFrom) HFRK_SWIGLU((swiglu_vec_kernel<DT_, uint32_t, true>)); \
+        else HFRK_SWIGLU((swiglu_vec_kernel<DT_, uint32_t, false>));                \
+    } while (0)
     if (io_dtype == HFRK_F16) {
         if (!vec) HFRK_SWIGLU(swiglu_scalar_kernel<HFRK_F16>);
-        else if (narrow) HFRK_SWIGLU((swiglu_vec_kernel<HFRK_F16, uint32_t>));
-        else HFRK_SWIGLU((swiglu_vec_kernel<HFRK_F16, uint64_t>));
+        else HFRK_SWIGLU_VEC(HFRK_F16);
     } else {
         if (!vec) HFRK_SWIGLU(swiglu_scalar_kernel<HFRK_BF16>);
-        else if (narrow) HFRK_SWIGLU((swiglu_vec_kernel<HFRK_BF16, uint32_t>));
-        else HFRK_SWIGLU((swiglu_vec_kernel<HFRK_BF16, uint64_t>));
+        else HFRK_SWIGLU_VEC(HFRK_BF16);
     }
+#undef HFRK_SWIGLU_VEC
 #undef HFRK_SWIGLU
     HFRK_HIP_TRY(hipGetLastError());
     return HFRK_SUCCESS;

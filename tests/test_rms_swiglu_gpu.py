@@ -451,3 +451,19 @@ def test_large_inputs_give_the_bits_of_their_halves(rows, cols, fp8, dtype):
     for part in (slice(0, half), slice(half, rows)):
         out, sum_ = residual_rms(x[part], res[part].clone(), w, 1e-5, scale)
         assert torch.equal(whole[part].view(torch.uint8), out.view(torch.uint8)) and torch.equal(sums[part], sum_)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("num_threads", [0, 192, 1024])
+@pytest.mark.parametrize("rows,cols", [(4007, 8272), (3909, 8192), (2001, 16384)])
+def test_large_swiglu_gives_the_bits_of_its_halves(rows, cols, num_threads, dtype):
+    """From 4 million pieces of 8 values on a workgroup's pieces follow one another; those of the halves are a launch apart."""
+    from hf_rocm_kernels import swiglu
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    gate_up = torch.randn(rows, 2 * cols, device="cuda", generator=g).to(dtype)
+    scale = torch.tensor([8.0 / 448], device="cuda")
+    whole = swiglu(gate_up, scale, num_threads=num_threads)
+    half = rows // 2
+    for part in (slice(0, half), slice(half, rows)):
+        assert torch.equal(whole[part].view(torch.uint8), swiglu(gate_up[part], scale).view(torch.uint8))
