@@ -1017,9 +1017,12 @@ int hfrk_skinny_gemm_fused(const void* A, const void* B, void* D, const void* ba
 
 int hfrk_linear_gemm(const void* A, const void* B, int packed, void* D, const void* base, int base_stride, const float* scale_a,
                      int sa_stride, const float* scale_b, int sb_stride, int m, int n, int k, int b_stride, int d_dtype, void* stream) {
-    // A k that ends inside a 256-byte chunk is handled by the skinny kernels for up to 32 rows; 33..64 rows were two launches over the
-    // same weight.  Measured, skinny / tiled: 4104 x 1936 at 33 rows 13.7 / 9.4 us, at 64 rows 15.9 / 10.3.  With whole chunks the
-    // skinny kernels stay, as on few columns of a very long k (1024 x 28656 at 33 rows 24.3 / 26.6; 2056 x 16400 28.2 / 19.0): one launch, and 4096 x 4096 at 64 rows 8.5 / 10.7, 28672 x 4096 25.0 / 31.8.
+    // Which kernel takes a call; fp8_linear.py's general path asks the same question.  Above 64 rows the tiled GEMM.  At 33..64 rows the
+    // skinny kernels take a k of whole 256-byte chunks in one launch and are faster on 108 of 120 measured points (at 64 rows 4096 x 4096
+    // 8.5 us skinny, 10.7 tiled; 28672 x 4096 25.0 / 31.8), but a k that ends inside a chunk in two launches over the same weight: there
+    // the tiled GEMM (4104 x 1936 at 33 rows 13.7 / 9.4, at 64 rows 15.9 / 10.3; 2056 x 16400 at 33 rows 28.2 / 19.0), except on few
+    // columns of a very long k, where its at most 4 splits leave it too few workgroups (1024 x 28656 at 33 rows 24.3 / 26.6).  The line
+    // k = 16 n stands between the last two.
     if ((m > HFRK_GEMM_MAX_M || (m > hfrk::kStreamMaxM && k % 256 != 0 && k <= 16L * n)) && hfrk::tiled_size_ok(m, n, k) && (packed || b_stride <= (1 << 21)))
         return hfrk_tiled_gemm(A, B, packed, D, base, base_stride, scale_a, sa_stride, scale_b, sb_stride, m, n, k, b_stride, d_dtype, nullptr, stream);
     if (base && base_stride != 0 && base_stride != n) return HFRK_BAD_SHAPE;

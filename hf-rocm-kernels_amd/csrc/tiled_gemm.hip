@@ -28,8 +28,9 @@ static int check_tiled_plan(int m, int n, int k, const hfrk_tiled_plan& p) {
 }
 
 // The shape and the number of k splits with the smallest predicted time, in us.  The constants are a least-squares fit of this very
-// expression to 4100 measured calls (11 weights from 1024 x 4096 to 8192 x 28672, 15 row counts from 65 to 4096, every shape and
-// 1..8 splits); over those 158 sizes the choice is 1.4 % slower than the best measured plan in the geometric mean, 10 % or more on 6.
+// expression to measured calls whose data was not kept.  Checked against a later sweep that was (profiles/tiled_gemm_plans.csv: 164 sizes,
+// 3543 calls, row-major weights out of the caches): the choice is 2.2 % slower than the best measured plan in the geometric mean, 10 % or
+// more on 13 sizes, most of them large weights at few rows that a split would serve better (8192 x 28672 at 128 rows 77 against 58 us).
 static float tiled_cost(int m, int n, int k, int shape, int splits) {
     struct Shape { float fixed, stage; };  // a workgroup's prologue and epilogue; one stage of 128 bytes of k on an idle chip
     static constexpr Shape kShape[kTiledShapeCount] = {{13.6f, 1.31f}, {7.9f, .67f}, {4.8f, .40f}, {1.4f, .32f}, {2.0f, .225f}};

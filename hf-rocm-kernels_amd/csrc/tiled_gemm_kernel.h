@@ -3,16 +3,19 @@
 // No counterpart in the reference, whose kernel stops at 32 rows (skinny_gemm_caller.cu:33-60); the linear layer ran such calls
 // as one skinny launch per 64 rows, each of which streamed the whole weight again.
 //
-//  * Bound: the matrix cores on the large tiles (v_mfma_f32_32x32x64_f8f6f4, 64 cycles each), L2 -> LDS traffic on the small
-//    ones.  A workgroup is four waves, one per SIMD; a wave owns TM x TN matrix tiles of 32 x 32.  On the largest tile
-//    (256 x 256, 128 x 128 per wave) an operand byte read from LDS feeds 128 multiply-adds, so the LDS pipe is half busy when the
-//    matrix cores are fully busy; accumulators fill the 256 accumulation registers, operands are double buffered in the others.
+//  * A workgroup is four waves, one per SIMD; a wave owns TM x TN matrix tiles of 32 x 32 (v_mfma_f32_32x32x64_f8f6f4, 64 cycles each).  On
+//    the largest tile (256 x 256, 128 x 128 per wave) an operand byte read from LDS feeds 128 multiply-adds; accumulators fill the
+//    256 accumulation registers, operands are double buffered in the others.
+//  * Bound (counters in profiles/tiled_gemm_counters_and_plans.txt, shares of the cycles in which a compute unit has work): 4096 x 28672 x
+//    4096 matrix cores 62 %, at the clock their power leaves, LDS 19 %; 512 x 4096 x 14336 packed 45 and 34 %; 201 x 6144 x 4096
+//    28 and 23 %.  On the small tiles neither is half busy: what remains is prologue, epilogue and the latency of each stage.
 //  * Operands go from memory to LDS without passing registers (buffer_load_dwordx4 ... lds), NST stages of 128 bytes of k deep, the
 //    stage NST ahead being requested behind the barrier that frees its slot.  One barrier per stage: a wave reads the operands of
 //    k step s + 1 (64 bytes) while it multiplies those of step s, so nothing in a step waits for LDS but its first instruction.
 //  * Such a load fills LDS in lane order, so the swizzle that keeps operand reads free of bank conflicts is applied to the memory
 //    side: the lane that fills slot c of row r fetches piece c ^ f(r) of that row (a permutation within one 128-byte line).
-//    Measured conflicts: none (SQ_LDS_BANK_CONFLICT = 0).  A packed weight is fetched as 512-byte runs into the same kind of layout.
+//    Measured conflicts: none on the 256 x 256 tile, 1 - 2 % of the LDS cycles on the smaller ones.  A packed weight is fetched as
+//    512-byte runs into the same kind of layout; its operand reads do conflict (128 x 128: a third of the LDS cycles).
 //  * Rows and columns past the edge, and the part of the last stage past k, are outside the buffers' ranges and read as zero.
 //  * Weights are the matrix instruction's A operand with their rows permuted so that a lane's 16 results of a tile are consecutive
 //    columns; results go through LDS in fp32 and leave as whole rows, scaled, added to their addend and rounded once.

@@ -6,8 +6,8 @@ usual (input, weight, weight_scale, input_scale, bias) signature, and an nn.Modu
 
 A call runs as one quantisation kernel (skipped when the caller already holds fp8 activations and their scales, e.g. from
 `residual_rms_dynamic` / `swiglu_dynamic`) and one GEMM with the scales, the bias or residual folded into its epilogue: a
-skinny GEMM for decode batches (up to 64 tokens; 32 where k ends inside a 256-byte chunk), the tiled GEMM for everything larger,
-up to whole prompts.
+skinny GEMM for decode batches (up to 64 tokens; 32 where k ends inside a 256-byte chunk and is at most 16 n), the tiled GEMM for
+everything larger, up to whole prompts.
 """
 from typing import Optional, Sequence, Tuple, Union
 
@@ -47,7 +47,7 @@ def apply_fp8_linear(
       its scale(s): one float32 or one per token
     - weight: (n, k) float8_e4m3fn row-major, or its PackedWeight; weight_scale: one float32 or one per output channel,
       or None for a PackedWeight that carries its scales
-    - bias: (n,) in the output dtype; residual: (..., n) in the output dtype, added in the GEMM's epilogue (fp32 sum
+    - bias: (n,) in the output dtype (any shape and dtype that broadcasts to the output is taken); residual: (..., n) in the output dtype, added in the GEMM's epilogue (fp32 sum
       with the product, one rounding).  Given both, the bias is added to the residual first (one 16-bit add).
     - out_dtype: float16/bfloat16; defaults to the input's (bfloat16 for an fp8 input)
     """

@@ -96,7 +96,8 @@ int hfrk_version(void);
  * stream's first launch and kept from then on; launches on different streams are therefore independent of each other,
  * as the reference's are (it needs no workspace: it adds fp16 atomics into the caller's zeroed output,
  * csrc/op_src/skinny_gemm/consumers/mfma_16x16x32_consumer.cu:155-163).
- *   hfrk_init             allocates the first 4 workspaces of the current device.  Idempotent, thread-safe.  The pool
+ *   hfrk_init             allocates the first 4 workspaces of the current device and waits until their counters are clear, as
+ *                         every call does that finds the pool empty.  Idempotent, thread-safe.  The pool
  *                         grows by itself (up to 64) when a fifth stream appears, except while that stream is being
  *                         captured into a graph (no allocation inside a capture): then the call returns
  *                         HFRK_NOT_INITIALISED, so run hfrk_init, and one launch per further stream, before capturing.
@@ -268,9 +269,10 @@ int hfrk_skinny_gemm_packed(const void* A, const void* B_packed, void* D, const 
                             int sa_stride, const float* scale_b, int sb_stride, const float* out_scale, int m, int n,
                             int k, int d_dtype, int epilogue, const hfrk_gemm_plan* plan, void* stream);
 
-/* The linear layer's GEMM for any number of rows, under the library's own plan: a skinny GEMM up to 64 rows (32 where k % 256 != 0),
- * hfrk_tiled_gemm (below, same arguments) above, or one skinny GEMM per 64 rows where a size is beyond the tiled kernel's.  base_stride is 0 (one row of n
- * values added to every row of D: a bias) or, where a skinny GEMM runs, n. */
+/* The linear layer's GEMM for any number of rows, under the library's own plan: hfrk_tiled_gemm (below, same arguments) above 64 rows and at
+ * 33..64 rows where k % 256 != 0 and k <= 16 n; a skinny GEMM otherwise; one skinny GEMM per 64 rows where a size is beyond the tiled
+ * kernel's.  Plan tables apply to skinny GEMMs.  base_stride is 0 (one row of n values added to every row of D: a bias) or, where a
+ * skinny GEMM runs, n. */
 int hfrk_linear_gemm(const void* A, const void* B, int packed, void* D, const void* base, int base_stride, const float* scale_a,
                      int sa_stride, const float* scale_b, int sb_stride, int m, int n, int k, int b_stride, int d_dtype, void* stream);
 
@@ -292,10 +294,12 @@ int hfrk_tiled_gemm_plan(int m, int n, int k, hfrk_tiled_plan* plan);
  *   A  fp8 e4m3fn [m,k] row-major     B  the weight: row-major with row stride b_stride (packed == 0) or the buffer
  *   D  16-bit [m,n] row-major            hfrk_pack_weight wrote (packed == 1, b_stride unused)
  *   base  16-bit addend of D's type or NULL; base_stride elements between its rows, 0: one row for all (a bias)
- * fp32 accumulation, one rounding, bit-reproducible.  k % 16 == 0 (256 for a packed weight); n, k and the strides at most 2^21.
+ * fp32 accumulation, one rounding.  Bit-reproducible under one plan; without a plan the split of k, and with it the order of the sums,
+ * depends on whether the stream has a workspace.  k % 16 == 0 (256 for a packed weight); n, k and the strides at most 2^21, m at most
+ * 2^24, fewer than 2^24 tiles of 64 x 64.
  * A and B 16-byte aligned, b_stride a multiple of 16; D and base may have any alignment, 16 bytes with n % 8 == 0 is the fast one.
- * A plan whose k is split needs the stream's workspace like the skinny GEMMs (see hfrk_init); without a plan and without a
- * workspace k is not split. */
+ * A plan whose k is split needs the stream's workspace like the skinny GEMMs (see hfrk_init); without a plan k is not split where there is
+ * none: the 65th stream, one first met in a capture, or no memory for it. */
 int hfrk_tiled_gemm(const void* A, const void* B, int packed, void* D, const void* base, int base_stride, const float* scale_a,
                     int sa_stride, const float* scale_b, int sb_stride, int m, int n, int k, int b_stride, int d_dtype,
                     const hfrk_tiled_plan* plan, void* stream);
