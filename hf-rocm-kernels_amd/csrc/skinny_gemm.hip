@@ -493,18 +493,13 @@ static uint64_t stream_key(hipStream_t stream) {
     return key;
 }
 
-// The counters are zero before any stream may launch on them.  hipMemset does not do: it returns while the null stream still works (83 ms
-// early behind an 84 ms kernel), and a launch on another stream then counted its arrivals on memory that was cleared under it.  That
-// call's output stayed unwritten, and the counts stayed wrong for every later split on the workspace.
+// The counters are zero before any stream may launch on them.  hipMemset alone does not do: it returns while the null stream still works
+// (83 ms early behind an 84 ms kernel), and a launch on another stream then counted its arrivals on memory that was cleared under it.
+// That call's output stayed unwritten, and the counts stayed wrong for every later split on the workspace.
+// Cleared and waited for on the null stream, once per workspace: no stream, and no hardware queue behind it, is made for it.
 static hipError_t zero_and_wait(int* p, int count) {
-    hipStream_t s = nullptr;
-    hipError_t e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);  // its own: the null stream may have a queue of work
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(zero_ints_kernel, dim3((count + 255) / 256), dim3(256), 0, s, p, count);
-    e = hipGetLastError();
-    const hipError_t waited = hipStreamSynchronize(s);
-    (void)hipStreamDestroy(s);
-    return e != hipSuccess ? e : waited;
+    const hipError_t e = hipMemset(p, 0, count * sizeof(int));
+    return e != hipSuccess ? e : hipStreamSynchronize(nullptr);
 }
 
 // caller holds g_mutex

@@ -25,7 +25,7 @@ int hipFree(void* p) { return 0; }
 int hipMemset(void* p, int v, size_t n) { clearing = 1; return 0; }  /* does not wait for the device */
 int hipStreamCreateWithFlags(void** s, unsigned flags) { *s = &own_stream; return 0; }
 int hipStreamDestroy(void* s) { return 0; }
-int hipStreamSynchronize(void* s) { clearing = 0; return 0; }
+int hipStreamSynchronize(void* s) { if (!s || s == &own_stream) clearing = 0; return 0; }
 int hipDeviceSynchronize(void) { clearing = 0; return 0; }
 int stand_in_early(void) { return early; }
 int hipStreamIsCapturing(void* s, int* state) { *state = capturing; return 0; }
