@@ -28,12 +28,11 @@ struct TiledGemmArgs {
 };
 
 constexpr int kTiledStage = 128;    // bytes of k per pipeline stage
-constexpr int kTiledThreads = 256;  // four waves
 
 // TM x TN matrix tiles of 32 x 32 per wave, WM x WN waves, NST stages of operands in LDS, WGS workgroups per compute unit.
 // X(index, TM, TN, WM, WN, NST, WGS)
 #define HFRK_TILED_SHAPES(X) \
-    X(0, 4, 4, 2, 2, 2, 1)   \
+    X(0, 4, 2, 2, 4, 2, 1)   \
     X(1, 4, 2, 2, 2, 3, 1)   \
     X(2, 2, 2, 2, 2, 5, 1)   \
     X(3, 2, 1, 2, 2, 3, 2)   \

@@ -3,12 +3,17 @@
 // No counterpart in the reference, whose kernel stops at 32 rows (skinny_gemm_caller.cu:33-60); the linear layer ran such calls
 // as one skinny launch per 64 rows, each of which streamed the whole weight again.
 //
-//  * A workgroup is four waves, one per SIMD; a wave owns TM x TN matrix tiles of 32 x 32 (v_mfma_f32_32x32x64_f8f6f4, 64 cycles each).  On
-//    the largest tile (256 x 256, 128 x 128 per wave) an operand byte read from LDS feeds 128 multiply-adds; accumulators fill the
-//    256 accumulation registers, operands are double buffered in the others.
+//  * A wave owns TM x TN matrix tiles of 32 x 32 (v_mfma_f32_32x32x64_f8f6f4, 64 cycles each).  The largest tile (256 x 256) runs on eight
+//    waves of 128 x 64, two per SIMD: with four of 128 x 128 an operand byte read from LDS fed a third more multiply-adds, but nothing ran
+//    while the one wave of a SIMD waited for its stage or stored (4096 x 28672 x 4096 432 -> 409 us, 4096 x 4096 x 4096 62.7 -> 57,
+//    2048 x 6144 x 4096 56 -> 52; 12 % in the mean over 70 weights and rows where tiles are few).  The others have four waves, one per
+//    SIMD: 128 x 128 on eight or sixteen waves takes the same time.
 //  * Bound (counters in profiles/tiled_gemm_counters_and_plans.txt, shares of the cycles in which a compute unit has work): 4096 x 28672 x
 //    4096 matrix cores 62 %, at the clock their power leaves, LDS 19 %; 512 x 4096 x 14336 packed 45 and 34 %; 201 x 6144 x 4096
-//    28 and 23 %.  On the small tiles neither is half busy: what remains is prologue, epilogue and the latency of each stage.
+//    28 and 23 %.  On the small tiles neither is half busy.  (The first of the three before its tile ran on eight waves.)
+//    What bounds the small tiles is what a compute unit can fetch: without matrix instructions and operand reads a launch takes the same
+//    time (201 x 6144 x 4096, 512 x 4096 x 14336), and so it does with 4, 5 or 6 stages in flight.  A unit gets about 75 GB/s, 47 where
+//    nothing it reads is in its L2 yet and 128 - 148 where everything is.
 //  * Operands go from memory to LDS without passing registers (buffer_load_dwordx4 ... lds), NST stages of 128 bytes of k deep, the
 //    stage NST ahead being requested behind the barrier that frees its slot.  One barrier per stage: a wave reads the operands of
 //    k step s + 1 (64 bytes) while it multiplies those of step s, so nothing in a step waits for LDS but its first instruction.
@@ -25,7 +30,7 @@
 //    adds them in split order (bit-reproducible), as in the skinny workgroup kernel.
 //
 // Measured (row-major / packed, us, bf16 out): 4096 x 28672 x 4096 412 / 395 (2.3 / 2.4 PFLOP/s; 1550 as 64 skinny launches; a loop that
-// stays resident clocks at 1.8 - 2.0 GHz, so the matrix cores' power bounds it before their issue rate does), 512 x 4096 x 14336
+// stays resident clocks at 1.8 - 2.0 GHz, so the matrix cores' power bounds it before their issue rate does; on eight waves 409), 512 x 4096 x 14336
 // 38 / 37 (150), 201 x 6144 x 4096 13.2 / 13.1 (46), 65 x 4096 x 4096 10.5 / 9.9 (16).  The epilogue is written with little code on
 // purpose: with a branch per value for NaN and 64-bit addresses it took 18 us of a 256 x 256 tile, now 7.
 #pragma once
@@ -67,12 +72,12 @@ __device__ __forceinline__ uint32_t pack_pair(float lo, float hi) {
 }
 
 template <int TM, int TN, int WM, int WN, int NST, int WGS, bool PACKED>
-__global__ void __launch_bounds__(kTiledThreads, WGS) tiled_gemm_kernel(const TiledGemmArgs a) {
-    static_assert(WM * WN == 4, "a workgroup is 4 waves");
+__global__ void __launch_bounds__(64 * WM * WN, WGS * WM * WN / 4) tiled_gemm_kernel(const TiledGemmArgs a) {
+    constexpr int NW = WM * WN;
     constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN;
     constexpr int KB = kTiledStage;
     constexpr int A_BYTES = BM * KB, B_BYTES = BN * KB, STAGE = A_BYTES + B_BYTES;
-    constexpr int LA = A_BYTES / 4096, LB = B_BYTES / 4096;  // load instructions per wave and stage, 1 KB each
+    constexpr int LA = A_BYTES / (1024 * NW), LB = B_BYTES / (1024 * NW);  // load instructions per wave and stage, 1 KB each
     constexpr int NMMA = TM * TN;
     constexpr int kOutside = 0x7ffffff0;  // beyond any tile's range
 
@@ -117,7 +122,7 @@ __global__ void __launch_bounds__(kTiledThreads, WGS) tiled_gemm_kernel(const Ti
     int pa[LA], pb[LB];  // k byte of the lane's piece within its stage (for the last, partial stage)
 #pragma unroll
     for (int q = 0; q < LA; ++q) {
-        const int row = (q * 4 + wave) * 8 + (lane >> 3);
+        const int row = (q * NW + wave) * 8 + (lane >> 3);
         pa[q] = ((lane & 7) ^ ((row >> 1) & 7)) * 16;
         va[q] = row * a.k + pa[q];
     }
@@ -125,12 +130,12 @@ __global__ void __launch_bounds__(kTiledThreads, WGS) tiled_gemm_kernel(const Ti
     for (int q = 0; q < LB; ++q) {
         if constexpr (PACKED) {
             // LDS block (16-row tile, half of the stage): [piece j][k group][row slot], 1 KB
-            const int blk = q * 4 + wave, t16 = blk >> 1, s = blk & 1, group = (lane >> 4) & 1;
+            const int blk = q * NW + wave, t16 = blk >> 1, s = blk & 1, group = (lane >> 4) & 1;
             const int row = (lane & 15) ^ ((t16 & 1) << 3) ^ group << 2;
             vb[q] = t16 * a.k * 16 + (lane >> 5) * 1024 + s * 512 + group * 256 + row * 16;
             pb[q] = 0;
         } else {
-            const int row = (q * 4 + wave) * 8 + (lane >> 3);
+            const int row = (q * NW + wave) * 8 + (lane >> 3);
             pb[q] = ((lane & 7) ^ (((row >> 1) & 3) | ((row >> 4) & 1) << 2)) * 16;
             vb[q] = row * a.b_stride + pb[q];
         }
@@ -144,12 +149,12 @@ __global__ void __launch_bounds__(kTiledThreads, WGS) tiled_gemm_kernel(const Ti
     auto issue_a = [&](int q) __attribute__((always_inline)) {
         int off = va[q];
         if (issued == tail_stage) off = pa[q] < k_tail ? off : kOutside;
-        load_to_lds(ra, off, lds0 + slot_issue + (uint32_t)(q * 4 + wave) * 1024u);
+        load_to_lds(ra, off, lds0 + slot_issue + (uint32_t)(q * NW + wave) * 1024u);
     };
     auto issue_b = [&](int q) __attribute__((always_inline)) {
         int off = vb[q];
         if (!PACKED && issued == tail_stage) off = pb[q] < k_tail ? off : kOutside;
-        load_to_lds(rb, off, lds0 + slot_issue + A_BYTES + (uint32_t)(q * 4 + wave) * 1024u);
+        load_to_lds(rb, off, lds0 + slot_issue + A_BYTES + (uint32_t)(q * NW + wave) * 1024u);
     };
     auto issue_end = [&]() __attribute__((always_inline)) {
         auto advance = [](v4i& r, uint32_t by) __attribute__((always_inline)) {
@@ -212,10 +217,13 @@ __global__ void __launch_bounds__(kTiledThreads, WGS) tiled_gemm_kernel(const Ti
             issue_begin();
         }
         constexpr int READS = TM + TN, LOADS = S == 1 ? LA + LB : 0;
+        // two stages leave a load one stage to arrive in: there the requests stand in front of the first half of the matrix instructions
+        // (4096 x 4096 x 4096 58.5 -> 56.8 us, 1024 x 8192 x 8192 95 -> 91); deeper pipelines lose up to 4 % by that
+        constexpr int kHaste = NST == 2 ? 2 : 1;
         int reads = 0, loads = 0;
 #pragma unroll
         for (int t = 0; t < NMMA; ++t) {
-            const int reads_to = NMMA <= 2 ? READS : min(READS, (t + 1) * READS * 4 / (3 * NMMA) + 1), loads_to = (t + 1) * LOADS / NMMA;
+            const int reads_to = NMMA <= 2 ? READS : min(READS, (t + 1) * READS * 4 / (3 * NMMA) + 1), loads_to = min(LOADS, (t + 1) * LOADS * kHaste / NMMA);
 #pragma unroll
             for (int r = 0; r < READS; ++r)
                 if (r >= reads && r < reads_to) {
@@ -268,7 +276,7 @@ __global__ void __launch_bounds__(kTiledThreads, WGS) tiled_gemm_kernel(const Ti
         const __amdgpu_buffer_rsrc_t ws = make_rsrc(a.ws, a.ws_bytes);
         constexpr int kCoherent = 17;  // sc0 | sc1: written through to memory, read past the caches (the XCDs' L2s are not coherent)
         auto ws_off = [&](int sp, int t, int p) __attribute__((always_inline)) {
-            return ((((tile * a.splits + sp) * 4 + wave) * NMMA + t) * 4 + p) * 1024 + lane * 16;
+            return ((((tile * a.splits + sp) * NW + wave) * NMMA + t) * 4 + p) * 1024 + lane * 16;
         };
 #pragma unroll
         for (int t = 0; t < NMMA; ++t)
@@ -320,7 +328,7 @@ __global__ void __launch_bounds__(kTiledThreads, WGS) tiled_gemm_kernel(const Ti
     constexpr int RPI = 64 / LPR;          // rows per pass
     constexpr int PASSES = 32 / RPI;
     constexpr int RS = TN * 32 + 4;        // floats between rows: 16 rows of one column lie in different banks
-    static_assert(4 * 32 * RS * 4 <= NST * STAGE, "the staging fits in the operands' LDS");
+    static_assert(NW * 32 * RS * 4 <= NST * STAGE, "the staging fits in the operands' LDS");
     float* const stage = reinterpret_cast<float*>(lds) + wave * (32 * RS);
     const int row0 = wm * TM * 32, col = wn * TN * 32 + (lane % LPR) * 8;
     // buffers over the tile's rows: what lies outside reads as zero and is not stored.  A column past n is marked by bits that no row
@@ -408,7 +416,7 @@ static int launch_tiled_shape(const TiledGemmArgs& args, int lds_bytes, hipStrea
         HFRK_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes));
         if (dev >= 0 && dev < kMaxDevices) attr_done[dev] = true;
     }
-    hipLaunchKernelGGL(kern, dim3(args.tiles_m * args.tiles_n * args.splits), dim3(kTiledThreads), lds_bytes, stream, args);
+    hipLaunchKernelGGL(kern, dim3(args.tiles_m * args.tiles_n * args.splits), dim3(64 * WM * WN), lds_bytes, stream, args);
     HFRK_HIP_TRY(hipGetLastError());
     return HFRK_SUCCESS;
 }

@@ -169,3 +169,46 @@ def test_largest_sizes(m, n, k):
             audit(m, n, k, 1 << 21, forced, False, 1 << 21)
             if k % 256 == 0:
                 audit(m, n, k, k, forced, True, 0)
+
+
+# TM, TN, WM, WN, stages in LDS as the kernel is built: the 256 x 256 tile runs on eight waves
+BUILT = [(4, 2, 2, 4, 2)] + SHAPES[1:]
+
+
+@pytest.mark.parametrize("shape", range(5))
+def test_every_wave_has_its_part_of_the_tile(shape):
+    """The parts that the waves of a workgroup load, multiply, leave as partial sums and store are the whole tile, each once."""
+    TM, TN, WM, WN, NST = BUILT[shape]
+    NW, BM, BN = WM * WN, 32 * TM * WM, 32 * TN * WN
+    assert (BM, BN) == (32 * SHAPES[shape][0] * SHAPES[shape][2], 32 * SHAPES[shape][1] * SHAPES[shape][3])
+    stage = (BM + BN) * KB
+    assert stage * NST <= 160 * 1024 and NW % 4 == 0
+    wave = np.arange(NW)[None, :, None]
+    loads = 0
+    for rows in (BM, BN):  # A and row-major B: 8 rows of 8 pieces a load; packed B: half a 16-row tile's stage
+        per_wave = rows * KB // (1024 * NW)
+        assert per_wave * 1024 * NW == rows * KB
+        loads += per_wave
+        piece = np.arange(per_wave)[:, None, None] * NW + wave
+        assert (np.sort(piece.ravel()) == np.arange(rows // 8)).all()            # KB of LDS it fills
+        row = piece * 8 + (LANE >> 3)
+        for f in ((row >> 1) & 7, ((row >> 1) & 3) | (((row >> 4) & 1) << 2)):
+            assert len(np.unique(row * 8 + ((LANE & 7) ^ f))) == rows * 8
+        t16, half, group = piece >> 1, piece & 1, (LANE >> 4) & 1
+        slot = (LANE & 15) ^ ((t16 & 1) << 3) ^ (group << 2)
+        assert len(np.unique(t16 * 128 + (((LANE >> 5) * 1024 + half * 512 + group * 256 + slot * 16) >> 4))) == rows * 8
+    assert (NST - 1) * loads <= 63                                               # outstanding loads a wait can name
+    # a matrix tile's rows and columns: lane lr of wave (wm, wn)
+    rows = {w // WN * TM * 32 + i * 32 + lr for w in range(NW) for i in range(TM) for lr in range(32)}
+    cols = {w % WN * TN * 32 + j * 32 + c for w in range(NW) for j in range(TN) for c in range(32)}
+    assert rows == set(range(BM)) and cols == set(range(BN))
+    # partial sums of a tile, in KB
+    nmma = TM * TN
+    at = {(w * nmma + t) * 4 + p for w in range(NW) for t in range(nmma) for p in range(4)}
+    assert at == set(range(BM * BN * 4 // 1024))
+    # epilogue: a wave's rows of 32 in LDS, then 8 columns a lane
+    assert NW * 32 * (TN * 32 + 4) * 4 <= stage * NST
+    lpr = 4 * TN
+    out = [(w // WN * TM * 32 + i * 32 + r * (64 // lpr) + lane // lpr, w % WN * TN * 32 + lane % lpr * 8)
+           for w in range(NW) for i in range(TM) for r in range(lpr // 2) for lane in range(64)]
+    assert len(out) == len(set(out)) == BM * BN // 8 and max(out) == (BM - 1, BN - 8)
