@@ -196,4 +196,11 @@ __device__ __forceinline__ void store_fp8_piece(__amdgpu_buffer_rsrc_t row, int 
     __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2i, x), row, v * 8, 0, 0);
 }
 
+// residual <- input + residual_in, output <- e4m3fn(rmsnorm(residual) * weight / scale), and input_copy <- input where it is not null
+// (residual_rms.hip); residual and input_copy may be residual_in and input.  _takes: whether sizes and alignment allow it.
+bool residual_rms_into_takes(const void* input, const void* residual_in, const void* residual, const void* input_copy, const void* weight,
+                             const void* output, int cols);
+int residual_rms_into(const void* input, const void* residual_in, void* residual, void* input_copy, const void* weight, const float* scale_tensor,
+                      float epsilon, void* output, int rows, int cols, int io_dtype, hipStream_t stream);
+
 }  // namespace hfrk

@@ -42,16 +42,18 @@ __device__ __forceinline__ void zero_next_buffer_row(uint16_t* next_buffer, int 
 
 // 8 elements (16 bytes) per thread per iteration, ITERS iterations cached in registers: cols <= 8*blockDim*ITERS.
 // READ_ONCE: the input is read past the caches (kReadOnceFrom).
+// residual_in is residual itself, or another tensor that stays as it is; input_copy, where not null, becomes a copy of the input.  Every
+// thread has read its pieces of the inputs before it writes any, and nobody else's: either may be its own source.
 template <int DT, bool FP8_OUT, int ITERS, bool READ_ONCE>
 __global__ void __launch_bounds__(kRmsMaxThreads) residual_rms_vec_kernel(
-    const uint16_t* __restrict__ input, uint16_t* __restrict__ residual, const uint16_t* __restrict__ weight,
+    const uint16_t* input, const uint16_t* residual_in, uint16_t* residual, uint16_t* input_copy, const uint16_t* __restrict__ weight,
     const float* __restrict__ scale_tensor, void* __restrict__ output, uint16_t* __restrict__ next_buffer,
     float epsilon, int cols, int buffer_cols) {
     __shared__ __align__(16) float red[16];
     const long row_off = (long)blockIdx.x * cols;
     const uint32_t row_bytes = (uint32_t)cols * 2u;
-    const __amdgpu_buffer_rsrc_t rin = make_rsrc(input + row_off, row_bytes), rres = make_rsrc(residual + row_off, row_bytes),
-                                 rweight = make_rsrc(weight, row_bytes);
+    const __amdgpu_buffer_rsrc_t rin = make_rsrc(input + row_off, row_bytes), rres_in = make_rsrc(residual_in + row_off, row_bytes),
+                                 rres = make_rsrc(residual + row_off, row_bytes), rweight = make_rsrc(weight, row_bytes);
     const __amdgpu_buffer_rsrc_t rout = FP8_OUT ? make_rsrc(static_cast<uint8_t*>(output) + row_off, (uint32_t)cols)
                                                 : make_rsrc(static_cast<uint16_t*>(output) + row_off, row_bytes);
     uint4 a[ITERS], z[ITERS], wreg[ITERS];
@@ -63,7 +65,7 @@ __global__ void __launch_bounds__(kRmsMaxThreads) residual_rms_vec_kernel(
     for (int it = 0; it < ITERS; ++it) {
         const int v = threadIdx.x + it * blockDim.x;
         a[it] = load_piece<READ_ONCE>(rin, v);
-        z[it] = load_piece(rres, v);
+        z[it] = load_piece(rres_in, v);
     }
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) wreg[it] = load_piece(rweight, threadIdx.x + it * blockDim.x);
@@ -71,6 +73,11 @@ __global__ void __launch_bounds__(kRmsMaxThreads) residual_rms_vec_kernel(
     for (int it = 0; it < ITERS; ++it) {
         z[it] = rms_add_square<DT>(a[it], z[it], ssq);
         store_piece(rres, threadIdx.x + it * blockDim.x, z[it]);
+    }
+    if (input_copy) {
+        const __amdgpu_buffer_rsrc_t rcopy = make_rsrc(input_copy + row_off, row_bytes);
+#pragma unroll
+        for (int it = 0; it < ITERS; ++it) store_piece(rcopy, threadIdx.x + it * blockDim.x, a[it]);
     }
     const float total = block_sum(ssq, red);
     const float norm = rsqrtf(total / (float)cols + epsilon);
@@ -135,11 +142,13 @@ __global__ void __launch_bounds__(kRmsMaxThreads) residual_rms_scalar_kernel(
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 template <int DT, bool FP8_OUT>
-static int launch_rms(const void* input, void* residual, const void* weight, const float* scale_tensor, float epsilon,
+static int launch_rms(const void* input, const void* residual_in, void* residual, void* input_copy, const void* weight, const float* scale_tensor, float epsilon,
                       void* output, void* next_buffer, int rows, int cols, int buffer_cols, int num_threads,
                       bool force_scalar, hipStream_t stream) {
     const uint16_t* in = static_cast<const uint16_t*>(input);
+    const uint16_t* res_in = static_cast<const uint16_t*>(residual_in);
     uint16_t* res = static_cast<uint16_t*>(residual);
+    uint16_t* copy = static_cast<uint16_t*>(input_copy);
     const uint16_t* w = static_cast<const uint16_t*>(weight);
     uint16_t* nb = static_cast<uint16_t*>(next_buffer);
     // 16-byte path: aligned rows (cols % 8 == 0 keeps every row aligned) and an aligned output row
@@ -159,7 +168,7 @@ static int launch_rms(const void* input, void* residual, const void* weight, con
         if (iters > 4) vec = false;  // would not fit the register cache: fall through to the strided kernel
         else {
 #define HFRK_RMS_LAUNCH(IT, ONCE)                                                                                          \
-    hipLaunchKernelGGL((residual_rms_vec_kernel<DT, FP8_OUT, IT, ONCE>), dim3(rows), dim3(threads), 0, stream, in, res, w, \
+    hipLaunchKernelGGL((residual_rms_vec_kernel<DT, FP8_OUT, IT, ONCE>), dim3(rows), dim3(threads), 0, stream, in, res_in, res, copy, w, \
                        scale_tensor, output, nb, epsilon, cols, buffer_cols)
 #define HFRK_RMS_ITERS(ONCE)                         \
     do {                                             \
@@ -174,6 +183,7 @@ static int launch_rms(const void* input, void* residual, const void* weight, con
         }
     }
     if (!vec) {
+        if (res_in != res || copy) return HFRK_BAD_ALIGNMENT;  // residual_rms_into's callers ask first
         if (threads == 0) {
             threads = ((cols + 63) / 64) * 64;
             if (threads > kRmsMaxThreads) threads = kRmsMaxThreads;
@@ -183,6 +193,19 @@ static int launch_rms(const void* input, void* residual, const void* weight, con
     }
     HFRK_HIP_TRY(hipGetLastError());
     return HFRK_SUCCESS;
+}
+
+bool residual_rms_into_takes(const void* input, const void* residual_in, const void* residual, const void* input_copy, const void* weight, const void* output,
+                             int cols) {
+    return cols % 8 == 0 && cols <= 4 * 8 * kRmsMaxThreads && aligned16(input) && aligned16(residual_in) && aligned16(residual) && aligned16(input_copy) &&
+           aligned16(weight) && (reinterpret_cast<uintptr_t>(output) & 7) == 0;
+}
+
+int residual_rms_into(const void* input, const void* residual_in, void* residual, void* input_copy, const void* weight, const float* scale_tensor,
+                      float epsilon, void* output, int rows, int cols, int io_dtype, hipStream_t stream) {
+    return io_dtype == HFRK_F16
+               ? launch_rms<HFRK_F16, true>(input, residual_in, residual, input_copy, weight, scale_tensor, epsilon, output, nullptr, rows, cols, 0, 0, false, stream)
+               : launch_rms<HFRK_BF16, true>(input, residual_in, residual, input_copy, weight, scale_tensor, epsilon, output, nullptr, rows, cols, 0, 0, false, stream);
 }
 
 }  // namespace hfrk
@@ -203,9 +226,9 @@ extern "C" int hfrk_residual_rms(const void* input, void* residual, const void* 
     const bool fs = force_scalar != 0;
     const bool fp8 = out_dtype == HFRK_FP8_E4M3FN;
     if (io_dtype == HFRK_F16) {
-        return fp8 ? launch_rms<HFRK_F16, true>(input, residual, weight, scale_tensor, epsilon, output, next_buffer, rows, cols, buffer_cols, num_threads, fs, s)
-                   : launch_rms<HFRK_F16, false>(input, residual, weight, scale_tensor, epsilon, output, next_buffer, rows, cols, buffer_cols, num_threads, fs, s);
+        return fp8 ? launch_rms<HFRK_F16, true>(input, residual, residual, nullptr, weight, scale_tensor, epsilon, output, next_buffer, rows, cols, buffer_cols, num_threads, fs, s)
+                   : launch_rms<HFRK_F16, false>(input, residual, residual, nullptr, weight, scale_tensor, epsilon, output, next_buffer, rows, cols, buffer_cols, num_threads, fs, s);
     }
-    return fp8 ? launch_rms<HFRK_BF16, true>(input, residual, weight, scale_tensor, epsilon, output, next_buffer, rows, cols, buffer_cols, num_threads, fs, s)
-               : launch_rms<HFRK_BF16, false>(input, residual, weight, scale_tensor, epsilon, output, next_buffer, rows, cols, buffer_cols, num_threads, fs, s);
+    return fp8 ? launch_rms<HFRK_BF16, true>(input, residual, residual, nullptr, weight, scale_tensor, epsilon, output, next_buffer, rows, cols, buffer_cols, num_threads, fs, s)
+               : launch_rms<HFRK_BF16, false>(input, residual, residual, nullptr, weight, scale_tensor, epsilon, output, next_buffer, rows, cols, buffer_cols, num_threads, fs, s);
 }

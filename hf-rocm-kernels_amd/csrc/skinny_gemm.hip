@@ -659,6 +659,7 @@ static int choose_plan(int m, int n, int k, bool packed, hfrk_gemm_plan* plan) {
 // D = (base ? base : 0) + scale_a x scale_b x A.B   (epilogue 0), or the fused SwiGLU form (epilogue 1).
 // use_static: partial sums and counters go to this device's `scratch` array instead of the stream's workspace.
 // base_row: base is one row of n values, added to every row.
+// only_check: everything that can refuse the call (arguments, plan, the stream's workspace), and no launch.
 // rms: the activations are not read from A but built by the kernel's RMSNorm prologue from these 16-bit tensors.
 struct RmsPrologue {
     const void* input;
@@ -672,7 +673,7 @@ struct RmsPrologue {
 static int gemm_launch(const void* A, const void* B, void* D, const void* base, const float* scale_a, int sa_stride,
                        const float* scale_b, int sb_stride, const float* out_scale, int m, int n, int k, int b_stride,
                        int d_dtype, int epilogue, const hfrk_gemm_plan* user_plan, hipStream_t stream, bool packed = false,
-                       bool use_static = false, const RmsPrologue* rms = nullptr, bool base_row = false) {
+                       bool use_static = false, const RmsPrologue* rms = nullptr, bool base_row = false, bool only_check = false) {
     if (packed) b_stride = k;
     if (m < 1 || m > HFRK_GEMM_MAX_M || n < 1 || k < 1 || b_stride < k) return HFRK_BAD_SHAPE;
     if (k % 16 != 0 || (packed && k % 256 != 0)) return HFRK_K_NOT_DIVISIBLE_BY_WARPTILE_K;
@@ -777,6 +778,7 @@ static int gemm_launch(const void* A, const void* B, void* D, const void* base, 
         if (rc != HFRK_SUCCESS) return rc;
     }
     if (plan_ws_bytes(p) > ws_bytes || plan_counters(p) > counters) return use_static ? HFRK_EXCEEDS_SCRATCH : HFRK_BAD_SHAPE;
+    if (only_check) return HFRK_SUCCESS;
     if (use_static) {
         // The array keeps whatever the last call (or a launch that never finished) left: the counters of this plan start at zero.
         const int count = (int)plan_counters(p);
@@ -1034,6 +1036,53 @@ int hfrk_linear_gemm(const void* A, const void* B, int packed, void* D, const vo
     }
     return hfrk::gemm_launch(A, B, D, base, scale_a, sa_stride, scale_b, sb_stride, nullptr, m, n, k, b_stride, d_dtype, HFRK_EPILOGUE_NONE,
                              nullptr, static_cast<hipStream_t>(stream), packed != 0, false, nullptr, base && base_stride == 0);
+}
+
+size_t hfrk_llama_mlp_scratch_bytes(int m, int hidden, int inter) {
+    if (m < 1 || hidden < 1 || inter < 1) return 0;
+    const size_t normalized = ((size_t)m * hidden + 255) / 256 * 256, activated = ((size_t)m * inter + 255) / 256 * 256;
+    return normalized + activated + (m > 16 ? (size_t)m * inter * 4 : 0);
+}
+
+int hfrk_llama_mlp(const void* input, const void* residual_in, void* residual, void* input_copy, const void* rms_weight, float epsilon,
+                   const float* gate_up_input_scale, const void* gate_up, int gate_up_packed, int gate_up_stride, const float* gate_up_output_scale,
+                   const float* down_input_scale, const void* down, int down_packed, int down_stride, const float* down_output_scale, int add_residual,
+                   void* output, void* scratch, int m, int hidden, int inter, int dtype, int* launched, void* stream) {
+    using namespace hfrk;
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    if (launched) *launched = 0;
+    if (!input || !residual_in || !residual || !rms_weight || !gate_up_input_scale || !down_input_scale || !output || !scratch) return HFRK_BAD_SHAPE;
+    if (m < 1 || m > HFRK_GEMM_MAX_M || hidden < 1 || inter < 1 || hidden % 256 != 0 || inter % 256 != 0 || inter > (1 << 28)) return HFRK_BAD_SHAPE;
+    if (!(epsilon > 0.f)) return HFRK_BAD_SHAPE;
+    if (dtype != HFRK_F16 && dtype != HFRK_BF16) return HFRK_BAD_DTYPE;
+    uint8_t* const normalized = static_cast<uint8_t*>(scratch);
+    uint8_t* const activated = normalized + ((size_t)m * hidden + 255) / 256 * 256;
+    void* const both = activated + ((size_t)m * inter + 255) / 256 * 256;  // gate and up where they are launched apart from the SwiGLU
+    if (!residual_rms_into_takes(input, residual_in, residual, input_copy, rms_weight, normalized, hidden)) return HFRK_BAD_ALIGNMENT;
+    auto gate_up_gemm = [&](bool fused, bool only_check) {
+        return gemm_launch(normalized, gate_up, fused ? activated : both, nullptr, gate_up_output_scale, 0, nullptr, 0, fused ? down_input_scale : nullptr, m,
+                           2 * inter, hidden, gate_up_stride, dtype, fused ? HFRK_EPILOGUE_SWIGLU : HFRK_EPILOGUE_NONE, nullptr, s, gate_up_packed != 0,
+                           false, nullptr, false, only_check);
+    };
+    auto down_gemm = [&](bool only_check) {
+        return gemm_launch(activated, down, output, add_residual ? residual : nullptr, down_output_scale, 0, nullptr, 0, nullptr, m, hidden, inter, down_stride,
+                           dtype, HFRK_EPILOGUE_NONE, nullptr, s, down_packed != 0, false, nullptr, false, only_check);
+    };
+    // Nothing is launched unless everything can be: a caller that goes another way must find the residual as it was.  Where the SwiGLU is
+    // the gate_up GEMM's epilogue: skinny_gemm_swiglu (operators/skinny_gemm/wrapped.py) has the same rule and the figures behind it.
+    const bool window = hidden == 2048 || hidden == 4096;
+    bool fused = m <= 16 || window || (m <= kRowsMaxM && !gate_up_packed && 2L * inter * hidden <= (128L << 20));
+    int rc = fused ? gate_up_gemm(true, true) : HFRK_BAD_SHAPE;
+    if (rc == HFRK_BAD_SHAPE && m > 16 && !(fused && window)) {
+        fused = false;
+        rc = gate_up_gemm(false, true);
+    }
+    if (rc != HFRK_SUCCESS || (rc = down_gemm(true)) != HFRK_SUCCESS) return rc;
+    if (launched) *launched = 1;
+    rc = residual_rms_into(input, residual_in, residual, input_copy, rms_weight, gate_up_input_scale, epsilon, normalized, m, hidden, dtype, s);
+    if (rc == HFRK_SUCCESS) rc = gate_up_gemm(fused, false);
+    if (rc == HFRK_SUCCESS && !fused) rc = hfrk_swiglu(both, down_input_scale, activated, nullptr, m, inter, 0, dtype, 0, 0, stream);
+    return rc == HFRK_SUCCESS ? down_gemm(false) : rc;
 }
 
 int hfrk_skinny_gemm_rms_plan(int m, int n, int k, int epilogue, hfrk_gemm_plan* plan) {

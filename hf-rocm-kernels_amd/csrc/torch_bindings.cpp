@@ -597,6 +597,69 @@ bool skinny_gemm_into(const at::Tensor& A, const at::Tensor& B, const at::Tensor
     return plain_gemm(A, B, scale, D, true) == HFRK_SUCCESS;
 }
 
+// The fused decoder MLP block (combined_ops/llama_mlp.py) as one operator: its Python side took about 35 us per call, the block of 8 rows
+// of 4096 x 14336 35 us of kernels and that of one row of 2048 x 6144 less than half of it.  residual_out <- input + residual (it may be
+// `residual`), input_copy <- input, and the block's output, into `output` where one is given.  Weights are [k, n] views or (n >= 0) packed buffers.
+// False, with nothing launched, for everything that the wrappers would convert, copy or refuse.
+bool llama_mlp(const at::Tensor& input, const at::Tensor& residual, at::Tensor& residual_out, const std::optional<at::Tensor>& input_copy,
+               const at::Tensor& rms_weight, double epsilon, const at::Tensor& gate_up, int64_t gate_up_n, const at::Tensor& gate_up_input_scale,
+               const at::Tensor& gate_up_output_scale, const at::Tensor& down, int64_t down_n, const at::Tensor& down_input_scale,
+               const at::Tensor& down_output_scale, bool add_residual, at::Tensor& output) {
+    if (!input.is_cuda() || input.dim() != 2 || !is_16bit(input.scalar_type())) return false;
+    const int64_t m = input.size(0), hidden = input.size(1);
+    auto like_input = [&](const at::Tensor& t) {
+        return t.is_contiguous() && t.sizes() == input.sizes() && t.scalar_type() == input.scalar_type() && t.device() == input.device();
+    };
+    if (m < 1 || m > HFRK_GEMM_MAX_M || hidden < 256 || hidden % 256 != 0 || hidden > 32768) return false;
+    if (!like_input(input) || !like_input(residual) || !like_input(residual_out) || !like_input(output)) return false;
+    if (input_copy.has_value() && !like_input(*input_copy)) return false;
+    // A tensor read may be one that is written (the same values, each read before it is written), but not overlap one, and a residual that
+    // would be overwritten by the input's copy first is left to the copies.
+    auto apart = [&](const at::Tensor& read, const at::Tensor& written) {
+        const char *r = static_cast<const char*>(read.data_ptr()), *w = static_cast<const char*>(written.data_ptr());
+        const size_t bytes = (size_t)(m * hidden) * 2;
+        return r == w || r + bytes <= w || w + bytes <= r;
+    };
+    if (!apart(input, residual_out) || !apart(residual, residual_out)) return false;
+    if (input_copy.has_value() && (!apart(input, *input_copy) || !apart(residual, *input_copy) || residual_out.data_ptr() == input_copy->data_ptr() ||
+                                   (residual.data_ptr() == input_copy->data_ptr() && input.data_ptr() != residual.data_ptr())))
+        return false;
+    if (at::GradMode::is_enabled() && (input.requires_grad() || residual.requires_grad())) return false;
+    if (rms_weight.dim() != 1 || rms_weight.size(0) != hidden || !rms_weight.is_contiguous() || rms_weight.scalar_type() != input.scalar_type() ||
+        rms_weight.device() != input.device() || !(epsilon > 0))
+        return false;
+    for (const at::Tensor* t : {&gate_up_input_scale, &gate_up_output_scale, &down_input_scale, &down_output_scale})
+        if (!one_float(*t, input)) return false;
+    // a weight's columns, or -1 where it is none of `k` rows that the GEMMs read as it is
+    auto columns = [&](const at::Tensor& w, int64_t n, int64_t k) -> int64_t {
+        if (w.scalar_type() != at::kFloat8_e4m3fn || w.device() != input.device()) return -1;
+        if (n >= 0) {
+            if (n < 1 || n >= (int64_t(1) << 24) || !w.is_contiguous()) return -1;
+            const size_t plain = hfrk_packed_weight_bytes((int)n, (int)k), have = (size_t)w.numel();
+            return plain != 0 && (have == plain || have == hfrk_packed_weight_bytes_scaled((int)n, (int)k)) ? n : -1;
+        }
+        if (w.dim() != 2 || w.size(0) != k || w.stride(0) != 1 || w.size(1) < 2 || w.size(1) >= (int64_t(1) << 24) || w.stride(1) < k ||
+            w.stride(1) >= (int64_t(1) << 30))
+            return -1;
+        return w.size(1);
+    };
+    const int64_t n = columns(gate_up, gate_up_n, hidden), inter = n / 2;
+    if (n < 512 || inter % 256 != 0 || n % 2 != 0 || columns(down, down_n, inter) != hidden) return false;
+
+    DeviceScope scope(input);
+    at::Tensor scratch = at::empty({(int64_t)hfrk_llama_mlp_scratch_bytes((int)m, (int)hidden, (int)inter)}, input.options().dtype(at::kByte));
+    int launched = 0;
+    const int status = hfrk_llama_mlp(
+        input.data_ptr(), residual.data_ptr(), residual_out.data_ptr(), input_copy.has_value() ? input_copy->data_ptr() : nullptr,
+        rms_weight.data_ptr(), (float)epsilon, gate_up_input_scale.data_ptr<float>(), gate_up.data_ptr(), gate_up_n >= 0 ? 1 : 0,
+        gate_up_n >= 0 ? (int)hidden : (int)gate_up.stride(1), gate_up_output_scale.data_ptr<float>(), down_input_scale.data_ptr<float>(),
+        down.data_ptr(), down_n >= 0 ? 1 : 0, down_n >= 0 ? (int)inter : (int)down.stride(1), down_output_scale.data_ptr<float>(),
+        add_residual ? 1 : 0, output.data_ptr(), scratch.data_ptr(), (int)m, (int)hidden, (int)inter,
+        input.scalar_type() == at::kBFloat16 ? HFRK_BF16 : HFRK_F16, &launched, current_stream(input));
+    if (launched) raise_on(status, "llama_mlp");
+    return status == HFRK_SUCCESS;
+}
+
 bool is_byte_tensor(const at::Tensor& t) {
     return t.scalar_type() == at::kByte || t.scalar_type() == at::kFloat8_e4m3fn || t.scalar_type() == at::kFloat8_e4m3fnuz;
 }
@@ -736,6 +799,13 @@ TORCH_LIBRARY(_HFRK_C, ops) {
     ops.impl("skinny_gemm_new", torch::dispatch(c10::DispatchKey::Autograd, torch::CppFunction::makeFallthrough()));
     ops.def("skinny_gemm_into(Tensor A, Tensor B, Tensor scale, Tensor! D) -> bool");
     ops.impl("skinny_gemm_into", c10::kCUDA, &skinny_gemm_into);
+
+    ops.def(
+        "llama_mlp(Tensor input, Tensor residual, Tensor(a!) residual_out, Tensor(b!)? input_copy, Tensor rms_weight, float epsilon, Tensor gate_up, "
+        "int gate_up_n, Tensor gate_up_input_scale, Tensor gate_up_output_scale, Tensor down, int down_n, Tensor down_input_scale, "
+        "Tensor down_output_scale, bool add_residual, Tensor(c!) output) -> bool");
+    ops.impl("llama_mlp", c10::kCUDA, &llama_mlp);
+    ops.impl("llama_mlp", torch::dispatch(c10::DispatchKey::Autograd, torch::CppFunction::makeFallthrough()));
 
     ops.def("quantize_fp8(Tensor input, Tensor? scale_tensor, Tensor! output, Tensor! scales) -> ()");
     ops.impl("quantize_fp8", c10::kCUDA, &quantize_fp8);

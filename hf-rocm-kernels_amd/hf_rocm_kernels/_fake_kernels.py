@@ -19,7 +19,7 @@ _RETURNS_NOTHING = ("increment", "residual_rms", "swiglu", "pack_weight", "pack_
 _RETURNS_STATUS = ("skinny_gemm_tb", "skinny_gemm_scaled", "skinny_gemm_fused", "skinny_gemm_packed", "skinny_gemm_rms_fused",
                    # a result of their own, _OTHER_RESULT; the wrappers keep fake calls away from these (utils/dispatch.py), a caller of
                    # torch.ops need not
-                   "fp8_linear", "skinny_gemm_new", "skinny_gemm_into")
+                   "fp8_linear", "skinny_gemm_new", "skinny_gemm_into", "llama_mlp")
 
 
 def _nothing(*args, **kwargs) -> None:
@@ -39,7 +39,8 @@ def _skinny_gemm_new(A, B, scale):
     return A.new_empty((A.shape[0], B.shape[1]), dtype=torch.float16)
 
 
-_OTHER_RESULT = {"fp8_linear": _fp8_linear, "skinny_gemm_new": _skinny_gemm_new, "skinny_gemm_into": lambda A, B, scale, D: True}
+_OTHER_RESULT = {"fp8_linear": _fp8_linear, "skinny_gemm_new": _skinny_gemm_new, "skinny_gemm_into": lambda A, B, scale, D: True,
+                 "llama_mlp": lambda *args: True}
 
 
 def register() -> None:

@@ -276,6 +276,19 @@ int hfrk_skinny_gemm_packed(const void* A, const void* B_packed, void* D, const 
 int hfrk_linear_gemm(const void* A, const void* B, int packed, void* D, const void* base, int base_stride, const float* scale_a,
                      int sa_stride, const float* scale_b, int sb_stride, int m, int n, int k, int b_stride, int d_dtype, void* stream);
 
+/* The fused decoder MLP block for up to 64 rows: hfrk_residual_rms, the gate_up GEMM with the SwiGLU as its epilogue (or behind it, where that
+ * is the faster way), and the down GEMM with or without the updated residual as its addend.
+ *   residual <- input + residual_in (which may be the same tensor);  input_copy <- input, where it is not NULL
+ *   output   <- (add_residual ? residual : 0) + down_output_scale * down(e4m3fn(silu(gate) * up / down_input_scale))
+ * input, residual_in, residual, input_copy, output: 16-bit (dtype) [m, hidden], the first four and rms_weight 16-byte aligned; weights
+ * row-major [2*inter, hidden] and [hidden, inter] with row strides, or the buffers hfrk_pack_weight wrote; hidden and inter multiples of 256;
+ * scratch: hfrk_llama_mlp_scratch_bytes, 16-byte aligned.  *launched (may be NULL): 0 if the call was refused with nothing written. */
+size_t hfrk_llama_mlp_scratch_bytes(int m, int hidden, int inter);
+int hfrk_llama_mlp(const void* input, const void* residual_in, void* residual, void* input_copy, const void* rms_weight, float epsilon,
+                   const float* gate_up_input_scale, const void* gate_up, int gate_up_packed, int gate_up_stride, const float* gate_up_output_scale,
+                   const float* down_input_scale, const void* down, int down_packed, int down_stride, const float* down_output_scale, int add_residual,
+                   void* output, void* scratch, int m, int hidden, int inter, int dtype, int* launched, void* stream);
+
 /* How one tiled GEMM call is decomposed: an index into the library's tile shapes (0: 256 x 256, 1: 256 x 128, 2: 128 x 128,
  * 3: 128 x 64, 4: 64 x 64 rows x columns of D per workgroup), how many workgroups share a tile's k, and how many rows of tiles
  * the workgroups walk side by side. */
