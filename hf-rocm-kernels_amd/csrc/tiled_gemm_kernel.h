@@ -27,7 +27,7 @@
 //  * Workgroup ids are dealt to the XCDs in contiguous ranges and walk the tiles in column-major groups of group_m rows of tiles, so
 //    that the workgroups of one L2 share both operands.
 //  * Few tiles and a long k: k is cut between `splits` workgroups.  Partial tiles are written through to memory, the last arriver
-//    adds them in split order (bit-reproducible), as in the skinny workgroup kernel.
+//    adds them in split order (bit-reproducible), its own from its registers.
 //
 // Measured (row-major / packed, us, bf16 out): 4096 x 28672 x 4096 412 / 395 (2.3 / 2.4 PFLOP/s; 1550 as 64 skinny launches; a loop that
 // stays resident clocks at 1.8 - 2.0 GHz, so the matrix cores' power bounds it before their issue rate does; on eight waves 409), 512 x 4096 x 14336
@@ -299,19 +299,53 @@ __global__ void __launch_bounds__(64 * WM * WN, WGS * WM * WN / 4) tiled_gemm_ke
         const int last = *flag;
         __syncthreads();  // the epilogue writes where the flag lies
         if (!last) return;
-        constexpr int CH = NMMA < 4 ? NMMA : 4;  // tiles whose shares are in flight together
+        // The last arriver adds the partials in split order, its own from its registers; up to four splits' are requested together, more
+        // one after the other.  What it costs is the round trips: with its own read back and one split at a time 512 x 4096 x 14336 in 2
+        // splits 43.8 -> 43.0 us, 64 x 4096 x 14336 in 4 17.5 -> 17.1, 1024 x 8192 x 8192 on 256 x 256 tiles in 2 82 -> 76.
+        constexpr int CH = NW > 4 ? 1 : NMMA <= 4 ? NMMA : 2;  // matrix tiles whose shares are in flight together: what fits the registers
+        auto load_shares = [&](v4i (&share)[CH * 4], int t0, int sp) __attribute__((always_inline)) {
+#pragma unroll
+            for (int p = 0; p < CH * 4; ++p) share[p] = __builtin_amdgcn_raw_buffer_load_b128(ws, ws_off(sp, t0 + p / 4, p % 4), 0, kCoherent);
+        };
 #pragma unroll
         for (int t0 = 0; t0 < NMMA; t0 += CH) {
             v4f sum[CH * 4];
 #pragma unroll
             for (int p = 0; p < CH * 4; ++p) sum[p] = v4f{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-            for (int sp = 0; sp < a.splits; ++sp) {
-                v4i share[CH * 4];
-#pragma unroll
-                for (int p = 0; p < CH * 4; ++p) share[p] = __builtin_amdgcn_raw_buffer_load_b128(ws, ws_off(sp, t0 + p / 4, p % 4), 0, kCoherent);
+            auto add = [&](const v4i (&share)[CH * 4]) __attribute__((always_inline)) {
 #pragma unroll
                 for (int p = 0; p < CH * 4; ++p) sum[p] += __builtin_bit_cast(v4f, share[p]);
+            };
+            auto add_own = [&]() __attribute__((always_inline)) {
+#pragma unroll
+                for (int p = 0; p < CH * 4; ++p) {
+                    const v16f& x = acc[(t0 + p / 4) / TN][(t0 + p / 4) % TN];
+                    sum[p] += v4f{x[4 * (p % 4)], x[4 * (p % 4) + 1], x[4 * (p % 4) + 2], x[4 * (p % 4) + 3]};
+                }
+            };
+            if (a.splits <= 4) {
+                v4i other[3][CH * 4];
+#pragma unroll
+                for (int j = 0; j < 3; ++j)
+                    if (j + 1 < a.splits) load_shares(other[j], t0, j + (j >= split ? 1 : 0));
+#pragma unroll
+                for (int sp = 0; sp < 4; ++sp) {
+                    if (sp >= a.splits) continue;
+                    if (sp == split) add_own();
+                    else if (sp < split) add(other[sp < 3 ? sp : 2]);
+                    else add(other[sp > 0 ? sp - 1 : 0]);
+                }
+            } else {
+#pragma unroll 1
+                for (int sp = 0; sp < a.splits; ++sp) {
+                    if (sp == split) {
+                        add_own();
+                        continue;
+                    }
+                    v4i share[CH * 4];
+                    load_shares(share, t0, sp);
+                    add(share);
+                }
             }
 #pragma unroll
             for (int t = 0; t < CH; ++t)
