@@ -33,7 +33,7 @@ constexpr int kTiledStage = 128;    // bytes of k per pipeline stage
 // X(index, TM, TN, WM, WN, NST, WGS)
 #define HFRK_TILED_SHAPES(X) \
     X(0, 4, 2, 2, 4, 2, 1)   \
-    X(1, 4, 2, 2, 2, 3, 1)   \
+    X(1, 2, 2, 4, 2, 3, 1)   \
     X(2, 2, 2, 2, 2, 5, 1)   \
     X(3, 2, 1, 2, 2, 3, 2)   \
     X(4, 1, 1, 2, 2, 8, 1)

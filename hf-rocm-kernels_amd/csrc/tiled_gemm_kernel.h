@@ -6,8 +6,10 @@
 //  * A wave owns TM x TN matrix tiles of 32 x 32 (v_mfma_f32_32x32x64_f8f6f4, 64 cycles each).  The largest tile (256 x 256) runs on eight
 //    waves of 128 x 64, two per SIMD: with four of 128 x 128 an operand byte read from LDS fed a third more multiply-adds, but nothing ran
 //    while the one wave of a SIMD waited for its stage or stored (4096 x 28672 x 4096 432 -> 409 us, 4096 x 4096 x 4096 62.7 -> 57,
-//    2048 x 6144 x 4096 56 -> 52; 12 % in the mean over 70 weights and rows where tiles are few).  The others have four waves, one per
-//    SIMD: 128 x 128 on eight or sixteen waves takes the same time.
+//    2048 x 6144 x 4096 56 -> 52; 12 % in the mean over 70 weights and rows where tiles are few).  The 256 x 128 tile has eight
+//    waves of 64 x 64 for the same reason (four of 128 x 64 before: 4096 x 6144 x 4096 106 -> 97 us, 4096 x 2048 x 2048 23.0 -> 21.0,
+//    300 x 20000 x 4096 56.3 -> 53.5, 1024 x 8192 x 8192 64.6 -> 64; 512 x 10240 x 8192 54.6 -> 55.4 is the loss).  The others have
+//    four waves, one per SIMD: 128 x 128 on eight or sixteen takes the same time.
 //  * Bound (counters in profiles/tiled_gemm_counters_and_plans.txt, shares of the cycles in which a compute unit has work): 4096 x 28672 x
 //    4096 matrix cores 62 %, at the clock their power leaves, LDS 19 %; 512 x 4096 x 14336 packed 45 and 34 %; 201 x 6144 x 4096
 //    28 and 23 %.  On the small tiles neither is half busy.  (The first of the three before its tile ran on eight waves.)

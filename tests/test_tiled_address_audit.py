@@ -171,8 +171,8 @@ def test_largest_sizes(m, n, k):
                 audit(m, n, k, k, forced, True, 0)
 
 
-# TM, TN, WM, WN, stages in LDS as the kernel is built: the 256 x 256 tile runs on eight waves
-BUILT = [(4, 2, 2, 4, 2)] + SHAPES[1:]
+# TM, TN, WM, WN, stages in LDS as the kernel is built: the 256-row tiles run on eight waves
+BUILT = [(4, 2, 2, 4, 2), (2, 2, 4, 2, 3)] + SHAPES[2:]
 
 
 @pytest.mark.parametrize("shape", range(5))
