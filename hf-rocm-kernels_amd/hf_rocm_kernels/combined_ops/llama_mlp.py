@@ -159,9 +159,9 @@ class LlamaMlpGraph:
         The usual call does the same without the graph: the RMSNorm reads the inputs where they are and writes the copies, and the launches
         go out from native code, which costs the GPU less than starting a graph (8 rows of 4096 x 14336: 46.6 us with two copies in front,
         41.9 for the replay alone, 35.9 this way; one row of 2048 x 6144 31.6, 23.4, 17.0)."""
-        if self._fused and runs_now(attn_output) and _native_block(attn_output, residual, self.residual, self.attn_output, self.mlp_output,
-                                                                   *self._operands, self._add_residual):
-            return self.mlp_output, self.residual
+        if self._fused and runs_now(attn_output) and not torch.cuda.is_current_stream_capturing():
+            if _native_block(attn_output, residual, self.residual, self.attn_output, self.mlp_output, *self._operands, self._add_residual):
+                return self.mlp_output, self.residual
         self.attn_output.copy_(attn_output)
         self.residual.copy_(residual)
         self.graph.replay()

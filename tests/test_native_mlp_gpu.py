@@ -1,6 +1,7 @@
 """The fused MLP block as one native operator against the launches of its wrappers (same kernels: same bits), and the calls it leaves
 to them."""
 import itertools
+import sys
 
 import pytest
 import torch
@@ -9,7 +10,7 @@ from hf_rocm_kernels.combined_ops.llama_mlp import LlamaMlpGraph, llama_mlp_comb
 from hf_rocm_kernels.utils.weight_format import pack_weight
 
 pytestmark = pytest.mark.gpu
-MODULE = __import__("sys").modules["hf_rocm_kernels.combined_ops.llama_mlp"]
+MODULE = sys.modules["hf_rocm_kernels.combined_ops.llama_mlp"]
 
 
 def _block(hidden, inter, dtype, packed=(False, False), wide=0, seed=0):
