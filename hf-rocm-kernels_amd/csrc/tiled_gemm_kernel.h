@@ -31,9 +31,9 @@
 //  * Few tiles and a long k: k is cut between `splits` workgroups.  Partial tiles are written through to memory, the last arriver
 //    adds them in split order (bit-reproducible), its own from its registers.
 //
-// Measured (row-major / packed, us, bf16 out): 4096 x 28672 x 4096 412 / 395 (2.3 / 2.4 PFLOP/s; 1550 as 64 skinny launches; a loop that
-// stays resident clocks at 1.8 - 2.0 GHz, so the matrix cores' power bounds it before their issue rate does; on eight waves 409), 512 x 4096 x 14336
-// 38 / 37 (150), 201 x 6144 x 4096 13.2 / 13.1 (46), 65 x 4096 x 4096 10.5 / 9.9 (16).  The epilogue is written with little code on
+// Measured (us, bf16 out): 4096 x 28672 x 4096 409 (2.35 PFLOP/s; 1550 as 64 skinny launches; a loop that stays resident clocks at 1.8 - 2.0
+// GHz, so the matrix cores' power bounds it before their issue rate does), 512 x 4096 x 14336 packed 36 (150), 201 x 6144 x 4096
+// 13.4 (46), 65 x 4096 x 4096 10.5, packed 9.9 (16).  The epilogue is written with little code on
 // purpose: with a branch per value for NaN and 64-bit addresses it took 18 us of a 256 x 256 tile, now 7.
 #pragma once
 
