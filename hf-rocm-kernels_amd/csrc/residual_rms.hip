@@ -42,18 +42,20 @@ __device__ __forceinline__ void zero_next_buffer_row(uint16_t* next_buffer, int 
 
 // 8 elements (16 bytes) per thread per iteration, ITERS iterations cached in registers: cols <= 8*blockDim*ITERS.
 // READ_ONCE: the input is read past the caches (kReadOnceFrom).
-// residual_in is residual itself, or another tensor that stays as it is; input_copy, where not null, becomes a copy of the input.  Every
-// thread has read its pieces of the inputs before it writes any, and nobody else's: either may be its own source.
-template <int DT, bool FP8_OUT, int ITERS, bool READ_ONCE>
-__global__ void __launch_bounds__(kRmsMaxThreads) residual_rms_vec_kernel(
-    const uint16_t* input, const uint16_t* residual_in, uint16_t* residual, uint16_t* input_copy, const uint16_t* __restrict__ weight,
-    const float* __restrict__ scale_tensor, void* __restrict__ output, uint16_t* __restrict__ next_buffer,
-    float epsilon, int cols, int buffer_cols) {
+// INTO: the residual is read from residual_in, which stays as it is unless it is `residual` itself, and input_copy, where not null,
+// becomes a copy of the input.  Every thread has read its pieces of the inputs before it writes any, and nobody else's: either may be its
+// own source.  Two kernels call this: with the further pointers and without __restrict__ the four-piece instances of the plain one take 62
+// to 69 registers instead of 60 to 64, and beyond 64 a compute unit holds one workgroup of 16 waves instead of two.
+template <int DT, bool FP8_OUT, int ITERS, bool READ_ONCE, bool INTO>
+__device__ __forceinline__ void residual_rms_vec(
+    const uint16_t* input, const uint16_t* residual_in, uint16_t* residual, uint16_t* input_copy, const uint16_t* weight,
+    const float* scale_tensor, void* output, uint16_t* next_buffer, float epsilon, int cols, int buffer_cols) {
     __shared__ __align__(16) float red[16];
     const long row_off = (long)blockIdx.x * cols;
     const uint32_t row_bytes = (uint32_t)cols * 2u;
-    const __amdgpu_buffer_rsrc_t rin = make_rsrc(input + row_off, row_bytes), rres_in = make_rsrc(residual_in + row_off, row_bytes),
-                                 rres = make_rsrc(residual + row_off, row_bytes), rweight = make_rsrc(weight, row_bytes);
+    const __amdgpu_buffer_rsrc_t rin = make_rsrc(input + row_off, row_bytes), rres = make_rsrc(residual + row_off, row_bytes),
+                                 rweight = make_rsrc(weight, row_bytes);
+    const __amdgpu_buffer_rsrc_t rres_in = INTO ? make_rsrc(residual_in + row_off, row_bytes) : rres;
     const __amdgpu_buffer_rsrc_t rout = FP8_OUT ? make_rsrc(static_cast<uint8_t*>(output) + row_off, (uint32_t)cols)
                                                 : make_rsrc(static_cast<uint16_t*>(output) + row_off, row_bytes);
     uint4 a[ITERS], z[ITERS], wreg[ITERS];
@@ -74,7 +76,7 @@ __global__ void __launch_bounds__(kRmsMaxThreads) residual_rms_vec_kernel(
         z[it] = rms_add_square<DT>(a[it], z[it], ssq);
         store_piece(rres, threadIdx.x + it * blockDim.x, z[it]);
     }
-    if (input_copy) {
+    if (INTO && input_copy) {
         const __amdgpu_buffer_rsrc_t rcopy = make_rsrc(input_copy + row_off, row_bytes);
 #pragma unroll
         for (int it = 0; it < ITERS; ++it) store_piece(rcopy, threadIdx.x + it * blockDim.x, a[it]);
@@ -104,6 +106,23 @@ __global__ void __launch_bounds__(kRmsMaxThreads) residual_rms_vec_kernel(
         }
     }
     zero_next_buffer_row(next_buffer, buffer_cols);
+}
+
+template <int DT, bool FP8_OUT, int ITERS, bool READ_ONCE>
+__global__ void __launch_bounds__(kRmsMaxThreads) residual_rms_vec_kernel(
+    const uint16_t* __restrict__ input, uint16_t* __restrict__ residual, const uint16_t* __restrict__ weight,
+    const float* __restrict__ scale_tensor, void* __restrict__ output, uint16_t* __restrict__ next_buffer,
+    float epsilon, int cols, int buffer_cols) {
+    residual_rms_vec<DT, FP8_OUT, ITERS, READ_ONCE, false>(input, residual, residual, nullptr, weight, scale_tensor, output, next_buffer, epsilon, cols,
+                                                           buffer_cols);
+}
+
+// For the MLP block (residual_rms_into): at most 64 rows, so nothing is read past the caches.
+template <int DT, int ITERS>
+__global__ void __launch_bounds__(kRmsMaxThreads) residual_rms_into_kernel(
+    const uint16_t* input, const uint16_t* residual_in, uint16_t* residual, uint16_t* input_copy, const uint16_t* __restrict__ weight,
+    const float* __restrict__ scale_tensor, void* __restrict__ output, float epsilon, int cols) {
+    residual_rms_vec<DT, true, ITERS, false, true>(input, residual_in, residual, input_copy, weight, scale_tensor, output, nullptr, epsilon, cols, 0);
 }
 
 // One element per thread per iteration; no alignment or divisibility requirement.  The second pass re-reads the
@@ -141,14 +160,20 @@ __global__ void __launch_bounds__(kRmsMaxThreads) residual_rms_scalar_kernel(
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
+// threads per row of nvec 16-byte pieces: enough for one or two each, whole wavefronts, at most 1024
+static int rms_threads(int nvec) {
+    int threads = ((nvec + 63) / 64) * 64;
+    if (threads > 512) threads = ((nvec + 127) / 128) * 64;
+    if (threads > kRmsMaxThreads) threads = kRmsMaxThreads;
+    return threads < 64 ? 64 : threads;
+}
+
 template <int DT, bool FP8_OUT>
-static int launch_rms(const void* input, const void* residual_in, void* residual, void* input_copy, const void* weight, const float* scale_tensor, float epsilon,
+static int launch_rms(const void* input, void* residual, const void* weight, const float* scale_tensor, float epsilon,
                       void* output, void* next_buffer, int rows, int cols, int buffer_cols, int num_threads,
                       bool force_scalar, hipStream_t stream) {
     const uint16_t* in = static_cast<const uint16_t*>(input);
-    const uint16_t* res_in = static_cast<const uint16_t*>(residual_in);
     uint16_t* res = static_cast<uint16_t*>(residual);
-    uint16_t* copy = static_cast<uint16_t*>(input_copy);
     const uint16_t* w = static_cast<const uint16_t*>(weight);
     uint16_t* nb = static_cast<uint16_t*>(next_buffer);
     // 16-byte path: aligned rows (cols % 8 == 0 keeps every row aligned) and an aligned output row
@@ -157,18 +182,12 @@ static int launch_rms(const void* input, const void* residual_in, void* residual
     int threads = num_threads;
     if (vec) {
         const int nvec = cols / 8;
-        if (threads == 0) {
-            // enough threads for one or two 16-byte pieces each, whole wavefronts, at most 1024
-            threads = ((nvec + 63) / 64) * 64;
-            if (threads > 512) threads = ((nvec + 127) / 128) * 64;
-            if (threads > kRmsMaxThreads) threads = kRmsMaxThreads;
-            if (threads < 64) threads = 64;
-        }
+        if (threads == 0) threads = rms_threads(nvec);
         const int iters = (nvec + threads - 1) / threads;
         if (iters > 4) vec = false;  // would not fit the register cache: fall through to the strided kernel
         else {
 #define HFRK_RMS_LAUNCH(IT, ONCE)                                                                                          \
-    hipLaunchKernelGGL((residual_rms_vec_kernel<DT, FP8_OUT, IT, ONCE>), dim3(rows), dim3(threads), 0, stream, in, res_in, res, copy, w, \
+    hipLaunchKernelGGL((residual_rms_vec_kernel<DT, FP8_OUT, IT, ONCE>), dim3(rows), dim3(threads), 0, stream, in, res, w, \
                        scale_tensor, output, nb, epsilon, cols, buffer_cols)
 #define HFRK_RMS_ITERS(ONCE)                         \
     do {                                             \
@@ -183,7 +202,6 @@ static int launch_rms(const void* input, const void* residual_in, void* residual
         }
     }
     if (!vec) {
-        if (res_in != res || copy) return HFRK_BAD_ALIGNMENT;  // residual_rms_into's callers ask first
         if (threads == 0) {
             threads = ((cols + 63) / 64) * 64;
             if (threads > kRmsMaxThreads) threads = kRmsMaxThreads;
@@ -201,11 +219,27 @@ bool residual_rms_into_takes(const void* input, const void* residual_in, const v
            aligned16(weight) && (reinterpret_cast<uintptr_t>(output) & 7) == 0;
 }
 
+template <int DT>
+static int launch_rms_into(const void* input, const void* residual_in, void* residual, void* input_copy, const void* weight, const float* scale_tensor,
+                           float epsilon, void* output, int rows, int cols, hipStream_t stream) {
+    const int threads = rms_threads(cols / 8), iters = (cols / 8 + threads - 1) / threads;
+#define HFRK_RMS_LAUNCH(IT)                                                                                                         \
+    hipLaunchKernelGGL((residual_rms_into_kernel<DT, IT>), dim3(rows), dim3(threads), 0, stream, static_cast<const uint16_t*>(input), \
+                       static_cast<const uint16_t*>(residual_in), static_cast<uint16_t*>(residual), static_cast<uint16_t*>(input_copy), \
+                       static_cast<const uint16_t*>(weight), scale_tensor, output, epsilon, cols)
+    if (iters <= 1) HFRK_RMS_LAUNCH(1);
+    else if (iters == 2) HFRK_RMS_LAUNCH(2);
+    else HFRK_RMS_LAUNCH(4);
+#undef HFRK_RMS_LAUNCH
+    HFRK_HIP_TRY(hipGetLastError());
+    return HFRK_SUCCESS;
+}
+
 int residual_rms_into(const void* input, const void* residual_in, void* residual, void* input_copy, const void* weight, const float* scale_tensor,
                       float epsilon, void* output, int rows, int cols, int io_dtype, hipStream_t stream) {
-    return io_dtype == HFRK_F16
-               ? launch_rms<HFRK_F16, true>(input, residual_in, residual, input_copy, weight, scale_tensor, epsilon, output, nullptr, rows, cols, 0, 0, false, stream)
-               : launch_rms<HFRK_BF16, true>(input, residual_in, residual, input_copy, weight, scale_tensor, epsilon, output, nullptr, rows, cols, 0, 0, false, stream);
+    if (!residual_rms_into_takes(input, residual_in, residual, input_copy, weight, output, cols)) return HFRK_BAD_ALIGNMENT;
+    return io_dtype == HFRK_F16 ? launch_rms_into<HFRK_F16>(input, residual_in, residual, input_copy, weight, scale_tensor, epsilon, output, rows, cols, stream)
+                                : launch_rms_into<HFRK_BF16>(input, residual_in, residual, input_copy, weight, scale_tensor, epsilon, output, rows, cols, stream);
 }
 
 }  // namespace hfrk
@@ -226,9 +260,9 @@ extern "C" int hfrk_residual_rms(const void* input, void* residual, const void* 
     const bool fs = force_scalar != 0;
     const bool fp8 = out_dtype == HFRK_FP8_E4M3FN;
     if (io_dtype == HFRK_F16) {
-        return fp8 ? launch_rms<HFRK_F16, true>(input, residual, residual, nullptr, weight, scale_tensor, epsilon, output, next_buffer, rows, cols, buffer_cols, num_threads, fs, s)
-                   : launch_rms<HFRK_F16, false>(input, residual, residual, nullptr, weight, scale_tensor, epsilon, output, next_buffer, rows, cols, buffer_cols, num_threads, fs, s);
+        return fp8 ? launch_rms<HFRK_F16, true>(input, residual, weight, scale_tensor, epsilon, output, next_buffer, rows, cols, buffer_cols, num_threads, fs, s)
+                   : launch_rms<HFRK_F16, false>(input, residual, weight, scale_tensor, epsilon, output, next_buffer, rows, cols, buffer_cols, num_threads, fs, s);
     }
-    return fp8 ? launch_rms<HFRK_BF16, true>(input, residual, residual, nullptr, weight, scale_tensor, epsilon, output, next_buffer, rows, cols, buffer_cols, num_threads, fs, s)
-               : launch_rms<HFRK_BF16, false>(input, residual, residual, nullptr, weight, scale_tensor, epsilon, output, next_buffer, rows, cols, buffer_cols, num_threads, fs, s);
+    return fp8 ? launch_rms<HFRK_BF16, true>(input, residual, weight, scale_tensor, epsilon, output, next_buffer, rows, cols, buffer_cols, num_threads, fs, s)
+               : launch_rms<HFRK_BF16, false>(input, residual, weight, scale_tensor, epsilon, output, next_buffer, rows, cols, buffer_cols, num_threads, fs, s);
 }

@@ -70,3 +70,10 @@ def test_row_split_kernels_keep_their_registers(source, tmp_path):
     """The loop of the 32-row instances fills all 256: at most one pair of registers lives in scratch."""
     sizes = [int(x) for x in re.findall(r"\.private_segment_fixed_size: (\d+)", "".join(_assembly(source, tmp_path)))]
     assert len(sizes) >= 30 and max(sizes) <= 8
+
+
+def test_rms_kernels_leave_room_for_two_workgroups(tmp_path):
+    """A row of more than 16384 values takes 16 waves with four pieces a thread: above 64 registers a compute unit holds one such workgroup."""
+    text = "".join(_assembly("residual_rms.hip", tmp_path))
+    registers = {m[1]: int(m[2]) for m in re.finditer(r"\.name:\s+_ZN4hfrk\d+residual_rms_vec_kernelI(\S+?)EEEv.*?\.vgpr_count:\s+(\d+)", text, re.S)}
+    assert len(registers) == 24 and max(registers.values()) <= 64, registers

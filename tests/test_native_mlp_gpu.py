@@ -57,7 +57,7 @@ def test_same_bits_as_the_wrappers(m, hidden, inter, monkeypatch):
     assert taken == [True] * 8
 
 
-@pytest.mark.parametrize("m,hidden,inter", [(1, 2048, 2816), (8, 4096, 1536), (40, 1280, 1024)])
+@pytest.mark.parametrize("m,hidden,inter", [(1, 2048, 2816), (8, 4096, 1536), (40, 1280, 1024), (3, 16640, 512), (2, 32768, 512)])
 def test_graph_call_leaves_what_copies_and_a_replay_leave(m, hidden, inter, monkeypatch):
     taken = _counted(monkeypatch)
     args = _block(hidden, inter, torch.bfloat16)
