@@ -37,6 +37,8 @@ constexpr int kTiledStage = 128;    // bytes of k per pipeline stage
     X(2, 2, 2, 2, 2, 5, 1)   \
     X(3, 2, 1, 2, 2, 3, 2)   \
     X(4, 1, 1, 2, 2, 8, 1)
+// Shape 1 on four waves, for row-major operands whose rows begin inside a 128-byte line (tiled_gemm_rowmajor.hip).
+#define HFRK_TILED_FOUR_WAVES(X) X(1, 4, 2, 2, 2, 3, 1)
 
 struct TiledShape {
     int bm, bn, stages, per_cu;
@@ -44,6 +46,10 @@ struct TiledShape {
 #define HFRK_TILED_ROW(I, TM, TN, WM, WN, NST, WGS) {32 * TM * WM, 32 * TN * WN, NST, WGS},
 constexpr TiledShape kTiledShapes[] = {HFRK_TILED_SHAPES(HFRK_TILED_ROW)};
 #undef HFRK_TILED_ROW
+#define HFRK_TILED_SAME(I, TM, TN, WM, WN, NST, WGS) \
+    static_assert(kTiledShapes[I].bm == 32 * TM * WM && kTiledShapes[I].bn == 32 * TN * WN && kTiledShapes[I].stages == NST && kTiledShapes[I].per_cu == WGS);
+HFRK_TILED_FOUR_WAVES(HFRK_TILED_SAME)
+#undef HFRK_TILED_SAME
 constexpr int kTiledShapeCount = sizeof(kTiledShapes) / sizeof(kTiledShapes[0]);
 constexpr int tiled_lds_bytes(const TiledShape& s) { return (s.bm + s.bn) * kTiledStage * s.stages; }
 

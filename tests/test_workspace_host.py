@@ -14,10 +14,11 @@ typedef struct { uint32_t x, y, z; } dim3_;
 static int allocations, capturing, last_error;
 static int clearing, early;          // memory is being cleared by work that nobody has waited for; a launch met it so
 static char own_stream;
-static uint32_t grid;
+static uint32_t grid, threads;
 static uintptr_t next_block = 1 << 20;
 void stand_in(int allocs, int capture) { allocations = allocs; capturing = capture; grid = 0; }
 uint32_t stand_in_grid(void) { return grid; }
+uint32_t stand_in_threads(void) { return threads; }
 static int fail(int e) { return last_error = e; }
 int hipGetDevice(int* d) { *d = 0; return 0; }
 int hipMalloc(void** p, size_t n) { if (allocations-- <= 0) return fail(2); *p = (void*)next_block; next_block += (n + 4095) & ~(size_t)4095; return 0; }
@@ -36,6 +37,7 @@ int __hipPushCallConfiguration(dim3_ grid_, dim3_ block_, size_t lds, void* stre
 int __hipPopCallConfiguration(dim3_* grid_, dim3_* block_, size_t* lds, void** stream) { *grid_ = g; *block_ = b; *lds = l; *stream = s; return 0; }
 int hipLaunchKernel(const void* f, dim3_ grid_, dim3_ block_, void** args, size_t lds, void* stream) {
     grid = grid_.x;
+    threads = block_.x;
     if (stream == &own_stream) clearing = 1;
     else if (clearing) early = 1;
     return 0;
@@ -105,6 +107,28 @@ stand_in.stand_in(2, 0)
 assert skinny(1) == _capi.SUCCESS
 """,
 }
+
+
+_CASES["waves of the 256 x 128 tile"] = """
+def waves(m, n, k, stride=None, packed=0, splits=1, shape=1):
+    stand_in.stand_in(100, 0)
+    plan = ctypes.byref(_capi.TiledPlan(shape, splits, 1))
+    assert lib.hfrk_tiled_gemm(4096, 8192, packed, 16384, None, 0, 64, 0, None, 0, m, n, k, stride or k, _capi.BF16, plan, 1) == _capi.SUCCESS
+    return stand_in.stand_in_threads() // 64
+
+for m in (65, 127, 128, 256, 300, 384, 512, 784, 1040, 1536, 4096):
+    for n in (8, 4104, 10240, 28672):
+        few = -(-m // 256) * -(-n // 128) <= 384
+        eight = m % 256 in range(1, 128) and (m <= 1024 or few)  # a last row of tiles less than half full, one of four or of few workgroups
+        for k in (128, 4096, 8320):
+            assert waves(m, n, k) == waves(m, n, k, k + 256) == 8
+            assert waves(m, n, k, k + 16) == waves(m, n, k, k + 64) == (8 if eight else 4)
+        for k in (16, 4112, 8256):
+            assert waves(m, n, k) == waves(m, n, k, k + 112) == waves(m, n, k, -(-k // 128) * 128) == (8 if eight else 4), (m, n, k)
+        assert waves(m, n, 4096, packed=1) == 8
+        assert waves(m, n, 4112, shape=0) == 8 and all(waves(m, n, 4112, shape=s) == 4 for s in (2, 3, 4))
+assert waves(1040, 4104, 4112) == 8 and waves(1040, 4104, 4112, splits=3) == 4  # 165 workgroups, 495
+"""
 
 
 @pytest.fixture(scope="module")
