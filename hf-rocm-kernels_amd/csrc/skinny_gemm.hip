@@ -1058,6 +1058,21 @@ int hfrk_llama_mlp(const void* input, const void* residual_in, void* residual, v
     uint8_t* const normalized = static_cast<uint8_t*>(scratch);
     uint8_t* const activated = normalized + ((size_t)m * hidden + 255) / 256 * 256;
     void* const both = activated + ((size_t)m * inter + 255) / 256 * 256;  // gate and up where they are launched apart from the SwiGLU
+    {
+        // A result that lies on another result or on the scratch is lost; an input that lies across one is read half overwritten.  The inputs may
+        // be `residual` or input_copy (the RMSNorm reads before it writes, piece by piece) and may lie on the output (nothing reads them by then).
+        const size_t bytes = (size_t)m * hidden * 2, scratch_bytes = hfrk_llama_mlp_scratch_bytes(m, hidden, inter);
+        auto apart = [](const void* p, size_t p_bytes, const void* q, size_t q_bytes) {
+            const uintptr_t a = reinterpret_cast<uintptr_t>(p), b = reinterpret_cast<uintptr_t>(q);
+            return !p || !q || a + p_bytes <= b || b + q_bytes <= a;
+        };
+        if (!apart(residual, bytes, input_copy, bytes) || !apart(residual, bytes, output, bytes) || !apart(input_copy, bytes, output, bytes)) return HFRK_BAD_SHAPE;
+        for (const void* in : {input, residual_in})
+            for (const void* out : {static_cast<const void*>(residual), static_cast<const void*>(input_copy)})
+                if (in != out && !apart(in, bytes, out, bytes)) return HFRK_BAD_SHAPE;
+        for (const void* t : {input, residual_in, static_cast<const void*>(residual), static_cast<const void*>(input_copy), static_cast<const void*>(output)})
+            if (!apart(t, bytes, scratch, scratch_bytes)) return HFRK_BAD_SHAPE;
+    }
     if (!residual_rms_into_takes(input, residual_in, residual, input_copy, rms_weight, normalized, hidden)) return HFRK_BAD_ALIGNMENT;
     auto gate_up_gemm = [&](bool fused, bool only_check) {
         return gemm_launch(normalized, gate_up, fused ? activated : both, nullptr, gate_up_output_scale, 0, nullptr, 0, fused ? down_input_scale : nullptr, m,

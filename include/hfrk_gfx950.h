@@ -282,7 +282,9 @@ int hfrk_linear_gemm(const void* A, const void* B, int packed, void* D, const vo
  *   output   <- (add_residual ? residual : 0) + down_output_scale * down(e4m3fn(silu(gate) * up / down_input_scale))
  * input, residual_in, residual, input_copy, output: 16-bit (dtype) [m, hidden], the first four and rms_weight 16-byte aligned; weights
  * row-major [2*inter, hidden] and [hidden, inter] with row strides, or the buffers hfrk_pack_weight wrote; hidden and inter multiples of 256;
- * scratch: hfrk_llama_mlp_scratch_bytes, 16-byte aligned.  *launched (may be NULL): 0 if the call was refused with nothing written. */
+ * scratch: hfrk_llama_mlp_scratch_bytes, 16-byte aligned.  residual, input_copy, output and scratch must not overlap (HFRK_BAD_SHAPE); input
+ * and residual_in may each be residual or input_copy, or lie apart from them, and may lie anywhere on the output.
+ * *launched (may be NULL): 0 if the call was refused with nothing written. */
 size_t hfrk_llama_mlp_scratch_bytes(int m, int hidden, int inter);
 int hfrk_llama_mlp(const void* input, const void* residual_in, void* residual, void* input_copy, const void* rms_weight, float epsilon,
                    const float* gate_up_input_scale, const void* gate_up, int gate_up_packed, int gate_up_stride, const float* gate_up_output_scale,

@@ -115,3 +115,15 @@ def test_calls_that_are_left_to_the_wrappers(monkeypatch):
         with pytest.raises(error):
             llama_mlp_combined_ops(x, res.clone(), *bad, add_residual=True, fused=True)
     assert not any(taken[2:])
+
+
+def test_results_that_overlap_are_not_written():
+    hidden = 512
+    norm, eps, w1, s1, s2, w2, s3, s4 = _block(hidden, 1024, torch.bfloat16)
+    x, res = _rows(4, hidden, torch.bfloat16)
+    out, before = torch.zeros_like(x), (x.clone(), res.clone())
+    half = torch.zeros(6 * hidden, dtype=torch.bfloat16, device="cuda")
+    for residual_out, copy, output in ((res, None, res), (res, res, out), (out, None, out), (half[:4 * hidden].view(4, hidden), half[2 * hidden:].view(4, hidden), out)):
+        assert not MODULE._llama_mlp(x, res, residual_out, copy, norm, eps, w1, -1, s1, s2, w2, -1, s3, s4, True, output)
+        torch.cuda.synchronize()
+        assert torch.equal(x, before[0]) and torch.equal(res, before[1]) and not out.any() and not half.any()

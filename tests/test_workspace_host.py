@@ -14,9 +14,10 @@ typedef struct { uint32_t x, y, z; } dim3_;
 static int allocations, capturing, last_error;
 static int clearing, early;          // memory is being cleared by work that nobody has waited for; a launch met it so
 static char own_stream;
-static uint32_t grid, threads;
+static uint32_t grid, threads, launches;
 static uintptr_t next_block = 1 << 20;
-void stand_in(int allocs, int capture) { allocations = allocs; capturing = capture; grid = 0; }
+void stand_in(int allocs, int capture) { allocations = allocs; capturing = capture; grid = launches = 0; }
+uint32_t stand_in_launches(void) { return launches; }
 uint32_t stand_in_grid(void) { return grid; }
 uint32_t stand_in_threads(void) { return threads; }
 static int fail(int e) { return last_error = e; }
@@ -38,6 +39,7 @@ int __hipPopCallConfiguration(dim3_* grid_, dim3_* block_, size_t* lds, void** s
 int hipLaunchKernel(const void* f, dim3_ grid_, dim3_ block_, void** args, size_t lds, void* stream) {
     grid = grid_.x;
     threads = block_.x;
+    ++launches;
     if (stream == &own_stream) clearing = 1;
     else if (clearing) early = 1;
     return 0;
@@ -58,6 +60,17 @@ def tiled(stream, plan=None):
 
 def skinny(stream, plan=None):  # (64 rows of a narrow weight: k is split between workgroups)
     return lib.hfrk_skinny_gemm_fused(4096, 8192, 16384, None, 64, 0, None, 0, None, 64, 64, 16384, 16384, _capi.BF16, 0, plan, stream)
+
+def block(stream=1, m=4, hidden=512, inter=512, **at):
+    # tensors of m * hidden 16-bit values, `place` apart unless `at` says where one lies, in units of one tensor
+    place, launched, size = 1 << 24, ctypes.c_int(7), m * hidden * 2
+    names = ["input", "residual_in", "residual", "input_copy", "output", "scratch"]
+    where = {{x: (i + 1) * place for i, x in enumerate(names)}}
+    where.update((x, v if v is None else int((names.index(v[0]) + 1) * place + v[1] * size)) for x, v in at.items())
+    status = lib.hfrk_llama_mlp(where["input"], where["residual_in"], where["residual"], where["input_copy"], 4096, 1e-5, 64, 1 << 30, 0, hidden,
+                                64, 64, 1 << 31, 0, inter, 64, 1, where["output"], where["scratch"], m, hidden, inter, _capi.BF16,
+                                ctypes.byref(launched), stream)
+    return status, launched.value, stand_in.stand_in_launches()
 
 chosen = _capi.TiledPlan()
 assert lib.hfrk_tiled_gemm_plan(m, n, k, ctypes.byref(chosen)) == _capi.SUCCESS and chosen.splits > 1
@@ -128,6 +141,24 @@ for m in (65, 127, 128, 256, 300, 384, 512, 784, 1040, 1536, 4096):
         assert waves(m, n, 4096, packed=1) == 8
         assert waves(m, n, 4112, shape=0) == 8 and all(waves(m, n, 4112, shape=s) == 4 for s in (2, 3, 4))
 assert waves(1040, 4104, 4112) == 8 and waves(1040, 4104, 4112, splits=3) == 4  # 165 workgroups, 495
+"""
+
+
+_CASES["a block whose results would overlap is refused"] = """
+for m in (1, 4, 64):
+    for at in ({"input_copy": ("residual", 0)}, {"output": ("residual", 0)}, {"output": ("input_copy", 0)}, {"output": ("residual", .5)},
+               {"input_copy": ("residual", -.5)}, {"input": ("residual", .5)}, {"residual_in": ("residual", -.25)}, {"input": ("input_copy", .75)},
+               {"residual_in": ("input_copy", .25)}, {"scratch": ("input", 0)}, {"scratch": ("residual_in", .5)}, {"scratch": ("residual", 0)},
+               {"scratch": ("input_copy", 0)}, {"scratch": ("output", .5)}, {"output": ("scratch", .125)}):
+        stand_in.stand_in(100, 0)
+        assert block(m=m, **at) == (_capi.BAD_SHAPE, 0, 0), (m, at)
+    for at in ({}, {"input_copy": None}, {"residual": ("residual_in", 0)}, {"input_copy": ("input", 0)}, {"input": ("residual_in", 0)},
+               {"input": ("residual", 0)}, {"residual_in": ("input_copy", 0)}, {"output": ("input", 0)}, {"output": ("residual_in", .5)},
+               {"residual": ("input_copy", 1)}, {"residual": ("input_copy", -1)},
+               {"residual": ("residual_in", 0), "input_copy": None, "output": ("input", 0)}):
+        stand_in.stand_in(100, 0)
+        status, launched, launches = block(m=m, **at)
+        assert (status, launched) == (_capi.SUCCESS, 1) and launches >= 3, (m, at, status, launches)
 """
 
 
