@@ -27,6 +27,7 @@
 //    every slab of the panel it writes D directly, otherwise it parks its fp32 partial in the workspace and the
 //    workgroup that arrives last (per-panel counter) adds the partials in workgroup order -- a fixed order, so
 //    results are bit-reproducible -- applies the scales once, adds D (accumulate mode) and rounds once.
+#include <algorithm>
 #include <functional>
 #include <mutex>
 #include <thread>
@@ -659,7 +660,8 @@ static int choose_plan(int m, int n, int k, bool packed, hfrk_gemm_plan* plan) {
 // D = (base ? base : 0) + scale_a x scale_b x A.B   (epilogue 0), or the fused SwiGLU form (epilogue 1).
 // use_static: partial sums and counters go to this device's `scratch` array instead of the stream's workspace.
 // base_row: base is one row of n values, added to every row.
-// only_check: everything that can refuse the call (arguments, plan, the stream's workspace), and no launch.
+// given: partial sums and counters go to this memory instead of the stream's workspace.
+// needs: raised to what the call takes of a workspace; everything else that can refuse it is checked, and nothing is launched.
 // rms: the activations are not read from A but built by the kernel's RMSNorm prologue from these 16-bit tensors.
 struct RmsPrologue {
     const void* input;
@@ -670,10 +672,21 @@ struct RmsPrologue {
     float epsilon;
     int dtype;
 };
+constexpr int kGivenCounters = 1 << 16;  // at the front of a given workspace, partial sums behind them
+struct GivenWorkspace {
+    unsigned char* ptr;
+    size_t bytes;
+};
+struct GemmNeeds {
+    size_t ws_bytes;
+    long counters;
+    size_t given_bytes() const { return ws_bytes || counters ? kGivenCounters * sizeof(int) + ws_bytes : 0; }
+};
 static int gemm_launch(const void* A, const void* B, void* D, const void* base, const float* scale_a, int sa_stride,
                        const float* scale_b, int sb_stride, const float* out_scale, int m, int n, int k, int b_stride,
                        int d_dtype, int epilogue, const hfrk_gemm_plan* user_plan, hipStream_t stream, bool packed = false,
-                       bool use_static = false, const RmsPrologue* rms = nullptr, bool base_row = false, bool only_check = false) {
+                       bool use_static = false, const RmsPrologue* rms = nullptr, bool base_row = false,
+                       const GivenWorkspace* given = nullptr, GemmNeeds* needs = nullptr) {
     if (packed) b_stride = k;
     if (m < 1 || m > HFRK_GEMM_MAX_M || n < 1 || k < 1 || b_stride < k) return HFRK_BAD_SHAPE;
     if (k % 16 != 0 || (packed && k % 256 != 0)) return HFRK_K_NOT_DIVISIBLE_BY_WARPTILE_K;
@@ -715,12 +728,12 @@ static int gemm_launch(const void* A, const void* B, void* D, const void* base, 
         const int first = kStreamMaxM;
         const size_t row_bytes = (size_t)n * 2;
         int rc = gemm_launch(A, B, D, base, scale_a, sa_stride, scale_b, sb_stride, out_scale, first, n, k, b_stride, d_dtype,
-                             epilogue, nullptr, stream, packed, use_static, nullptr, base_row);
+                             epilogue, nullptr, stream, packed, use_static, nullptr, base_row, given, needs);
         if (rc != HFRK_SUCCESS) return rc;
         return gemm_launch(static_cast<const uint8_t*>(A) + (size_t)first * k, B, static_cast<uint8_t*>(D) + first * row_bytes,
                            base && !base_row ? static_cast<const uint8_t*>(base) + first * row_bytes : base, scale_a + (size_t)first * sa_stride,
                            sa_stride, scale_b, sb_stride, out_scale, m - first, n, k, b_stride, d_dtype, epilogue, nullptr, stream,
-                           packed, use_static, nullptr, base_row);
+                           packed, use_static, nullptr, base_row, given, needs);
     }
     hfrk_gemm_plan p;
     if (user_plan) {
@@ -756,6 +769,12 @@ static int gemm_launch(const void* A, const void* B, void* D, const void* base, 
         if (rc != HFRK_SUCCESS) return rc;
     }
 
+    if (needs) {
+        if (plan_ws_bytes(p) > kWsFloats * sizeof(float) || plan_counters(p) > kMaxPanels) return HFRK_BAD_SHAPE;
+        needs->ws_bytes = std::max(needs->ws_bytes, plan_ws_bytes(p));
+        needs->counters = std::max(needs->counters, plan_counters(p));
+        return HFRK_SUCCESS;
+    }
     int dev = 0;
     HFRK_HIP_TRY(hipGetDevice(&dev));
     Workspace st;
@@ -773,12 +792,16 @@ static int gemm_launch(const void* A, const void* B, void* D, const void* base, 
         st.counters = reinterpret_cast<int*>(ptr + kStaticWsBytes);
         ws_bytes = kStaticWsBytes;
         counters = kStaticCounters;
+    } else if (given) {
+        counters = kGivenCounters;
+        ws_bytes = given->bytes < counters * sizeof(int) ? 0 : given->bytes - counters * sizeof(int);
+        st.counters = reinterpret_cast<int*>(given->ptr);
+        st.ws = reinterpret_cast<float*>(given->ptr + counters * sizeof(int));
     } else {
         const int rc = workspace_for(dev, stream, &st);
         if (rc != HFRK_SUCCESS) return rc;
     }
-    if (plan_ws_bytes(p) > ws_bytes || plan_counters(p) > counters) return use_static ? HFRK_EXCEEDS_SCRATCH : HFRK_BAD_SHAPE;
-    if (only_check) return HFRK_SUCCESS;
+    if (plan_ws_bytes(p) > ws_bytes || plan_counters(p) > counters) return use_static || given ? HFRK_EXCEEDS_SCRATCH : HFRK_BAD_SHAPE;
     if (use_static) {
         // The array keeps whatever the last call (or a launch that never finished) left: the counters of this plan start at zero.
         const int count = (int)plan_counters(p);
@@ -873,6 +896,47 @@ static int gemm_launch(const void* A, const void* B, void* D, const void* base, 
     }
     return HFRK_INVALID_CONFIG;
 }
+
+// ---- the MLP block: what it launches behind its RMSNorm --------------------------------------------------------------------
+static bool block_sizes_ok(int m, int hidden, int inter) {
+    return m >= 1 && m <= HFRK_GEMM_MAX_M && hidden >= 1 && inter >= 1 && hidden % 256 == 0 && inter % 256 == 0 && inter <= (1 << 28);
+}
+
+struct BlockGemms {
+    uint8_t *normalized, *activated;
+    void* both;  // gate and up where they are launched apart from the SwiGLU
+    void* output;
+    const void* addend;
+    const void *gate_up, *down;
+    bool gate_up_packed, down_packed;
+    int gate_up_stride, down_stride;
+    const float *gate_up_scale, *activation_scale, *down_scale;
+    int m, hidden, inter, dtype;
+    hipStream_t stream;
+    const GivenWorkspace* given;
+
+    int gate_up_gemm(bool fused, GemmNeeds* needs = nullptr) const {
+        return gemm_launch(normalized, gate_up, fused ? static_cast<void*>(activated) : both, nullptr, gate_up_scale, 0, nullptr, 0,
+                           fused ? activation_scale : nullptr, m, 2 * inter, hidden, gate_up_stride, dtype,
+                           fused ? HFRK_EPILOGUE_SWIGLU : HFRK_EPILOGUE_NONE, nullptr, stream, gate_up_packed, false, nullptr, false, given, needs);
+    }
+    int down_gemm(GemmNeeds* needs = nullptr) const {
+        return gemm_launch(activated, down, output, addend, down_scale, 0, nullptr, 0, nullptr, m, hidden, inter, down_stride, dtype, HFRK_EPILOGUE_NONE,
+                           nullptr, stream, down_packed, false, nullptr, false, given, needs);
+    }
+    // Whether both can run, what they take of a workspace, and whether the SwiGLU is the gate_up GEMM's epilogue: skinny_gemm_swiglu
+    // (operators/skinny_gemm/wrapped.py) has the same rule and the figures behind it.
+    int check(bool* fused, GemmNeeds* needs) const {
+        const bool window = hidden == 2048 || hidden == 4096;
+        *fused = m <= 16 || window || (m <= kRowsMaxM && !gate_up_packed && 2L * inter * hidden <= (128L << 20));
+        int rc = *fused ? gate_up_gemm(true, needs) : HFRK_BAD_SHAPE;
+        if (rc == HFRK_BAD_SHAPE && m > 16 && !(*fused && window)) {
+            *fused = false;
+            rc = gate_up_gemm(false, needs);
+        }
+        return rc == HFRK_SUCCESS ? down_gemm(needs) : rc;
+    }
+};
 
 }  // namespace hfrk
 
@@ -1044,15 +1108,36 @@ size_t hfrk_llama_mlp_scratch_bytes(int m, int hidden, int inter) {
     return normalized + activated + (m > 16 ? (size_t)m * inter * 4 : 0);
 }
 
+size_t hfrk_llama_mlp_workspace_bytes(int m, int hidden, int inter, int gate_up_packed, int down_packed) {
+    if (!hfrk::block_sizes_ok(m, hidden, inter)) return 0;
+    unsigned char* const any = reinterpret_cast<unsigned char*>(4096);  // looked at for its alignment only
+    float* const scale = reinterpret_cast<float*>(any);
+    const hfrk::BlockGemms gemms{any, any, any, any, nullptr, any, any, gate_up_packed != 0, down_packed != 0, hidden, inter, scale, scale, scale,
+                                 m, hidden, inter, HFRK_BF16, nullptr, nullptr};
+    bool fused = false;
+    hfrk::GemmNeeds needs{};
+    return gemms.check(&fused, &needs) == HFRK_SUCCESS ? needs.given_bytes() : 0;
+}
+
 int hfrk_llama_mlp(const void* input, const void* residual_in, void* residual, void* input_copy, const void* rms_weight, float epsilon,
                    const float* gate_up_input_scale, const void* gate_up, int gate_up_packed, int gate_up_stride, const float* gate_up_output_scale,
                    const float* down_input_scale, const void* down, int down_packed, int down_stride, const float* down_output_scale, int add_residual,
                    void* output, void* scratch, int m, int hidden, int inter, int dtype, int* launched, void* stream) {
+    return hfrk_llama_mlp_owned(input, residual_in, residual, input_copy, rms_weight, epsilon, gate_up_input_scale, gate_up, gate_up_packed, gate_up_stride,
+                                gate_up_output_scale, down_input_scale, down, down_packed, down_stride, down_output_scale, add_residual, output, scratch,
+                                nullptr, 0, m, hidden, inter, dtype, launched, stream);
+}
+
+int hfrk_llama_mlp_owned(const void* input, const void* residual_in, void* residual, void* input_copy, const void* rms_weight, float epsilon,
+                         const float* gate_up_input_scale, const void* gate_up, int gate_up_packed, int gate_up_stride, const float* gate_up_output_scale,
+                         const float* down_input_scale, const void* down, int down_packed, int down_stride, const float* down_output_scale, int add_residual,
+                         void* output, void* scratch, void* workspace, size_t workspace_bytes, int m, int hidden, int inter, int dtype, int* launched,
+                         void* stream) {
     using namespace hfrk;
     const hipStream_t s = static_cast<hipStream_t>(stream);
     if (launched) *launched = 0;
     if (!input || !residual_in || !residual || !rms_weight || !gate_up_input_scale || !down_input_scale || !output || !scratch) return HFRK_BAD_SHAPE;
-    if (m < 1 || m > HFRK_GEMM_MAX_M || hidden < 1 || inter < 1 || hidden % 256 != 0 || inter % 256 != 0 || inter > (1 << 28)) return HFRK_BAD_SHAPE;
+    if (!block_sizes_ok(m, hidden, inter)) return HFRK_BAD_SHAPE;
     if (!(epsilon > 0.f)) return HFRK_BAD_SHAPE;
     if (dtype != HFRK_F16 && dtype != HFRK_BF16) return HFRK_BAD_DTYPE;
     uint8_t* const normalized = static_cast<uint8_t*>(scratch);
@@ -1071,33 +1156,33 @@ int hfrk_llama_mlp(const void* input, const void* residual_in, void* residual, v
             for (const void* out : {static_cast<const void*>(residual), static_cast<const void*>(input_copy)})
                 if (in != out && !apart(in, bytes, out, bytes)) return HFRK_BAD_SHAPE;
         for (const void* t : {input, residual_in, static_cast<const void*>(residual), static_cast<const void*>(input_copy), static_cast<const void*>(output)})
-            if (!apart(t, bytes, scratch, scratch_bytes)) return HFRK_BAD_SHAPE;
+            if (!apart(t, bytes, scratch, scratch_bytes) || !apart(t, bytes, workspace, workspace_bytes)) return HFRK_BAD_SHAPE;
+        if (!apart(scratch, scratch_bytes, workspace, workspace_bytes)) return HFRK_BAD_SHAPE;
     }
     if (!residual_rms_into_takes(input, residual_in, residual, input_copy, rms_weight, normalized, hidden)) return HFRK_BAD_ALIGNMENT;
-    auto gate_up_gemm = [&](bool fused, bool only_check) {
-        return gemm_launch(normalized, gate_up, fused ? activated : both, nullptr, gate_up_output_scale, 0, nullptr, 0, fused ? down_input_scale : nullptr, m,
-                           2 * inter, hidden, gate_up_stride, dtype, fused ? HFRK_EPILOGUE_SWIGLU : HFRK_EPILOGUE_NONE, nullptr, s, gate_up_packed != 0,
-                           false, nullptr, false, only_check);
-    };
-    auto down_gemm = [&](bool only_check) {
-        return gemm_launch(activated, down, output, add_residual ? residual : nullptr, down_output_scale, 0, nullptr, 0, nullptr, m, hidden, inter, down_stride,
-                           dtype, HFRK_EPILOGUE_NONE, nullptr, s, down_packed != 0, false, nullptr, false, only_check);
-    };
-    // Nothing is launched unless everything can be: a caller that goes another way must find the residual as it was.  Where the SwiGLU is
-    // the gate_up GEMM's epilogue: skinny_gemm_swiglu (operators/skinny_gemm/wrapped.py) has the same rule and the figures behind it.
-    const bool window = hidden == 2048 || hidden == 4096;
-    bool fused = m <= 16 || window || (m <= kRowsMaxM && !gate_up_packed && 2L * inter * hidden <= (128L << 20));
-    int rc = fused ? gate_up_gemm(true, true) : HFRK_BAD_SHAPE;
-    if (rc == HFRK_BAD_SHAPE && m > 16 && !(fused && window)) {
-        fused = false;
-        rc = gate_up_gemm(false, true);
+    if (reinterpret_cast<uintptr_t>(workspace) & 15) return HFRK_BAD_ALIGNMENT;
+    const GivenWorkspace given{static_cast<unsigned char*>(workspace), workspace_bytes};
+    const BlockGemms gemms{normalized, activated, both, output, add_residual ? residual : nullptr, gate_up, down, gate_up_packed != 0, down_packed != 0,
+                           gate_up_stride, down_stride, gate_up_output_scale, down_input_scale, down_output_scale, m, hidden, inter, dtype, s,
+                           workspace ? &given : nullptr};
+    // Nothing is launched unless everything can be: a caller that goes another way must find the residual as it was.
+    bool fused = false;
+    GemmNeeds needs{};
+    int rc = gemms.check(&fused, &needs);
+    if (rc != HFRK_SUCCESS) return rc;
+    if (workspace) {
+        if (needs.given_bytes() > workspace_bytes || needs.counters > kGivenCounters) return HFRK_EXCEEDS_SCRATCH;
+    } else if (needs.given_bytes() != 0) {
+        int dev = 0;
+        Workspace st;
+        HFRK_HIP_TRY(hipGetDevice(&dev));
+        if ((rc = workspace_for(dev, s, &st)) != HFRK_SUCCESS) return rc;
     }
-    if (rc != HFRK_SUCCESS || (rc = down_gemm(true)) != HFRK_SUCCESS) return rc;
     if (launched) *launched = 1;
     rc = residual_rms_into(input, residual_in, residual, input_copy, rms_weight, gate_up_input_scale, epsilon, normalized, m, hidden, dtype, s);
-    if (rc == HFRK_SUCCESS) rc = gate_up_gemm(fused, false);
+    if (rc == HFRK_SUCCESS) rc = gemms.gate_up_gemm(fused);
     if (rc == HFRK_SUCCESS && !fused) rc = hfrk_swiglu(both, down_input_scale, activated, nullptr, m, inter, 0, dtype, 0, 0, stream);
-    return rc == HFRK_SUCCESS ? down_gemm(false) : rc;
+    return rc == HFRK_SUCCESS ? gemms.down_gemm() : rc;
 }
 
 int hfrk_skinny_gemm_rms_plan(int m, int n, int k, int epilogue, hfrk_gemm_plan* plan) {

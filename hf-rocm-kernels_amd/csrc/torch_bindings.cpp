@@ -600,11 +600,12 @@ bool skinny_gemm_into(const at::Tensor& A, const at::Tensor& B, const at::Tensor
 // The fused decoder MLP block (combined_ops/llama_mlp.py) as one operator: its Python side took about 35 us per call, the block of 8 rows
 // of 4096 x 14336 35 us of kernels and that of one row of 2048 x 6144 less than half of it.  residual_out <- input + residual (it may be
 // `residual`), input_copy <- input, and the block's output, into `output` where one is given.  Weights are [k, n] views or (n >= 0) packed buffers.
-// False, with nothing launched, for everything that the wrappers would convert, copy or refuse.
+// False, with nothing launched, for everything that the wrappers would convert, copy or refuse.  memory: scratch, and behind it the workspace of
+// hfrk_llama_mlp_owned; without it scratch is allocated and the workspace is the stream's.
 bool llama_mlp(const at::Tensor& input, const at::Tensor& residual, at::Tensor& residual_out, const std::optional<at::Tensor>& input_copy,
                const at::Tensor& rms_weight, double epsilon, const at::Tensor& gate_up, int64_t gate_up_n, const at::Tensor& gate_up_input_scale,
                const at::Tensor& gate_up_output_scale, const at::Tensor& down, int64_t down_n, const at::Tensor& down_input_scale,
-               const at::Tensor& down_output_scale, bool add_residual, at::Tensor& output) {
+               const at::Tensor& down_output_scale, bool add_residual, at::Tensor& output, const std::optional<at::Tensor>& memory) {
     if (!input.is_cuda() || input.dim() != 2 || !is_16bit(input.scalar_type())) return false;
     const int64_t m = input.size(0), hidden = input.size(1);
     auto like_input = [&](const at::Tensor& t) {
@@ -638,15 +639,20 @@ bool llama_mlp(const at::Tensor& input, const at::Tensor& residual, at::Tensor& 
     if (n < 512 || inter % 256 != 0 || n % 2 != 0 || columns(down, down_n, inter) != hidden) return false;
 
     DeviceScope scope(input);
-    at::Tensor scratch = at::empty({(int64_t)hfrk_llama_mlp_scratch_bytes((int)m, (int)hidden, (int)inter)}, input.options().dtype(at::kByte));
+    const size_t scratch_bytes = hfrk_llama_mlp_scratch_bytes((int)m, (int)hidden, (int)inter);
+    if (memory.has_value() && (memory->scalar_type() != at::kByte || !memory->is_contiguous() || memory->device() != input.device() ||
+                               (size_t)memory->numel() < scratch_bytes))
+        return false;
+    at::Tensor scratch = memory.has_value() ? *memory : at::empty({(int64_t)scratch_bytes}, input.options().dtype(at::kByte));
+    uint8_t* const workspace = memory.has_value() ? scratch.data_ptr<uint8_t>() + scratch_bytes : nullptr;
     int launched = 0;
-    const int status = hfrk_llama_mlp(
+    const int status = hfrk_llama_mlp_owned(
         input.data_ptr(), residual.data_ptr(), residual_out.data_ptr(), input_copy.has_value() ? input_copy->data_ptr() : nullptr,
         rms_weight.data_ptr(), (float)epsilon, gate_up_input_scale.data_ptr<float>(), gate_up.data_ptr(), gate_up_n >= 0 ? 1 : 0,
         gate_up_n >= 0 ? (int)hidden : (int)gate_up.stride(1), gate_up_output_scale.data_ptr<float>(), down_input_scale.data_ptr<float>(),
         down.data_ptr(), down_n >= 0 ? 1 : 0, down_n >= 0 ? (int)inter : (int)down.stride(1), down_output_scale.data_ptr<float>(),
-        add_residual ? 1 : 0, output.data_ptr(), scratch.data_ptr(), (int)m, (int)hidden, (int)inter,
-        input.scalar_type() == at::kBFloat16 ? HFRK_BF16 : HFRK_F16, &launched, current_stream(input));
+        add_residual ? 1 : 0, output.data_ptr(), scratch.data_ptr(), workspace, workspace ? (size_t)scratch.numel() - scratch_bytes : 0, (int)m,
+        (int)hidden, (int)inter, input.scalar_type() == at::kBFloat16 ? HFRK_BF16 : HFRK_F16, &launched, current_stream(input));
     if (launched) raise_on(status, "llama_mlp");
     return status == HFRK_SUCCESS;
 }
@@ -794,7 +800,7 @@ TORCH_LIBRARY(_HFRK_C, ops) {
     ops.def(
         "llama_mlp(Tensor input, Tensor residual, Tensor(a!) residual_out, Tensor(b!)? input_copy, Tensor rms_weight, float epsilon, Tensor gate_up, "
         "int gate_up_n, Tensor gate_up_input_scale, Tensor gate_up_output_scale, Tensor down, int down_n, Tensor down_input_scale, "
-        "Tensor down_output_scale, bool add_residual, Tensor(c!) output) -> bool");
+        "Tensor down_output_scale, bool add_residual, Tensor(c!) output, Tensor(d!)? memory=None) -> bool");
     ops.impl("llama_mlp", c10::kCUDA, &llama_mlp);
     ops.impl("llama_mlp", torch::dispatch(c10::DispatchKey::Autograd, torch::CppFunction::makeFallthrough()));
 

@@ -90,6 +90,8 @@ SIGNATURES = {
     "hfrk_linear_gemm": (_i, [_p, _p, _i, _p, _p, _i, _p, _i, _p, _i, _i, _i, _i, _i, _i, _p]),
     "hfrk_llama_mlp_scratch_bytes": (ctypes.c_size_t, [_i, _i, _i]),
     "hfrk_llama_mlp": (_i, [_p] * 5 + [_f, _p, _p, _i, _i, _p, _p, _p, _i, _i, _p, _i, _p, _p, _i, _i, _i, _i, ctypes.POINTER(_i), _p]),
+    "hfrk_llama_mlp_workspace_bytes": (ctypes.c_size_t, [_i] * 5),
+    "hfrk_llama_mlp_owned": (_i, [_p] * 5 + [_f, _p, _p, _i, _i, _p, _p, _p, _i, _i, _p, _i, _p, _p, _p, ctypes.c_size_t, _i, _i, _i, _i, ctypes.POINTER(_i), _p]),
     "hfrk_tiled_gemm_plan": (_i, [_i, _i, _i, ctypes.POINTER(TiledPlan)]),
     "hfrk_tiled_gemm": (_i, [_p, _p, _i, _p, _p, _i, _p, _i, _p, _i, _i, _i, _i, _i, _i, ctypes.POINTER(TiledPlan), _p]),
     "hfrk_residual_rms": (_i, [_p, _p, _p, _p, _f, _p, _p, _i, _i, _i, _i, _i, _i, _i, _p]),

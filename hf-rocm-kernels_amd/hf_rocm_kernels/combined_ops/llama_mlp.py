@@ -5,6 +5,7 @@ from torch import Tensor
 
 from hf_rocm_kernels import residual_rms, skinny_gemm, skinny_gemm_add, skinny_gemm_rms, skinny_gemm_scaled, skinny_gemm_swiglu, swiglu
 
+from .. import _capi
 from ..utils.dispatch import runs_now
 from ..utils.weight_format import PackedWeight
 
@@ -12,14 +13,23 @@ _llama_mlp = torch.ops._HFRK_C.llama_mlp.default
 
 
 def _native_block(attn_output, residual, residual_out, attn_copy, output, rms_weight, rms_epsilon, gate_up_weight, gate_up_input_scale,
-                  gate_up_output_scale, down_weight, down_input_scale, down_output_scale, add_residual) -> bool:
+                  gate_up_output_scale, down_weight, down_input_scale, down_output_scale, add_residual, memory=None) -> bool:
     """The fused block as one native operator, into the given tensors; False, with nothing written, if this is not one of its calls.
-    For calls that run now (utils/dispatch.py)."""
+    For calls that run now (utils/dispatch.py).  memory: bytes of `_block_memory`; without them scratch is allocated and partial sums go to the
+    stream's workspace."""
     gate_up_packed, down_packed = isinstance(gate_up_weight, PackedWeight), isinstance(down_weight, PackedWeight)
     return _llama_mlp(attn_output, residual, residual_out, attn_copy, rms_weight, rms_epsilon,
                       gate_up_weight.data if gate_up_packed else gate_up_weight, gate_up_weight.n if gate_up_packed else -1,
                       gate_up_input_scale, gate_up_output_scale, down_weight.data if down_packed else down_weight,
-                      down_weight.n if down_packed else -1, down_input_scale, down_output_scale, add_residual, output)
+                      down_weight.n if down_packed else -1, down_input_scale, down_output_scale, add_residual, output, memory)
+
+
+def _block_memory(rows, hidden, gate_up_weight, down_weight, device) -> Tensor:
+    """Scratch and workspace of a block's calls, the workspace's arrival counters clear."""
+    lib, inter = _capi.load(), down_weight.size(0)
+    size = lib.hfrk_llama_mlp_scratch_bytes(rows, hidden, inter)
+    size += lib.hfrk_llama_mlp_workspace_bytes(rows, hidden, inter, isinstance(gate_up_weight, PackedWeight), isinstance(down_weight, PackedWeight))
+    return torch.zeros(size, dtype=torch.uint8, device=device)
 
 
 def llama_mlp_combined_ops(
@@ -151,6 +161,8 @@ class LlamaMlpGraph:
             with torch.cuda.graph(self.graph, stream=self._stream):
                 self.mlp_output, residual_out = llama_mlp_combined_ops(self.attn_output, self.residual, *args, **kwargs)
         assert residual_out.data_ptr() == self.residual.data_ptr()  # updated in place
+        # a call allocates nothing and needs no workspace of the stream it is made on, as a replay
+        self._memory = _block_memory(rows, hidden, gate_up_weight, down_weight, device) if fused else None
         torch.cuda.synchronize(device)
 
     def __call__(self, attn_output: Tensor, residual: Tensor) -> Tuple[Tensor, Tensor]:
@@ -160,7 +172,8 @@ class LlamaMlpGraph:
         go out from native code, which costs the GPU less than starting a graph (8 rows of 4096 x 14336: 46.6 us with two copies in front,
         41.9 for the replay alone, 35.9 this way; one row of 2048 x 6144 31.6, 23.4, 17.0)."""
         if self._fused and runs_now(attn_output) and not torch.cuda.is_current_stream_capturing():
-            if _native_block(attn_output, residual, self.residual, self.attn_output, self.mlp_output, *self._operands, self._add_residual):
+            if _native_block(attn_output, residual, self.residual, self.attn_output, self.mlp_output, *self._operands, self._add_residual,
+                             self._memory):
                 return self.mlp_output, self.residual
         self.attn_output.copy_(attn_output)
         self.residual.copy_(residual)

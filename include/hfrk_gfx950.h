@@ -43,7 +43,7 @@ enum hfrk_status {
     HFRK_NOT_INITIALISED = 11,              /* workspace missing and the stream is capturing (call hfrk_init first) */
     HFRK_BAD_FILE = 12,                     /* a plan-table file that cannot be read or is not a plan table */
     HFRK_NO_WORKSPACE = 13,                 /* more streams hold a split-K workspace than the library allows (hfrk_release_stream) */
-    HFRK_EXCEEDS_SCRATCH = 14               /* hfrk_skinny_gemm_noalloc: the plan needs more than the built-in scratch array holds */
+    HFRK_EXCEEDS_SCRATCH = 14               /* a plan needs more than the built-in scratch array (hfrk_skinny_gemm_noalloc) or the given workspace holds */
 };
 
 /* Element types of 16-bit tensors. */
@@ -290,6 +290,18 @@ int hfrk_llama_mlp(const void* input, const void* residual_in, void* residual, v
                    const float* gate_up_input_scale, const void* gate_up, int gate_up_packed, int gate_up_stride, const float* gate_up_output_scale,
                    const float* down_input_scale, const void* down, int down_packed, int down_stride, const float* down_output_scale, int add_residual,
                    void* output, void* scratch, int m, int hidden, int inter, int dtype, int* launched, void* stream);
+
+/* The same on memory of the caller's: partial sums and arrival counters go to `workspace` instead of one that the stream owns, so the call
+ * allocates nothing and claims nothing on a stream first met, under a capture neither.  hfrk_llama_mlp_workspace_bytes of it (0: the plans chosen
+ * now need none), 16-byte aligned and apart from every tensor, zero before its first call and used by one call at a time; a call leaves its
+ * counters zero.  A call whose plans have come to need more
+ * (hfrk_plan_table_set) is refused with HFRK_EXCEEDS_SCRATCH.  workspace NULL: the stream's. */
+size_t hfrk_llama_mlp_workspace_bytes(int m, int hidden, int inter, int gate_up_packed, int down_packed);
+int hfrk_llama_mlp_owned(const void* input, const void* residual_in, void* residual, void* input_copy, const void* rms_weight, float epsilon,
+                         const float* gate_up_input_scale, const void* gate_up, int gate_up_packed, int gate_up_stride, const float* gate_up_output_scale,
+                         const float* down_input_scale, const void* down, int down_packed, int down_stride, const float* down_output_scale, int add_residual,
+                         void* output, void* scratch, void* workspace, size_t workspace_bytes, int m, int hidden, int inter, int dtype, int* launched,
+                         void* stream);
 
 /* How one tiled GEMM call is decomposed: an index into the library's tile shapes (0: 256 x 256, 1: 256 x 128, 2: 128 x 128,
  * 3: 128 x 64, 4: 64 x 64 rows x columns of D per workgroup), how many workgroups share a tile's k, and how many rows of tiles

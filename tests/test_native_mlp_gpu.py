@@ -8,6 +8,7 @@ import torch
 
 from hf_rocm_kernels.combined_ops.llama_mlp import LlamaMlpGraph, llama_mlp_combined_ops
 from hf_rocm_kernels.utils.weight_format import pack_weight
+from test_gemm_gpu import all_plans
 
 pytestmark = pytest.mark.gpu
 MODULE = sys.modules["hf_rocm_kernels.combined_ops.llama_mlp"]
@@ -127,3 +128,67 @@ def test_results_that_overlap_are_not_written():
         assert not MODULE._llama_mlp(x, res, residual_out, copy, norm, eps, w1, -1, s1, s2, w2, -1, s3, s4, True, output)
         torch.cuda.synchronize()
         assert torch.equal(x, before[0]) and torch.equal(res, before[1]) and not out.any() and not half.any()
+
+
+@pytest.mark.parametrize("m,packed", [(8, False), (16, True), (64, False), (64, True)])
+def test_graph_call_takes_no_memory_and_no_workspace(m, packed, monkeypatch):
+    """As a replay: the object holds what its calls need, also on a stream that has launched nothing before."""
+    from hf_rocm_kernels import _capi
+    lib, taken = _capi.load(), _counted(monkeypatch)
+    hidden, inter = 1024, 5120
+    args = _block(hidden, inter, torch.bfloat16, (packed, packed))
+    block = LlamaMlpGraph(m, hidden, *args)
+    rows = [_rows(m, hidden, torch.bfloat16, seed) for seed in range(4)]
+    want = [[t.clone() for t in llama_mlp_combined_ops(x, res.clone(), *args, add_residual=True, fused=True)] for x, res in rows]
+    assert lib.hfrk_llama_mlp_workspace_bytes(64, hidden, inter, 0, 0) > 0  # k is split between workgroups in one of the two
+    torch.cuda.synchronize()
+    del taken[:]
+    for stream in [torch.cuda.Stream() for _ in range(3)]:
+        if lib.hfrk_workspace_id(stream.cuda_stream) >= 0:
+            continue  # a handle that an earlier test's stream had
+        for (x, res), expected in zip(rows, want):
+            before = torch.cuda.memory_stats()["allocation.all.allocated"]
+            with torch.cuda.stream(stream):
+                got = block(x, res)
+            assert torch.cuda.memory_stats()["allocation.all.allocated"] == before
+            torch.cuda.synchronize()
+            _same(got, expected)
+        assert lib.hfrk_workspace_id(stream.cuda_stream) == -1
+    assert taken and all(taken)
+
+
+def test_graph_call_whose_plan_has_grown_replays(monkeypatch):
+    import ctypes
+    from hf_rocm_kernels import _capi
+    lib, taken = _capi.load(), _counted(monkeypatch)
+    m, hidden, inter = 8, 1024, 5120
+    args = _block(hidden, inter, torch.bfloat16)
+    block = LlamaMlpGraph(m, hidden, *args)
+    x, res = _rows(m, hidden, torch.bfloat16)
+    want = [t.clone() for t in block(x, res)]
+    assert lib.hfrk_llama_mlp_workspace_bytes(m, hidden, inter, 0, 0) == 0
+    plan = next(p for p in all_plans(m, hidden, inter) if p.wn > 0)  # partial sums between workgroups
+    try:
+        assert lib.hfrk_plan_table_set(m, hidden, inter, 0, ctypes.byref(plan)) == 0
+        assert lib.hfrk_llama_mlp_workspace_bytes(m, hidden, inter, 0, 0) > 0
+        got = block(x, res)
+        torch.cuda.synchronize()
+        assert taken[-1] is False
+        _same(got, want)
+    finally:
+        lib.hfrk_plan_table_set(m, hidden, inter, 0, None)
+    block(x, res)
+    assert taken[-1] is True
+
+
+def test_graph_call_is_refused_while_a_caller_captures():
+    """A graph is not replayed into another; what can be captured is llama_mlp_combined_ops."""
+    args = _block(512, 1024, torch.bfloat16)
+    block = LlamaMlpGraph(4, 512, *args)
+    x, res = _rows(4, 512, torch.bfloat16)
+    want = [t.clone() for t in block(x, res)]
+    with pytest.raises(RuntimeError):
+        with torch.cuda.graph(torch.cuda.CUDAGraph(), stream=torch.cuda.Stream()):
+            block(x, res)
+    torch.cuda.synchronize()
+    _same(block(x, res), want)

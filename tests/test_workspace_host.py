@@ -61,14 +61,15 @@ def tiled(stream, plan=None):
 def skinny(stream, plan=None):  # (64 rows of a narrow weight: k is split between workgroups)
     return lib.hfrk_skinny_gemm_fused(4096, 8192, 16384, None, 64, 0, None, 0, None, 64, 64, 16384, 16384, _capi.BF16, 0, plan, stream)
 
-def block(stream=1, m=4, hidden=512, inter=512, **at):
+def block(stream=1, m=4, hidden=512, inter=512, workspace=None, **at):
     # tensors of m * hidden 16-bit values, `place` apart unless `at` says where one lies, in units of one tensor
     place, launched, size = 1 << 24, ctypes.c_int(7), m * hidden * 2
     names = ["input", "residual_in", "residual", "input_copy", "output", "scratch"]
     where = {{x: (i + 1) * place for i, x in enumerate(names)}}
     where.update((x, v if v is None else int((names.index(v[0]) + 1) * place + v[1] * size)) for x, v in at.items())
-    status = lib.hfrk_llama_mlp(where["input"], where["residual_in"], where["residual"], where["input_copy"], 4096, 1e-5, 64, 1 << 30, 0, hidden,
-                                64, 64, 1 << 31, 0, inter, 64, 1, where["output"], where["scratch"], m, hidden, inter, _capi.BF16,
+    workspace = workspace or (None, 0)
+    status = lib.hfrk_llama_mlp_owned(where["input"], where["residual_in"], where["residual"], where["input_copy"], 4096, 1e-5, 64, 1 << 30, 0, hidden,
+                                64, 64, 1 << 31, 0, inter, 64, 1, where["output"], where["scratch"], *workspace, m, hidden, inter, _capi.BF16,
                                 ctypes.byref(launched), stream)
     return status, launched.value, stand_in.stand_in_launches()
 
@@ -159,6 +160,37 @@ for m in (1, 4, 64):
         stand_in.stand_in(100, 0)
         status, launched, launches = block(m=m, **at)
         assert (status, launched) == (_capi.SUCCESS, 1) and launches >= 3, (m, at, status, launches)
+"""
+
+
+_CASES["a block on memory of its own"] = """
+size = lambda m, hidden, inter, packed=0: lib.hfrk_llama_mlp_workspace_bytes(m, hidden, inter, packed, packed)
+own, m, hidden, inter = 1 << 40, 64, 1024, 5120
+need = size(m, hidden, inter)
+assert need > 0 and size(1, hidden, inter) == 0 and size(65, hidden, inter) == size(8, 1000, inter) == size(8, hidden, 0) == 0
+for capturing in (0, 1):  # no memory to be had, no workspace of the stream's
+    for stream in (1, 2):
+        stand_in.stand_in(0, capturing)
+        status, launched, launches = block(stream, m, hidden, inter, (own, need))
+        assert (status, launched) == (_capi.SUCCESS, 1) and launches >= 3
+        assert lib.hfrk_workspace_id(stream) == -1
+        stand_in.stand_in(0, capturing)
+        assert block(stream, m, hidden, inter)[1:] == (0, 0)
+stand_in.stand_in(100, 0)
+assert block(1, m, hidden, inter, (own, need - 1)) == block(1, m, hidden, inter, (own, 0)) == (_capi.EXCEEDS_SCRATCH, 0, 0)
+assert block(1, m, hidden, inter, (own + 8, need)) == (_capi.BAD_ALIGNMENT, 0, 0)
+for place in range(1, 7):
+    assert block(1, m, hidden, inter, ((place << 24) + 4096, need)) == (_capi.BAD_SHAPE, 0, 0)
+assert block(1, 1, hidden, inter, (own, 0))[:2] == (_capi.SUCCESS, 1)
+assert block(1, m, hidden, inter)[:2] == (_capi.SUCCESS, 1) and lib.hfrk_workspace_id(1) >= 0
+for m in (1, 8, 16, 17, 32, 33, 64):
+    for hidden in (256, 1024, 2048, 4096, 8192):
+        for inter in (256, 2816, 14336):
+            need = size(m, hidden, inter)
+            stand_in.stand_in(0, 1)
+            assert block(3, m, hidden, inter, (own, need))[:2] == (_capi.SUCCESS, 1), (m, hidden, inter)
+            if need:
+                assert block(3, m, hidden, inter, (own, need - 1))[0] == _capi.EXCEEDS_SCRATCH
 """
 
 
