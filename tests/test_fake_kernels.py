@@ -124,6 +124,17 @@ def test_a_traced_call_records_operators_that_check_their_arguments():
             hf_rocm_kernels.skinny_gemm(_fp8(8, 512), _fp8(256, 768).t(), torch.empty(1, device="cuda"))
 
 
+def test_whole_call_operators_take_no_meta_tensors():
+    """One meta tensor among device tensors sends a call to the shape-only implementations; a result of theirs would be one that nobody
+    computed."""
+    meta = lambda *shape, dtype=FP8: torch.empty(*shape, device="meta", dtype=dtype)
+    ops, one, x = torch.ops._HFRK_C, meta(1, dtype=torch.float32), meta(4, 512, dtype=torch.bfloat16)
+    assert ops.fp8_linear(x, meta(256, 512), -1, one, None, None, None, None) is None
+    assert ops.skinny_gemm_new(meta(4, 512), meta(256, 512).t(), one) is None
+    assert ops.skinny_gemm_into(meta(4, 512), meta(256, 512).t(), one, meta(4, 256, dtype=torch.float16)) is False
+    assert ops.llama_mlp(x, x, x, None, meta(512, dtype=torch.bfloat16), 1e-5, meta(1024, 512).t(), -1, one, one, meta(512, 512).t(), -1, one, one, True, x) is False
+
+
 def _interceptors():
     """Ways a call is recorded, batched or replaced: each runs its argument with a tensor."""
     from torch.fx.experimental.proxy_tensor import make_fx

@@ -192,3 +192,16 @@ def test_graph_call_is_refused_while_a_caller_captures():
             block(x, res)
     torch.cuda.synchronize()
     _same(block(x, res), want)
+
+
+def test_a_meta_tensor_is_refused():
+    hidden = 512
+    args = _block(hidden, 1024, torch.bfloat16)
+    block = LlamaMlpGraph(4, hidden, *args)
+    x, res = _rows(4, hidden, torch.bfloat16)
+    with pytest.raises(AssertionError):
+        llama_mlp_combined_ops(x, res.to("meta"), *args, add_residual=True, fused=True)
+    with pytest.raises(AssertionError):
+        llama_mlp_combined_ops(x, res, args[0], 1e-5, args[2].to("meta"), *args[3:], add_residual=True, fused=True)
+    with pytest.raises((RuntimeError, NotImplementedError)):
+        block(x, res.to("meta"))
