@@ -924,13 +924,12 @@ struct BlockGemms {
         return gemm_launch(activated, down, output, addend, down_scale, 0, nullptr, 0, nullptr, m, hidden, inter, down_stride, dtype, HFRK_EPILOGUE_NONE,
                            nullptr, stream, down_packed, false, nullptr, false, given, needs);
     }
-    // Whether both can run, what they take of a workspace, and whether the SwiGLU is the gate_up GEMM's epilogue: skinny_gemm_swiglu
-    // (operators/skinny_gemm/wrapped.py) has the same rule and the figures behind it.
+    // Whether both can run, what they take of a workspace, and whether the SwiGLU is the gate_up GEMM's epilogue.
     int check(bool* fused, GemmNeeds* needs) const {
-        const bool window = hidden == 2048 || hidden == 4096;
-        *fused = m <= 16 || window || (m <= kRowsMaxM && !gate_up_packed && 2L * inter * hidden <= (128L << 20));
+        const int route = hfrk_swiglu_in_epilogue(m, 2 * inter, hidden, gate_up_packed);
+        *fused = route != 0;
         int rc = *fused ? gate_up_gemm(true, needs) : HFRK_BAD_SHAPE;
-        if (rc == HFRK_BAD_SHAPE && m > 16 && !(*fused && window)) {
+        if (rc == HFRK_BAD_SHAPE && route != 1) {
             *fused = false;
             rc = gate_up_gemm(false, needs);
         }
@@ -1100,6 +1099,14 @@ int hfrk_linear_gemm(const void* A, const void* B, int packed, void* D, const vo
     }
     return hfrk::gemm_launch(A, B, D, base, scale_a, sa_stride, scale_b, sb_stride, nullptr, m, n, k, b_stride, d_dtype, HFRK_EPILOGUE_NONE,
                              nullptr, static_cast<hipStream_t>(stream), packed != 0, false, nullptr, base && base_stride == 0);
+}
+
+// skinny_gemm_swiglu (operators/skinny_gemm/wrapped.py) has the same rule, for tracers, and the figures behind it.
+int hfrk_swiglu_in_epilogue(int m, int n, int k, int packed) {
+    const bool window = k == 2048 || k == 4096;
+    if (m < 1 || m > HFRK_GEMM_MAX_M || n % 32 != 0 || (m > hfrk::kRowsMaxM && !window)) return 0;
+    if (m <= 16 || window) return 1;
+    return !packed && (long)n * k <= (128L << 20) ? 2 : 0;
 }
 
 size_t hfrk_llama_mlp_scratch_bytes(int m, int hidden, int inter) {

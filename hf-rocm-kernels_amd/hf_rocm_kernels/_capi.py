@@ -88,6 +88,7 @@ SIGNATURES = {
     "hfrk_packed_weight_scales": (_p, [_p, _i, _i]),
     "hfrk_skinny_gemm_packed": (_i, [_p, _p, _p, _p, _p, _i, _p, _i, _p, _i, _i, _i, _i, _i, ctypes.POINTER(GemmPlan), _p]),
     "hfrk_linear_gemm": (_i, [_p, _p, _i, _p, _p, _i, _p, _i, _p, _i, _i, _i, _i, _i, _i, _p]),
+    "hfrk_swiglu_in_epilogue": (_i, [_i] * 4),
     "hfrk_llama_mlp_scratch_bytes": (ctypes.c_size_t, [_i, _i, _i]),
     "hfrk_llama_mlp": (_i, [_p] * 5 + [_f, _p, _p, _i, _i, _p, _p, _p, _i, _i, _p, _i, _p, _p, _i, _i, _i, _i, ctypes.POINTER(_i), _p]),
     "hfrk_llama_mlp_workspace_bytes": (ctypes.c_size_t, [_i] * 5),

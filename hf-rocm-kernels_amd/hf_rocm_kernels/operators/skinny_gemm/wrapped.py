@@ -219,6 +219,22 @@ def skinny_gemm_add(
     return output
 
 
+def _swiglu_route(m: int, n: int, k: int, packed: bool) -> int:
+    """Where gate_up and SwiGLU are one launch: 1, or 2 if the library has a plan, which its status says; 0: two launches.  The rule of
+    `hfrk_swiglu_in_epilogue`, in a form that a tracer follows.
+    17..32 rows on other k than 2048 and 4096: one launch where the library's row-split kernel takes the shape (row-major weights whose
+    output columns deal out over the workgroups) and where it is the faster way: measured on
+    k = 8192 at 20 / 32 rows, 16384 columns 25.8 / 26.5 us fused against 26.0 / 26.1 in two launches, 28672 columns 44.0 /
+    46.4 against 40.7 / 41.0, 57344 columns 78.3 / 84.4 against 77.3 / 78.0 (above 16 rows the workgroup kernel is the
+    faster GEMM on large weights, by more than the SwiGLU launch costs)."""
+    window = k in (2048, 4096)
+    if n % 32 != 0 or (m > 32 and not window):
+        return 0
+    if m <= 16 or window:
+        return 1
+    return 0 if packed or n * k > (128 << 20) else 2
+
+
 def skinny_gemm_swiglu(
     skinny_a: Tensor,
     gate_up_weight: Tensor,
@@ -250,15 +266,9 @@ def skinny_gemm_swiglu(
         return output
 
     k = skinny_a.size(1)
-    if n % 32 != 0 or (m > 32 and k not in (2048, 4096)):
-        return two_launches()
-    # 17..32 rows on other k: one launch where the library's row-split kernel takes the shape (row-major weights whose
-    # output columns deal out over the workgroups), which its status says -- and where it is the faster way: measured on
-    # k = 8192 at 20 / 32 rows, 16384 columns 25.8 / 26.5 us fused against 26.0 / 26.1 in two launches, 28672 columns 44.0 /
-    # 46.4 against 40.7 / 41.0, 57344 columns 78.3 / 84.4 against 77.3 / 78.0 (above 16 rows the workgroup kernel is the
-    # faster GEMM on large weights, by more than the SwiGLU launch costs)
-    maybe = m > 16 and k not in (2048, 4096)
-    if maybe and (isinstance(gate_up_weight, PackedWeight) or torch.compiler.is_compiling() or n * k > (128 << 20)):
+    route = _swiglu_route(m, n, k, isinstance(gate_up_weight, PackedWeight))
+    maybe = route == 2
+    if route == 0 or (maybe and torch.compiler.is_compiling()):
         return two_launches()
     if output is None:
         output = torch.empty(size=(m, n // 2), dtype=torch.float8_e4m3fn, device=skinny_a.device)

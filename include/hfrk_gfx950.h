@@ -276,6 +276,10 @@ int hfrk_skinny_gemm_packed(const void* A, const void* B_packed, void* D, const 
 int hfrk_linear_gemm(const void* A, const void* B, int packed, void* D, const void* base, int base_stride, const float* scale_a,
                      int sa_stride, const float* scale_b, int sb_stride, int m, int n, int k, int b_stride, int d_dtype, void* stream);
 
+/* Whether gate_up and SwiGLU are better one launch (HFRK_EPILOGUE_SWIGLU) than the GEMM and hfrk_swiglu behind it, n the columns of gate_up:
+ * 1 yes, 0 no, 2 yes if the fused entry point takes the shape (it returns HFRK_BAD_SHAPE where no plan does). */
+int hfrk_swiglu_in_epilogue(int m, int n, int k, int packed);
+
 /* The fused decoder MLP block for up to 64 rows: hfrk_residual_rms, the gate_up GEMM with the SwiGLU as its epilogue (or behind it, where that
  * is the faster way), and the down GEMM with or without the updated residual as its addend.
  *   residual <- input + residual_in (which may be the same tensor);  input_copy <- input, where it is not NULL

@@ -784,3 +784,17 @@ def test_fp8_linear_keeps_its_quantised_buffers_through_dtype_casts():
     twin.half().load_state_dict(state)
     assert torch.equal(twin[0].weight_data.view(torch.uint8), weight_bits) and torch.equal(twin[0].weight_scale, scale)
     assert twin[0].weight is twin[0].weight_data
+
+
+def test_one_rule_says_where_the_swiglu_is_an_epilogue():
+    """The wrapper's form of the rule, which a tracer can follow, and the library's, which the native MLP block goes by."""
+    from hf_rocm_kernels.operators.skinny_gemm.wrapped import _swiglu_route
+    lib = _capi.load()
+    seen = set()
+    for m in (1, 15, 16, 17, 31, 32, 33, 63, 64):
+        for n in (32, 48, 512, 1000, 16384, 16416, 28672, 32768, 32800, 65536, 65568):
+            for k in (256, 2048, 2304, 4080, 4096, 8192, 28672):
+                for packed in (False, True):
+                    assert _swiglu_route(m, n, k, packed) == lib.hfrk_swiglu_in_epilogue(m, n, k, packed), (m, n, k, packed)
+                    seen.add(_swiglu_route(m, n, k, packed))
+    assert seen == {0, 1, 2}
