@@ -2,7 +2,9 @@
 tiles, first and last stages, all pieces of a stage and all lanes, and checked against what it points into (the rules are those of
 test_address_audit.py: a live access lies inside its buffer, a suppressed one at or beyond its end without wrapping round)."""
 import ctypes
+import os
 import random
+import re
 
 import numpy as np
 import pytest
@@ -10,7 +12,22 @@ import pytest
 from hf_rocm_kernels import _capi
 from test_address_audit import MAX_PANELS, U32, WS_BYTES
 
-SHAPES = [(4, 4, 2, 2, 2), (4, 2, 2, 2, 3), (2, 2, 2, 2, 5), (2, 1, 2, 2, 3), (1, 1, 2, 2, 8)]  # TM, TN, WM, WN, stages in LDS
+
+
+def _built():
+    """Shape index -> the kernels built for it as (TM, TN, WM, WN, stages in LDS), from the header that instantiates them."""
+    header = os.path.join(os.path.dirname(_capi.LIB_PATH), os.pardir, "csrc", "tiled_gemm.h")
+    with open(header) as f:
+        rows = re.findall(r"X\((\d), (\d), (\d), (\d), (\d), (\d), \d\)", f.read())
+    built = {}
+    for index, *shape in rows:
+        built.setdefault(int(index), []).append(tuple(map(int, shape)))
+    assert sorted(built) == list(range(5)) and [len(built[i]) for i in range(5)] == [1, 2, 1, 1, 1]
+    return built
+
+
+BUILT = _built()
+KERNELS = [(shape, kernel) for shape in sorted(BUILT) for kernel in BUILT[shape]]
 KB, OUTSIDE = 128, 0x7FFFFFF0
 LANE = np.arange(64)
 
@@ -27,12 +44,17 @@ def _edge(count):
 
 
 def audit(m, n, k, b_stride, plan, packed, base_stride, sa_stride=1):
-    TM, TN, WM, WN, NST = SHAPES[plan.shape]
-    BM, BN = 32 * TM * WM, 32 * TN * WN
+    for kernel in BUILT[plan.shape]:
+        _audit(kernel, m, n, k, b_stride, plan, packed, base_stride, sa_stride)
+
+
+def _audit(kernel, m, n, k, b_stride, plan, packed, base_stride, sa_stride):
+    TM, TN, WM, WN, NST = kernel
+    NW, BM, BN = WM * WN, 32 * TM * WM, 32 * TN * WN
     tiles_m, tiles_n = -(-m // BM), -(-n // BN)
     tiles, stages = tiles_m * tiles_n, -(-k // KB)
     grid = tiles * plan.splits
-    assert grid * 256 < U32 and (BM + BN) * KB * NST <= 160 * 1024
+    assert grid * 64 * NW < U32 and (BM + BN) * KB * NST <= 160 * 1024
 
     # workgroup -> id: a bijection; tile -> (tm, tn): every tile once, whatever the group height
     per, extra = grid >> 3, grid & 7
@@ -53,12 +75,12 @@ def audit(m, n, k, b_stride, plan, packed, base_stride, sa_stride=1):
     begins = [s * q + min(s, r) for s in range(plan.splits + 1)]
     assert begins[-1] == stages and all(b > a for a, b in zip(begins, begins[1:]))
 
-    la, lb = BM * KB // 4096, BN * KB // 4096
+    la, lb = BM * KB // (1024 * NW), BN * KB // (1024 * NW)
     k_tail, tail_stage = k % KB, k // KB if k % KB else -1
-    wave = np.arange(4)[:, None]
+    wave = np.arange(NW)[:, None]
     for tm in _edge(tiles_m):
         m0, rows_a = tm * BM, min(BM, m - tm * BM)
-        piece = np.arange(la)[:, None, None] * 4 + wave[None]          # (load, wave, lane)
+        piece = np.arange(la)[:, None, None] * NW + wave[None]         # (load, wave, lane)
         row = piece * 8 + (LANE >> 3)
         pa = ((LANE & 7) ^ ((row >> 1) & 7)) * 16
         assert len(np.unique(row * 8 + (pa >> 4))) == BM * 8           # every 16-byte piece of the stage is fetched once
@@ -74,7 +96,7 @@ def audit(m, n, k, b_stride, plan, packed, base_stride, sa_stride=1):
     for tn in _edge(tiles_n):
         n0 = tn * BN
         for s in {0, stages - 1, *(b - 1 for b in begins[1:]), *begins[:-1]}:
-            piece = np.arange(lb)[:, None, None] * 4 + wave[None]
+            piece = np.arange(lb)[:, None, None] * NW + wave[None]
             if packed:
                 tiles16 = min(BN // 16, (n + 15) // 16 - n0 // 16)
                 t16, half, group = piece >> 1, piece & 1, (LANE >> 4) & 1
@@ -100,12 +122,12 @@ def audit(m, n, k, b_stride, plan, packed, base_stride, sa_stride=1):
     LPR = 4 * TN
     RPI = 64 // LPR
     passes = 32 // RPI
-    assert 4 * 32 * (TN * 32 + 4) * 4 <= (BM + BN) * KB * NST
+    assert NW * 32 * (TN * 32 + 4) * 4 <= (BM + BN) * KB * NST
     for tm in _edge(tiles_m):
         m0, rows_a = tm * BM, min(BM, m - tm * BM)
         for tn in _edge(tiles_n):
             n0 = tn * BN
-            for w in range(4):
+            for w in range(NW):
                 row0, col = (w // WN) * TM * 32, (w % WN) * TN * 32 + (LANE % LPR) * 8
                 outside = np.where(n0 + col < n, 0, OUTSIDE)
                 step = (np.arange(TM)[:, None, None] * passes + np.arange(passes)[None, :, None])
@@ -125,7 +147,7 @@ def audit(m, n, k, b_stride, plan, packed, base_stride, sa_stride=1):
     if plan.splits > 1:
         assert tiles <= MAX_PANELS
         nmma = TM * TN
-        last = ((((tiles - 1) * plan.splits + plan.splits - 1) * 4 + 3) * nmma + nmma - 1) * 4 + 3
+        last = ((((tiles - 1) * plan.splits + plan.splits - 1) * NW + NW - 1) * nmma + nmma - 1) * 4 + 3
         assert (last + 1) * 1024 == tiles * plan.splits * BM * BN * 4 <= WS_BYTES < 1 << 31
 
 
@@ -140,7 +162,7 @@ def _plan(m, n, k):
                                           (600, 520, 768, 1), (200, 72, 16, 1), (33, 4104, 1936, 4), (70, 1032, 2064, 8), (300, 40, 784, 7)])
 def test_forced_plans(shape, m, n, k, splits):
     for group_m in (1, 2):
-        if group_m > -(-m // (32 * SHAPES[shape][0] * SHAPES[shape][2])):
+        if group_m > -(-m // (32 * BUILT[shape][0][0] * BUILT[shape][0][2])):
             continue
         plan = _capi.TiledPlan(shape, splits, group_m)
         for base_stride in (0, n):
@@ -171,16 +193,12 @@ def test_largest_sizes(m, n, k):
                 audit(m, n, k, k, forced, True, 0)
 
 
-# TM, TN, WM, WN, stages in LDS as the kernel is built: the 256-row tiles run on eight waves
-BUILT = [(4, 2, 2, 4, 2), (2, 2, 4, 2, 3)] + SHAPES[2:]
-
-
-@pytest.mark.parametrize("shape", range(5))
-def test_every_wave_has_its_part_of_the_tile(shape):
+@pytest.mark.parametrize("shape,kernel", KERNELS)
+def test_every_wave_has_its_part_of_the_tile(shape, kernel):
     """The parts that the waves of a workgroup load, multiply, leave as partial sums and store are the whole tile, each once."""
-    TM, TN, WM, WN, NST = BUILT[shape]
+    TM, TN, WM, WN, NST = kernel
     NW, BM, BN = WM * WN, 32 * TM * WM, 32 * TN * WN
-    assert (BM, BN) == (32 * SHAPES[shape][0] * SHAPES[shape][2], 32 * SHAPES[shape][1] * SHAPES[shape][3])
+    assert (BM, BN) == [(256, 256), (256, 128), (128, 128), (128, 64), (64, 64)][shape]
     stage = (BM + BN) * KB
     assert stage * NST <= 160 * 1024 and NW % 4 == 0
     wave = np.arange(NW)[None, :, None]
