@@ -354,10 +354,13 @@ def test_dynamic_ops_reject_rows_they_cannot_hold():
 
 
 @pytest.mark.parametrize("packed", [False, True])
-def test_captured_mlp_block_replays_like_the_eager_block(packed):
+def test_captured_mlp_block_replays_like_the_eager_block(packed, monkeypatch):
     """LlamaMlpGraph: the fused block as one graph launch.  Replayed several times with fresh inputs, with the
-    program's own eager launches and synchronisations in between; every replay must equal the eager result bit for bit."""
+    program's own eager launches and synchronisations in between; every replay, and every call of the object, must equal the launches of the
+    wrappers (without the native block) bit for bit."""
+    import sys
     from hf_rocm_kernels.combined_ops.llama_mlp import LlamaMlpGraph, llama_mlp_combined_ops
+    module = sys.modules["hf_rocm_kernels.combined_ops.llama_mlp"]
     from hf_rocm_kernels.utils.fp8 import amax_scale, fp8_quantize
     from hf_rocm_kernels.utils.weight_format import pack_weight
     g = torch.Generator().manual_seed(5)
@@ -375,8 +378,17 @@ def test_captured_mlp_block_replays_like_the_eager_block(packed):
     for step in range(4):
         x = torch.randn(m, hidden, generator=g).to(torch.bfloat16).cuda()
         res = torch.randn(m, hidden, generator=g).to(torch.bfloat16).cuda()
-        want, want_res = llama_mlp_combined_ops(x, res.clone(), *args, add_residual=True, fused=True)
+        with monkeypatch.context() as patch:
+            patch.setattr(module, "_llama_mlp", lambda *a: False)
+            want, want_res = llama_mlp_combined_ops(x, res.clone(), *args, add_residual=True, fused=True)
         torch.cuda.synchronize()
+        block.attn_output.copy_(x)
+        block.residual.copy_(res)
+        block.mlp_output.zero_()
+        block.graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(block.mlp_output, want) and torch.equal(block.residual, want_res), step
+        block.mlp_output.zero_()
         got, got_res = block(x, res)
         torch.cuda.synchronize()
         assert torch.equal(got, want) and torch.equal(got_res, want_res), step
