@@ -28,15 +28,18 @@ static int check_tiled_plan(int m, int n, int k, const hfrk_tiled_plan& p) {
 }
 
 // The shape and the number of k splits with the smallest predicted time, in us.  The constants are fitted to a sweep so that the choices come
-// out right (profiles/tiled_gemm_plans.csv: 260 sizes, 3640 calls, row-major weights rotated through 768 MB): the choice is 0.25 % slower
-// than the best measured plan in the geometric mean, 5 % or more on 6 sizes, 14 % on the worst (613 x 23408 x 3584 90 us instead of 79); on
-// every third size, with the others fitted, 0.4 %, and with the quantisation kernel in front of each call 0.2 %.  Against the
-// constants before, which were for these tiles on four waves, 54 choices differ, 10 % faster in the mean; one is 6 % slower.  A term for
-// the operands' traffic out of L2, which an earlier fit had, came out idle.
+// out right (profiles/tiled_gemm_plans.csv: 260 sizes, 3640 calls, row-major weights rotated through 768 MB, k whole stages; on four sizes the
+// choice is a split that the sweep does not have): the choice is 0.25 % slower than the best measured plan in the geometric mean, 5 % or
+// more on 6 sizes, 14 % on the worst (613 x 23408 x 3584 90 us instead of 79, with 782 x 16888 x 3584 8 % the same: 128 x 128 where 256 x 128
+// is faster); on every third size, with the others fitted, 0.4 %, and with the quantisation kernel in front of each call 0.2 %.  Against the
+// constants before, which were for these tiles on four waves, 54 choices differ, 10 % faster in the mean; one is 6 % slower.  On 73 drawn sizes
+// where the two differ the choices are 9 % faster in the mean on weights from memory, and 1.5 % on one weight that the 256 MB cache holds from call
+// to call; there 12 of them are 7 to 23 % slower, most of them splits of a long k (722 x 2000 x 16384 33.7 / 41.3 us, from memory 40.5 / 40.6).
+// Terms for the operands' traffic out of L2 and for the weight's out of memory came out idle.
 static float tiled_cost(int m, int n, int k, int shape, int splits) {
     struct Shape { float fixed, stage; };  // a workgroup's prologue and epilogue; one stage of 128 bytes of k
     static constexpr Shape kShape[kTiledShapeCount] = {{8.81f, 1.28f}, {8.88f, .643f}, {5.10f, .491f}, {2.97f, .398f}, {3.53f, .240f}};
-    constexpr float kHbm = 8.37e6f, kShares = 6.41e6f;       // bytes per us: weights, partial sums
+    constexpr float kShares = 6.41e6f;                       // bytes per us of partial sums
     constexpr float kPairFixed = 1.29f, kPairStage = 1.61f;  // two workgroups on a compute unit against one
     const TiledShape& s = kTiledShapes[shape];
     const long wgs = (long)div_up(m, s.bm) * div_up(n, s.bn) * splits, slots = (long)kNumCU * s.per_cu;
@@ -47,8 +50,6 @@ static float tiled_cost(int m, int n, int k, int shape, int splits) {
         return kShape[shape].fixed * (pair ? kPairFixed : 1.f) + stages * kShape[shape].stage * (pair ? kPairStage : 1.f);
     };
     float t = (float)(wgs / slots) * round_us(slots) + round_us(wgs % slots);
-    const float stream = (float)n * k / kHbm;
-    if (t < stream) t = stream;
     if (splits > 1) t += .451f + .797f * splits + (float)wgs * s.bm * s.bn * 8.f / kShares;
     return t;
 }

@@ -1,5 +1,7 @@
 """The tiled GEMM's planner: whatever it chooses is a plan that the entry point would accept from a caller."""
+import csv
 import ctypes
+import os
 import random
 
 from hf_rocm_kernels import _capi
@@ -42,3 +44,22 @@ def test_plans_of_few_rows_and_of_small_weights():
         tiles, stages = -(-m // bm) * -(-n // bn), -(-k // 128)
         assert 1 <= plan.splits <= stages and 1 <= plan.group_m <= -(-m // bm), (m, n, k, plan.shape, plan.splits)
         assert plan.splits == 1 or (tiles * plan.splits * bm * bn * 4 <= WORKSPACE_BYTES and tiles <= MAX_COUNTERS and stages >= 2 * plan.splits)
+
+
+def test_choices_are_those_of_the_recorded_sweep():
+    """The figures beside the planner's constants are of the choices that the sweep's file marks."""
+    lib = _capi.load()
+    sweep = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "profiles", "tiled_gemm_plans.csv")
+    measured = {}
+    with open(sweep) as f:
+        for row in csv.DictReader(f):
+            size = tuple(int(row[x]) for x in ("m", "n", "k"))
+            measured.setdefault(size, {})[int(row["shape"]), int(row["splits"])] = int(row["chosen"])
+    missing = 0
+    for size, plans in measured.items():
+        plan = _capi.TiledPlan()
+        assert lib.hfrk_tiled_gemm_plan(*size, ctypes.byref(plan)) == _capi.SUCCESS
+        choice = (plan.shape, plan.splits)
+        missing += choice not in plans
+        assert [p for p, chosen in plans.items() if chosen] == ([choice] if choice in plans else []), size
+    assert len(measured) == 260 and missing == 4  # four are split 5 ways
