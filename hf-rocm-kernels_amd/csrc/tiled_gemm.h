@@ -37,7 +37,7 @@ constexpr int kTiledStage = 128;    // bytes of k per pipeline stage
     X(2, 2, 2, 2, 2, 5, 1)   \
     X(3, 2, 1, 2, 2, 3, 2)   \
     X(4, 1, 1, 2, 2, 8, 1)
-// Shape 1 on four waves, for row-major operands whose rows begin inside a 128-byte line (tiled_gemm_rowmajor.hip).
+// Shape 1 on four waves, for row-major operands whose rows begin inside a 128-byte line and a long k (tiled_gemm_rowmajor.hip).
 #define HFRK_TILED_FOUR_WAVES(X) X(1, 4, 2, 2, 2, 3, 1)
 
 struct TiledShape {

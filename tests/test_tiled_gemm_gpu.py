@@ -27,8 +27,9 @@ def _operands(m, n, k, seed):
 # (m, n, k, splits): one row; one tile and one stage; one row and eight columns past a tile, k past a stage and cut unevenly;
 # rows of D that are not 16-byte aligned; a last stage cut short; several groups of tiles; fewer stages than the pipeline is deep
 SIZES = [(1, 64, 256, 1), (64, 256, 128, 1), (257, 264, 1280, 3), (130, 203, 512, 2), (65, 136, 1008, 1), (600, 520, 768, 1), (200, 72, 16, 1),
-         # the 256 x 128 tile on four waves (k no multiple of 128, the last row of tiles at least half full, or many workgroups), and next to it
-         (128, 136, 144, 1), (127, 136, 144, 1), (384, 200, 1040, 3), (512, 264, 2064, 4), (1032, 520, 2064, 16)]
+         # the 256 x 128 tile on four waves (k no multiple of 128 and 44 stages or more, the last row of tiles more than half full, or many
+         # workgroups), and next to it
+         (144, 136, 5520, 1), (143, 136, 5520, 1), (144, 136, 5488, 1), (400, 200, 11280, 2), (512, 264, 5520, 1), (512, 264, 2064, 4)]
 
 
 @pytest.mark.parametrize("add", ["none", "bias", "residual"])

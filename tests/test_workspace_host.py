@@ -130,18 +130,20 @@ def waves(m, n, k, stride=None, packed=0, splits=1, shape=1):
     assert lib.hfrk_tiled_gemm(4096, 8192, packed, 16384, None, 0, 64, 0, None, 0, m, n, k, stride or k, _capi.BF16, plan, 1) == _capi.SUCCESS
     return stand_in.stand_in_threads() // 64
 
-for m in (65, 127, 128, 256, 300, 384, 512, 784, 1040, 1536, 4096):
+for m in (65, 143, 144, 256, 300, 400, 512, 784, 1040, 1536, 4096):
     for n in (8, 4104, 10240, 28672):
         few = -(-m // 256) * -(-n // 128) <= 384
-        eight = m % 256 in range(1, 128) and (m <= 1024 or few)  # a last row of tiles less than half full, one of four or of few workgroups
+        eight = m % 256 in range(1, 144) and (m <= 1024 or few)  # a last row of tiles about half full or less, one of four or of few workgroups
         for k in (128, 4096, 8320):
             assert waves(m, n, k) == waves(m, n, k, k + 256) == 8
-            assert waves(m, n, k, k + 16) == waves(m, n, k, k + 64) == (8 if eight else 4)
-        for k in (16, 4112, 8256):
+            assert waves(m, n, k, k + 16) == waves(m, n, k, k + 64) == (8 if eight or k < 8320 else 4)
+        for k in (5520, 8256):  # 44 stages or more
             assert waves(m, n, k) == waves(m, n, k, k + 112) == waves(m, n, k, -(-k // 128) * 128) == (8 if eight else 4), (m, n, k)
-        assert waves(m, n, 4096, packed=1) == 8
-        assert waves(m, n, 4112, shape=0) == 8 and all(waves(m, n, 4112, shape=s) == 4 for s in (2, 3, 4))
-assert waves(1040, 4104, 4112) == 8 and waves(1040, 4104, 4112, splits=3) == 4  # 165 workgroups, 495
+        assert waves(m, n, 16) == waves(m, n, 4112) == waves(m, n, 5488) == 8
+        assert waves(m, n, 8192, packed=1) == 8
+        assert waves(m, n, 8208, shape=0) == 8 and all(waves(m, n, 8208, shape=s) == 4 for s in (2, 3, 4))
+assert waves(1040, 5000, 16400) == 8 and waves(1040, 5000, 16400, splits=2) == 4  # 200 workgroups, 400
+assert waves(512, 4104, 16400, splits=2) == 4 and waves(512, 4104, 28656, splits=3) == 8 and waves(512, 4104, 8208, splits=2) == 8
 """
 
 
