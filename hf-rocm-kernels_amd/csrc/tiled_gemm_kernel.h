@@ -8,14 +8,16 @@
 //    while the one wave of a SIMD waited for its stage or stored (4096 x 28672 x 4096 432 -> 409 us, 4096 x 4096 x 4096 62.7 -> 57,
 //    2048 x 6144 x 4096 56 -> 52; 12 % in the mean over 70 weights and rows where tiles are few).  The 256 x 128 tile has eight
 //    waves of 64 x 64 for the same reason (four of 128 x 64 before: 4096 x 6144 x 4096 106 -> 97 us, 4096 x 2048 x 2048 23.0 -> 21.0,
-//    300 x 20000 x 4096 56.3 -> 53.5, 1024 x 8192 x 8192 64.6 -> 64; 512 x 10240 x 8192 54.6 -> 55.4 is the loss).  The others have
-//    four waves, one per SIMD: 128 x 128 on eight or sixteen takes the same time.
+//    300 x 20000 x 4096 56.3 -> 53.5, 1024 x 8192 x 8192 64.6 -> 64; 512 x 10240 x 8192 54.6 -> 55.4 is the loss), but for a long k in rows that
+//    begin inside a 128-byte line, where four are the faster (tiled_gemm_rowmajor.hip).  A long k on the largest tile is what eight cost
+//    there: 2513 x 11824 x 13312 314 -> 322, 1415 x 6304 x 18944 188 -> 193.  The others have four waves, one per SIMD: 128 x 128 on
+//    eight or sixteen takes the same time.
 //  * Bound (counters in profiles/tiled_gemm_counters_and_plans.txt, shares of the cycles in which a compute unit has work): 4096 x 28672 x
-//    4096 matrix cores 62 %, at the clock their power leaves, LDS 19 %; 512 x 4096 x 14336 packed 45 and 34 %; 201 x 6144 x 4096
-//    28 and 23 %.  On the small tiles neither is half busy.  (The first of the three before its tile ran on eight waves.)
-//    What bounds the small tiles is what a compute unit can fetch: without matrix instructions and operand reads a launch takes the same
-//    time (201 x 6144 x 4096, 512 x 4096 x 14336), and so it does with 4, 5 or 6 stages in flight.  A unit gets about 75 GB/s, 47 where
-//    nothing it reads is in its L2 yet and 128 - 148 where everything is.
+//    4096 matrix cores 69 %, at the clock their power leaves, LDS 31 % (62 and 19 on four waves); 512 x 4096 x 14336 packed 45 and 35 %;
+//    201 x 6144 x 4096 28 and 23 %.  On the small tiles neither is half busy.
+//    They wait for what a compute unit fetches: without matrix instructions and operand reads a launch takes the same time (201 x 6144 x
+//    4096, 512 x 4096 x 14336), and so it does with 4, 5 or 6 stages in flight.  A unit gets about 75 GB/s, a mixture of the 47 of lines that
+//    are new to its L2 and the 128 - 148 of lines in it: the tile decides how much of each, so it is no limit of the sizes.
 //  * Operands go from memory to LDS without passing registers (buffer_load_dwordx4 ... lds), NST stages of 128 bytes of k deep, the
 //    stage NST ahead being requested behind the barrier that frees its slot.  One barrier per stage: a wave reads the operands of
 //    k step s + 1 (64 bytes) while it multiplies those of step s, so nothing in a step waits for LDS but its first instruction.
@@ -31,7 +33,7 @@
 //  * Few tiles and a long k: k is cut between `splits` workgroups.  Partial tiles are written through to memory, the last arriver
 //    adds them in split order (bit-reproducible), its own from its registers.
 //
-// Measured (us, bf16 out): 4096 x 28672 x 4096 409 (2.35 PFLOP/s; 1550 as 64 skinny launches; a loop that stays resident clocks at 1.8 - 2.0
+// Measured (us, bf16 out): 4096 x 28672 x 4096 392 - 409 (2.35 - 2.45 PFLOP/s; 1550 as 64 skinny launches; a loop that stays resident clocks at 1.8 - 2.0
 // GHz, so the matrix cores' power bounds it before their issue rate does), 512 x 4096 x 14336 packed 36 (150), 201 x 6144 x 4096
 // 13.4 (46), 65 x 4096 x 4096 10.5, packed 9.9 (16).  The epilogue is written with little code on
 // purpose: with a branch per value for NaN and 64-bit addresses it took 18 us of a 256 x 256 tile, now 7.

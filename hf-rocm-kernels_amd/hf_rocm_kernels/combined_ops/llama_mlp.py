@@ -132,14 +132,16 @@ def llama_mlp_combined_ops(
 
 
 class LlamaMlpGraph:
-    """The decoder MLP sub-block captured once into a HIP graph: one host call per token step instead of three or four
-    operator launches (the reference times its kernels inside graphs, operators/skinny_gemm/benchmarking_fn.py:62-92,
-    but ships no captured block).
+    """The decoder MLP sub-block for a fixed number of rows: captured once into a HIP graph (`graph`; the reference times its kernels
+    inside graphs, operators/skinny_gemm/benchmarking_fn.py:62-92, but ships no captured block), and callable.
 
-    The graph reads `attn_output` and `residual` from buffers owned by this object: write the step's inputs with
-    `copy_` (or pass them to `__call__`, which does) and read the results from `mlp_output` / `residual`, which are
-    overwritten by every replay.  Weights and scales are the tensors given here; replace their contents in place if
-    they change.  Capturing needs the library's workspace to exist, so one eager run happens first."""
+    The graph reads `attn_output` and `residual` from buffers owned by this object: write the step's inputs with `copy_`, replay, and read the
+    results from `mlp_output` / `residual`, which every replay overwrites.  A call leaves the same in the same buffers.  The usual call
+    does not replay: it launches the native block on the inputs where they are, which is faster than the graph but costs about 15 us of
+    host, and takes no memory and no workspace of the stream it is made on (the object owns both).  A call during a caller's capture
+    is refused; `llama_mlp_combined_ops` can be captured.  Calls and replays of one object share its buffers: one at a time.
+    Weights and scales are the tensors given here; replace their contents in place if they change.  Capturing needs the library's
+    workspace to exist, so one eager run happens first."""
 
     def __init__(self, rows: int, hidden: int, rms_weight: Tensor, rms_epsilon: float, gate_up_weight, gate_up_input_scale: Tensor,
                  gate_up_output_scale: Tensor, down_weight, down_input_scale: Tensor, down_output_scale: Tensor,
@@ -166,11 +168,13 @@ class LlamaMlpGraph:
         torch.cuda.synchronize(device)
 
     def __call__(self, attn_output: Tensor, residual: Tensor) -> Tuple[Tensor, Tensor]:
-        """Copy the inputs in, replay, return (mlp_output, residual) -- views of this object's buffers.
+        """The block on these inputs; returns (mlp_output, residual), this object's buffers, with the inputs' sum and a copy of the first input in
+        them as a replay leaves them.
 
-        The usual call does the same without the graph: the RMSNorm reads the inputs where they are and writes the copies, and the launches
-        go out from native code, which costs the GPU less than starting a graph (8 rows of 4096 x 14336: 46.6 us with two copies in front,
-        41.9 for the replay alone, 35.9 this way; one row of 2048 x 6144 31.6, 23.4, 17.0)."""
+        What the native block does not take (inputs to convert, to broadcast or to copy) is copied in and replayed.  In a loop, us, with two
+        copies and a replay / the replay alone / this way: 8 rows of 4096 x 14336 43.0 / 38.9 / 32.2, on six objects in turn, which
+        reads every weight from memory, 44.3 / 40.2 / 33.6; one row of 2048 x 6144 34.4 / 22.6 / 15.0 and 34.9 / 23.1 / 16.4.  Starting a graph
+        costs the GPU about 6 us more than the launches in it."""
         if self._fused and runs_now(attn_output) and not torch.cuda.is_current_stream_capturing():
             if _native_block(attn_output, residual, self.residual, self.attn_output, self.mlp_output, *self._operands, self._add_residual,
                              self._memory):
