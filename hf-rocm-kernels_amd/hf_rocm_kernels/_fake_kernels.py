@@ -39,18 +39,19 @@ def _skinny_gemm_new(A, B, scale):
     return A.new_empty((A.shape[0], B.shape[1]), dtype=torch.float16)
 
 
-def _unless_meta(answer, refusal):
+def _unless_mixed(answer, refusal):
     """A whole-call operator also lands here when one tensor among device tensors is a meta tensor, which the wrapper's look at its first
     argument does not show: that is no call of the operator's, and the general way refuses it."""
     def fake(*args, **kwargs):
-        if any(isinstance(a, torch.Tensor) and a.device.type == "meta" for a in (*args, *kwargs.values())):
+        devices = {a.device.type for a in (*args, *kwargs.values()) if isinstance(a, torch.Tensor)}
+        if "meta" in devices and len(devices) > 1:
             return refusal
         return answer(*args, **kwargs)
     return fake
 
 
-_OTHER_RESULT = {"fp8_linear": _unless_meta(_fp8_linear, None), "skinny_gemm_new": _unless_meta(_skinny_gemm_new, None),
-                 "skinny_gemm_into": _unless_meta(lambda A, B, scale, D: True, False), "llama_mlp": _unless_meta(lambda *args, **kwargs: True, False)}
+_OTHER_RESULT = {"fp8_linear": _unless_mixed(_fp8_linear, None), "skinny_gemm_new": _unless_mixed(_skinny_gemm_new, None),
+                 "skinny_gemm_into": _unless_mixed(lambda A, B, scale, D: True, False), "llama_mlp": _unless_mixed(lambda *args, **kwargs: True, False)}
 
 
 def register() -> None:

@@ -298,7 +298,7 @@ int hfrk_llama_mlp(const void* input, const void* residual_in, void* residual, v
 /* The same on memory of the caller's: partial sums and arrival counters go to `workspace` instead of one that the stream owns, so the call
  * allocates nothing and claims nothing on a stream first met, under a capture neither.  hfrk_llama_mlp_workspace_bytes of it (0: the plans chosen
  * now need none), 16-byte aligned and apart from every tensor, zero before its first call and used by one call at a time; a call leaves its
- * counters zero.  A call whose plans have come to need more
+ * counters zero (hfrk_reset_workspace does not know them).  A call whose plans have come to need more
  * (hfrk_plan_table_set) is refused with HFRK_EXCEEDS_SCRATCH.  workspace NULL: the stream's. */
 size_t hfrk_llama_mlp_workspace_bytes(int m, int hidden, int inter, int gate_up_packed, int down_packed);
 int hfrk_llama_mlp_owned(const void* input, const void* residual_in, void* residual, void* input_copy, const void* rms_weight, float epsilon,

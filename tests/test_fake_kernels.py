@@ -124,15 +124,26 @@ def test_a_traced_call_records_operators_that_check_their_arguments():
             hf_rocm_kernels.skinny_gemm(_fp8(8, 512), _fp8(256, 768).t(), torch.empty(1, device="cuda"))
 
 
-def test_whole_call_operators_take_no_meta_tensors():
-    """One meta tensor among device tensors sends a call to the shape-only implementations; a result of theirs would be one that nobody
-    computed."""
-    meta = lambda *shape, dtype=FP8: torch.empty(*shape, device="meta", dtype=dtype)
-    ops, one, x = torch.ops._HFRK_C, meta(1, dtype=torch.float32), meta(4, 512, dtype=torch.bfloat16)
-    assert ops.fp8_linear(x, meta(256, 512), -1, one, None, None, None, None) is None
-    assert ops.skinny_gemm_new(meta(4, 512), meta(256, 512).t(), one) is None
-    assert ops.skinny_gemm_into(meta(4, 512), meta(256, 512).t(), one, meta(4, 256, dtype=torch.float16)) is False
-    assert ops.llama_mlp(x, x, x, None, meta(512, dtype=torch.bfloat16), 1e-5, meta(1024, 512).t(), -1, one, one, meta(512, 512).t(), -1, one, one, True, x) is False
+def test_whole_call_operators_take_no_meta_tensor_among_others():
+    """One meta tensor among tensors with data sends a call to the shape-only implementations; a result of theirs would be one that nobody
+    computed.  A call on meta tensors alone asks for shapes."""
+    def tensors(device, *others):
+        make = lambda i, *shape, dtype=FP8: torch.empty(*shape, device=others[0] if others and i == others[1] else device, dtype=dtype)
+        return [make(0, 4, 512, dtype=torch.bfloat16), make(1, 256, 512), make(2, 1, dtype=torch.float32), make(3, 4, 512), make(4, 4, 256, dtype=torch.float16),
+                make(5, 512, dtype=torch.bfloat16), make(6, 1024, 512), make(7, 512, 512)]
+
+    ops = torch.ops._HFRK_C
+    linear = lambda x, w, one, q, d, norm, gate_up, down: ops.fp8_linear(x, w, -1, one, None, None, None, None)
+    new = lambda x, w, one, q, d, norm, gate_up, down: ops.skinny_gemm_new(q, w.t(), one)
+    into = lambda x, w, one, q, d, norm, gate_up, down: ops.skinny_gemm_into(q, w.t(), one, d)
+    mlp = lambda x, w, one, q, d, norm, gate_up, down: ops.llama_mlp(x, x, x, None, norm, 1e-5, gate_up.t(), -1, one, one, down.t(), -1, one, one, True, x)
+    alone = tensors("meta")
+    assert linear(*alone).shape == (4, 256) and new(*alone).shape == (4, 256) and into(*alone) is True and mlp(*alone) is True
+    for at in (1, 2):
+        assert linear(*tensors("cpu", "meta", at)) is None and linear(*tensors("meta", "cpu", at)) is None
+        assert new(*tensors("cpu", "meta", at)) is None and into(*tensors("cpu", "meta", at)) is False
+    for at in (0, 2, 5, 6, 7):
+        assert mlp(*tensors("cpu", "meta", at)) is False
 
 
 def _interceptors():
