@@ -40,6 +40,9 @@ constexpr int kTiledStage = 128;    // bytes of k per pipeline stage
 // Shape 1 on four waves, for row-major operands whose rows begin inside a 128-byte line and a long k (tiled_gemm_rowmajor.hip).
 #define HFRK_TILED_FOUR_WAVES(X) X(1, 4, 2, 2, 2, 3, 1)
 
+// Waves of a workgroup that only load, beside the WM x WN that multiply (tiled_gemm_kernel.h).
+constexpr int tiled_loader_waves(int tm) { return tm < 4 ? 4 : 0; }
+
 struct TiledShape {
     int bm, bn, stages, per_cu;
 };

@@ -18,6 +18,14 @@
 //    They wait for what a compute unit fetches: without matrix instructions and operand reads a launch takes the same time (201 x 6144 x
 //    4096, 512 x 4096 x 14336), and so it does with 4, 5 or 6 stages in flight.  A unit gets about 75 GB/s, a mixture of the 47 of lines that
 //    are new to its L2 and the 128 - 148 of lines in it: the tile decides how much of each, so it is no limit of the sizes.
+//  * On every tile but the largest four more waves do nothing but load, one per SIMD.  A compute unit takes a load instruction of 1 KB in 16
+//    cycles and holds back the wave whose turn has not come: where the multiplying waves loaded for themselves, a stage took about as long as its
+//    loads and its matrix instructions after one another (201 x 6144 x 4096 with the weight in the 256 MB cache: 11.6 us without matrix instructions
+//    and operand reads, 9.0 without loads, 15.4 whole).  Now, weight in that cache / from memory: that size 14.1 -> 13.0 / 17.0 -> 17.0, 512 x
+//    4096 x 4096 18.1 -> 15.8 / 22.1 -> 22.1, 65 x 4096 x 4096 10.7 -> 9.1 / 11.2 -> 10.6, 244 x 2752 x 3072 9.3 -> 8.2 / 10.2 -> 9.8, 1024 x 4096 x
+//    4096 25.5 -> 23.3 / 29.1 -> 28.9; the worst 64 x 8192 x 28672 49.2 -> 50.1 / 50.1 -> 50.3 and, packed, 84 x 8088 x 3584 9.9 -> 9.4 / 11.0 ->
+//    11.5.  Eight loading waves are no faster, a higher priority for either kind changes nothing.  The tiles whose waves hold 128 x 64 (TM = 4)
+//    have no registers left for a third wave per SIMD.
 //  * Operands go from memory to LDS without passing registers (buffer_load_dwordx4 ... lds), NST stages of 128 bytes of k deep, the
 //    stage NST ahead being requested behind the barrier that frees its slot.  One barrier per stage: a wave reads the operands of
 //    k step s + 1 (64 bytes) while it multiplies those of step s, so nothing in a step waits for LDS but its first instruction.
@@ -76,12 +84,12 @@ __device__ __forceinline__ uint32_t pack_pair(float lo, float hi) {
 }
 
 template <int TM, int TN, int WM, int WN, int NST, int WGS, bool PACKED>
-__global__ void __launch_bounds__(64 * WM * WN, WGS * WM * WN / 4) tiled_gemm_kernel(const TiledGemmArgs a) {
-    constexpr int NW = WM * WN;
+__global__ void __launch_bounds__(64 * (WM * WN + tiled_loader_waves(TM)), WGS * (WM * WN + tiled_loader_waves(TM)) / 4) tiled_gemm_kernel(const TiledGemmArgs a) {
+    constexpr int NW = WM * WN, LW = tiled_loader_waves(TM), NL = LW ? LW : NW;  // waves that multiply, that only load, that load
     constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN;
     constexpr int KB = kTiledStage;
     constexpr int A_BYTES = BM * KB, B_BYTES = BN * KB, STAGE = A_BYTES + B_BYTES;
-    constexpr int LA = A_BYTES / (1024 * NW), LB = B_BYTES / (1024 * NW);  // load instructions per wave and stage, 1 KB each
+    constexpr int LA = A_BYTES / (1024 * NL), LB = B_BYTES / (1024 * NL);  // load instructions per loading wave and stage, 1 KB each
     constexpr int NMMA = TM * TN;
     constexpr int kOutside = 0x7ffffff0;  // beyond any tile's range
 
@@ -90,6 +98,7 @@ __global__ void __launch_bounds__(64 * WM * WN, WGS * WM * WN / 4) tiled_gemm_ke
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int loader = wave - (LW ? NW : 0);  // number among the waves that load
     const int wm = wave / WN, wn = wave % WN;
     const int lr = lane & 31, lg = lane >> 5;
 
@@ -126,7 +135,7 @@ __global__ void __launch_bounds__(64 * WM * WN, WGS * WM * WN / 4) tiled_gemm_ke
     int pa[LA], pb[LB];  // k byte of the lane's piece within its stage (for the last, partial stage)
 #pragma unroll
     for (int q = 0; q < LA; ++q) {
-        const int row = (q * NW + wave) * 8 + (lane >> 3);
+        const int row = (q * NL + loader) * 8 + (lane >> 3);
         pa[q] = ((lane & 7) ^ ((row >> 1) & 7)) * 16;
         va[q] = row * a.k + pa[q];
     }
@@ -134,12 +143,12 @@ __global__ void __launch_bounds__(64 * WM * WN, WGS * WM * WN / 4) tiled_gemm_ke
     for (int q = 0; q < LB; ++q) {
         if constexpr (PACKED) {
             // LDS block (16-row tile, half of the stage): [piece j][k group][row slot], 1 KB
-            const int blk = q * NW + wave, t16 = blk >> 1, s = blk & 1, group = (lane >> 4) & 1;
+            const int blk = q * NL + loader, t16 = blk >> 1, s = blk & 1, group = (lane >> 4) & 1;
             const int row = (lane & 15) ^ ((t16 & 1) << 3) ^ group << 2;
             vb[q] = t16 * a.k * 16 + (lane >> 5) * 1024 + s * 512 + group * 256 + row * 16;
             pb[q] = 0;
         } else {
-            const int row = (q * NW + wave) * 8 + (lane >> 3);
+            const int row = (q * NL + loader) * 8 + (lane >> 3);
             pb[q] = ((lane & 7) ^ (((row >> 1) & 3) | ((row >> 4) & 1) << 2)) * 16;
             vb[q] = row * a.b_stride + pb[q];
         }
@@ -153,12 +162,12 @@ __global__ void __launch_bounds__(64 * WM * WN, WGS * WM * WN / 4) tiled_gemm_ke
     auto issue_a = [&](int q) __attribute__((always_inline)) {
         int off = va[q];
         if (issued == tail_stage) off = pa[q] < k_tail ? off : kOutside;
-        load_to_lds(ra, off, lds0 + slot_issue + (uint32_t)(q * NW + wave) * 1024u);
+        load_to_lds(ra, off, lds0 + slot_issue + (uint32_t)(q * NL + loader) * 1024u);
     };
     auto issue_b = [&](int q) __attribute__((always_inline)) {
         int off = vb[q];
         if (!PACKED && issued == tail_stage) off = pb[q] < k_tail ? off : kOutside;
-        load_to_lds(rb, off, lds0 + slot_issue + A_BYTES + (uint32_t)(q * NW + wave) * 1024u);
+        load_to_lds(rb, off, lds0 + slot_issue + A_BYTES + (uint32_t)(q * NL + loader) * 1024u);
     };
     auto issue_end = [&]() __attribute__((always_inline)) {
         auto advance = [](v4i& r, uint32_t by) __attribute__((always_inline)) {
@@ -215,12 +224,13 @@ __global__ void __launch_bounds__(64 * WM * WN, WGS * WM * WN / 4) tiled_gemm_ke
     auto half = [&](auto sel) __attribute__((always_inline)) {
         constexpr int S = decltype(sel)::value;
         if constexpr (S == 1) {
-            wait_loads_and_lds<(NST - 2) * (LA + LB)>();
+            if constexpr (LW) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            else wait_loads_and_lds<(NST - 2) * (LA + LB)>();
             workgroup_barrier();
             slot_read = slot_read + STAGE == NST * STAGE ? 0 : slot_read + STAGE;
-            issue_begin();
+            if constexpr (!LW) issue_begin();
         }
-        constexpr int READS = TM + TN, LOADS = S == 1 ? LA + LB : 0;
+        constexpr int READS = TM + TN, LOADS = S == 1 && !LW ? LA + LB : 0;
         // two stages leave a load one stage to arrive in: there the requests stand in front of the first half of the matrix instructions
         // (4096 x 4096 x 4096 58.5 -> 56.8 us, 1024 x 8192 x 8192 95 -> 91); deeper pipelines lose up to 4 % by that
         constexpr int kHaste = NST == 2 ? 2 : 1;
@@ -245,23 +255,38 @@ __global__ void __launch_bounds__(64 * WM * WN, WGS * WM * WN / 4) tiled_gemm_ke
             acc[t / TN][t % TN] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(frb[S][t % TN], fra[S][t / TN], acc[t / TN][t % TN], 0, 0, 0, 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
         }
-        if constexpr (S == 1) issue_end();
+        if constexpr (S == 1 && !LW) issue_end();
     };
 
     // ---- main loop ---------------------------------------------------------------------------------------------------
-    // A load may read a scalar that a vector instruction wrote (v_readfirstlane) only five cycles later, and nobody looks after that
-    // for a load in inline assembly: both buffers pass through the wait.  From here on scalar instructions move them.
-    asm volatile("s_nop 4" : "+s"(ra), "+s"(rb) : : "memory");
-#pragma unroll 1
-    for (int s = 0; s < NST; ++s) {
+    auto issue_stage = [&]() __attribute__((always_inline)) {
         issue_begin();
 #pragma unroll
         for (int q = 0; q < LA; ++q) issue_a(q);
 #pragma unroll
         for (int q = 0; q < LB; ++q) issue_b(q);
         issue_end();
+    };
+    if (!LW || wave >= NW) {
+        // A load may read a scalar that a vector instruction wrote (v_readfirstlane) only five cycles later, and nobody looks after that
+        // for a load in inline assembly: both buffers pass through the wait.  From here on scalar instructions move them.
+        asm volatile("s_nop 4" : "+s"(ra), "+s"(rb) : : "memory");
+#pragma unroll 1
+        for (int s = 0; s < NST; ++s) issue_stage();
+        wait_loads_and_lds<(NST - 1) * (LA + LB)>();
+        if constexpr (LW) {  // the barriers of the multiplying waves: one in front of the loop, one per stage, one behind the loop
+            workgroup_barrier();
+#pragma unroll 1
+            for (int s = s_begin; s < s_end; ++s) {
+                wait_loads_and_lds<(NST - 2) * (LA + LB)>();
+                workgroup_barrier();
+                issue_stage();
+            }
+            wait_loads_and_lds<0>();
+            workgroup_barrier();
+            return;  // later barriers wait for the waves that are left
+        }
     }
-    wait_loads_and_lds<(NST - 1) * (LA + LB)>();
     workgroup_barrier();
 #pragma unroll
     for (int j = 0; j < TN; ++j) read_b(frb[0][j], j, 0);
@@ -303,54 +328,42 @@ __global__ void __launch_bounds__(64 * WM * WN, WGS * WM * WN / 4) tiled_gemm_ke
         const int last = *flag;
         __syncthreads();  // the epilogue writes where the flag lies
         if (!last) return;
-        // The last arriver adds the partials in split order, its own from its registers; up to four splits' are requested together, more
-        // one after the other.  What it costs is the round trips: with its own read back and one split at a time 512 x 4096 x 14336 in 2
-        // splits 43.8 -> 43.0 us, 64 x 4096 x 14336 in 4 17.5 -> 17.1, 1024 x 8192 x 8192 on 256 x 256 tiles in 2 82 -> 76.
-        constexpr int CH = NW > 4 ? 1 : NMMA <= 4 ? NMMA : 2;  // matrix tiles whose shares are in flight together: what fits the registers
-        auto load_shares = [&](v4i (&share)[CH * 4], int t0, int sp) __attribute__((always_inline)) {
-#pragma unroll
-            for (int p = 0; p < CH * 4; ++p) share[p] = __builtin_amdgcn_raw_buffer_load_b128(ws, ws_off(sp, t0 + p / 4, p % 4), 0, kCoherent);
-        };
+        // The last arriver adds the partials in split order, its own from its registers; the others' are requested FLY at a time.  What it costs
+        // is the round trips: with its own read back and one split at a time 512 x 4096 x 14336 in 2 splits 43.8 -> 43.0 us, 64 x 4096 x 14336 in
+        // 4 17.5 -> 17.1, 1024 x 8192 x 8192 on 256 x 256 tiles in 2 82 -> 76.
+        // CH matrix tiles' shares of FLY splits are in flight together: what fits the registers.
+        constexpr int CH = NMMA == 1 || WGS * (NW + LW) > 8 || (LW == 0 && NW > 4) ? 1 : 2, FLY = NMMA == 1 ? 7 : 3;
 #pragma unroll
         for (int t0 = 0; t0 < NMMA; t0 += CH) {
             v4f sum[CH * 4];
 #pragma unroll
             for (int p = 0; p < CH * 4; ++p) sum[p] = v4f{0.f, 0.f, 0.f, 0.f};
-            auto add = [&](const v4i (&share)[CH * 4]) __attribute__((always_inline)) {
-#pragma unroll
-                for (int p = 0; p < CH * 4; ++p) sum[p] += __builtin_bit_cast(v4f, share[p]);
-            };
-            auto add_own = [&]() __attribute__((always_inline)) {
-#pragma unroll
-                for (int p = 0; p < CH * 4; ++p) {
-                    const v16f& x = acc[(t0 + p / 4) / TN][(t0 + p / 4) % TN];
-                    sum[p] += v4f{x[4 * (p % 4)], x[4 * (p % 4) + 1], x[4 * (p % 4) + 2], x[4 * (p % 4) + 3]};
-                }
-            };
-            if (a.splits <= 4) {
-                v4i other[3][CH * 4];
-#pragma unroll
-                for (int j = 0; j < 3; ++j)
-                    if (j + 1 < a.splits) load_shares(other[j], t0, j + (j >= split ? 1 : 0));
-#pragma unroll
-                for (int sp = 0; sp < 4; ++sp) {
-                    if (sp >= a.splits) continue;
-                    if (sp == split) add_own();
-                    else if (sp < split) add(other[sp < 3 ? sp : 2]);
-                    else add(other[sp > 0 ? sp - 1 : 0]);
-                }
-            } else {
+            auto add_shares = [&](int first, int end) __attribute__((always_inline)) {
 #pragma unroll 1
-                for (int sp = 0; sp < a.splits; ++sp) {
-                    if (sp == split) {
-                        add_own();
-                        continue;
-                    }
-                    v4i share[CH * 4];
-                    load_shares(share, t0, sp);
-                    add(share);
+                for (; first < end; first += FLY) {
+                    v4i share[FLY][CH * 4];
+#pragma unroll
+                    for (int j = 0; j < FLY; ++j)
+                        if (first + j < end) {
+#pragma unroll
+                            for (int p = 0; p < CH * 4; ++p)
+                                share[j][p] = __builtin_amdgcn_raw_buffer_load_b128(ws, ws_off(first + j, t0 + p / 4, p % 4), 0, kCoherent);
+                        }
+#pragma unroll
+                    for (int j = 0; j < FLY; ++j)
+                        if (first + j < end) {
+#pragma unroll
+                            for (int p = 0; p < CH * 4; ++p) sum[p] += __builtin_bit_cast(v4f, share[j][p]);
+                        }
                 }
+            };
+            add_shares(0, split);
+#pragma unroll
+            for (int p = 0; p < CH * 4; ++p) {
+                const v16f& x = acc[(t0 + p / 4) / TN][(t0 + p / 4) % TN];
+                sum[p] += v4f{x[4 * (p % 4)], x[4 * (p % 4) + 1], x[4 * (p % 4) + 2], x[4 * (p % 4) + 3]};
             }
+            add_shares(split + 1, a.splits);
 #pragma unroll
             for (int t = 0; t < CH; ++t)
 #pragma unroll
@@ -454,7 +467,7 @@ static int launch_tiled_shape(const TiledGemmArgs& args, int lds_bytes, hipStrea
         HFRK_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes));
         if (dev >= 0 && dev < kMaxDevices) attr_done[dev] = true;
     }
-    hipLaunchKernelGGL(kern, dim3(args.tiles_m * args.tiles_n * args.splits), dim3(64 * WM * WN), lds_bytes, stream, args);
+    hipLaunchKernelGGL(kern, dim3(args.tiles_m * args.tiles_n * args.splits), dim3(64 * (WM * WN + tiled_loader_waves(TM))), lds_bytes, stream, args);
     HFRK_HIP_TRY(hipGetLastError());
     return HFRK_SUCCESS;
 }

@@ -29,6 +29,12 @@ def _built():
 BUILT = _built()
 KERNELS = [(shape, kernel) for shape in sorted(BUILT) for kernel in BUILT[shape]]
 KB, OUTSIDE = 128, 0x7FFFFFF0
+
+
+def _loading_waves(TM, NW):
+    return 4 if TM < 4 else NW
+
+
 LANE = np.arange(64)
 
 
@@ -75,12 +81,13 @@ def _audit(kernel, m, n, k, b_stride, plan, packed, base_stride, sa_stride):
     begins = [s * q + min(s, r) for s in range(plan.splits + 1)]
     assert begins[-1] == stages and all(b > a for a, b in zip(begins, begins[1:]))
 
-    la, lb = BM * KB // (1024 * NW), BN * KB // (1024 * NW)
+    NL = _loading_waves(TM, NW)
+    la, lb = BM * KB // (1024 * NL), BN * KB // (1024 * NL)
     k_tail, tail_stage = k % KB, k // KB if k % KB else -1
-    wave = np.arange(NW)[:, None]
+    wave = np.arange(NL)[:, None]
     for tm in _edge(tiles_m):
         m0, rows_a = tm * BM, min(BM, m - tm * BM)
-        piece = np.arange(la)[:, None, None] * NW + wave[None]         # (load, wave, lane)
+        piece = np.arange(la)[:, None, None] * NL + wave[None]         # (load, wave, lane)
         row = piece * 8 + (LANE >> 3)
         pa = ((LANE & 7) ^ ((row >> 1) & 7)) * 16
         assert len(np.unique(row * 8 + (pa >> 4))) == BM * 8           # every 16-byte piece of the stage is fetched once
@@ -96,7 +103,7 @@ def _audit(kernel, m, n, k, b_stride, plan, packed, base_stride, sa_stride):
     for tn in _edge(tiles_n):
         n0 = tn * BN
         for s in {0, stages - 1, *(b - 1 for b in begins[1:]), *begins[:-1]}:
-            piece = np.arange(lb)[:, None, None] * NW + wave[None]
+            piece = np.arange(lb)[:, None, None] * NL + wave[None]
             if packed:
                 tiles16 = min(BN // 16, (n + 15) // 16 - n0 // 16)
                 t16, half, group = piece >> 1, piece & 1, (LANE >> 4) & 1
@@ -201,13 +208,14 @@ def test_every_wave_has_its_part_of_the_tile(shape, kernel):
     assert (BM, BN) == [(256, 256), (256, 128), (128, 128), (128, 64), (64, 64)][shape]
     stage = (BM + BN) * KB
     assert stage * NST <= 160 * 1024 and NW % 4 == 0
-    wave = np.arange(NW)[None, :, None]
+    NL = _loading_waves(TM, NW)
+    wave = np.arange(NL)[None, :, None]
     loads = 0
     for rows in (BM, BN):  # A and row-major B: 8 rows of 8 pieces a load; packed B: half a 16-row tile's stage
-        per_wave = rows * KB // (1024 * NW)
-        assert per_wave * 1024 * NW == rows * KB
+        per_wave = rows * KB // (1024 * NL)
+        assert per_wave * 1024 * NL == rows * KB
         loads += per_wave
-        piece = np.arange(per_wave)[:, None, None] * NW + wave
+        piece = np.arange(per_wave)[:, None, None] * NL + wave
         assert (np.sort(piece.ravel()) == np.arange(rows // 8)).all()            # KB of LDS it fills
         row = piece * 8 + (LANE >> 3)
         for f in ((row >> 1) & 7, ((row >> 1) & 3) | (((row >> 4) & 1) << 2)):
