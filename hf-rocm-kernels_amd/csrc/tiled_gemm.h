@@ -29,10 +29,10 @@ struct TiledGemmArgs {
 
 constexpr int kTiledStage = 128;    // bytes of k per pipeline stage
 
-// TM x TN matrix tiles of 32 x 32 per wave, WM x WN waves, NST stages of operands in LDS, WGS workgroups per compute unit.
+// TM x TN matrix tiles of 32 x 32 per wave, WM x WN waves, NST stages (or halves of them) of operands in LDS, WGS workgroups per compute unit.
 // X(index, TM, TN, WM, WN, NST, WGS)
 #define HFRK_TILED_SHAPES(X) \
-    X(0, 4, 2, 2, 4, 2, 1)   \
+    X(0, 4, 2, 2, 4, 5, 1)   \
     X(1, 2, 2, 4, 2, 3, 1)   \
     X(2, 2, 2, 2, 2, 5, 1)   \
     X(3, 2, 1, 2, 2, 3, 2)   \
@@ -40,13 +40,16 @@ constexpr int kTiledStage = 128;    // bytes of k per pipeline stage
 // Shape 1 on four waves, for row-major operands whose rows begin inside a 128-byte line and a long k (tiled_gemm_rowmajor.hip).
 #define HFRK_TILED_FOUR_WAVES(X) X(1, 4, 2, 2, 2, 3, 1)
 
+// Whether LDS holds halves of stages (the 256 x 256 tile: five halves, 160 KB; two whole stages are 128).
+constexpr bool tiled_half_stages(int tm, int waves) { return tm * waves >= 32; }
 // Waves of a workgroup that only load, beside the WM x WN that multiply (tiled_gemm_kernel.h).
 constexpr int tiled_loader_waves(int tm) { return tm < 4 ? 4 : 0; }
 
 struct TiledShape {
     int bm, bn, stages, per_cu;
+    bool halves;
 };
-#define HFRK_TILED_ROW(I, TM, TN, WM, WN, NST, WGS) {32 * TM * WM, 32 * TN * WN, NST, WGS},
+#define HFRK_TILED_ROW(I, TM, TN, WM, WN, NST, WGS) {32 * TM * WM, 32 * TN * WN, NST, WGS, tiled_half_stages(TM, WM * WN)},
 constexpr TiledShape kTiledShapes[] = {HFRK_TILED_SHAPES(HFRK_TILED_ROW)};
 #undef HFRK_TILED_ROW
 #define HFRK_TILED_SAME(I, TM, TN, WM, WN, NST, WGS) \
@@ -54,7 +57,7 @@ constexpr TiledShape kTiledShapes[] = {HFRK_TILED_SHAPES(HFRK_TILED_ROW)};
 HFRK_TILED_FOUR_WAVES(HFRK_TILED_SAME)
 #undef HFRK_TILED_SAME
 constexpr int kTiledShapeCount = sizeof(kTiledShapes) / sizeof(kTiledShapes[0]);
-constexpr int tiled_lds_bytes(const TiledShape& s) { return (s.bm + s.bn) * kTiledStage * s.stages; }
+constexpr int tiled_lds_bytes(const TiledShape& s) { return (s.bm + s.bn) * (s.halves ? kTiledStage / 2 : kTiledStage) * s.stages; }
 
 bool tiled_size_ok(int m, int n, int k);  // tiled_gemm.hip
 int launch_tiled_rowmajor(const TiledGemmArgs& args, int shape, hipStream_t stream);  // tiled_gemm_rowmajor.hip

@@ -29,6 +29,12 @@
 //  * Operands go from memory to LDS without passing registers (buffer_load_dwordx4 ... lds), NST stages of 128 bytes of k deep, the
 //    stage NST ahead being requested behind the barrier that frees its slot.  One barrier per stage: a wave reads the operands of
 //    k step s + 1 (64 bytes) while it multiplies those of step s, so nothing in a step waits for LDS but its first instruction.
+//  * The 256 x 256 tile has room for two such stages, which left a load one stage to arrive in, so LDS holds five halves instead (64 bytes of
+//    k each): a stage is requested when the first half of the one before it is free, one and a half stages ahead.  A load then covers 64 bytes
+//    of 16 rows, the two halves of a line one after the other.  Two stages -> five halves, weight in the 256 MB cache / from memory: 4096 x
+//    28672 x 4096 396 -> 384 / 398 -> 384 us, 2048 x 28672 x 4096 219 -> 212 / 221 -> 213, 418 x 16920 x 6656 packed 74.1 -> 68.4 / 75.4 -> 68.7,
+//    1024 x 8192 x 8192 in 2 splits 75.8 -> 72.2 / 75.7 -> 72.9, 4096 x 4096 x 4096 58.4 -> 57.3 / 58.7 -> 57.9.  On operands of zeros the first takes
+//    313 us and took 345: the rest of it is the clock that the matrix cores' power leaves.
 //  * Such a load fills LDS in lane order, so the swizzle that keeps operand reads free of bank conflicts is applied to the memory
 //    side: the lane that fills slot c of row r fetches piece c ^ f(r) of that row (a permutation within one 128-byte line).
 //    Measured conflicts: none on the 256 x 256 tile, 1 - 2 % of the LDS cycles on the smaller ones.  A packed weight is fetched as
@@ -91,6 +97,9 @@ __global__ void __launch_bounds__(64 * (WM * WN + tiled_loader_waves(TM)), WGS *
     constexpr int A_BYTES = BM * KB, B_BYTES = BN * KB, STAGE = A_BYTES + B_BYTES;
     constexpr int LA = A_BYTES / (1024 * NL), LB = B_BYTES / (1024 * NL);  // load instructions per loading wave and stage, 1 KB each
     constexpr int NMMA = TM * TN;
+    // NST counts whole stages, or (HALF) the halves of stages, 64 bytes of k each, that LDS holds.
+    constexpr bool HALF = tiled_half_stages(TM, NW);
+    constexpr int ROW = HALF ? KB / 2 : KB, SLOT = HALF ? STAGE / 2 : STAGE, RING = NST * SLOT, AHEAD = HALF ? NST / 2 : NST;  // AHEAD: stages requested in front
     constexpr int kOutside = 0x7ffffff0;  // beyond any tile's range
 
     extern __shared__ __align__(16) uint8_t lds[];
@@ -135,26 +144,28 @@ __global__ void __launch_bounds__(64 * (WM * WN + tiled_loader_waves(TM)), WGS *
     int pa[LA], pb[LB];  // k byte of the lane's piece within its stage (for the last, partial stage)
 #pragma unroll
     for (int q = 0; q < LA; ++q) {
-        const int row = (q * NL + loader) * 8 + (lane >> 3);
-        pa[q] = ((lane & 7) ^ ((row >> 1) & 7)) * 16;
+        const int row = HALF ? ((q >> 1) * NL + loader) * 16 + (lane >> 2) : (q * NL + loader) * 8 + (lane >> 3);
+        pa[q] = HALF ? ((lane & 3) ^ ((row >> 2) & 3)) * 16 + (q & 1) * ROW : ((lane & 7) ^ ((row >> 1) & 7)) * 16;
         va[q] = row * a.k + pa[q];
     }
 #pragma unroll
     for (int q = 0; q < LB; ++q) {
         if constexpr (PACKED) {
             // LDS block (16-row tile, half of the stage): [piece j][k group][row slot], 1 KB
-            const int blk = q * NL + loader, t16 = blk >> 1, s = blk & 1, group = (lane >> 4) & 1;
+            const int blk = HALF ? ((q >> 1) * NL + loader) * 2 + (q & 1) : q * NL + loader, t16 = blk >> 1, s = blk & 1, group = (lane >> 4) & 1;
             const int row = (lane & 15) ^ ((t16 & 1) << 3) ^ group << 2;
             vb[q] = t16 * a.k * 16 + (lane >> 5) * 1024 + s * 512 + group * 256 + row * 16;
             pb[q] = 0;
         } else {
-            const int row = (q * NL + loader) * 8 + (lane >> 3);
-            pb[q] = ((lane & 7) ^ (((row >> 1) & 3) | ((row >> 4) & 1) << 2)) * 16;
+            const int row = HALF ? ((q >> 1) * NL + loader) * 16 + (lane >> 2) : (q * NL + loader) * 8 + (lane >> 3);
+            pb[q] = HALF ? ((lane & 3) ^ (((row >> 2) & 1) | ((row >> 4) & 1) << 1)) * 16 + (q & 1) * ROW
+                         : ((lane & 7) ^ (((row >> 1) & 3) | ((row >> 4) & 1) << 2)) * 16;
             vb[q] = row * a.b_stride + pb[q];
         }
     }
     int issued = s_begin;
-    uint32_t slot_issue = 0;
+    uint32_t slot_issue = 0, slot_issue_odd = SLOT;  // where the next stage goes (HALF: its first and second half)
+    auto next_slot = [](uint32_t slot) __attribute__((always_inline)) { return slot + SLOT == RING ? 0u : slot + SLOT; };
     const int k_tail = a.k & (KB - 1), tail_stage = k_tail ? a.k / KB : -1;
     auto issue_begin = [&]() __attribute__((always_inline)) {
         if (issued >= s_end) { ra[2] = 0; rb[2] = 0; }  // past the end: as many loads as ever, nothing is read
@@ -162,12 +173,12 @@ __global__ void __launch_bounds__(64 * (WM * WN + tiled_loader_waves(TM)), WGS *
     auto issue_a = [&](int q) __attribute__((always_inline)) {
         int off = va[q];
         if (issued == tail_stage) off = pa[q] < k_tail ? off : kOutside;
-        load_to_lds(ra, off, lds0 + slot_issue + (uint32_t)(q * NL + loader) * 1024u);
+        load_to_lds(ra, off, lds0 + (HALF && (q & 1) ? slot_issue_odd : slot_issue) + (uint32_t)((HALF ? q >> 1 : q) * NL + loader) * 1024u);
     };
     auto issue_b = [&](int q) __attribute__((always_inline)) {
         int off = vb[q];
         if (!PACKED && issued == tail_stage) off = pb[q] < k_tail ? off : kOutside;
-        load_to_lds(rb, off, lds0 + slot_issue + A_BYTES + (uint32_t)(q * NL + loader) * 1024u);
+        load_to_lds(rb, off, lds0 + (HALF && (q & 1) ? slot_issue_odd : slot_issue) + ROW * BM + (uint32_t)((HALF ? q >> 1 : q) * NL + loader) * 1024u);
     };
     auto issue_end = [&]() __attribute__((always_inline)) {
         auto advance = [](v4i& r, uint32_t by) __attribute__((always_inline)) {
@@ -181,31 +192,32 @@ __global__ void __launch_bounds__(64 * (WM * WN + tiled_loader_waves(TM)), WGS *
             advance(rb, kStepB);
         }
         ++issued;
-        slot_issue = slot_issue + STAGE == NST * STAGE ? 0 : slot_issue + STAGE;
+        slot_issue = next_slot(HALF ? slot_issue_odd : slot_issue);
+        slot_issue_odd = next_slot(slot_issue);
     };
 
     // ---- operand reads -----------------------------------------------------------------------------------------------
     // matrix row r of a weight tile is weight row perm(r): a lane's 16 results of a tile are then 16 consecutive columns
     const int perm = ((lr >> 2) & 1) * 16 + (lr >> 3) * 4 + (lr & 3);
-    const int fa = (lr >> 1) & 7, fb = ((perm >> 1) & 3) | ((perm >> 4) & 1) << 2;
-    const int a_row = (wm * TM * 32 + lr) * KB;
-    const int b_row = A_BYTES + (PACKED ? (wn * TN * 2 + (perm >> 4)) * 2048 + lg * 256 + ((perm & 15) ^ ((perm >> 4) << 3) ^ (lg << 2)) * 16
-                                        : (wn * TN * 32 + perm) * KB);
+    const int fa = HALF ? (lr >> 2) & 3 : (lr >> 1) & 7, fb = HALF ? ((perm >> 2) & 1) | ((perm >> 4) & 1) << 1 : ((perm >> 1) & 3) | ((perm >> 4) & 1) << 2;
+    const int a_row = (wm * TM * 32 + lr) * ROW;
+    const int b_row = ROW * BM + (PACKED ? (wn * TN * 2 + (perm >> 4)) * 16 * ROW + lg * 256 + ((perm & 15) ^ ((perm >> 4) << 3) ^ (lg << 2)) * 16
+                                        : (wn * TN * 32 + perm) * ROW);
     uint32_t slot_read = 0;
     v8i fra[2][TM], frb[2][TN];
     auto read16 = [&](int off) __attribute__((always_inline)) { return *reinterpret_cast<const v4i*>(lds + off); };
     auto join = [](v4i lo, v4i hi) __attribute__((always_inline)) { return v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]}; };
     auto read_a = [&](v8i& dst, int i, int s) __attribute__((always_inline)) {
-        const int off = (int)slot_read + a_row + (((2 * lg) ^ fa ^ (4 * s)) << 4);
-        dst = join(read16(off + i * 32 * KB), read16((off ^ 16) + i * 32 * KB));
+        const int off = (int)slot_read + a_row + (((2 * lg) ^ fa ^ (HALF ? 0 : 4 * s)) << 4);
+        dst = join(read16(off + i * 32 * ROW), read16((off ^ 16) + i * 32 * ROW));
     };
     auto read_b = [&](v8i& dst, int j, int s) __attribute__((always_inline)) {
         if constexpr (PACKED) {
-            const int off = (int)slot_read + b_row + j * 4096 + s * 1024;
+            const int off = (int)slot_read + b_row + j * 32 * ROW + (HALF ? 0 : s * 1024);
             dst = join(read16(off), read16(off + 512));
         } else {
-            const int off = (int)slot_read + b_row + (((2 * lg) ^ fb ^ (4 * s)) << 4);
-            dst = join(read16(off + j * 32 * KB), read16((off ^ 16) + j * 32 * KB));
+            const int off = (int)slot_read + b_row + (((2 * lg) ^ fb ^ (HALF ? 0 : 4 * s)) << 4);
+            dst = join(read16(off + j * 32 * ROW), read16((off ^ 16) + j * 32 * ROW));
         }
     };
 
@@ -218,26 +230,33 @@ __global__ void __launch_bounds__(64 * (WM * WN + tiled_loader_waves(TM)), WGS *
             for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
 
     // Half a stage (64 bytes of k): multiply the operands read half a stage ago (register set S) while the next half's are read into
-    // the other set.  The second half reads from the next stage, so it opens with the wait for that stage and the barrier behind
-    // which this stage's slot is free and the stage NST ahead is requested into it.  The schedule is fixed: operand reads in front
-    // of the first three quarters of the matrix instructions, loads spread over all of them.
+    // the other set.  The second half reads from the next stage, so it opens with the wait for that stage and a barrier behind it.  With
+    // whole stages in LDS that barrier also frees this stage's slot, and the stage NST ahead is requested into it behind the barrier.
+    // With halves, the first half's slot is free half a stage earlier, behind a barrier of its own: the five halves then hold one that is
+    // being read, a whole stage in flight, and the two into which the stage after that is requested.
+    // The schedule is fixed: operand reads in front of the first three quarters of the matrix instructions, loads spread over all of them.
+    constexpr int kFirstLoads = HALF ? (LA + LB) / 2 : 0;  // of a stage's loads, those in the first half
     auto half = [&](auto sel) __attribute__((always_inline)) {
         constexpr int S = decltype(sel)::value;
+        if constexpr (HALF && S == 0) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            workgroup_barrier();
+            issue_begin();
+        }
         if constexpr (S == 1) {
-            if constexpr (LW) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            if constexpr (HALF) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kFirstLoads) : "memory");
+            else if constexpr (LW) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             else wait_loads_and_lds<(NST - 2) * (LA + LB)>();
             workgroup_barrier();
-            slot_read = slot_read + STAGE == NST * STAGE ? 0 : slot_read + STAGE;
-            if constexpr (!LW) issue_begin();
+            if constexpr (!LW && !HALF) issue_begin();
         }
-        constexpr int READS = TM + TN, LOADS = S == 1 && !LW ? LA + LB : 0;
-        // two stages leave a load one stage to arrive in: there the requests stand in front of the first half of the matrix instructions
-        // (4096 x 4096 x 4096 58.5 -> 56.8 us, 1024 x 8192 x 8192 95 -> 91); deeper pipelines lose up to 4 % by that
-        constexpr int kHaste = NST == 2 ? 2 : 1;
+        if constexpr (HALF || S == 1) slot_read = next_slot(slot_read);
+        constexpr int READS = TM + TN, FIRST = S == 1 ? kFirstLoads : 0;
+        constexpr int LOADS = LW ? 0 : HALF ? (S == 0 ? kFirstLoads : LA + LB - kFirstLoads) : S == 1 ? LA + LB : 0;
         int reads = 0, loads = 0;
 #pragma unroll
         for (int t = 0; t < NMMA; ++t) {
-            const int reads_to = NMMA <= 2 ? READS : min(READS, (t + 1) * READS * 4 / (3 * NMMA) + 1), loads_to = min(LOADS, (t + 1) * LOADS * kHaste / NMMA);
+            const int reads_to = NMMA <= 2 ? READS : min(READS, (t + 1) * READS * 4 / (3 * NMMA) + 1), loads_to = min(LOADS, (t + 1) * LOADS / NMMA);
 #pragma unroll
             for (int r = 0; r < READS; ++r)
                 if (r >= reads && r < reads_to) {
@@ -247,8 +266,8 @@ __global__ void __launch_bounds__(64 * (WM * WN + tiled_loader_waves(TM)), WGS *
 #pragma unroll
             for (int l = 0; l < LOADS; ++l)
                 if (l >= loads && l < loads_to) {
-                    if (l < LA) issue_a(l);
-                    else issue_b(l - LA);
+                    if (FIRST + l < LA) issue_a(FIRST + l);
+                    else issue_b(FIRST + l - LA);
                 }
             reads = reads_to;
             loads = loads_to;
@@ -272,8 +291,8 @@ __global__ void __launch_bounds__(64 * (WM * WN + tiled_loader_waves(TM)), WGS *
         // for a load in inline assembly: both buffers pass through the wait.  From here on scalar instructions move them.
         asm volatile("s_nop 4" : "+s"(ra), "+s"(rb) : : "memory");
 #pragma unroll 1
-        for (int s = 0; s < NST; ++s) issue_stage();
-        wait_loads_and_lds<(NST - 1) * (LA + LB)>();
+        for (int s = 0; s < AHEAD; ++s) issue_stage();
+        wait_loads_and_lds<(AHEAD - 1) * (LA + LB)>();
         if constexpr (LW) {  // the barriers of the multiplying waves: one in front of the loop, one per stage, one behind the loop
             workgroup_barrier();
 #pragma unroll 1
@@ -379,7 +398,7 @@ __global__ void __launch_bounds__(64 * (WM * WN + tiled_loader_waves(TM)), WGS *
     constexpr int RPI = 64 / LPR;          // rows per pass
     constexpr int PASSES = 32 / RPI;
     constexpr int RS = TN * 32 + 4;        // floats between rows: 16 rows of one column lie in different banks
-    static_assert(NW * 32 * RS * 4 <= NST * STAGE, "the staging fits in the operands' LDS");
+    static_assert(NW * 32 * RS * 4 <= RING, "the staging fits in the operands' LDS");
     float* const stage = reinterpret_cast<float*>(lds) + wave * (32 * RS);
     const int row0 = wm * TM * 32, col = wn * TN * 32 + (lane % LPR) * 8;
     // buffers over the tile's rows: what lies outside reads as zero and is not stored.  A column past n is marked by bits that no row

@@ -35,6 +35,24 @@ def _loading_waves(TM, NW):
     return 4 if TM < 4 else NW
 
 
+def _half_stages(TM, NW):
+    return TM * NW >= 32
+
+
+def _pieces(rows, TM, NW):
+    """(load, wave, lane) -> row, its 16-byte piece of the stage for A and for a row-major B before the swizzle is undone, and the block of a
+    packed B that a load of a stage of `rows` rows fetches."""
+    NL = _loading_waves(TM, NW)
+    q, wave = np.arange(rows * KB // (1024 * NL))[:, None, None], np.arange(NL)[None, :, None]
+    if _half_stages(TM, NW):
+        row = ((q >> 1) * NL + wave) * 16 + (LANE >> 2)
+        swizzled = [((LANE & 3) ^ f) | (q & 1) << 2 for f in ((row >> 2) & 3, ((row >> 2) & 1) | (((row >> 4) & 1) << 1))]
+        return row, *swizzled, ((q >> 1) * NL + wave) * 2 + (q & 1)
+    row = (q * NL + wave) * 8 + (LANE >> 3)
+    swizzled = [(LANE & 7) ^ f for f in ((row >> 1) & 7, ((row >> 1) & 3) | (((row >> 4) & 1) << 2))]
+    return row, *swizzled, q * NL + wave
+
+
 LANE = np.arange(64)
 
 
@@ -60,7 +78,8 @@ def _audit(kernel, m, n, k, b_stride, plan, packed, base_stride, sa_stride):
     tiles_m, tiles_n = -(-m // BM), -(-n // BN)
     tiles, stages = tiles_m * tiles_n, -(-k // KB)
     grid = tiles * plan.splits
-    assert grid * 64 * NW < U32 and (BM + BN) * KB * NST <= 160 * 1024
+    ring = (BM + BN) * (KB // 2 if _half_stages(TM, NW) else KB) * NST
+    assert grid * 64 * (NW + 4) < U32 and ring <= 160 * 1024
 
     # workgroup -> id: a bijection; tile -> (tm, tn): every tile once, whatever the group height
     per, extra = grid >> 3, grid & 7
@@ -81,15 +100,11 @@ def _audit(kernel, m, n, k, b_stride, plan, packed, base_stride, sa_stride):
     begins = [s * q + min(s, r) for s in range(plan.splits + 1)]
     assert begins[-1] == stages and all(b > a for a, b in zip(begins, begins[1:]))
 
-    NL = _loading_waves(TM, NW)
-    la, lb = BM * KB // (1024 * NL), BN * KB // (1024 * NL)
     k_tail, tail_stage = k % KB, k // KB if k % KB else -1
-    wave = np.arange(NL)[:, None]
     for tm in _edge(tiles_m):
         m0, rows_a = tm * BM, min(BM, m - tm * BM)
-        piece = np.arange(la)[:, None, None] * NL + wave[None]         # (load, wave, lane)
-        row = piece * 8 + (LANE >> 3)
-        pa = ((LANE & 7) ^ ((row >> 1) & 7)) * 16
+        row, pa, _, _ = _pieces(BM, TM, NW)
+        pa = pa * 16
         assert len(np.unique(row * 8 + (pa >> 4))) == BM * 8           # every 16-byte piece of the stage is fetched once
         for s in {0, stages - 1, *(b - 1 for b in begins[1:]), *begins[:-1]}:
             records = rows_a * k - s * KB
@@ -103,10 +118,11 @@ def _audit(kernel, m, n, k, b_stride, plan, packed, base_stride, sa_stride):
     for tn in _edge(tiles_n):
         n0 = tn * BN
         for s in {0, stages - 1, *(b - 1 for b in begins[1:]), *begins[:-1]}:
-            piece = np.arange(lb)[:, None, None] * NL + wave[None]
+            row, _, pb, block = _pieces(BN, TM, NW)
+            pb = pb * 16
             if packed:
                 tiles16 = min(BN // 16, (n + 15) // 16 - n0 // 16)
-                t16, half, group = piece >> 1, piece & 1, (LANE >> 4) & 1
+                t16, half, group = block >> 1, block & 1, (LANE >> 4) & 1
                 slot = (LANE & 15) ^ ((t16 & 1) << 3) ^ (group << 2)
                 within = (LANE >> 5) * 1024 + half * 512 + group * 256 + slot * 16
                 assert len(np.unique(t16 * 128 + (within >> 4))) == BN * 8 and (within < 2048).all()
@@ -114,8 +130,6 @@ def _audit(kernel, m, n, k, b_stride, plan, packed, base_stride, sa_stride):
                 _check(t16 * k * 16 + within, 16, records, t16 < tiles16, ("packed B", tn, s))
                 assert (n0 // 16) * k * 16 + s * 2048 + records == ((n0 // 16) + tiles16) * k * 16 <= (n + 15) // 16 * k * 16
             else:
-                row = piece * 8 + (LANE >> 3)
-                pb = ((LANE & 7) ^ (((row >> 1) & 3) | (((row >> 4) & 1) << 2))) * 16
                 assert len(np.unique(row * 8 + (pb >> 4))) == BN * 8
                 rows_b = min(BN, n - n0)
                 records = (rows_b - 1) * b_stride + k - s * KB
@@ -129,7 +143,7 @@ def _audit(kernel, m, n, k, b_stride, plan, packed, base_stride, sa_stride):
     LPR = 4 * TN
     RPI = 64 // LPR
     passes = 32 // RPI
-    assert NW * 32 * (TN * 32 + 4) * 4 <= (BM + BN) * KB * NST
+    assert NW * 32 * (TN * 32 + 4) * 4 <= ring
     for tm in _edge(tiles_m):
         m0, rows_a = tm * BM, min(BM, m - tm * BM)
         for tn in _edge(tiles_n):
@@ -206,24 +220,24 @@ def test_every_wave_has_its_part_of_the_tile(shape, kernel):
     TM, TN, WM, WN, NST = kernel
     NW, BM, BN = WM * WN, 32 * TM * WM, 32 * TN * WN
     assert (BM, BN) == [(256, 256), (256, 128), (128, 128), (128, 64), (64, 64)][shape]
+    halves = _half_stages(TM, NW)
     stage = (BM + BN) * KB
-    assert stage * NST <= 160 * 1024 and NW % 4 == 0
+    ring = stage * NST // 2 if halves else stage * NST
+    assert ring <= 160 * 1024 and NW % 4 == 0
     NL = _loading_waves(TM, NW)
-    wave = np.arange(NL)[None, :, None]
     loads = 0
-    for rows in (BM, BN):  # A and row-major B: 8 rows of 8 pieces a load; packed B: half a 16-row tile's stage
+    for rows in (BM, BN):  # A and row-major B: 8 rows of 8 pieces a load, or 16 rows of 4; packed B: half a 16-row tile's stage
         per_wave = rows * KB // (1024 * NL)
-        assert per_wave * 1024 * NL == rows * KB
+        assert per_wave * 1024 * NL == rows * KB and (not halves or per_wave % 2 == 0)
         loads += per_wave
-        piece = np.arange(per_wave)[:, None, None] * NL + wave
-        assert (np.sort(piece.ravel()) == np.arange(rows // 8)).all()            # KB of LDS it fills
-        row = piece * 8 + (LANE >> 3)
-        for f in ((row >> 1) & 7, ((row >> 1) & 3) | (((row >> 4) & 1) << 2)):
-            assert len(np.unique(row * 8 + ((LANE & 7) ^ f))) == rows * 8
-        t16, half, group = piece >> 1, piece & 1, (LANE >> 4) & 1
+        row, *pieces, block = _pieces(rows, TM, NW)
+        assert (np.sort(block.ravel()) == np.arange(rows // 8)).all()            # KB of LDS it fills
+        for piece in pieces:
+            assert len(np.unique(row * 8 + piece)) == rows * 8
+        t16, half, group = block >> 1, block & 1, (LANE >> 4) & 1
         slot = (LANE & 15) ^ ((t16 & 1) << 3) ^ (group << 2)
         assert len(np.unique(t16 * 128 + (((LANE >> 5) * 1024 + half * 512 + group * 256 + slot * 16) >> 4))) == rows * 8
-    assert (NST - 1) * loads <= 63                                               # outstanding loads a wait can name
+    assert (NST // 2 - 1 if halves else NST - 1) * loads <= 63                   # outstanding loads a wait can name
     # a matrix tile's rows and columns: lane lr of wave (wm, wn)
     rows = {w // WN * TM * 32 + i * 32 + lr for w in range(NW) for i in range(TM) for lr in range(32)}
     cols = {w % WN * TN * 32 + j * 32 + c for w in range(NW) for j in range(TN) for c in range(32)}
@@ -233,7 +247,7 @@ def test_every_wave_has_its_part_of_the_tile(shape, kernel):
     at = {(w * nmma + t) * 4 + p for w in range(NW) for t in range(nmma) for p in range(4)}
     assert at == set(range(BM * BN * 4 // 1024))
     # epilogue: a wave's rows of 32 in LDS, then 8 columns a lane
-    assert NW * 32 * (TN * 32 + 4) * 4 <= stage * NST
+    assert NW * 32 * (TN * 32 + 4) * 4 <= ring
     lpr = 4 * TN
     out = [(w // WN * TM * 32 + i * 32 + r * (64 // lpr) + lane // lpr, w % WN * TN * 32 + lane % lpr * 8)
            for w in range(NW) for i in range(TM) for r in range(lpr // 2) for lane in range(64)]
