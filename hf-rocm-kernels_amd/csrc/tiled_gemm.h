@@ -22,6 +22,7 @@ struct TiledGemmArgs {
     int tiles_m, tiles_n, group_m;
     int stages_q, stages_r;       // k stages per split, the first stages_r splits one more
     int splits;
+    int window, phase_m, phase_n;  // stages within which a workgroup's start in k is turned; 65536ths of a turn per row and column of tiles
     float* ws;
     uint32_t ws_bytes;
     int* counters;

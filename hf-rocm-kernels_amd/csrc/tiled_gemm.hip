@@ -91,6 +91,27 @@ static void make_tiled_plan(int m, int n, int k, int max_splits, hfrk_tiled_plan
     }
 }
 
+// The workgroups of an XCD share rows of A and of the weight.  Walking k in step they all ask for a line while it is on its way into their
+// L2, and where rows are a multiple of some KB apart they all ask the same channels.  So each starts at a stage of its own: row and column of
+// tiles turn the start so that those who share an operand are spread evenly, within a window of k whose operands (of the workgroups that an XCD
+// runs at a time) take 700 KB of its 4 MB L2; a window of one stage is no turn.  As layer calls with the quantisation in front, us: 201 x 6144 x
+// 4096 16.1 -> 15.3, 300 x 4096 x 4096 16.9 -> 15.9, 512 x 4096 x 14336 packed 40.9 -> 39.2, 474 x 11744 x 11520 packed 78.3 -> 72.6, 507 x 14160 x
+// 15872 115 -> 109, 3385 x 2352 x 25600 packed 328 -> 289, 3605 x 2392 x 18928 242 -> 210; the worst 209 x 6752 x 3328 14.8 -> 15.0, 156 x 7920 x 2848
+// 16.0 -> 16.3.  Windows of 400 KB gain a third of that, of 1.2 to 3 MB as much on the sizes above and lose up to 7 % on others (1192 x 5488 x 2048 23.1 ->
+// 24.6); k turned as a whole loses up to twice the time where it does not fit L2.  64 x 64 tiles start together: they lose 1 to 3 % by it
+// (187 x 4024 x 7872 21.6 -> 22.2, 317 x 1800 x 6400 18.2 -> 18.7).
+static void turn_k(TiledGemmArgs* a, int shape) {
+    const TiledShape& s = kTiledShapes[shape];
+    const int grid = a->tiles_m * a->tiles_n * a->splits, resident = kNumCU * s.per_cu;
+    const int per_xcd = div_up(grid < resident ? grid : resident, 8);
+    int columns = div_up(per_xcd, a->group_m);
+    columns = columns < a->tiles_n ? columns : a->tiles_n;
+    a->phase_m = 65536 / a->group_m;
+    a->phase_n = 65536 / columns;
+    a->window = shape == 4 ? 1 : 700 * 1024 / ((a->group_m * s.bm + columns * s.bn) * kTiledStage);
+    a->window = a->window < 1 ? 1 : a->window;
+}
+
 }  // namespace hfrk
 
 extern "C" {
@@ -157,6 +178,7 @@ int hfrk_tiled_gemm(const void* A, const void* B, int packed, void* D, const voi
     args.splits = p.splits;
     args.stages_q = stages / p.splits;
     args.stages_r = stages % p.splits;
+    turn_k(&args, p.shape);
     return packed ? launch_tiled_packed(args, p.shape, static_cast<hipStream_t>(stream))
                   : launch_tiled_rowmajor(args, p.shape, static_cast<hipStream_t>(stream));
 }

@@ -124,21 +124,21 @@ __global__ void __launch_bounds__(64 * (WM * WN + tiled_loader_waves(TM)), WGS *
     const int gm = min(a.group_m, a.tiles_m - grp * a.group_m);
     const int tn = in_grp / gm, tm = grp * a.group_m + in_grp - tn * gm;
     const int m0 = tm * BM, n0 = tn * BN;
+    const uint32_t phase = ((uint32_t)(in_grp - tn * gm) * (uint32_t)a.phase_m + (uint32_t)tn * (uint32_t)a.phase_n) & 0xffff;  // in 65536ths
     const int s_begin = split * a.stages_q + min(split, a.stages_r), s_end = s_begin + a.stages_q + (split < a.stages_r ? 1 : 0);
 
     // ---- operand streams ---------------------------------------------------------------------------------------------
-    // buffers over this tile's rows from the current stage on
+    // buffers over this tile's rows, moved to the stage that is requested
     const int rows_a = min(BM, a.m - m0);
-    v4i ra = tile_rsrc(a.A + (long)m0 * a.k + (long)s_begin * KB, (uint32_t)rows_a * (uint32_t)a.k - (uint32_t)(s_begin * KB));
+    v4i ra = tile_rsrc(a.A + (long)m0 * a.k, (uint32_t)rows_a * (uint32_t)a.k);
     v4i rb;
     constexpr int kStepB = PACKED ? 2048 : KB;  // a stage of a packed 16-row tile is half of a 4 KB chunk
     if constexpr (PACKED) {
         const int tiles16 = min(BN / 16, (a.n + 15) / 16 - n0 / 16);
-        rb = tile_rsrc(a.B + (long)(n0 / 16) * a.k * 16 + (long)s_begin * kStepB, (uint32_t)tiles16 * (uint32_t)a.k * 16u - (uint32_t)(s_begin * kStepB));
+        rb = tile_rsrc(a.B + (long)(n0 / 16) * a.k * 16, (uint32_t)tiles16 * (uint32_t)a.k * 16u);
     } else {
         const int rows_b = min(BN, a.n - n0);
-        rb = tile_rsrc(a.B + (long)n0 * a.b_stride + (long)s_begin * kStepB,
-                       (uint32_t)(rows_b - 1) * (uint32_t)a.b_stride + (uint32_t)a.k - (uint32_t)(s_begin * kStepB));
+        rb = tile_rsrc(a.B + (long)n0 * a.b_stride, (uint32_t)(rows_b - 1) * (uint32_t)a.b_stride + (uint32_t)a.k);
     }
     int va[LA], vb[LB];
     int pa[LA], pb[LB];  // k byte of the lane's piece within its stage (for the last, partial stage)
@@ -163,35 +163,43 @@ __global__ void __launch_bounds__(64 * (WM * WN + tiled_loader_waves(TM)), WGS *
             vb[q] = row * a.b_stride + pb[q];
         }
     }
-    int issued = s_begin;
+    // The stages of a window of k are requested from `phase` of it on and round to there; then those of the next window.
+    int issued = s_begin, window = s_begin, window_end = min(s_begin + a.window, s_end), window_left = window_end - window;
+    int at = window + (int)((phase * (uint32_t)window_left) >> 16);  // the stage to request next
+    const uint64_t base_a = (uint64_t)(uint32_t)ra[1] << 32 | (uint32_t)ra[0], base_b = (uint64_t)(uint32_t)rb[1] << 32 | (uint32_t)rb[0];
+    const int range_a = ra[2], range_b = rb[2];
     uint32_t slot_issue = 0, slot_issue_odd = SLOT;  // where the next stage goes (HALF: its first and second half)
     auto next_slot = [](uint32_t slot) __attribute__((always_inline)) { return slot + SLOT == RING ? 0u : slot + SLOT; };
     const int k_tail = a.k & (KB - 1), tail_stage = k_tail ? a.k / KB : -1;
     auto issue_begin = [&]() __attribute__((always_inline)) {
-        if (issued >= s_end) { ra[2] = 0; rb[2] = 0; }  // past the end: as many loads as ever, nothing is read
+        auto seek = [&](v4i& r, uint64_t base, int range, int by) __attribute__((always_inline)) {
+            const uint64_t p = base + (uint32_t)by;
+            r[0] = (int)(uint32_t)p;
+            r[1] = (int)(uint32_t)(p >> 32);
+            r[2] = issued < s_end ? range - by : 0;  // past the end: as many loads as ever, nothing is read
+        };
+        seek(ra, base_a, range_a, at * KB);
+        seek(rb, base_b, range_b, at * kStepB);
     };
     auto issue_a = [&](int q) __attribute__((always_inline)) {
         int off = va[q];
-        if (issued == tail_stage) off = pa[q] < k_tail ? off : kOutside;
+        if (at == tail_stage) off = pa[q] < k_tail ? off : kOutside;
         load_to_lds(ra, off, lds0 + (HALF && (q & 1) ? slot_issue_odd : slot_issue) + (uint32_t)((HALF ? q >> 1 : q) * NL + loader) * 1024u);
     };
     auto issue_b = [&](int q) __attribute__((always_inline)) {
         int off = vb[q];
-        if (!PACKED && issued == tail_stage) off = pb[q] < k_tail ? off : kOutside;
+        if (!PACKED && at == tail_stage) off = pb[q] < k_tail ? off : kOutside;
         load_to_lds(rb, off, lds0 + (HALF && (q & 1) ? slot_issue_odd : slot_issue) + ROW * BM + (uint32_t)((HALF ? q >> 1 : q) * NL + loader) * 1024u);
     };
     auto issue_end = [&]() __attribute__((always_inline)) {
-        auto advance = [](v4i& r, uint32_t by) __attribute__((always_inline)) {
-            const uint64_t p = ((uint64_t)(uint32_t)r[1] << 32 | (uint32_t)r[0]) + by;
-            r[0] = (int)(uint32_t)p;
-            r[1] = (int)(uint32_t)(p >> 32);
-            r[2] -= (int)by;
-        };
-        if (issued < s_end) {
-            advance(ra, KB);
-            advance(rb, kStepB);
-        }
         ++issued;
+        at = at + 1 == window_end ? window : at + 1;
+        if (--window_left == 0) {
+            window = window_end;
+            window_end = min(window_end + a.window, s_end);
+            window_left = window_end - window;
+            at = window + (int)((phase * (uint32_t)window_left) >> 16);
+        }
         slot_issue = next_slot(HALF ? slot_issue_odd : slot_issue);
         slot_issue_odd = next_slot(slot_issue);
     };

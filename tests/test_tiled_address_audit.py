@@ -172,6 +172,26 @@ def _audit(kernel, m, n, k, b_stride, plan, packed, base_stride, sa_stride):
         assert (last + 1) * 1024 == tiles * plan.splits * BM * BN * 4 <= WS_BYTES < 1 << 31
 
 
+def test_a_turned_start_requests_every_stage_once():
+    rng = random.Random(4)
+    for _ in range(2000):
+        begin, window, phase = rng.randint(0, 50), rng.randint(1, 43), rng.choice((0, 1, 65535, rng.randint(0, 65535)))
+        end = begin + rng.randint(1, 100)
+        first, last = begin, min(begin + window, end)
+        left = last - first
+        at, seen = first + (phase * left >> 16), []
+        for _ in range(begin, end):
+            assert first <= at < last
+            seen.append(at)
+            at = first if at + 1 == last else at + 1
+            left -= 1
+            if left == 0:
+                first, last = last, min(last + window, end)
+                left = last - first
+                at = first + (phase * left >> 16)
+        assert sorted(seen) == list(range(begin, end))
+
+
 def _plan(m, n, k):
     plan = _capi.TiledPlan()
     assert _capi.load().hfrk_tiled_gemm_plan(m, n, k, ctypes.byref(plan)) == _capi.SUCCESS

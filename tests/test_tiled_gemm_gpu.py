@@ -29,7 +29,9 @@ def _operands(m, n, k, seed):
 SIZES = [(1, 64, 256, 1), (64, 256, 128, 1), (257, 264, 1280, 3), (130, 203, 512, 2), (65, 136, 1008, 1), (600, 520, 768, 1), (200, 72, 16, 1),
          # the 256 x 128 tile on four waves (k no multiple of 128 and 44 stages or more, the last row of tiles more than half full, or many
          # workgroups), and next to it
-         (144, 136, 5520, 1), (143, 136, 5520, 1), (144, 136, 5488, 1), (400, 200, 11280, 2), (512, 264, 5520, 1), (512, 264, 2064, 4)]
+         (144, 136, 5520, 1), (143, 136, 5520, 1), (144, 136, 5488, 1), (400, 200, 11280, 2), (512, 264, 5520, 1), (512, 264, 2064, 4),
+         # several rows and columns of tiles, each with a start in k of its own, over several windows, the last of them shorter
+         (600, 520, 5008, 2)]
 
 
 @pytest.mark.parametrize("add", ["none", "bias", "residual"])
