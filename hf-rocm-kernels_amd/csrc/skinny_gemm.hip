@@ -640,7 +640,8 @@ static bool plan_key(int m, int n, int k, int packed, uint64_t* key) {
 // same kernel instance on the same work: for m <= 16 the same number of 4-row activation loads (m' = 8 serves 5..8),
 // above that the same number of 16-row tiles (m' = 32 serves 17..32); rows past m are out of the buffer's range and
 // cost no traffic.  The nearest such entry wins.
-static int choose_plan(int m, int n, int k, bool packed, hfrk_gemm_plan* plan) {
+static int choose_plan(int m, int n, int k, bool packed, hfrk_gemm_plan* plan, bool* tuned = nullptr) {
+    if (tuned) *tuned = false;
     uint64_t key;
     if (plan_key(m, n, k, packed, &key)) {
         const int top = m <= 16 ? (m + 3) / 4 * 4 : (m + 15) / 16 * 16;
@@ -650,6 +651,7 @@ static int choose_plan(int m, int n, int k, bool packed, hfrk_gemm_plan* plan) {
             const auto it = g_plan_table.find(key);
             if (it != g_plan_table.end() && check_plan(m, n, k, false, &it->second, packed) == HFRK_SUCCESS) {
                 *plan = it->second;
+                if (tuned) *tuned = true;
                 return HFRK_SUCCESS;
             }
         }
@@ -736,6 +738,8 @@ static int gemm_launch(const void* A, const void* B, void* D, const void* base, 
                            packed, use_static, nullptr, base_row, given, needs);
     }
     hfrk_gemm_plan p;
+    hfrk_tiled_plan tiled{};
+    bool use_tiled = false;
     if (user_plan) {
         p = *user_plan;
         const int rc = check_plan(m, swiglu ? n / 2 : n, k, swiglu, &p, packed);
@@ -764,15 +768,21 @@ static int gemm_launch(const void* A, const void* B, void* D, const void* base, 
                 p.lds_bytes = stream_lds_bytes(p.ch, 2);
             }
         } else {
-            rc = choose_plan(m, n, k, packed, &p);
+            bool tuned = false;
+            rc = choose_plan(m, n, k, packed, &p, &tuned);
+            // a table's entry is run as it stands; rows of D or base that are not 16-byte aligned are the tiled kernel's slow ones
+            use_tiled = rc == HFRK_SUCCESS && !tuned && n % 8 == 0 && ((reinterpret_cast<uintptr_t>(D) | reinterpret_cast<uintptr_t>(base)) & 15) == 0 &&
+                        b_stride <= (1 << 21) && tiled_instead(m, n, k, p, &tiled);
         }
         if (rc != HFRK_SUCCESS) return rc;
     }
 
+    size_t need_bytes = use_tiled ? tiled_plan_ws_bytes(tiled, m, n) : plan_ws_bytes(p);
+    long need_counters = use_tiled ? tiled_plan_counters(tiled, m, n) : plan_counters(p);
     if (needs) {
-        if (plan_ws_bytes(p) > kWsFloats * sizeof(float) || plan_counters(p) > kMaxPanels) return HFRK_BAD_SHAPE;
-        needs->ws_bytes = std::max(needs->ws_bytes, plan_ws_bytes(p));
-        needs->counters = std::max(needs->counters, plan_counters(p));
+        if (need_bytes > kWsFloats * sizeof(float) || need_counters > kMaxPanels) return HFRK_BAD_SHAPE;
+        needs->ws_bytes = std::max(needs->ws_bytes, need_bytes);
+        needs->counters = std::max(needs->counters, need_counters);
         return HFRK_SUCCESS;
     }
     int dev = 0;
@@ -780,7 +790,7 @@ static int gemm_launch(const void* A, const void* B, void* D, const void* base, 
     Workspace st;
     size_t ws_bytes = kWsFloats * sizeof(float);
     long counters = kMaxPanels;
-    if (plan_ws_bytes(p) == 0 && plan_counters(p) == 0) {
+    if (need_bytes == 0 && need_counters == 0) {
         ws_bytes = 0;  // nothing crosses workgroups under this plan: no workspace is taken
         counters = 0;
         use_static = false;
@@ -799,15 +809,24 @@ static int gemm_launch(const void* A, const void* B, void* D, const void* base, 
         st.ws = reinterpret_cast<float*>(given->ptr + counters * sizeof(int));
     } else {
         const int rc = workspace_for(dev, stream, &st);
-        if (rc != HFRK_SUCCESS) return rc;
+        if (rc != HFRK_SUCCESS) {
+            if (!use_tiled || plan_ws_bytes(p) != 0 || plan_counters(p) != 0) return rc;
+            use_tiled = false;  // the skinny plan needs no workspace
+            need_bytes = ws_bytes = 0;
+            need_counters = counters = 0;
+        }
     }
-    if (plan_ws_bytes(p) > ws_bytes || plan_counters(p) > counters) return use_static || given ? HFRK_EXCEEDS_SCRATCH : HFRK_BAD_SHAPE;
+    if (need_bytes > ws_bytes || need_counters > counters) return use_static || given ? HFRK_EXCEEDS_SCRATCH : HFRK_BAD_SHAPE;
     if (use_static) {
         // The array keeps whatever the last call (or a launch that never finished) left: the counters of this plan start at zero.
-        const int count = (int)plan_counters(p);
+        const int count = (int)need_counters;
         hipLaunchKernelGGL(zero_ints_kernel, dim3((count + 255) / 256), dim3(256), 0, stream, st.counters, count);
         HFRK_HIP_TRY(hipGetLastError());
     }
+
+    if (use_tiled)
+        return tiled_launch(A, B, packed, D, base, base_row ? 0 : n, scale_a, sa_stride, scale_b, sb_stride, m, n, k, b_stride, d_dtype, tiled, st.ws, ws_bytes,
+                            st.counters, stream);
 
     GemmArgs args{};
     args.A = static_cast<const uint8_t*>(A);
@@ -1077,13 +1096,11 @@ int hfrk_skinny_gemm_fused(const void* A, const void* B, void* D, const void* ba
 
 int hfrk_linear_gemm(const void* A, const void* B, int packed, void* D, const void* base, int base_stride, const float* scale_a,
                      int sa_stride, const float* scale_b, int sb_stride, int m, int n, int k, int b_stride, int d_dtype, void* stream) {
-    // Which kernel takes a call; fp8_linear.py's general path asks the same question.  Above 64 rows the tiled GEMM.  At 33..64 rows the
-    // skinny kernels take a k of whole 256-byte chunks in one launch and are faster on 108 of 120 measured points (at 64 rows 4096 x 4096
-    // 8.5 us skinny, 10.7 tiled; 28672 x 4096 25.0 / 31.8), but a k that ends inside a chunk in two launches over the same weight: there
-    // the tiled GEMM (4104 x 1936 at 33 rows 13.7 / 9.4, at 64 rows 15.9 / 10.3; 2056 x 16400 at 33 rows 28.2 / 19.0), except on few
-    // columns of a very long k, where its at most 4 splits leave it too few workgroups (1024 x 28656 at 33 rows 24.3 / 26.6).  The line
-    // k = 16 n stands between the last two.
-    if ((m > HFRK_GEMM_MAX_M || (m > hfrk::kStreamMaxM && k % 256 != 0 && k <= 16L * n)) && hfrk::tiled_size_ok(m, n, k) && (packed || b_stride <= (1 << 21)))
+    // Which kernel takes a call; fp8_linear.py's general path asks the same question.  Above 64 rows the tiled GEMM.  Up to there
+    // the skinny GEMM, which weighs its plan against tiles (tiled_instead), but a k that ends inside a 256-byte chunk would take it two
+    // launches over the same weight from 33 rows on: there the tiled GEMM too (4104 x 1936 at 33 rows 13.7 / 9.4, at 64 rows 15.9 / 10.3;
+    // 1024 x 28656 at 33 rows 22.8 / 13.6, 1280 x 27632 at 50 rows 32.7 / 14.6).
+    if ((m > HFRK_GEMM_MAX_M || (m > hfrk::kStreamMaxM && k % 256 != 0)) && hfrk::tiled_size_ok(m, n, k) && (packed || b_stride <= (1 << 21)))
         return hfrk_tiled_gemm(A, B, packed, D, base, base_stride, scale_a, sa_stride, scale_b, sb_stride, m, n, k, b_stride, d_dtype, nullptr, stream);
     if (base && base_stride != 0 && base_stride != n) return HFRK_BAD_SHAPE;
     if (m > HFRK_GEMM_MAX_M) {  // beyond the tiled kernel's 32-bit offsets: one skinny GEMM per 64 rows

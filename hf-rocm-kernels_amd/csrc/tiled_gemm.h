@@ -60,7 +60,16 @@ HFRK_TILED_FOUR_WAVES(HFRK_TILED_SAME)
 constexpr int kTiledShapeCount = sizeof(kTiledShapes) / sizeof(kTiledShapes[0]);
 constexpr int tiled_lds_bytes(const TiledShape& s) { return (s.bm + s.bn) * (s.halves ? kTiledStage / 2 : kTiledStage) * s.stages; }
 
-bool tiled_size_ok(int m, int n, int k);  // tiled_gemm.hip
+// tiled_gemm.hip
+bool tiled_size_ok(int m, int n, int k);
+// Whether the tiled GEMM is the faster one for a call that the skinny GEMM would run under `skinny`, and the plan it then takes.
+bool tiled_instead(int m, int n, int k, const hfrk_gemm_plan& skinny, hfrk_tiled_plan* plan);
+size_t tiled_plan_ws_bytes(const hfrk_tiled_plan& p, int m, int n);
+long tiled_plan_counters(const hfrk_tiled_plan& p, int m, int n);
+// The launch alone: arguments are checked and the plan fits them and the workspace.
+int tiled_launch(const void* A, const void* B, bool packed, void* D, const void* base, int base_stride, const float* scale_a, int sa_stride,
+                 const float* scale_b, int sb_stride, int m, int n, int k, int b_stride, int d_dtype, const hfrk_tiled_plan& p, float* ws, size_t ws_bytes,
+                 int* counters, hipStream_t stream);
 int launch_tiled_rowmajor(const TiledGemmArgs& args, int shape, hipStream_t stream);  // tiled_gemm_rowmajor.hip
 int launch_tiled_packed(const TiledGemmArgs& args, int shape, hipStream_t stream);    // tiled_gemm_packed.hip
 

@@ -18,6 +18,12 @@ static size_t tiled_ws_bytes(const TiledShape& s, int m, int n, int splits) {
     return splits <= 1 ? 0 : (size_t)div_up(m, s.bm) * div_up(n, s.bn) * splits * s.bm * s.bn * sizeof(float);
 }
 
+size_t tiled_plan_ws_bytes(const hfrk_tiled_plan& p, int m, int n) { return tiled_ws_bytes(kTiledShapes[p.shape], m, n, p.splits); }
+long tiled_plan_counters(const hfrk_tiled_plan& p, int m, int n) {
+    const TiledShape& s = kTiledShapes[p.shape];
+    return p.splits <= 1 ? 0 : (long)div_up(m, s.bm) * div_up(n, s.bn);
+}
+
 static int check_tiled_plan(int m, int n, int k, const hfrk_tiled_plan& p) {
     if (p.shape < 0 || p.shape >= kTiledShapeCount || p.splits < 1 || p.group_m < 1) return HFRK_INVALID_CONFIG;
     const TiledShape& s = kTiledShapes[p.shape];
@@ -56,18 +62,80 @@ static float tiled_cost(int m, int n, int k, int shape, int splits) {
 
 constexpr int kTiledMaxSplits = 8;
 
+// Up to 64 rows: one row of tiles streams the weight.  64 x 64 tiles with k in up to 8 parts of 4 stages or more on at most 512 workgroups, or,
+// where they take a second round, 128 x 64 tiles, two on a compute unit.  In us, the constants fitted to 1500 sizes of 17 to 64 rows, weights from memory
+// and from the 256 MB cache alike (5300 calls; median error 2.6 %, 90 % of them within 8 %).
+static float few_rows_cost(int m, int n, int k, int shape, int splits) {
+    struct Shape { float fixed, stage, rows, bytes_per_us, start, overlap; };
+    static constexpr Shape kWide = {4.15f, .221f, .292f, 5.69e6f, .576f, .389f}, kNarrow = {2.45f, .090f, .109f, 9.04e6f, 2.79f, .548f};
+    const Shape& c = shape == 3 ? kWide : kNarrow;
+    const long wgs = (long)div_up(n, 64) * splits;
+    const int rounds = shape == 3 ? 1 : div_up(wgs, kNumCU);
+    const float work = rounds * (c.fixed + (float)div_up(k, kTiledStage) / splits * (c.stage + c.rows * (m + 64) / 128.f));
+    const float stream = (float)n * k / c.bytes_per_us + c.start;
+    float t = fmaxf(work, stream) + c.overlap * fminf(work, stream);
+    if (splits > 1) t += .708f + .344f * splits + 1.579f * wgs / kNumCU;
+    return t;
+}
+
+static float make_few_rows_plan(int m, int n, int k, int max_splits, hfrk_tiled_plan* plan) {
+    const int stages = div_up(k, kTiledStage);
+    const long tiles = div_up(n, 64);
+    float best = INFINITY;
+    auto offer = [&](int shape, int splits) {
+        const float t = few_rows_cost(m, n, k, shape, splits);
+        if (t < best) {
+            best = t;
+            *plan = {shape, splits, 1};
+        }
+    };
+    offer(4, 1);
+    if (tiles > kNumCU && tiles <= 2 * kNumCU) offer(3, 1);
+    for (int splits = 2; splits <= max_splits && 4 * splits <= stages && tiles * splits <= 2 * kNumCU; ++splits) offer(4, splits);
+    return best;
+}
+
+// What the workgroup kernel (skinny_gemm.hip) takes under a plan of its own, in us: its unit is a panel's rows and a slab of k, workgroups that
+// share a panel exchange their sums.  Fitted to 1079 of the same calls by the number of waves along k (median error 6 %, 90 % of them within 12 to 18 %).
+static float workgroup_kernel_cost(int m, int n, int k, const hfrk_gemm_plan& p) {
+    struct Waves { float fixed, bytes, rows, bytes_per_us, overlap, exchange, share; };
+    static constexpr Waves kWaves[3] = {{3.45f, .000869f, 36.8f, 19.1e6f, 2.53f, 4.98f, .0073f},
+                                        {3.72f, .00150f, 15.1f, 8.94e6f, .968f, 3.65f, .0124f},
+                                        {4.87f, .00162f, 19.7f, 5.85e6f, 0.f, 1.01f, .0516f}};
+    const Waves& c = kWaves[p.wk >= 4 ? 2 : p.wk - 1];
+    const long units = (long)p.panels * p.slabs, per = units / p.grid;
+    const int padded = 16 * div_up(m, 16);
+    const float work = (float)div_up(units, p.grid) * c.bytes * (16 * p.wn + c.rows * padded) * (p.wk * p.ch) * .25f;
+    const float stream = (float)n * k / c.bytes_per_us;
+    float t = c.fixed + fmaxf(work, stream) + c.overlap * fminf(work, stream);
+    if (p.panels % p.grid != 0) {  // panels are shared
+        const bool ragged = units % p.grid != 0 || (per % p.slabs != 0 && p.slabs % per != 0);
+        const long sharers = div_up(p.slabs, per) + (ragged ? 1 : 0);
+        t += c.exchange + c.share * (float)(sharers < p.slabs ? sharers : p.slabs) * 16 * p.wn * padded * 4 / 1024.f;
+    }
+    return t;
+}
+
+// 17 to 64 rows that the skinny GEMM's planner gives to its workgroup kernel.  That kernel was tuned on weights whose rows and k deal out in whole
+// panels and slabs over the compute units; elsewhere the shares of a panel lie with up to twenty workgroups, whose sums one of them collects.  Over 1079
+// such calls (n and k drawn from 1024 to 28672, 40 % of them multiples of 256, 512 or 1024; row-major and packed) the choice below is 23 % faster in
+// the mean: 57 x 2832 x 1792 14.5 -> 6.4 us, 50 x 6176 x 3072 15.5 -> 8.5 from the 256 MB cache and 15.4 -> 11.2 from memory, 57 x 1752 x 14592 19.5 -> 12.0,
+// 64 x 11096 x 5120 21.5 -> 13.7 / 21.8 -> 20.1.  The margins are the fits' errors: whole panels, where nothing is exchanged, and weights above 76 MB, where
+// memory bounds both, are predicted less well.  Above 112 MB at most 2 % could be gained (64 x 8192 x 28672 44 us and 50 on tiles).  What it loses is 7 % at
+// most (40 x 3072 x 8192), 3 % or more on 5 of the 1079.  The row-split and K-split kernels stay: the tiled kernel is 3 to 60 % slower than they are on
+// all but a few of their sizes.
+bool tiled_instead(int m, int n, int k, const hfrk_gemm_plan& skinny, hfrk_tiled_plan* plan) {
+    if (m <= 16 || skinny.wn < 1 || (long)n * k > (112L << 20) || !tiled_size_ok(m, n, k)) return false;
+    const bool whole_panels = skinny.panels % skinny.grid == 0, large = (long)n * k > (76L << 20);
+    const float margin = (whole_panels ? 1.15f : 1.08f) + (large ? .07f : 0.f);
+    return margin * make_few_rows_plan(m, n, k, kTiledMaxSplits, plan) < workgroup_kernel_cost(m, n, k, skinny);
+}
+
 static void make_tiled_plan(int m, int n, int k, int max_splits, hfrk_tiled_plan* plan) {
     float best = INFINITY;
     const int stages = div_up(k, kTiledStage);
-    if (m <= 64) {
-        // One row of tiles streams the weight: the deepest pipeline (64 x 64), k split up to one workgroup per compute unit but
-        // at most 4 ways and not below 8 stages.  The fit below starts at 65 rows and splits too little here: 4096 x 14336 at 64 rows
-        // 24.4 -> 18.1 us, 8192 x 28672 at 33 rows 67 -> 45, 4104 x 1936 at 64 rows 11.8 -> 10.3.
-        int splits = kNumCU / div_up(n, 64);
-        splits = splits < stages / 8 ? splits : stages / 8;
-        splits = splits < 4 ? splits : 4;
-        splits = splits < max_splits ? splits : max_splits;
-        *plan = {4, splits < 1 ? 1 : splits, 1};
+    if (m <= 64) {  // (the fit below starts at 65 rows)
+        make_few_rows_plan(m, n, k, max_splits, plan);
         return;
     }
     for (int shape = 0; shape < kTiledShapeCount; ++shape) {
@@ -112,6 +180,41 @@ static void turn_k(TiledGemmArgs* a, int shape) {
     a->window = a->window < 1 ? 1 : a->window;
 }
 
+int tiled_launch(const void* A, const void* B, bool packed, void* D, const void* base, int base_stride, const float* scale_a, int sa_stride,
+                 const float* scale_b, int sb_stride, int m, int n, int k, int b_stride, int d_dtype, const hfrk_tiled_plan& p, float* ws, size_t ws_bytes,
+                 int* counters, hipStream_t stream) {
+    TiledGemmArgs args{};
+    const TiledShape& s = kTiledShapes[p.shape];
+    args.A = static_cast<const uint8_t*>(A);
+    args.B = static_cast<const uint8_t*>(B);
+    args.D = D;
+    args.base = base;
+    args.base_stride = base ? base_stride : 0;
+    args.scale_a = scale_a;
+    args.scale_b = scale_b;
+    args.sa_stride = sa_stride;
+    args.sb_stride = sb_stride;
+    args.m = m;
+    args.n = n;
+    args.k = k;
+    args.b_stride = b_stride;
+    args.d_dtype = d_dtype;
+    args.vec = n % 8 == 0 && args.base_stride % 8 == 0 && ((reinterpret_cast<uintptr_t>(D) | reinterpret_cast<uintptr_t>(base)) & 15) == 0;
+    args.tiles_m = div_up(m, s.bm);
+    args.tiles_n = div_up(n, s.bn);
+    args.group_m = p.group_m;
+    const int stages = div_up(k, kTiledStage);
+    args.splits = p.splits;
+    args.ws = ws;
+    args.ws_bytes = (uint32_t)ws_bytes;
+    args.counters = counters;
+    args.stages_q = stages / p.splits;
+    args.stages_r = stages % p.splits;
+    turn_k(&args, p.shape);
+    return packed ? launch_tiled_packed(args, p.shape, stream)
+                  : launch_tiled_rowmajor(args, p.shape, stream);
+}
+
 }  // namespace hfrk
 
 extern "C" {
@@ -144,43 +247,21 @@ int hfrk_tiled_gemm(const void* A, const void* B, int packed, void* D, const voi
     } else {
         make_tiled_plan(m, n, k, kTiledMaxSplits, &p);
     }
-    TiledGemmArgs args{};
+    float* ws = nullptr;
+    size_t ws_bytes = 0;
+    int* counters = nullptr;
     if (p.splits > 1) {
-        size_t bytes = 0;
-        const int rc = stream_workspace(static_cast<hipStream_t>(stream), &args.ws, &bytes, &args.counters);
-        if (rc == HFRK_SUCCESS) args.ws_bytes = (uint32_t)bytes;
-        // no workspace left, no memory for one (a caching allocator may hold it all), or none before a capture began: a call that names
-        // no plan runs without splitting k
-        else if (!plan && (rc == HFRK_NO_WORKSPACE || rc == HFRK_NOT_INITIALISED ||
-                           (rc == HFRK_HIP_ERROR && hfrk_last_hip_error() == (int)hipErrorOutOfMemory))) make_tiled_plan(m, n, k, 1, &p);
-        else return rc;
+        const int rc = stream_workspace(static_cast<hipStream_t>(stream), &ws, &ws_bytes, &counters);
+        if (rc != HFRK_SUCCESS) {
+            // no workspace left, no memory for one (a caching allocator may hold it all), or none before a capture began: a call that names
+            // no plan runs without splitting k
+            const bool none = rc == HFRK_NO_WORKSPACE || rc == HFRK_NOT_INITIALISED || (rc == HFRK_HIP_ERROR && hfrk_last_hip_error() == (int)hipErrorOutOfMemory);
+            if (plan || !none) return rc;
+            make_tiled_plan(m, n, k, 1, &p);
+        }
     }
-    const TiledShape& s = kTiledShapes[p.shape];
-    args.A = static_cast<const uint8_t*>(A);
-    args.B = static_cast<const uint8_t*>(B);
-    args.D = D;
-    args.base = base;
-    args.base_stride = base ? base_stride : 0;
-    args.scale_a = scale_a;
-    args.scale_b = scale_b;
-    args.sa_stride = sa_stride;
-    args.sb_stride = sb_stride;
-    args.m = m;
-    args.n = n;
-    args.k = k;
-    args.b_stride = b_stride;
-    args.d_dtype = d_dtype;
-    args.vec = n % 8 == 0 && args.base_stride % 8 == 0 && ((reinterpret_cast<uintptr_t>(D) | reinterpret_cast<uintptr_t>(base)) & 15) == 0;
-    args.tiles_m = div_up(m, s.bm);
-    args.tiles_n = div_up(n, s.bn);
-    args.group_m = p.group_m;
-    const int stages = div_up(k, kTiledStage);
-    args.splits = p.splits;
-    args.stages_q = stages / p.splits;
-    args.stages_r = stages % p.splits;
-    turn_k(&args, p.shape);
-    return packed ? launch_tiled_packed(args, p.shape, static_cast<hipStream_t>(stream))
-                  : launch_tiled_rowmajor(args, p.shape, static_cast<hipStream_t>(stream));
+    return tiled_launch(A, B, packed != 0, D, base, base_stride, scale_a, sa_stride, scale_b, sb_stride, m, n, k, b_stride, d_dtype, p, ws, ws_bytes,
+                        counters, static_cast<hipStream_t>(stream));
 }
 
 }  // extern "C"

@@ -6,8 +6,8 @@ usual (input, weight, weight_scale, input_scale, bias) signature, and an nn.Modu
 
 A call runs as one quantisation kernel (skipped when the caller already holds fp8 activations and their scales, e.g. from
 `residual_rms_dynamic` / `swiglu_dynamic`) and one GEMM with the scales, the bias or residual folded into its epilogue: a
-skinny GEMM for decode batches (up to 64 tokens; 32 where k ends inside a 256-byte chunk and is at most 16 n), the tiled GEMM for
-everything larger, up to whole prompts.
+skinny GEMM for decode batches (up to 64 tokens; 32 where k ends inside a 256-byte chunk), the tiled GEMM for everything larger, up to
+whole prompts, and for the sizes of 17 to 64 tokens that the skinny GEMM itself hands to it.
 """
 from typing import Optional, Sequence, Tuple, Union
 
@@ -78,7 +78,7 @@ def apply_fp8_linear(
     m = q.size(0)
     if sa.numel() != 1:
         sa = sa[:m]  # a buffer of scales may be longer than the batch
-    tiled = m > _capi.GEMM_MAX_M or (m > 32 and k % 256 != 0 and k <= 16 * n)  # as hfrk_linear_gemm has it
+    tiled = m > _capi.GEMM_MAX_M or (m > 32 and k % 256 != 0)  # as hfrk_linear_gemm has it
     base = None
     if residual is not None:
         base = residual.reshape(m, n)

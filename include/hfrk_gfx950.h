@@ -127,7 +127,9 @@ int hfrk_skinny_gemm_validate(int m, int n, int k, int b_stride, int split_k, in
                               int consumers, int a_lanes, int b_lanes, int qsize, int op_m, int ops);
 
 /* Pure host function: choose the decomposition for a shape (counterpart of infer_skinny_gemm_params,
- * hf_rocm_kernels/operators/skinny_gemm/wrapped.py:42-102).  Returns HFRK_SUCCESS or a shape error. */
+ * hf_rocm_kernels/operators/skinny_gemm/wrapped.py:42-102).  Returns HFRK_SUCCESS or a shape error.  Where this is the workgroup
+ * decomposition (wn >= 1) a call of 17 to 64 rows that names no plan and has none in the table may run on the tiled kernel instead
+ * (hfrk_tiled_gemm), as the library's cost estimates of the two have it; every entry point then does, with the same bits. */
 int hfrk_skinny_gemm_plan(int m, int n, int k, hfrk_gemm_plan* plan);
 
 /* Plan table (host only, thread-safe): tuned decompositions, keyed (m, n, k, packed), that take the planner's place
@@ -270,7 +272,7 @@ int hfrk_skinny_gemm_packed(const void* A, const void* B_packed, void* D, const 
                             int k, int d_dtype, int epilogue, const hfrk_gemm_plan* plan, void* stream);
 
 /* The linear layer's GEMM for any number of rows, under the library's own plan: hfrk_tiled_gemm (below, same arguments) above 64 rows and at
- * 33..64 rows where k % 256 != 0 and k <= 16 n; a skinny GEMM otherwise; one skinny GEMM per 64 rows where a size is beyond the tiled
+ * 33..64 rows where k % 256 != 0; a skinny GEMM otherwise; one skinny GEMM per 64 rows where a size is beyond the tiled
  * kernel's.  Plan tables apply to skinny GEMMs.  base_stride is 0 (one row of n values added to every row of D: a bias) or, where a
  * skinny GEMM runs, n. */
 int hfrk_linear_gemm(const void* A, const void* B, int packed, void* D, const void* base, int base_stride, const float* scale_a,

@@ -111,6 +111,55 @@ def test_weights_beyond_the_tiled_kernels_sizes_run_in_pieces():
         assert torch.equal(whole[r0:r1], apply_fp8_linear(a[r0:r1], w, sw, sa[r0:r1], bias=bias))
 
 
+# (m, n, k) that the skinny entry points hand to the tiled kernel: one tile's height and the smallest row count, ragged columns, k in one and in
+# several parts, tiles in pairs on a compute unit
+@pytest.mark.parametrize("m,n,k", [(17, 1112, 6912), (64, 3800, 1792), (33, 2136, 15104), (44, 17152, 1792), (64, 1040, 2560)])
+def test_skinny_calls_that_run_on_tiles(m, n, k):
+    import hf_rocm_kernels as h
+    from hf_rocm_kernels import _capi
+    from hf_rocm_kernels.utils.weight_format import pack_weight
+    lib = _capi.load()
+    a, w, sa, sw = _operands(m, n, k, seed=m + n)
+    da, dw, dsa, dsw = (t.cuda() for t in (a, w, sa, sw))
+    g = torch.Generator().manual_seed(5)
+    base = torch.randn(m, n, generator=g).to(torch.bfloat16)
+    check = oracle_checker(a, w.t(), sa, sw, torch.bfloat16, base=base)
+    outs = []
+    for weight in (dw.t(), pack_weight(dw)):
+        out = torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
+        outs.append(h.skinny_gemm_add(da, weight, dsa, dsw, base.cuda(), output=out))
+        check(outs[-1])
+    for entry in (lib.hfrk_skinny_gemm_ex, lib.hfrk_skinny_gemm_noalloc):  # added to what is there, in place
+        out = base.cuda()
+        _capi.check(entry(da.data_ptr(), dw.data_ptr(), out.data_ptr(), dsa.data_ptr(), 1, dsw.data_ptr(), 1, m, n, k, k, _capi.BF16, 1, None,
+                          torch.cuda.current_stream().cuda_stream), "accumulate")
+        torch.cuda.synchronize()
+        assert torch.equal(out, outs[0])
+    # captured and replayed between other work; the workspace is the capture stream's
+    stream, out = torch.cuda.Stream(), torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        h.skinny_gemm_add(da, dw.t(), dsa, dsw, base.cuda(), output=out)
+        torch.cuda.synchronize()
+        addend, graph = base.cuda(), torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            h.skinny_gemm_add(da, dw.t(), dsa, dsw, addend, output=out)
+    for _ in range(3):
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, outs[0])
+    del graph
+    lib.hfrk_release_stream(stream.cuda_stream)
+    # rows that are not 16-byte aligned stay where they were
+    off = torch.empty(m * n + 4, dtype=torch.bfloat16, device="cuda")[4:].view(m, n)
+    off.copy_(base)
+    _capi.check(lib.hfrk_skinny_gemm_ex(da.data_ptr(), dw.data_ptr(), off.data_ptr(), dsa.data_ptr(), 1, dsw.data_ptr(), 1, m, n, k, k, _capi.BF16, 1, None,
+                                        torch.cuda.current_stream().cuda_stream), "8-byte rows")
+    check(off)
+
+
 # A process of its own: it takes every workspace there is.
 _NO_WORKSPACE = """
 import ctypes, torch
