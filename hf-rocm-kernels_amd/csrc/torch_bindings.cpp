@@ -657,6 +657,69 @@ bool llama_mlp(const at::Tensor& input, const at::Tensor& residual, at::Tensor& 
     return status == HFRK_SUCCESS;
 }
 
+// The row kernels beside the GEMMs as their wrappers are usually called: no buffer to clear, the launcher's own choice of threads, and nothing that
+// autograd would have to know of.  In Python the checks, two to four allocations and the operator took 8 to 10 us a call, the kernels 2 to 4; now 5.5 to 6.3.
+bool plain_rows(const at::Tensor& x) {
+    return x.is_cuda() && x.dim() == 2 && is_16bit(x.scalar_type()) && x.is_contiguous() && x.numel() > 0 && x.size(0) < (int64_t(1) << 24) &&
+           x.size(1) < (int64_t(1) << 24) && !(at::GradMode::is_enabled() && x.requires_grad());
+}
+
+bool plain_rms(const at::Tensor& input, const at::Tensor& residual, const at::Tensor& weight, double epsilon) {
+    return plain_rows(input) && plain_rows(residual) && residual.sizes() == input.sizes() && residual.scalar_type() == input.scalar_type() &&
+           residual.device() == input.device() && weight.dim() == 1 && weight.size(0) == input.size(1) && weight.is_contiguous() &&
+           weight.scalar_type() == input.scalar_type() && weight.device() == input.device() && !(at::GradMode::is_enabled() && weight.requires_grad()) &&
+           epsilon > 0;
+}
+
+// Rows that the dynamic kernels take: whole 16-byte pieces, held in registers.
+bool dynamic_columns(int64_t cols) { return cols % 8 == 0 && cols <= 32768; }
+
+at::Tensor residual_rms_new(const at::Tensor& input, at::Tensor& residual, const at::Tensor& weight, double epsilon, const std::optional<at::Tensor>& scale) {
+    if (!plain_rms(input, residual, weight, epsilon) || (scale.has_value() && !one_float(*scale, input))) return {};
+    DeviceScope scope(input);
+    const int io = dtype16(input, "input");
+    at::Tensor output = at::empty(input.sizes(), input.options().dtype(scale.has_value() ? at::kFloat8_e4m3fn : input.scalar_type()));
+    return hfrk_residual_rms(input.data_ptr(), residual.data_ptr(), weight.data_ptr(), scale.has_value() ? scale->data_ptr<float>() : nullptr, (float)epsilon,
+                             output.data_ptr(), nullptr, (int)input.size(0), (int)input.size(1), 0, io, scale.has_value() ? HFRK_FP8_E4M3FN : io, 0, 0,
+                             current_stream(input)) == HFRK_SUCCESS
+               ? output
+               : at::Tensor();
+}
+
+std::tuple<at::Tensor, at::Tensor> residual_rms_dynamic_new(const at::Tensor& input, at::Tensor& residual, const at::Tensor& weight, double epsilon) {
+    if (!plain_rms(input, residual, weight, epsilon) || !dynamic_columns(input.size(1))) return {};
+    DeviceScope scope(input);
+    at::Tensor output = at::empty(input.sizes(), input.options().dtype(at::kFloat8_e4m3fn));
+    at::Tensor scales = at::empty({input.size(0)}, input.options().dtype(at::kFloat));
+    if (hfrk_residual_rms_dynamic(input.data_ptr(), residual.data_ptr(), weight.data_ptr(), (float)epsilon, output.data_ptr(), scales.data_ptr<float>(), nullptr,
+                                  (int)input.size(0), (int)input.size(1), 0, dtype16(input, "input"), current_stream(input)) != HFRK_SUCCESS)
+        return {};
+    return {output, scales};
+}
+
+at::Tensor swiglu_new(const at::Tensor& gate_up, const at::Tensor& scale) {
+    if (!plain_rows(gate_up) || gate_up.size(1) % 2 != 0 || !one_float(scale, gate_up)) return {};
+    DeviceScope scope(gate_up);
+    const int64_t rows = gate_up.size(0), cols = gate_up.size(1) / 2;
+    at::Tensor output = at::empty({rows, cols}, gate_up.options().dtype(at::kFloat8_e4m3fn));
+    return hfrk_swiglu(gate_up.data_ptr(), scale.data_ptr<float>(), output.data_ptr(), nullptr, (int)rows, (int)cols, 0, dtype16(gate_up, "gate_up"), 0, 0,
+                       current_stream(gate_up)) == HFRK_SUCCESS
+               ? output
+               : at::Tensor();
+}
+
+std::tuple<at::Tensor, at::Tensor> swiglu_dynamic_new(const at::Tensor& gate_up) {
+    if (!plain_rows(gate_up) || gate_up.size(1) % 2 != 0 || !dynamic_columns(gate_up.size(1) / 2)) return {};
+    DeviceScope scope(gate_up);
+    const int64_t rows = gate_up.size(0), cols = gate_up.size(1) / 2;
+    at::Tensor output = at::empty({rows, cols}, gate_up.options().dtype(at::kFloat8_e4m3fn));
+    at::Tensor scales = at::empty({rows}, gate_up.options().dtype(at::kFloat));
+    if (hfrk_swiglu_dynamic(gate_up.data_ptr(), output.data_ptr(), scales.data_ptr<float>(), nullptr, (int)rows, (int)cols, 0, dtype16(gate_up, "gate_up"),
+                            current_stream(gate_up)) != HFRK_SUCCESS)
+        return {};
+    return {output, scales};
+}
+
 bool is_byte_tensor(const at::Tensor& t) {
     return t.scalar_type() == at::kByte || t.scalar_type() == at::kFloat8_e4m3fn || t.scalar_type() == at::kFloat8_e4m3fnuz;
 }
@@ -803,6 +866,17 @@ TORCH_LIBRARY(_HFRK_C, ops) {
         "Tensor down_output_scale, bool add_residual, Tensor(c!) output, Tensor(d!)? memory=None) -> bool");
     ops.impl("llama_mlp", c10::kCUDA, &llama_mlp);
     ops.impl("llama_mlp", torch::dispatch(c10::DispatchKey::Autograd, torch::CppFunction::makeFallthrough()));
+
+    ops.def("residual_rms_new(Tensor input, Tensor(a!) residual, Tensor weight, float epsilon, Tensor? scale) -> Tensor");
+    ops.impl("residual_rms_new", c10::kCUDA, &residual_rms_new);
+    ops.def("residual_rms_dynamic_new(Tensor input, Tensor(a!) residual, Tensor weight, float epsilon) -> (Tensor, Tensor)");
+    ops.impl("residual_rms_dynamic_new", c10::kCUDA, &residual_rms_dynamic_new);
+    ops.def("swiglu_new(Tensor gate_up, Tensor scale) -> Tensor");
+    ops.impl("swiglu_new", c10::kCUDA, &swiglu_new);
+    ops.def("swiglu_dynamic_new(Tensor gate_up) -> (Tensor, Tensor)");
+    ops.impl("swiglu_dynamic_new", c10::kCUDA, &swiglu_dynamic_new);
+    for (const char* name : {"residual_rms_new", "residual_rms_dynamic_new", "swiglu_new", "swiglu_dynamic_new"})
+        ops.impl(name, torch::dispatch(c10::DispatchKey::Autograd, torch::CppFunction::makeFallthrough()));
 
     ops.def("quantize_fp8(Tensor input, Tensor? scale_tensor, Tensor! output, Tensor! scales) -> ()");
     ops.impl("quantize_fp8", c10::kCUDA, &quantize_fp8);

@@ -19,7 +19,8 @@ _RETURNS_NOTHING = ("increment", "residual_rms", "swiglu", "pack_weight", "pack_
 _RETURNS_STATUS = ("skinny_gemm_tb", "skinny_gemm_scaled", "skinny_gemm_fused", "skinny_gemm_packed", "skinny_gemm_rms_fused",
                    # a result of their own, _OTHER_RESULT; the wrappers keep fake calls away from these (utils/dispatch.py), a caller of
                    # torch.ops need not
-                   "fp8_linear", "skinny_gemm_new", "skinny_gemm_into", "llama_mlp")
+                   "fp8_linear", "skinny_gemm_new", "skinny_gemm_into", "llama_mlp", "residual_rms_new", "residual_rms_dynamic_new", "swiglu_new",
+                   "swiglu_dynamic_new")
 
 
 def _nothing(*args, **kwargs) -> None:
@@ -39,6 +40,22 @@ def _skinny_gemm_new(A, B, scale):
     return A.new_empty((A.shape[0], B.shape[1]), dtype=torch.float16)
 
 
+def _residual_rms_new(input, residual, weight, epsilon, scale):
+    return input.new_empty(input.shape, dtype=input.dtype if scale is None else torch.float8_e4m3fn)
+
+
+def _residual_rms_dynamic_new(input, residual, weight, epsilon):
+    return input.new_empty(input.shape, dtype=torch.float8_e4m3fn), input.new_empty((input.shape[0],), dtype=torch.float32)
+
+
+def _swiglu_new(gate_up, scale=None):
+    return gate_up.new_empty((gate_up.shape[0], gate_up.shape[1] // 2), dtype=torch.float8_e4m3fn)
+
+
+def _swiglu_dynamic_new(gate_up):
+    return _swiglu_new(gate_up), gate_up.new_empty((gate_up.shape[0],), dtype=torch.float32)
+
+
 def _unless_mixed(answer, refusal):
     """A whole-call operator also lands here when one tensor among device tensors is a meta tensor, which the wrapper's look at its first
     argument does not show: that is no call of the operator's, and the general way refuses it."""
@@ -51,7 +68,9 @@ def _unless_mixed(answer, refusal):
 
 
 _OTHER_RESULT = {"fp8_linear": _unless_mixed(_fp8_linear, None), "skinny_gemm_new": _unless_mixed(_skinny_gemm_new, None),
-                 "skinny_gemm_into": _unless_mixed(lambda A, B, scale, D: True, False), "llama_mlp": _unless_mixed(lambda *args, **kwargs: True, False)}
+                 "skinny_gemm_into": _unless_mixed(lambda A, B, scale, D: True, False), "llama_mlp": _unless_mixed(lambda *args, **kwargs: True, False),
+                 "residual_rms_new": _unless_mixed(_residual_rms_new, None), "residual_rms_dynamic_new": _unless_mixed(_residual_rms_dynamic_new, (None, None)),
+                 "swiglu_new": _unless_mixed(_swiglu_new, None), "swiglu_dynamic_new": _unless_mixed(_swiglu_dynamic_new, (None, None))}
 
 
 def register() -> None:

@@ -167,8 +167,12 @@ class Fp8Linear(torch.nn.Module):
 
     def forward(self, input: Tensor, input_scale: Optional[Tensor] = None, residual: Optional[Tensor] = None) -> Tensor:
         """`input` 16-bit (quantised here) or fp8 with `input_scale`; `residual` is added in the GEMM's epilogue."""
-        scale = input_scale if input_scale is not None else self.input_scale
-        return apply_fp8_linear(input, self._operand, self.weight_scale, scale, self.bias, residual)
+        buffers = self._buffers
+        if "weight_scale" in buffers and "input_scale" in buffers and "bias" in buffers:  # by name a module finds each 0.6 us later
+            weight_scale, scale, bias = buffers["weight_scale"], buffers["input_scale"], buffers["bias"]
+        else:  # one was replaced by a parameter
+            weight_scale, scale, bias = self.weight_scale, self.input_scale, self.bias
+        return apply_fp8_linear(input, self._operand, weight_scale, scale if input_scale is None else input_scale, bias, residual)
 
     def extra_repr(self) -> str:
         kind = "packed" if self.packed else "row-major"

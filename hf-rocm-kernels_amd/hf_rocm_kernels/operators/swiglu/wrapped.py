@@ -3,9 +3,12 @@ from typing import Optional, Tuple
 import torch
 from torch import Tensor
 
+from ...utils.dispatch import runs_now
 from .binding import _swiglu
 
 
+_swiglu_new = torch.ops._HFRK_C.swiglu_new.default
+_swiglu_dynamic_new = torch.ops._HFRK_C.swiglu_dynamic_new.default
 MAX_THREADS_PER_SM = 1024
 _IO_DTYPES = (torch.bfloat16, torch.float16)
 
@@ -60,6 +63,10 @@ def swiglu(
     Outputs:
         - a float8_e4m3fn tensor of shape (rows, cols) in row-major format
     """
+    if next_buffer is None and not force_scalar and num_threads == -1 and runs_now(gate_up_proj):
+        output = _swiglu_new(gate_up_proj, scale_tensor)  # the usual call as one native operator; None: not one of those
+        if output is not None:
+            return output
     if next_buffer is None:
         next_buffer = torch.empty(size=(gate_up_proj.size(0), 0), device=gate_up_proj.device, dtype=gate_up_proj.dtype)
     swiglu_checks(gate_up_proj, scale_tensor, next_buffer)
@@ -86,6 +93,10 @@ def swiglu_dynamic(
 ) -> Tuple[Tensor, Tensor]:
     """SwiGLU with per-row dynamic quantisation to float8_e4m3fn (scale = row amax / 448).
     Returns (output fp8 (rows, cols), scales fp32 (rows,)).  cols % 8 == 0 and cols <= 32768."""
+    if next_buffer is None and runs_now(gate_up_proj):
+        output, scales = _swiglu_dynamic_new(gate_up_proj)
+        if output is not None:
+            return output, scales
     if next_buffer is None:
         next_buffer = torch.empty(size=(gate_up_proj.size(0), 0), device=gate_up_proj.device, dtype=gate_up_proj.dtype)
     swiglu_checks(gate_up_proj, torch.empty(1, dtype=torch.float32, device=gate_up_proj.device), next_buffer)

@@ -122,3 +122,51 @@ def test_recorded_and_batched_calls_go_the_general_way(rows):
         torch.jit.trace(layer, x, check_trace=False)
     with pytest.raises(RuntimeError):
         torch.vmap(layer)(x.view(2, rows // 2, 512))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,cols", [(1, 8), (3, 2050), (5, 14648), (130, 4096), (2, 32768), (2, 40960)])
+def test_row_kernels_same_bits_as_the_general_path(rows, cols, dtype, monkeypatch):
+    from hf_rocm_kernels.operators.residual_rms import wrapped as rms
+    from hf_rocm_kernels.operators.swiglu import wrapped as swi
+    gen = torch.Generator(device="cuda").manual_seed(rows + cols)
+    x, res = (torch.randn(rows, cols, generator=gen, device="cuda").to(dtype) for _ in range(2))
+    w = torch.randn(cols, generator=gen, device="cuda").to(dtype)
+    both = torch.randn(rows, 2 * cols, generator=gen, device="cuda").to(dtype)
+    scale = torch.tensor([0.02], device="cuda")
+    calls = [lambda r: rms.residual_rms(x, r, w, 1e-5, scale), lambda r: rms.residual_rms(x, r, w, 1e-5), lambda r: (swi.swiglu(both, scale),)]
+    if cols % 8 == 0 and cols <= 32768:
+        calls += [lambda r: rms.residual_rms_dynamic(x, r, w, 1e-5), lambda r: swi.swiglu_dynamic(both)]
+    for call in calls:
+        native = call(res.clone())
+        with monkeypatch.context() as patch:
+            patch.setattr(rms, "_residual_rms_new", lambda *args: None)
+            patch.setattr(swi, "_swiglu_new", lambda *args: None)
+            patch.setattr(rms, "_residual_rms_dynamic_new", lambda *args: (None, None))
+            patch.setattr(swi, "_swiglu_dynamic_new", lambda *args: (None, None))
+            general = call(res.clone())
+        assert len(native) == len(general)
+        for got, want in zip(native, general):
+            assert got.shape == want.shape and got.dtype == want.dtype and torch.equal(_bits(got), _bits(want))
+
+
+def test_row_kernels_refuse_what_they_refused():
+    from hf_rocm_kernels import residual_rms, residual_rms_dynamic, swiglu, swiglu_dynamic
+    x, w, one = torch.zeros(4, 512, device="cuda", dtype=torch.bfloat16), torch.ones(512, device="cuda", dtype=torch.bfloat16), torch.ones(1, device="cuda")
+    keep = x.clone()
+    for call in (lambda: residual_rms(x, x[:2], w, 1e-5, one), lambda: residual_rms(x, x.clone(), w[:256], 1e-5, one), lambda: residual_rms(x, x.clone().half(), w, 1e-5, one),
+                 lambda: residual_rms(x.t(), x.t().clone(), w[:4], 1e-5, one), lambda: residual_rms(x, x.clone(), w, 0.0, one), lambda: residual_rms(x, x.cpu(), w, 1e-5, one),
+                 lambda: residual_rms(x, x.clone(), w, 1e-5, one.cpu()), lambda: residual_rms(x.float(), x.float(), w, 1e-5, one),
+                 lambda: residual_rms_dynamic(x[:, :508].contiguous(), x[:, :508].contiguous(), w[:508], 1e-5), lambda: swiglu(x[:, :511].contiguous(), one),
+                 lambda: swiglu(x.t(), one), lambda: swiglu(x, torch.ones(2, device="cuda")), lambda: swiglu_dynamic(x[:, :24].contiguous())):
+        with pytest.raises(AssertionError):
+            call()
+    with pytest.raises(RuntimeError):
+        swiglu(x, one.half())
+    assert torch.equal(x, keep)
+    # a tensor that autograd follows goes the general way, which has always taken it
+    weight = w.clone().requires_grad_()
+    got, want = residual_rms(x, x.clone(), weight, 1e-5, one), residual_rms(x, x.clone(), w, 1e-5, one)
+    assert torch.equal(_bits(got[0]), _bits(want[0]))
+    with torch.inference_mode():
+        assert torch.equal(_bits(swiglu(x, one)), _bits(swiglu(x.clone(), one)))
