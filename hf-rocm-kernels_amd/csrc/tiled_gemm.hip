@@ -63,18 +63,18 @@ static float tiled_cost(int m, int n, int k, int shape, int splits) {
 constexpr int kTiledMaxSplits = 8;
 
 // Up to 64 rows: one row of tiles streams the weight.  64 x 64 tiles with k in up to 8 parts of 4 stages or more on at most 512 workgroups, or,
-// where they take a second round, 128 x 64 tiles, two on a compute unit.  In us, the constants fitted to 1500 sizes of 17 to 64 rows, weights from memory
-// and from the 256 MB cache alike (5300 calls; median error 2.6 %, 90 % of them within 8 %).
+// where they take a second round, 128 x 64 tiles, two on a compute unit.  In us, the constants fitted to 1300 sizes of 17 to 64 rows with weights from
+// memory (5300 calls; median error 2.7 %, 90 % of them within 8 %); weights that the 256 MB cache holds are up to 45 % faster.
 static float few_rows_cost(int m, int n, int k, int shape, int splits) {
     struct Shape { float fixed, stage, rows, bytes_per_us, start, overlap; };
-    static constexpr Shape kWide = {4.15f, .221f, .292f, 5.69e6f, .576f, .389f}, kNarrow = {2.45f, .090f, .109f, 9.04e6f, 2.79f, .548f};
+    static constexpr Shape kWide = {3.15f, .334f, .204f, 7.82e6f, 3.97f, .501f}, kNarrow = {2.31f, .0566f, .209f, 8.74e6f, 3.08f, .469f};
     const Shape& c = shape == 3 ? kWide : kNarrow;
     const long wgs = (long)div_up(n, 64) * splits;
     const int rounds = shape == 3 ? 1 : div_up(wgs, kNumCU);
     const float work = rounds * (c.fixed + (float)div_up(k, kTiledStage) / splits * (c.stage + c.rows * (m + 64) / 128.f));
     const float stream = (float)n * k / c.bytes_per_us + c.start;
     float t = fmaxf(work, stream) + c.overlap * fminf(work, stream);
-    if (splits > 1) t += .708f + .344f * splits + 1.579f * wgs / kNumCU;
+    if (splits > 1) t += .552f + .335f * splits + 1.859f * wgs / kNumCU;
     return t;
 }
 
@@ -84,7 +84,7 @@ static float make_few_rows_plan(int m, int n, int k, int max_splits, hfrk_tiled_
     float best = INFINITY;
     auto offer = [&](int shape, int splits) {
         const float t = few_rows_cost(m, n, k, shape, splits);
-        if (t < best) {
+        if (t < .99f * best) {  // of equals the one with the fewest parts
             best = t;
             *plan = {shape, splits, 1};
         }
@@ -118,16 +118,16 @@ static float workgroup_kernel_cost(int m, int n, int k, const hfrk_gemm_plan& p)
 
 // 17 to 64 rows that the skinny GEMM's planner gives to its workgroup kernel.  That kernel was tuned on weights whose rows and k deal out in whole
 // panels and slabs over the compute units; elsewhere the shares of a panel lie with up to twenty workgroups, whose sums one of them collects.  Over 1079
-// such calls (n and k drawn from 1024 to 28672, 40 % of them multiples of 256, 512 or 1024; row-major and packed) the choice below is 23 % faster in
-// the mean: 57 x 2832 x 1792 14.5 -> 6.4 us, 50 x 6176 x 3072 15.5 -> 8.5 from the 256 MB cache and 15.4 -> 11.2 from memory, 57 x 1752 x 14592 19.5 -> 12.0,
-// 64 x 11096 x 5120 21.5 -> 13.7 / 21.8 -> 20.1.  The margins are the fits' errors: whole panels, where nothing is exchanged, and weights above 76 MB, where
-// memory bounds both, are predicted less well.  Above 112 MB at most 2 % could be gained (64 x 8192 x 28672 44 us and 50 on tiles).  What it loses is 7 % at
-// most (40 x 3072 x 8192), 3 % or more on 5 of the 1079.  The row-split and K-split kernels stay: the tiled kernel is 3 to 60 % slower than they are on
-// all but a few of their sizes.
+// such calls (n and k drawn from 1024 to 28672, 40 % of them multiples of 256, 512 or 1024; row-major and packed) the choice below is 19 % faster in
+// the mean with weights from memory and 26 % with weights from the 256 MB cache: 57 x 2832 x 1792 13.3 -> 6.4 us / 14.5 -> 6.4, 50 x 6176 x 3072 15.4 -> 11.2 / 15.5 ->
+// 8.5, 57 x 1752 x 14592 19.5 -> 12.0 from the cache, 64 x 11096 x 5120 21.8 -> 20.1 / 21.5 -> 13.7.  The margins are for the fits' errors: whole panels, where
+// nothing is exchanged, and weights above 76 MB, where memory bounds both, are predicted less well.  Above 112 MB at most 2 % could be gained (64 x 8192 x 28672
+// 44 us, 50 on tiles).  33 of the 1079 lose more than 3 % from one of the two, 7 more than 8 % (57 x 8192 x 8192 from memory 11 %, and from the cache 10 % faster).
+// The row-split and K-split kernels stay: the tiled kernel is 3 to 60 % slower than they are on all but a few of their sizes.
 bool tiled_instead(int m, int n, int k, const hfrk_gemm_plan& skinny, hfrk_tiled_plan* plan) {
     if (m <= 16 || skinny.wn < 1 || (long)n * k > (112L << 20) || !tiled_size_ok(m, n, k)) return false;
     const bool whole_panels = skinny.panels % skinny.grid == 0, large = (long)n * k > (76L << 20);
-    const float margin = (whole_panels ? 1.15f : 1.08f) + (large ? .07f : 0.f);
+    const float margin = (whole_panels ? 1.08f : 1.03f) + (large ? .05f : 0.f);
     return margin * make_few_rows_plan(m, n, k, kTiledMaxSplits, plan) < workgroup_kernel_cost(m, n, k, skinny);
 }
 
