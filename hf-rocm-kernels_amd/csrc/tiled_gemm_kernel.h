@@ -13,11 +13,11 @@
 //    there: 2513 x 11824 x 13312 314 -> 322, 1415 x 6304 x 18944 188 -> 193.  The others have four waves, one per SIMD: 128 x 128 on
 //    eight or sixteen takes the same time.
 //  * Bound (counters in profiles/tiled_gemm_counters_and_plans.txt, shares of the cycles in which a compute unit has work): 4096 x 28672 x
-//    4096 matrix cores 69 %, at the clock their power leaves, LDS 31 % (62 and 19 on four waves); 512 x 4096 x 14336 packed 45 and 35 %;
-//    201 x 6144 x 4096 28 and 23 %.  On the small tiles neither is half busy.
-//    They wait for what a compute unit fetches: without matrix instructions and operand reads a launch takes the same time (201 x 6144 x
-//    4096, 512 x 4096 x 14336), and so it does with 4, 5 or 6 stages in flight.  A unit gets about 75 GB/s, a mixture of the 47 of lines that
-//    are new to its L2 and the 128 - 148 of lines in it: the tile decides how much of each, so it is no limit of the sizes.
+//    4096 matrix cores 68 %, at the clock their power leaves, LDS 30 % (62 and 19 on four waves); 512 x 4096 x 14336 packed 52 and 40 %;
+//    201 x 6144 x 4096 32 and 27 %.
+//    The small tiles wait for what a compute unit fetches, 135 GB/s from its L2 and 58 where a stage waits for lines from memory: loads
+//    alone, without matrix instructions and operand reads, take 7 us of 201 x 6144 x 4096 with everything in L2, 10 from the 256 MB cache and
+//    15.6 from memory, with three stages in flight or six.
 //  * On every tile but the largest four more waves do nothing but load, one per SIMD.  A compute unit takes a load instruction of 1 KB in 16
 //    cycles and holds back the wave whose turn has not come: where the multiplying waves loaded for themselves, a stage took about as long as its
 //    loads and its matrix instructions after one another (201 x 6144 x 4096 with the weight in the 256 MB cache: 11.6 us without matrix instructions
@@ -37,7 +37,7 @@
 //    313 us and took 345: the rest of it is the clock that the matrix cores' power leaves.
 //  * Such a load fills LDS in lane order, so the swizzle that keeps operand reads free of bank conflicts is applied to the memory
 //    side: the lane that fills slot c of row r fetches piece c ^ f(r) of that row (a permutation within one 128-byte line).
-//    Measured conflicts: none on the 256 x 256 tile, 1 - 2 % of the LDS cycles on the smaller ones.  A packed weight is fetched as
+//    Measured conflicts: 3.5 % of the LDS cycles on the 256 x 256 tile, 1 - 2 % on the smaller ones.  A packed weight is fetched as
 //    512-byte runs into the same kind of layout; its operand reads do conflict (128 x 128: a third of the LDS cycles).
 //  * Rows and columns past the edge, and the part of the last stage past k, are outside the buffers' ranges and read as zero.
 //  * Weights are the matrix instruction's A operand with their rows permuted so that a lane's 16 results of a tile are consecutive
@@ -47,9 +47,9 @@
 //  * Few tiles and a long k: k is cut between `splits` workgroups.  Partial tiles are written through to memory, the last arriver
 //    adds them in split order (bit-reproducible), its own from its registers.
 //
-// Measured (us, bf16 out): 4096 x 28672 x 4096 392 - 409 (2.35 - 2.45 PFLOP/s; 1550 as 64 skinny launches; a loop that stays resident clocks at 1.8 - 2.0
-// GHz, so the matrix cores' power bounds it before their issue rate does), 512 x 4096 x 14336 packed 36 (150), 201 x 6144 x 4096
-// 13.4 (46), 65 x 4096 x 4096 10.5, packed 9.9 (16).  The epilogue is written with little code on
+// Measured (us, bf16 out): 4096 x 28672 x 4096 384 - 398 (2.42 - 2.51 PFLOP/s; 1550 as 64 skinny launches; a loop that stays resident clocks at 1.8 - 2.0
+// GHz, so the matrix cores' power bounds it before their issue rate does), 512 x 4096 x 14336 packed 33 (150), 201 x 6144 x 4096
+// 12 (46), 65 x 4096 x 4096 9.1 (16).  The epilogue is written with little code on
 // purpose: with a branch per value for NaN and 64-bit addresses it took 18 us of a 256 x 256 tile, now 7.
 #pragma once
 
