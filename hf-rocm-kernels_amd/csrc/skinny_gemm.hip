@@ -663,7 +663,8 @@ static int choose_plan(int m, int n, int k, bool packed, hfrk_gemm_plan* plan, b
 // use_static: partial sums and counters go to this device's `scratch` array instead of the stream's workspace.
 // base_row: base is one row of n values, added to every row.
 // given: partial sums and counters go to this memory instead of the stream's workspace.
-// needs: raised to what the call takes of a workspace; everything else that can refuse it is checked, and nothing is launched.
+// needs: raised to what the call takes of a workspace, for any alignment of D and base and any b_stride; everything else that can refuse
+// it is checked, and nothing is launched.
 // rms: the activations are not read from A but built by the kernel's RMSNorm prologue from these 16-bit tensors.
 struct RmsPrologue {
     const void* input;
@@ -682,6 +683,7 @@ struct GivenWorkspace {
 struct GemmNeeds {
     size_t ws_bytes;
     long counters;
+    bool taken;  // whether these arguments take any of it
     size_t given_bytes() const { return ws_bytes || counters ? kGivenCounters * sizeof(int) + ws_bytes : 0; }
 };
 static int gemm_launch(const void* A, const void* B, void* D, const void* base, const float* scale_a, int sa_stride,
@@ -739,7 +741,7 @@ static int gemm_launch(const void* A, const void* B, void* D, const void* base, 
     }
     hfrk_gemm_plan p;
     hfrk_tiled_plan tiled{};
-    bool use_tiled = false;
+    bool could_tile = false, use_tiled = false;
     if (user_plan) {
         p = *user_plan;
         const int rc = check_plan(m, swiglu ? n / 2 : n, k, swiglu, &p, packed);
@@ -771,8 +773,8 @@ static int gemm_launch(const void* A, const void* B, void* D, const void* base, 
             bool tuned = false;
             rc = choose_plan(m, n, k, packed, &p, &tuned);
             // a table's entry is run as it stands; rows of D or base that are not 16-byte aligned are the tiled kernel's slow ones
-            use_tiled = rc == HFRK_SUCCESS && !tuned && n % 8 == 0 && ((reinterpret_cast<uintptr_t>(D) | reinterpret_cast<uintptr_t>(base)) & 15) == 0 &&
-                        b_stride <= (1 << 21) && tiled_instead(m, n, k, p, &tiled);
+            could_tile = rc == HFRK_SUCCESS && !tuned && n % 8 == 0 && tiled_instead(m, n, k, p, &tiled);
+            use_tiled = could_tile && ((reinterpret_cast<uintptr_t>(D) | reinterpret_cast<uintptr_t>(base)) & 15) == 0 && b_stride <= (1 << 21);
         }
         if (rc != HFRK_SUCCESS) return rc;
     }
@@ -780,9 +782,18 @@ static int gemm_launch(const void* A, const void* B, void* D, const void* base, 
     size_t need_bytes = use_tiled ? tiled_plan_ws_bytes(tiled, m, n) : plan_ws_bytes(p);
     long need_counters = use_tiled ? tiled_plan_counters(tiled, m, n) : plan_counters(p);
     if (needs) {
-        if (need_bytes > kWsFloats * sizeof(float) || need_counters > kMaxPanels) return HFRK_BAD_SHAPE;
-        needs->ws_bytes = std::max(needs->ws_bytes, need_bytes);
-        needs->counters = std::max(needs->counters, need_counters);
+        auto fits = [](size_t bytes, long count) { return bytes <= kWsFloats * sizeof(float) && count <= kMaxPanels; };
+        auto raise = [&](size_t bytes, long count) {
+            needs->ws_bytes = std::max(needs->ws_bytes, bytes);
+            needs->counters = std::max(needs->counters, count);
+        };
+        if (!fits(need_bytes, need_counters)) return HFRK_BAD_SHAPE;
+        raise(need_bytes, need_counters);
+        needs->taken = needs->taken || need_bytes != 0 || need_counters != 0;
+        if (could_tile) {  // whoever asks for a size may call with tensors that go the other way
+            if (fits(plan_ws_bytes(p), plan_counters(p))) raise(plan_ws_bytes(p), plan_counters(p));
+            raise(tiled_plan_ws_bytes(tiled, m, n), tiled_plan_counters(tiled, m, n));
+        }
         return HFRK_SUCCESS;
     }
     int dev = 0;
@@ -1196,7 +1207,7 @@ int hfrk_llama_mlp_owned(const void* input, const void* residual_in, void* resid
     if (rc != HFRK_SUCCESS) return rc;
     if (workspace) {
         if (needs.given_bytes() > workspace_bytes || needs.counters > kGivenCounters) return HFRK_EXCEEDS_SCRATCH;
-    } else if (needs.given_bytes() != 0) {
+    } else if (needs.taken) {
         int dev = 0;
         Workspace st;
         HFRK_HIP_TRY(hipGetDevice(&dev));

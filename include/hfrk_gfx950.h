@@ -298,10 +298,11 @@ int hfrk_llama_mlp(const void* input, const void* residual_in, void* residual, v
                    void* output, void* scratch, int m, int hidden, int inter, int dtype, int* launched, void* stream);
 
 /* The same on memory of the caller's: partial sums and arrival counters go to `workspace` instead of one that the stream owns, so the call
- * allocates nothing and claims nothing on a stream first met, under a capture neither.  hfrk_llama_mlp_workspace_bytes of it (0: the plans chosen
- * now need none), 16-byte aligned and apart from every tensor, zero before its first call and used by one call at a time; a call leaves its
- * counters zero (hfrk_reset_workspace does not know them).  A call whose plans have come to need more
- * (hfrk_plan_table_set) is refused with HFRK_EXCEEDS_SCRATCH.  workspace NULL: the stream's. */
+ * allocates nothing and claims nothing on a stream first met, under a capture neither.  hfrk_llama_mlp_workspace_bytes of it
+ * (enough for any alignment of the output and any row strides; 0: the plans chosen now need none), 16-byte aligned and apart from every
+ * tensor, zero before its first call and used by one call at a time; a call leaves its counters zero (hfrk_reset_workspace does not know
+ * them).  A call whose plans have come to need more (hfrk_plan_table_set) is refused with HFRK_EXCEEDS_SCRATCH.  workspace NULL: the
+ * stream's. */
 size_t hfrk_llama_mlp_workspace_bytes(int m, int hidden, int inter, int gate_up_packed, int down_packed);
 int hfrk_llama_mlp_owned(const void* input, const void* residual_in, void* residual, void* input_copy, const void* rms_weight, float epsilon,
                          const float* gate_up_input_scale, const void* gate_up, int gate_up_packed, int gate_up_stride, const float* gate_up_output_scale,

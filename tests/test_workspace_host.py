@@ -197,6 +197,26 @@ for m in (1, 8, 16, 17, 32, 33, 64):
 """
 
 
+_CASES["a block's workspace is enough for any alignment and stride"] = """
+size = lambda m, hidden, inter, packed: lib.hfrk_llama_mlp_workspace_bytes(m, hidden, inter, packed, packed)
+own, launched = 1 << 40, ctypes.c_int()
+def aligned_to(m, hidden, inter, packed, need, output, down_stride):
+    place = 1 << 24
+    stand_in.stand_in(0, 1)  # nothing can be allocated, no stream has a workspace
+    return lib.hfrk_llama_mlp_owned(place, 2 * place, 3 * place, None, 4096, 1e-5, 64, 1 << 30, packed, hidden, 64, 64, 1 << 33, packed, down_stride, 64, 1,
+                                    4 * place + output, 5 * place, own, need, m, hidden, inter, _capi.BF16, ctypes.byref(launched), 9)
+for m in (17, 31, 32, 45, 51, 64):
+    for hidden, inter in ((1024, 2560), (2816, 8192), (4096, 13056), (2048, 6656), (256, 256), (512, 14336), (3584, 1024), (8192, 28672)):
+        for packed in (0, 1):
+            need = size(m, hidden, inter, packed)
+            for output in (0, 8):
+                assert aligned_to(m, hidden, inter, packed, need, output, inter) == _capi.SUCCESS, (m, hidden, inter, packed, output)
+            if not packed and hidden <= 512:  # (the weight's last offset is below 2^31)
+                assert aligned_to(m, hidden, inter, packed, need, 0, (1 << 21) + 16) == _capi.SUCCESS, (m, hidden, inter)
+assert lib.hfrk_workspace_id(9) == -1
+"""
+
+
 @pytest.fixture(scope="module")
 def stand_in(tmp_path_factory):
     directory = tmp_path_factory.mktemp("stand_in")
