@@ -779,8 +779,8 @@ static int gemm_launch(const void* A, const void* B, void* D, const void* base, 
         if (rc != HFRK_SUCCESS) return rc;
     }
 
-    size_t need_bytes = use_tiled ? tiled_plan_ws_bytes(tiled, m, n) : plan_ws_bytes(p);
-    long need_counters = use_tiled ? tiled_plan_counters(tiled, m, n) : plan_counters(p);
+    const size_t need_bytes = use_tiled ? tiled_plan_ws_bytes(tiled, m, n) : plan_ws_bytes(p);
+    const long need_counters = use_tiled ? tiled_plan_counters(tiled, m, n) : plan_counters(p);
     if (needs) {
         auto fits = [](size_t bytes, long count) { return bytes <= kWsFloats * sizeof(float) && count <= kMaxPanels; };
         auto raise = [&](size_t bytes, long count) {
@@ -820,12 +820,7 @@ static int gemm_launch(const void* A, const void* B, void* D, const void* base, 
         st.ws = reinterpret_cast<float*>(given->ptr + counters * sizeof(int));
     } else {
         const int rc = workspace_for(dev, stream, &st);
-        if (rc != HFRK_SUCCESS) {
-            if (!use_tiled || plan_ws_bytes(p) != 0 || plan_counters(p) != 0) return rc;
-            use_tiled = false;  // the skinny plan needs no workspace
-            need_bytes = ws_bytes = 0;
-            need_counters = counters = 0;
-        }
+        if (rc != HFRK_SUCCESS) return rc;
     }
     if (need_bytes > ws_bytes || need_counters > counters) return use_static || given ? HFRK_EXCEEDS_SCRATCH : HFRK_BAD_SHAPE;
     if (use_static) {
