@@ -49,8 +49,9 @@ constexpr int tiled_loader_waves(int tm) { return tm < 4 ? 4 : 0; }
 struct TiledShape {
     int bm, bn, stages, per_cu;
     bool halves;
+    int threads;  // per workgroup
 };
-#define HFRK_TILED_ROW(I, TM, TN, WM, WN, NST, WGS) {32 * TM * WM, 32 * TN * WN, NST, WGS, tiled_half_stages(TM, WM * WN)},
+#define HFRK_TILED_ROW(I, TM, TN, WM, WN, NST, WGS) {32 * TM * WM, 32 * TN * WN, NST, WGS, tiled_half_stages(TM, WM * WN), 64 * (WM * WN + tiled_loader_waves(TM))},
 constexpr TiledShape kTiledShapes[] = {HFRK_TILED_SHAPES(HFRK_TILED_ROW)};
 #undef HFRK_TILED_ROW
 #define HFRK_TILED_SAME(I, TM, TN, WM, WN, NST, WGS) \

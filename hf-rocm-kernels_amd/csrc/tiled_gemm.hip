@@ -184,8 +184,22 @@ static void turn_k(TiledGemmArgs* a, int shape) {
 int tiled_launch(const void* A, const void* B, bool packed, void* D, const void* base, int base_stride, const float* scale_a, int sa_stride,
                  const float* scale_b, int sb_stride, int m, int n, int k, int b_stride, int d_dtype, const hfrk_tiled_plan& p, float* ws, size_t ws_bytes,
                  int* counters, hipStream_t stream) {
-    TiledGemmArgs args{};
     const TiledShape& s = kTiledShapes[p.shape];
+    const int row_tiles = div_up(m, s.bm);
+    if ((uint64_t)row_tiles * div_up(n, s.bn) * p.splits * s.threads >> 32) {
+        // A launch holds fewer than 2^32 threads: 2^23 tiles or more that a plan cuts 64 columns wide go as two launches (or, halved once more,
+        // up to four), each of half the rows of tiles.  k is not split then, as the partial sums of so many tiles fit no workspace.
+        const int half = row_tiles / 2, rows = half * s.bm;
+        auto part = [&](int row, int count) {
+            const hfrk_tiled_plan q{p.shape, p.splits, p.group_m < half ? p.group_m : half};
+            return tiled_launch(static_cast<const uint8_t*>(A) + (size_t)row * k, B, packed, static_cast<uint8_t*>(D) + (size_t)row * n * 2,
+                                base ? static_cast<const uint8_t*>(base) + (size_t)row * base_stride * 2 : base, base_stride, scale_a + (size_t)row * sa_stride,
+                                sa_stride, scale_b, sb_stride, count, n, k, b_stride, d_dtype, q, ws, ws_bytes, counters, stream);
+        };
+        const int rc = part(0, rows);
+        return rc == HFRK_SUCCESS ? part(rows, m - rows) : rc;
+    }
+    TiledGemmArgs args{};
     args.A = static_cast<const uint8_t*>(A);
     args.B = static_cast<const uint8_t*>(B);
     args.D = D;
@@ -201,7 +215,7 @@ int tiled_launch(const void* A, const void* B, bool packed, void* D, const void*
     args.b_stride = b_stride;
     args.d_dtype = d_dtype;
     args.vec = n % 8 == 0 && args.base_stride % 8 == 0 && ((reinterpret_cast<uintptr_t>(D) | reinterpret_cast<uintptr_t>(base)) & 15) == 0;
-    args.tiles_m = div_up(m, s.bm);
+    args.tiles_m = row_tiles;
     args.tiles_n = div_up(n, s.bn);
     args.group_m = p.group_m;
     const int stages = div_up(k, kTiledStage);

@@ -1,7 +1,8 @@
-"""What a launch does when the split-K workspace is not to be had, on the CPU: the library runs over a stand-in for the HIP runtime that
-hands out a given number of allocations, can claim that a stream is capturing, keeps the last error as the runtime does, and notes the
-grid of every launch instead of running it."""
+"""What a call launches, and what it does when the split-K workspace is not to be had, on the CPU: the library runs over a stand-in for the
+HIP runtime that hands out a given number of allocations, can claim that a stream is capturing, keeps the last error as the runtime does,
+and notes the kernel, grid and (the tiled GEMM's) arguments of every launch instead of running it."""
 import os
+import re
 import subprocess
 import sys
 
@@ -11,12 +12,22 @@ _STAND_IN = r"""
 #include <stddef.h>
 #include <stdint.h>
 typedef struct { uint32_t x, y, z; } dim3_;
+%s  /* struct TiledGemmArgs */
+static struct TiledGemmArgs tiled_args[4];
+static int keep_args;                // the launches to come are the tiled GEMM's
+static const void* kernel;
+static uint64_t groups, most_threads;  // workgroups of all launches, threads of the largest
+void stand_in_keep_args(int on) { keep_args = on; }
+const struct TiledGemmArgs* stand_in_args(int launch) { return tiled_args + launch; }
+const void* stand_in_kernel(void) { return kernel; }
+uint64_t stand_in_groups(void) { return groups; }
+uint64_t stand_in_most_threads(void) { return most_threads; }
 static int allocations, capturing, last_error;
 static int clearing, early;          // memory is being cleared by work that nobody has waited for; a launch met it so
 static char own_stream;
 static uint32_t grid, threads, launches;
 static uintptr_t next_block = 1 << 20;
-void stand_in(int allocs, int capture) { allocations = allocs; capturing = capture; grid = launches = 0; }
+void stand_in(int allocs, int capture) { allocations = allocs; capturing = capture; grid = launches = 0; kernel = 0; groups = most_threads = 0; }
 uint32_t stand_in_launches(void) { return launches; }
 uint32_t stand_in_grid(void) { return grid; }
 uint32_t stand_in_threads(void) { return threads; }
@@ -39,6 +50,10 @@ int __hipPopCallConfiguration(dim3_* grid_, dim3_* block_, size_t* lds, void** s
 int hipLaunchKernel(const void* f, dim3_ grid_, dim3_ block_, void** args, size_t lds, void* stream) {
     grid = grid_.x;
     threads = block_.x;
+    kernel = f;
+    groups += grid;
+    if ((uint64_t)grid * threads > most_threads) most_threads = (uint64_t)grid * threads;
+    if (keep_args && launches < 4) tiled_args[launches] = *(struct TiledGemmArgs*)args[0];
     ++launches;
     if (stream == &own_stream) clearing = 1;
     else if (clearing) early = 1;
@@ -52,6 +67,13 @@ import ctypes, sys
 sys.path.insert(0, {package!r})
 import _capi
 lib, stand_in = _capi.load(), ctypes.CDLL({stand_in!r})
+for name in ("kernel", "groups", "most_threads"):
+    getattr(stand_in, "stand_in_" + name).restype = ctypes.c_uint64
+
+class TiledArgs(ctypes.Structure):
+    _fields_ = {fields!r}
+    _fields_ = [(name, getattr(ctypes, kind)) for name, kind in _fields_]
+stand_in.stand_in_args.restype = ctypes.POINTER(TiledArgs)
 m, n, k = 65, 64, 4096
 
 def tiled(stream, plan=None):
@@ -217,12 +239,50 @@ assert lib.hfrk_workspace_id(9) == -1
 """
 
 
+_CASES["more tiles than one launch holds threads"] = """
+def run(m, n, k, shape, group=1, base_stride=0, sa_stride=0):
+    stand_in.stand_in(0, 0)
+    plan = ctypes.byref(_capi.TiledPlan(shape, 1, group))
+    status = lib.hfrk_tiled_gemm(1 << 40, 8192, 0, 1 << 50, 1 << 45 if base_stride is not None else None, base_stride or 0, 1 << 42, sa_stride, None, 0,
+                                 m, n, k, k, _capi.BF16, plan, 1)
+    return status, stand_in.stand_in_launches(), stand_in.stand_in_groups(), stand_in.stand_in_most_threads()
+
+stand_in.stand_in_keep_args(1)
+for m, n, k, shape, bm, bn in ((1 << 24, 2112, 16, 4, 64, 64), (1 << 24, 4032, 32, 4, 64, 64), ((1 << 24) - 5, 64 * 63 - 7, 16, 4, 64, 64),
+                               ((1 << 24) - 191, 4095 * 64 // 65, 16, 3, 128, 64), (1 << 24, 2048, 16, 0, 256, 256)):
+    for group in (1, 3, -(-m // bm)):
+        for base_stride, sa_stride in ((None, 0), (0, 1), (n, 1), (n + 8, 0)):
+            status, launches, groups, threads = run(m, n, k, shape, group, base_stride, sa_stride)
+            assert status == _capi.SUCCESS and threads < 1 << 32 and groups == -(-m // bm) * -(-n // bn), (m, n, shape, launches, groups, threads)
+            row = 0
+            for i in range(launches):
+                a = stand_in.stand_in_args(i).contents
+                assert a.A == (1 << 40) + row * k and a.D == (1 << 50) + row * n * 2 and a.scale_a == (1 << 42) + 4 * row * sa_stride
+                assert a.base == (None if base_stride is None else (1 << 45) + row * base_stride * 2) and a.B == 8192
+                assert row % bm == 0 and 1 <= a.group_m <= a.tiles_m == -(-a.m // bm) and a.tiles_n == -(-n // bn)
+                row += a.m
+            assert row == m and launches <= 2
+"""
+
+
+_STRUCT = re.search(r"struct TiledGemmArgs \{.*?\n\};", open(os.path.join(os.path.dirname(__file__), "..", "hf-rocm-kernels_amd", "csrc", "tiled_gemm.h")).read(),
+                    re.S).group(0)
+
+
+def _fields():
+    out = []
+    for kind, names in re.findall(r"^    (?:const )?(\w+\*?) ([^;]+);", _STRUCT, re.M):
+        ctype = "c_void_p" if kind.endswith("*") else {"int": "c_int", "uint32_t": "c_uint32"}[kind]
+        out += [(name.strip(), ctype) for name in names.split(",")]
+    return out
+
+
 @pytest.fixture(scope="module")
 def stand_in(tmp_path_factory):
     directory = tmp_path_factory.mktemp("stand_in")
     source, library = os.path.join(directory, "stand_in.c"), os.path.join(directory, "libstand_in.so")
     with open(source, "w") as f:
-        f.write(_STAND_IN)
+        f.write(_STAND_IN % _STRUCT)
     subprocess.run(["gcc", "-O1", "-shared", "-fPIC", source, "-o", library], check=True)
     return library
 
@@ -231,5 +291,5 @@ def stand_in(tmp_path_factory):
 def test_launches_without_a_workspace(case, stand_in):
     from hf_rocm_kernels import _capi
     preload = ":".join(p for p in (stand_in, os.environ.get("LD_PRELOAD")) if p)
-    code = _PRELUDE.format(package=os.path.dirname(_capi.__file__), stand_in=stand_in) + _CASES[case]
+    code = _PRELUDE.format(package=os.path.dirname(_capi.__file__), stand_in=stand_in, fields=_fields()) + _CASES[case]
     subprocess.run([sys.executable, "-c", code], check=True, timeout=100, env=dict(os.environ, LD_PRELOAD=preload))
