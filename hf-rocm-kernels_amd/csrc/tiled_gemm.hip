@@ -177,7 +177,7 @@ static void turn_k(TiledGemmArgs* a, int shape) {
     columns = columns < a->tiles_n ? columns : a->tiles_n;
     a->phase_m = 65536 / a->group_m;
     a->phase_n = 65536 / columns;
-    a->window = shape == 4 ? 1 : 700 * 1024 / ((a->group_m * s.bm + columns * s.bn) * kTiledStage);
+    a->window = shape == 4 ? 1 : (int)(700 * 1024 / (((long)a->group_m * s.bm + (long)columns * s.bn) * kTiledStage));
     a->window = a->window < 1 ? 1 : a->window;
 }
 
