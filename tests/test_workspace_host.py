@@ -265,6 +265,47 @@ for m, n, k, shape, bm, bn in ((1 << 24, 2112, 16, 4, 64, 64), (1 << 24, 4032, 3
 """
 
 
+_CASES["which kernel takes 17 to 64 rows"] = """
+tiles = [(256, 256), (256, 128), (128, 128), (128, 64), (64, 64)]
+tiled_kernels = {}
+for shape in range(5):
+    for packed in (0, 1):
+        stand_in.stand_in(100, 0)
+        assert lib.hfrk_tiled_gemm(4096, 8192, packed, 16384, None, 0, 64, 1, 64, 1, 64, 1024, 1024, 1024, 1, ctypes.byref(_capi.TiledPlan(shape, 1, 1)), 1) == 0
+        tiled_kernels[stand_in.stand_in_kernel()] = shape
+assert len(tiled_kernels) == 10
+
+def on_tiles(m, n, k, packed=0, output=16384, call=lib.hfrk_linear_gemm):
+    # whether a call runs on tiles; if so, its grid is the plan's
+    stand_in.stand_in(100, 0)
+    assert call(4096, 8192, packed, output, None, 0, 64, 1, 64, 1, m, n, k, k, 1, 1) == _capi.SUCCESS
+    plan = _capi.TiledPlan()
+    assert lib.hfrk_tiled_gemm_plan(m, n, k, ctypes.byref(plan)) == _capi.SUCCESS
+    if stand_in.stand_in_kernel() not in tiled_kernels:
+        return False
+    assert tiled_kernels[stand_in.stand_in_kernel()] == plan.shape and stand_in.stand_in_launches() == 1
+    rows, columns = tiles[plan.shape]
+    assert stand_in.stand_in_grid() == -(-m // rows) * -(-n // columns) * plan.splits
+    return True
+
+skinny_plan = _capi.GemmPlan()
+for packed in (0, 1):
+    for m, n, k in ((17, 1112, 6912), (64, 3800, 1792), (33, 2136, 15104), (44, 17152, 1792), (64, 1040, 2560), (37, 4608, 3584), (50, 6176, 3072)):
+        assert on_tiles(m, n, k, packed) and not on_tiles(m, n, k, packed, output=16392)  # rows of the output that are not 16-byte aligned stay
+        assert lib.hfrk_plan_table_get(m, n, k, packed, ctypes.byref(skinny_plan)) == _capi.SUCCESS
+        assert stand_in.stand_in_grid() == skinny_plan.grid
+    # weights above 112 MB; fewer rows than 17; a third round of tiles; k of a slab or two
+    for m, n, k in ((64, 8192, 28672), (64, 28672, 8192), (17, 1024, 4096), (16, 1112, 6912), (34, 45008, 256), (37, 45056, 768), (34, 33000, 1280), (32, 42896, 256),
+                    (24, 48384, 256), (22, 16792, 512), (30, 608, 1024), (21, 296, 1024), (24, 22192, 1024), (33, 1296, 256)):
+        assert not on_tiles(m, n, k, packed), (m, n, k, packed)
+    assert on_tiles(60, 32016, 1024, packed) and on_tiles(33, 1296, 1024, packed) and on_tiles(32, 3296, 768, packed) and on_tiles(40, 20000, 512, packed)
+# a table's entry is run as it stands
+m, n, k = 64, 3800, 1792
+assert lib.hfrk_plan_table_get(m, n, k, 0, ctypes.byref(skinny_plan)) == lib.hfrk_plan_table_set(m, n, k, 0, ctypes.byref(skinny_plan)) == _capi.SUCCESS
+assert not on_tiles(m, n, k) and stand_in.stand_in_grid() == skinny_plan.grid and on_tiles(m, n, k, 1)
+"""
+
+
 _CASES["where a launch's workgroups start in k"] = """
 tiles = [(256, 256, 1), (256, 128, 1), (128, 128, 1), (128, 64, 2), (64, 64, 1)]  # rows, columns, workgroups per compute unit
 stand_in.stand_in_keep_args(1)
