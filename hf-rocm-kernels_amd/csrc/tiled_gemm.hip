@@ -79,9 +79,18 @@ static float few_rows_cost(int m, int n, int k, int shape, int splits) {
     return t;
 }
 
+// The fit's sizes have k in whole stages.  Rows of another k begin inside a 128-byte line, and from memory the fit then takes too few parts of it: up
+// to four of 8 stages or more are kept where a compute unit each has room for them (62 x 8096 x 3088 in two parts 13.3 us, in one 16.6; 55 x 3920 x 6416 in four
+// 13.9, in three 15.3; of 814 drawn sizes of 33 to 64 rows 30 had fewer, 7 % slower from memory and 12 % faster from the cache).  Below 13 stages it
+// takes two or three for nothing (54 x 192 x 1344 6.14 us in one, 6.64 in two; 17 sizes, 4 % slower from the cache, 1 % faster from memory).
 static float make_few_rows_plan(int m, int n, int k, int max_splits, hfrk_tiled_plan* plan) {
     const int stages = div_up(k, kTiledStage);
     const long tiles = div_up(n, 64);
+    int least = 1;
+    if (k % 256 != 0) {
+        for (least = 4; least > 1 && (least > max_splits || least * tiles > kNumCU || least * 8 > stages);) --least;
+        if (stages < 13) max_splits = 1;
+    }
     float best = INFINITY;
     auto offer = [&](int shape, int splits) {
         const float t = few_rows_cost(m, n, k, shape, splits);
@@ -90,9 +99,9 @@ static float make_few_rows_plan(int m, int n, int k, int max_splits, hfrk_tiled_
             *plan = {shape, splits, 1};
         }
     };
-    offer(4, 1);
+    if (least == 1) offer(4, 1);
     if (tiles > kNumCU && tiles <= 2 * kNumCU) offer(3, 1);
-    for (int splits = 2; splits <= max_splits && 4 * splits <= stages && tiles * splits <= 2 * kNumCU; ++splits) offer(4, splits);
+    for (int splits = least < 2 ? 2 : least; splits <= max_splits && 4 * splits <= stages && tiles * splits <= 2 * kNumCU; ++splits) offer(4, splits);
     return best;
 }
 

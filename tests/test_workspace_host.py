@@ -306,6 +306,24 @@ assert not on_tiles(m, n, k) and stand_in.stand_in_grid() == skinny_plan.grid an
 """
 
 
+_CASES["parts of a k that ends inside a 256-byte chunk, few rows"] = """
+parts = _capi.TiledPlan()
+for m in (17, 33, 49, 64):
+    for n in (8, 192, 1000, 2288, 3920, 5352, 7792, 8096, 8200, 16384, 16400, 32768, 40000):
+        tiles = -(-n // 64)
+        for k in (16, 272, 1008, 1328, 1520, 1552, 2032, 3088, 3376, 4448, 6416, 12400, 28656):
+            assert lib.hfrk_tiled_gemm_plan(m, n, k, ctypes.byref(parts)) == _capi.SUCCESS
+            stages = -(-k // 128)
+            least = max(min(256 // tiles, stages // 8, 4), 1)
+            assert least <= parts.splits <= (8 if stages > 12 else 1) and (parts.splits == 1 or parts.splits * 4 <= stages), (m, n, k, parts.splits)
+            assert parts.shape == 4 or (parts.shape == 3 and parts.splits == 1 and 256 < tiles <= 512)
+    assert lib.hfrk_tiled_gemm_plan(m, 1000, 28672, ctypes.byref(parts)) == _capi.SUCCESS and parts.splits > 4
+stand_in.stand_in(0, 0)  # no workspace: k in one part
+assert lib.hfrk_linear_gemm(4096, 8192, 0, 16384, None, 0, 64, 1, 64, 1, 64, 1000, 28656, 28656, 1, 1) == _capi.SUCCESS
+assert stand_in.stand_in_grid() == 16
+"""
+
+
 _CASES["where a launch's workgroups start in k"] = """
 tiles = [(256, 256, 1), (256, 128, 1), (128, 128, 1), (128, 64, 2), (64, 64, 1)]  # rows, columns, workgroups per compute unit
 stand_in.stand_in_keep_args(1)
