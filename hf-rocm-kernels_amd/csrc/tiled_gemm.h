@@ -41,6 +41,13 @@ constexpr int kTiledStage = 128;    // bytes of k per pipeline stage
 // Shape 1 on four waves, for row-major operands whose rows begin inside a 128-byte line and a long k (tiled_gemm_rowmajor.hip).
 #define HFRK_TILED_FOUR_WAVES(X) X(1, 4, 2, 2, 2, 3, 1)
 
+// The shapes whose multiplying waves load for themselves where a workgroup's k is one or two stages.  Waves that only load have nothing to run ahead
+// of there, and starting them costs: over 285 sizes of one stage and 274 of two on 128 x 64 tiles 3.5 and 1.7 % (165 x 9040 x 512 packed 6.9 us without, 7.7
+// with them), on eight of the 256 x 128 tile 3 %; from three stages on the two are level, from eight on they win.
+#define HFRK_TILED_SHORT_K(X) \
+    X(1, 2, 2, 4, 2, 3, 1)    \
+    X(3, 2, 1, 2, 2, 3, 2)
+
 // Whether LDS holds halves of stages (the 256 x 256 tile: five halves, 160 KB; two whole stages are 128).
 constexpr bool tiled_half_stages(int tm, int waves) { return tm * waves >= 32; }
 // Waves of a workgroup that only load, beside the WM x WN that multiply (tiled_gemm_kernel.h).
@@ -49,7 +56,7 @@ constexpr int tiled_loader_waves(int tm) { return tm < 4 ? 4 : 0; }
 struct TiledShape {
     int bm, bn, stages, per_cu;
     bool halves;
-    int threads;  // per workgroup
+    int threads;  // per workgroup, at most
 };
 #define HFRK_TILED_ROW(I, TM, TN, WM, WN, NST, WGS) {32 * TM * WM, 32 * TN * WN, NST, WGS, tiled_half_stages(TM, WM * WN), 64 * (WM * WN + tiled_loader_waves(TM))},
 constexpr TiledShape kTiledShapes[] = {HFRK_TILED_SHAPES(HFRK_TILED_ROW)};
@@ -57,6 +64,7 @@ constexpr TiledShape kTiledShapes[] = {HFRK_TILED_SHAPES(HFRK_TILED_ROW)};
 #define HFRK_TILED_SAME(I, TM, TN, WM, WN, NST, WGS) \
     static_assert(kTiledShapes[I].bm == 32 * TM * WM && kTiledShapes[I].bn == 32 * TN * WN && kTiledShapes[I].stages == NST && kTiledShapes[I].per_cu == WGS);
 HFRK_TILED_FOUR_WAVES(HFRK_TILED_SAME)
+HFRK_TILED_SHORT_K(HFRK_TILED_SAME)
 #undef HFRK_TILED_SAME
 constexpr int kTiledShapeCount = sizeof(kTiledShapes) / sizeof(kTiledShapes[0]);
 constexpr int tiled_lds_bytes(const TiledShape& s) { return (s.bm + s.bn) * (s.halves ? kTiledStage / 2 : kTiledStage) * s.stages; }

@@ -89,9 +89,10 @@ __device__ __forceinline__ uint32_t pack_pair(float lo, float hi) {
     else return __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{lo, hi}, v2h));
 }
 
-template <int TM, int TN, int WM, int WN, int NST, int WGS, bool PACKED>
-__global__ void __launch_bounds__(64 * (WM * WN + tiled_loader_waves(TM)), WGS * (WM * WN + tiled_loader_waves(TM)) / 4) tiled_gemm_kernel(const TiledGemmArgs a) {
-    constexpr int NW = WM * WN, LW = tiled_loader_waves(TM), NL = LW ? LW : NW;  // waves that multiply, that only load, that load
+// LW: waves that only load.
+template <int TM, int TN, int WM, int WN, int NST, int WGS, bool PACKED, int LW>
+__global__ void __launch_bounds__(64 * (WM * WN + LW), WGS * (WM * WN + LW) / 4) tiled_gemm_kernel(const TiledGemmArgs a) {
+    constexpr int NW = WM * WN, NL = LW ? LW : NW;  // waves that multiply, that load
     constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN;
     constexpr int KB = kTiledStage;
     constexpr int A_BYTES = BM * KB, B_BYTES = BN * KB, STAGE = A_BYTES + B_BYTES;
@@ -484,9 +485,9 @@ __global__ void __launch_bounds__(64 * (WM * WN + tiled_loader_waves(TM)), WGS *
     else write_back(std::integral_constant<int, HFRK_F16>{});
 }
 
-template <int TM, int TN, int WM, int WN, int NST, int WGS, bool PACKED>
+template <int TM, int TN, int WM, int WN, int NST, int WGS, bool PACKED, int LW = tiled_loader_waves(TM)>
 static int launch_tiled_shape(const TiledGemmArgs& args, int lds_bytes, hipStream_t stream) {
-    auto kern = tiled_gemm_kernel<TM, TN, WM, WN, NST, WGS, PACKED>;
+    auto kern = tiled_gemm_kernel<TM, TN, WM, WN, NST, WGS, PACKED, LW>;
     static bool attr_done[kMaxDevices] = {};
     int dev = 0;
     HFRK_HIP_TRY(hipGetDevice(&dev));
@@ -494,13 +495,21 @@ static int launch_tiled_shape(const TiledGemmArgs& args, int lds_bytes, hipStrea
         HFRK_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes));
         if (dev >= 0 && dev < kMaxDevices) attr_done[dev] = true;
     }
-    hipLaunchKernelGGL(kern, dim3(args.tiles_m * args.tiles_n * args.splits), dim3(64 * (WM * WN + tiled_loader_waves(TM))), lds_bytes, stream, args);
+    hipLaunchKernelGGL(kern, dim3(args.tiles_m * args.tiles_n * args.splits), dim3(64 * (WM * WN + LW)), lds_bytes, stream, args);
     HFRK_HIP_TRY(hipGetLastError());
     return HFRK_SUCCESS;
 }
 
 template <bool PACKED>
 static int launch_tiled(const TiledGemmArgs& args, int shape, hipStream_t stream) {
+    if (args.stages_q + (args.stages_r ? 1 : 0) <= 2) {
+        switch (shape) {
+#define HFRK_TILED_CASE(I, TM, TN, WM, WN, NST, WGS) \
+    case I: return launch_tiled_shape<TM, TN, WM, WN, NST, WGS, PACKED, 0>(args, tiled_lds_bytes(kTiledShapes[I]), stream);
+            HFRK_TILED_SHORT_K(HFRK_TILED_CASE)
+#undef HFRK_TILED_CASE
+        }
+    }
     switch (shape) {
 #define HFRK_TILED_CASE(I, TM, TN, WM, WN, NST, WGS) \
     case I: return launch_tiled_shape<TM, TN, WM, WN, NST, WGS, PACKED>(args, tiled_lds_bytes(kTiledShapes[I]), stream);

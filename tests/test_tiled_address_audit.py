@@ -15,14 +15,16 @@ from test_address_audit import MAX_PANELS, U32, WS_BYTES
 
 
 def _built():
-    """Shape index -> the kernels built for it as (TM, TN, WM, WN, stages in LDS), from the header that instantiates them."""
+    """Shape index -> the kernels built for it as (TM, TN, WM, WN, stages in LDS, waves that load), from the header that instantiates them."""
     header = os.path.join(os.path.dirname(_capi.LIB_PATH), os.pardir, "csrc", "tiled_gemm.h")
     with open(header) as f:
-        rows = re.findall(r"X\((\d), (\d), (\d), (\d), (\d), (\d), \d\)", f.read())
+        lists = re.findall(r"#define HFRK_TILED_(\w+)\(X\)((?:.*\\\n)*.*)", f.read())
     built = {}
-    for index, *shape in rows:
-        built.setdefault(int(index), []).append(tuple(map(int, shape)))
-    assert sorted(built) == list(range(5)) and [len(built[i]) for i in range(5)] == [1, 2, 1, 1, 1]
+    for name, rows in lists:
+        for row in re.findall(r"X\((\d), (\d), (\d), (\d), (\d), (\d), \d\)", rows):
+            index, TM, TN, WM, WN, NST = map(int, row)
+            built.setdefault(index, []).append((TM, TN, WM, WN, NST, 4 if TM < 4 and name != "SHORT_K" else WM * WN))
+    assert sorted(built) == list(range(5)) and [len(built[i]) for i in range(5)] == [1, 3, 1, 2, 1]
     return built
 
 
@@ -31,18 +33,13 @@ KERNELS = [(shape, kernel) for shape in sorted(BUILT) for kernel in BUILT[shape]
 KB, OUTSIDE = 128, 0x7FFFFFF0
 
 
-def _loading_waves(TM, NW):
-    return 4 if TM < 4 else NW
-
-
 def _half_stages(TM, NW):
     return TM * NW >= 32
 
 
-def _pieces(rows, TM, NW):
+def _pieces(rows, TM, NW, NL):
     """(load, wave, lane) -> row, its 16-byte piece of the stage for A and for a row-major B before the swizzle is undone, and the block of a
     packed B that a load of a stage of `rows` rows fetches."""
-    NL = _loading_waves(TM, NW)
     q, wave = np.arange(rows * KB // (1024 * NL))[:, None, None], np.arange(NL)[None, :, None]
     if _half_stages(TM, NW):
         row = ((q >> 1) * NL + wave) * 16 + (LANE >> 2)
@@ -73,7 +70,7 @@ def audit(m, n, k, b_stride, plan, packed, base_stride, sa_stride=1):
 
 
 def _audit(kernel, m, n, k, b_stride, plan, packed, base_stride, sa_stride):
-    TM, TN, WM, WN, NST = kernel
+    TM, TN, WM, WN, NST, NL = kernel
     NW, BM, BN = WM * WN, 32 * TM * WM, 32 * TN * WN
     tiles_m, tiles_n = -(-m // BM), -(-n // BN)
     tiles, stages = tiles_m * tiles_n, -(-k // KB)
@@ -103,7 +100,7 @@ def _audit(kernel, m, n, k, b_stride, plan, packed, base_stride, sa_stride):
     k_tail, tail_stage = k % KB, k // KB if k % KB else -1
     for tm in _edge(tiles_m):
         m0, rows_a = tm * BM, min(BM, m - tm * BM)
-        row, pa, _, _ = _pieces(BM, TM, NW)
+        row, pa, _, _ = _pieces(BM, TM, NW, NL)
         pa = pa * 16
         assert len(np.unique(row * 8 + (pa >> 4))) == BM * 8           # every 16-byte piece of the stage is fetched once
         for s in {0, stages - 1, *(b - 1 for b in begins[1:]), *begins[:-1]}:
@@ -118,7 +115,7 @@ def _audit(kernel, m, n, k, b_stride, plan, packed, base_stride, sa_stride):
     for tn in _edge(tiles_n):
         n0 = tn * BN
         for s in {0, stages - 1, *(b - 1 for b in begins[1:]), *begins[:-1]}:
-            row, _, pb, block = _pieces(BN, TM, NW)
+            row, _, pb, block = _pieces(BN, TM, NW, NL)
             pb = pb * 16
             if packed:
                 tiles16 = min(BN // 16, (n + 15) // 16 - n0 // 16)
@@ -237,20 +234,19 @@ def test_largest_sizes(m, n, k):
 @pytest.mark.parametrize("shape,kernel", KERNELS)
 def test_every_wave_has_its_part_of_the_tile(shape, kernel):
     """The parts that the waves of a workgroup load, multiply, leave as partial sums and store are the whole tile, each once."""
-    TM, TN, WM, WN, NST = kernel
+    TM, TN, WM, WN, NST, NL = kernel
     NW, BM, BN = WM * WN, 32 * TM * WM, 32 * TN * WN
     assert (BM, BN) == [(256, 256), (256, 128), (128, 128), (128, 64), (64, 64)][shape]
     halves = _half_stages(TM, NW)
     stage = (BM + BN) * KB
     ring = stage * NST // 2 if halves else stage * NST
     assert ring <= 160 * 1024 and NW % 4 == 0
-    NL = _loading_waves(TM, NW)
     loads = 0
     for rows in (BM, BN):  # A and row-major B: 8 rows of 8 pieces a load, or 16 rows of 4; packed B: half a 16-row tile's stage
         per_wave = rows * KB // (1024 * NL)
         assert per_wave * 1024 * NL == rows * KB and (not halves or per_wave % 2 == 0)
         loads += per_wave
-        row, *pieces, block = _pieces(rows, TM, NW)
+        row, *pieces, block = _pieces(rows, TM, NW, NL)
         assert (np.sort(block.ravel()) == np.arange(rows // 8)).all()            # KB of LDS it fills
         for piece in pieces:
             assert len(np.unique(row * 8 + piece)) == rows * 8

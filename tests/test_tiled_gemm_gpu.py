@@ -31,7 +31,9 @@ SIZES = [(1, 64, 256, 1), (64, 256, 128, 1), (257, 264, 1280, 3), (130, 203, 512
          # workgroups), and next to it
          (144, 136, 5520, 1), (143, 136, 5520, 1), (144, 136, 5488, 1), (400, 200, 11280, 2), (512, 264, 5520, 1), (512, 264, 2064, 4),
          # several rows and columns of tiles, each with a start in k of its own, over several windows, the last of them shorter
-         (600, 520, 5008, 2)]
+         (600, 520, 5008, 2),
+         # two stages a workgroup, the last one cut short
+         (600, 520, 400, 2)]
 
 
 @pytest.mark.parametrize("add", ["none", "bias", "residual"])

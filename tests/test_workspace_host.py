@@ -150,23 +150,31 @@ def waves(m, n, k, stride=None, packed=0, splits=1, shape=1):
     stand_in.stand_in(100, 0)
     plan = ctypes.byref(_capi.TiledPlan(shape, splits, 1))
     assert lib.hfrk_tiled_gemm(4096, 8192, packed, 16384, None, 0, 64, 0, None, 0, m, n, k, stride or k, _capi.BF16, plan, 1) == _capi.SUCCESS
-    total = stand_in.stand_in_threads() // 64
-    return total - (4 if shape and total != 4 else 0)  # four more only load, but on 256 x 256 and on the 256 x 128 tile of four
+    return stand_in.stand_in_threads() // 64  # four of twelve only load, and four of the smaller tiles' eight
 
 for m in (65, 143, 144, 256, 300, 400, 512, 784, 1040, 1536, 4096):
     for n in (8, 4104, 10240, 28672):
         few = -(-m // 256) * -(-n // 128) <= 384
-        eight = m % 256 in range(1, 144) and (m <= 1024 or few)  # a last row of tiles about half full or less, one of four or of few workgroups
-        for k in (128, 4096, 8320):
-            assert waves(m, n, k) == waves(m, n, k, k + 256) == 8
-            assert waves(m, n, k, k + 16) == waves(m, n, k, k + 64) == (8 if eight or k < 8320 else 4)
+        twelve = m % 256 in range(1, 144) and (m <= 1024 or few)  # a last row of tiles about half full or less, one of four or of few workgroups
+        for k in (384, 4096, 8320):
+            assert waves(m, n, k) == waves(m, n, k, k + 256) == 12
+            assert waves(m, n, k, k + 16) == waves(m, n, k, k + 64) == (12 if twelve or k < 8320 else 4)
         for k in (5520, 8256):  # 44 stages or more
-            assert waves(m, n, k) == waves(m, n, k, k + 112) == waves(m, n, k, -(-k // 128) * 128) == (8 if eight else 4), (m, n, k)
-        assert waves(m, n, 16) == waves(m, n, 4112) == waves(m, n, 5488) == 8
-        assert waves(m, n, 8192, packed=1) == 8
-        assert waves(m, n, 8208, shape=0) == 8 and all(waves(m, n, 8208, shape=s) == 4 for s in (2, 3, 4))
-assert waves(1040, 5000, 16400) == 8 and waves(1040, 5000, 16400, splits=2) == 4  # 200 workgroups, 400
-assert waves(512, 4104, 16400, splits=2) == 4 and waves(512, 4104, 28656, splits=3) == 8 and waves(512, 4104, 8208, splits=2) == 8
+            assert waves(m, n, k) == waves(m, n, k, k + 112) == waves(m, n, k, -(-k // 128) * 128) == (12 if twelve else 4), (m, n, k)
+        assert waves(m, n, 272) == waves(m, n, 4112) == waves(m, n, 5488) == 12
+        assert waves(m, n, 8192, packed=1) == 12
+        assert waves(m, n, 8208, shape=0) == 8 and all(waves(m, n, 8208, shape=s) == 8 for s in (2, 3, 4))
+        # one or two stages of k: nobody only loads on the 256 x 128 and the 128 x 64 tile
+        for k, splits in ((16, 1), (128, 1), (144, 1), (256, 1), (256, 2), (512, 2), (400, 2)):
+            if splits == 2 and (m > 512 or n > 10240):  # (more partial sums than the workspace holds)
+                continue
+            assert waves(m, n, k, splits=splits) == waves(m, n, k, k + 16, splits=splits) == 8 and waves(m, n, k, splits=splits, shape=3) == 4
+            assert waves(m, n, k, splits=splits, shape=2) == waves(m, n, k, splits=splits, shape=4) == 8
+            if k % 256 == 0:
+                assert waves(m, n, k, packed=1, splits=splits) == 8 and waves(m, n, k, packed=1, splits=splits, shape=3) == 4
+        assert waves(m, n, 272, shape=3) == 8 and (m > 512 or n > 10240 or (waves(m, n, 640, splits=2) == 12 and waves(m, n, 528, splits=2, shape=3) == 8))
+assert waves(1040, 5000, 16400) == 12 and waves(1040, 5000, 16400, splits=2) == 4  # 200 workgroups, 400
+assert waves(512, 4104, 16400, splits=2) == 4 and waves(512, 4104, 28656, splits=3) == 12 and waves(512, 4104, 8208, splits=2) == 12
 """
 
 
@@ -271,9 +279,10 @@ tiled_kernels = {}
 for shape in range(5):
     for packed in (0, 1):
         stand_in.stand_in(100, 0)
-        assert lib.hfrk_tiled_gemm(4096, 8192, packed, 16384, None, 0, 64, 1, 64, 1, 64, 1024, 1024, 1024, 1, ctypes.byref(_capi.TiledPlan(shape, 1, 1)), 1) == 0
-        tiled_kernels[stand_in.stand_in_kernel()] = shape
-assert len(tiled_kernels) == 10
+        for k in (256, 1024):  # (a short k has kernels of its own on two of the tiles)
+            assert lib.hfrk_tiled_gemm(4096, 8192, packed, 16384, None, 0, 64, 1, 64, 1, 64, 1024, k, k, 1, ctypes.byref(_capi.TiledPlan(shape, 1, 1)), 1) == 0
+            tiled_kernels[stand_in.stand_in_kernel()] = shape
+assert len(tiled_kernels) == 14
 
 def on_tiles(m, n, k, packed=0, output=16384, call=lib.hfrk_linear_gemm):
     # whether a call runs on tiles; if so, its grid is the plan's
