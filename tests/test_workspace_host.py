@@ -308,6 +308,7 @@ for packed in (0, 1):
                     (24, 48384, 256), (22, 16792, 512), (30, 608, 1024), (21, 296, 1024), (24, 22192, 1024), (33, 1296, 256)):
         assert not on_tiles(m, n, k, packed), (m, n, k, packed)
     assert on_tiles(60, 32016, 1024, packed) and on_tiles(33, 1296, 1024, packed) and on_tiles(32, 3296, 768, packed) and on_tiles(40, 20000, 512, packed)
+    assert on_tiles(22, 10352, 1024, packed) and on_tiles(32, 8560, 1024, packed)  # 324 and 268 panels, one round of tiles
 # a table's entry is run as it stands
 m, n, k = 64, 3800, 1792
 assert lib.hfrk_plan_table_get(m, n, k, 0, ctypes.byref(skinny_plan)) == lib.hfrk_plan_table_set(m, n, k, 0, ctypes.byref(skinny_plan)) == _capi.SUCCESS
