@@ -657,18 +657,18 @@ bool llama_mlp(const at::Tensor& input, const at::Tensor& residual, at::Tensor& 
     return status == HFRK_SUCCESS;
 }
 
-// The row kernels beside the GEMMs as their wrappers are usually called: no buffer to clear, the launcher's own choice of threads, and nothing that
-// autograd would have to know of.  In Python the checks, two to four allocations and the operator took 8 to 10 us a call, the kernels 2 to 4; now 5.5 to 6.3.
+// The row kernels beside the GEMMs as their wrappers are usually called: no buffer to clear and the launcher's own choice of threads.  In Python the
+// checks, two to four allocations and the operator took 8 to 10 us a call, the kernels 2 to 4; now 5.5 to 6.3.  A tensor that requires a gradient changes
+// nothing: the general operators return no tensor and record nothing either.
 bool plain_rows(const at::Tensor& x) {
-    return x.is_cuda() && x.dim() == 2 && is_16bit(x.scalar_type()) && x.is_contiguous() && x.numel() > 0 && x.size(0) < (int64_t(1) << 24) &&
-           x.size(1) < (int64_t(1) << 24) && !(at::GradMode::is_enabled() && x.requires_grad());
+    return x.is_cuda() && x.dim() == 2 && is_16bit(x.scalar_type()) && x.is_contiguous() && x.size(1) > 0 && x.size(0) < (int64_t(1) << 24) &&
+           x.size(1) < (int64_t(1) << 24);
 }
 
 bool plain_rms(const at::Tensor& input, const at::Tensor& residual, const at::Tensor& weight, double epsilon) {
     return plain_rows(input) && plain_rows(residual) && residual.sizes() == input.sizes() && residual.scalar_type() == input.scalar_type() &&
            residual.device() == input.device() && weight.dim() == 1 && weight.size(0) == input.size(1) && weight.is_contiguous() &&
-           weight.scalar_type() == input.scalar_type() && weight.device() == input.device() && !(at::GradMode::is_enabled() && weight.requires_grad()) &&
-           epsilon > 0;
+           weight.scalar_type() == input.scalar_type() && weight.device() == input.device() && epsilon > 0;
 }
 
 // Rows that the dynamic kernels take: whole 16-byte pieces, held in registers.

@@ -164,9 +164,32 @@ def test_row_kernels_refuse_what_they_refused():
     with pytest.raises(RuntimeError):
         swiglu(x, one.half())
     assert torch.equal(x, keep)
-    # a tensor that autograd follows goes the general way, which has always taken it
+    # a tensor that autograd follows is taken, as it always was
     weight = w.clone().requires_grad_()
     got, want = residual_rms(x, x.clone(), weight, 1e-5, one), residual_rms(x, x.clone(), w, 1e-5, one)
     assert torch.equal(_bits(got[0]), _bits(want[0]))
     with torch.inference_mode():
         assert torch.equal(_bits(swiglu(x, one)), _bits(swiglu(x.clone(), one)))
+
+
+@pytest.mark.parametrize("rows", [0, 3])
+def test_row_kernels_take_tensors_that_require_a_gradient_and_empty_batches(rows, monkeypatch):
+    """Such calls run as the native operator at once; the general way behind a refusal of it took them longer than it alone."""
+    from hf_rocm_kernels.operators.residual_rms import wrapped as rms
+    from hf_rocm_kernels.operators.swiglu import wrapped as swi
+    x, res, w = (torch.randn(*shape, device="cuda", dtype=torch.bfloat16) for shape in ((rows, 512), (rows, 512), (512,)))
+    scale = torch.tensor([0.02], device="cuda")
+    calls = {"static": lambda x, r, w: rms.residual_rms(x, r, w, 1e-5, scale), "16 bits": lambda x, r, w: rms.residual_rms(x, r, w, 1e-5),
+             "dynamic": lambda x, r, w: rms.residual_rms_dynamic(x, r, w, 1e-5), "swiglu": lambda x, r, w: (swi.swiglu(x, scale),),
+             "swiglu dynamic": lambda x, r, w: swi.swiglu_dynamic(x)}
+    with monkeypatch.context() as patch:  # the general way
+        patch.setattr(rms, "runs_now", lambda t: False)
+        patch.setattr(swi, "runs_now", lambda t: False)
+        want = {name: call(x, res.clone(), w) for name, call in calls.items()}
+    monkeypatch.setattr(rms, "residual_rms_checks", None)  # the general way ends here
+    monkeypatch.setattr(swi, "swiglu_checks", None)
+    for x_, w_ in ((x, w), (x, torch.nn.Parameter(w.clone())), (x.clone().requires_grad_(), w)):
+        for name, call in calls.items():
+            got = call(x_, res.clone(), w_)
+            for g, t in zip(got, want[name]):
+                assert g.shape == t.shape and g.dtype == t.dtype and not g.requires_grad and torch.equal(_bits(g), _bits(t)), name
