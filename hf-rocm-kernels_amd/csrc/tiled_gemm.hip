@@ -133,15 +133,14 @@ static float workgroup_kernel_cost(int m, int n, int k, const hfrk_gemm_plan& p)
 // 8.5, 57 x 1752 x 14592 19.5 -> 12.0 from the cache, 64 x 11096 x 5120 21.8 -> 20.1 / 21.5 -> 13.7.  The margins are for the fits' errors: whole panels, where
 // nothing is exchanged, and weights above 76 MB, where memory bounds both, are predicted less well.  Above 112 MB at most 2 % could be gained (64 x 8192 x 28672
 // 44 us, 50 on tiles).  33 of the 1079 lose more than 3 % from one of the two, 7 more than 8 % (57 x 8192 x 8192 from memory 11 %, and from the cache 10 % faster).
-// Three kinds of sizes outside that range stay, by 788 more drawn ones (n from 16 to 131072, k from 256 up) that the costs alone put on tiles: more tiles
-// than two rounds of compute units (37 x 45056 x 768 13.0 / 14.6 us, weight from the cache), k of one chunk, and, up to 32 rows, k of
-// one or two slabs (34 x 45008 x 256 packed 6.6 / 11.0, 32 x 42896 x 256 packed 5.5 / 11.0, 22 x 16792 x 512 packed 5.8 / 7.0, 30 x 608 x 1024 packed
-// 4.9 / 5.5), unless the panels take a second round that the tiles do not (22 x 10352 x 1024 6.7 / 5.8).  99 of the 788 are such, 17 % slower on tiles in
-// the mean; of the others 3 are more than 3 % slower and the mean is 30 % faster.
+// Three kinds of sizes outside that range stay: k up to 1024 with more tiles than two rounds of compute units (37 x 45056 x 768 13.0 / 14.6 us, weight from the
+// cache; of 260 drawn n from 32776 to 128056 the costs put 16 on tiles, the six of them with k = 768 4 % slower in the mean there, the ten from k = 1280 on 6 % faster), k of
+// one chunk, and, up to 32 rows, k of one or two slabs (34 x 45008 x 256 packed 6.6 / 11.0, 32 x 42896 x 256 packed 5.5 / 11.0, 22 x 16792 x 512 packed 5.8 / 7.0, 30 x
+// 608 x 1024 packed 4.9 / 5.5), unless the panels take a second round that the tiles do not (22 x 10352 x 1024 6.7 / 5.8).
 // The row-split and K-split kernels stay: the tiled kernel is 3 to 60 % slower than they are on all but a few of their sizes.
 bool tiled_instead(int m, int n, int k, const hfrk_gemm_plan& skinny, hfrk_tiled_plan* plan) {
     if (m <= 16 || skinny.wn < 1 || (long)n * k > (112L << 20) || !tiled_size_ok(m, n, k)) return false;
-    if (n > 64 * 2 * kNumCU || k <= 256) return false;
+    if (k <= (n > 64 * 2 * kNumCU ? 1024 : 256)) return false;
     if (m <= 32 && skinny.slabs < 3 && (skinny.panels <= skinny.grid || div_up(n, 64) > kNumCU)) return false;
     const bool whole_panels = skinny.panels % skinny.grid == 0, large = (long)n * k > (76L << 20);
     const float margin = (whole_panels ? 1.08f : 1.03f) + (large ? .05f : 0.f);

@@ -303,11 +303,12 @@ for packed in (0, 1):
         assert on_tiles(m, n, k, packed) and not on_tiles(m, n, k, packed, output=16392)  # rows of the output that are not 16-byte aligned stay
         assert lib.hfrk_plan_table_get(m, n, k, packed, ctypes.byref(skinny_plan)) == _capi.SUCCESS
         assert stand_in.stand_in_grid() == skinny_plan.grid
-    # weights above 112 MB; fewer rows than 17; a third round of tiles; k of a slab or two
-    for m, n, k in ((64, 8192, 28672), (64, 28672, 8192), (17, 1024, 4096), (16, 1112, 6912), (34, 45008, 256), (37, 45056, 768), (34, 33000, 1280), (32, 42896, 256),
+    # weights above 112 MB; fewer rows than 17; a third round of tiles and k up to 1024; k of a slab or two
+    for m, n, k in ((64, 8192, 28672), (64, 28672, 8192), (17, 1024, 4096), (16, 1112, 6912), (34, 45008, 256), (37, 45056, 768), (61, 48320, 768), (32, 42896, 256),
                     (24, 48384, 256), (22, 16792, 512), (30, 608, 1024), (21, 296, 1024), (24, 22192, 1024), (33, 1296, 256)):
         assert not on_tiles(m, n, k, packed), (m, n, k, packed)
     assert on_tiles(60, 32016, 1024, packed) and on_tiles(33, 1296, 1024, packed) and on_tiles(32, 3296, 768, packed) and on_tiles(40, 20000, 512, packed)
+    assert on_tiles(53, 45240, 1792, packed) and on_tiles(54, 46448, 1280, packed)  # a third round of a longer k
     assert on_tiles(22, 10352, 1024, packed) and on_tiles(32, 8560, 1024, packed)  # 324 and 268 panels, one round of tiles
 # a table's entry is run as it stands
 m, n, k = 64, 3800, 1792
