@@ -136,12 +136,13 @@ static float workgroup_kernel_cost(int m, int n, int k, const hfrk_gemm_plan& p)
 // Three kinds of sizes outside that range stay: k up to 1024 with more tiles than two rounds of compute units (37 x 45056 x 768 13.0 / 14.6 us, weight from the
 // cache; of 260 drawn n from 32776 to 128056 the costs put 16 on tiles, the six of them with k = 768 4 % slower in the mean there, the ten from k = 1280 on 6 % faster), k of
 // one chunk, and, up to 32 rows, k of one or two slabs (34 x 45008 x 256 packed 6.6 / 11.0, 32 x 42896 x 256 packed 5.5 / 11.0, 22 x 16792 x 512 packed 5.8 / 7.0, 30 x
-// 608 x 1024 packed 4.9 / 5.5), unless the panels take a second round that the tiles do not (22 x 10352 x 1024 6.7 / 5.8).
+// 608 x 1024 packed 4.9 / 5.5), unless the panels take a second round and the tiles do not (22 x 10352 x 1024 6.7 / 5.8) or k is two slabs (16390 to 32768 columns of k = 1024,
+// which then go by the costs: 69 drawn ones 13 % faster from the cache and 4 % from memory).
 // The row-split and K-split kernels stay: the tiled kernel is 3 to 60 % slower than they are on all but a few of their sizes.
 bool tiled_instead(int m, int n, int k, const hfrk_gemm_plan& skinny, hfrk_tiled_plan* plan) {
     if (m <= 16 || skinny.wn < 1 || (long)n * k > (112L << 20) || !tiled_size_ok(m, n, k)) return false;
     if (k <= (n > 64 * 2 * kNumCU ? 1024 : 256)) return false;
-    if (m <= 32 && skinny.slabs < 3 && (skinny.panels <= skinny.grid || div_up(n, 64) > kNumCU)) return false;
+    if (m <= 32 && skinny.slabs < 3 && (skinny.panels <= skinny.grid || (skinny.slabs == 1 && div_up(n, 64) > kNumCU))) return false;
     const bool whole_panels = skinny.panels % skinny.grid == 0, large = (long)n * k > (76L << 20);
     const float margin = (whole_panels ? 1.08f : 1.03f) + (large ? .05f : 0.f);
     return margin * make_few_rows_plan(m, n, k, kTiledMaxSplits, plan) < workgroup_kernel_cost(m, n, k, skinny);

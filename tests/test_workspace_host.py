@@ -305,11 +305,12 @@ for packed in (0, 1):
         assert stand_in.stand_in_grid() == skinny_plan.grid
     # weights above 112 MB; fewer rows than 17; a third round of tiles and k up to 1024; k of a slab or two
     for m, n, k in ((64, 8192, 28672), (64, 28672, 8192), (17, 1024, 4096), (16, 1112, 6912), (34, 45008, 256), (37, 45056, 768), (61, 48320, 768), (32, 42896, 256),
-                    (24, 48384, 256), (22, 16792, 512), (30, 608, 1024), (21, 296, 1024), (24, 22192, 1024), (33, 1296, 256)):
+                    (24, 48384, 256), (22, 16792, 512), (30, 608, 1024), (21, 296, 1024), (33, 1296, 256)):
         assert not on_tiles(m, n, k, packed), (m, n, k, packed)
     assert on_tiles(60, 32016, 1024, packed) and on_tiles(33, 1296, 1024, packed) and on_tiles(32, 3296, 768, packed) and on_tiles(40, 20000, 512, packed)
     assert on_tiles(53, 45240, 1792, packed) and on_tiles(54, 46448, 1280, packed)  # a third round of a longer k
     assert on_tiles(22, 10352, 1024, packed) and on_tiles(32, 8560, 1024, packed)  # 324 and 268 panels, one round of tiles
+    assert on_tiles(28, 26384, 1024, packed) and on_tiles(24, 22192, 1024, packed)  # two rounds of both, two slabs of k
 # a table's entry is run as it stands
 m, n, k = 64, 3800, 1792
 assert lib.hfrk_plan_table_get(m, n, k, 0, ctypes.byref(skinny_plan)) == lib.hfrk_plan_table_set(m, n, k, 0, ctypes.byref(skinny_plan)) == _capi.SUCCESS
