@@ -128,11 +128,13 @@ static float workgroup_kernel_cost(int m, int n, int k, const hfrk_gemm_plan& p)
 
 // 17 to 64 rows that the skinny GEMM's planner gives to its workgroup kernel.  That kernel was tuned on weights whose rows and k deal out in whole
 // panels and slabs over the compute units; elsewhere the shares of a panel lie with up to twenty workgroups, whose sums one of them collects.  Over 1079
-// such calls (n and k drawn from 1024 to 28672, 40 % of them multiples of 256, 512 or 1024; row-major and packed) the choice below is 19 % faster in
-// the mean with weights from memory and 26 % with weights from the 256 MB cache: 57 x 2832 x 1792 13.3 -> 6.4 us / 14.5 -> 6.4, 50 x 6176 x 3072 15.4 -> 11.2 / 15.5 ->
+// such calls (n and k drawn from 1024 to 28672, 40 % of them multiples of 256, 512 or 1024; row-major and packed) the choice below is 17 % faster in
+// the mean with weights from memory and 25 % with weights from the 256 MB cache: 57 x 2832 x 1792 13.3 -> 6.4 us / 14.5 -> 6.4, 50 x 6176 x 3072 15.4 -> 11.2 / 15.5 ->
 // 8.5, 57 x 1752 x 14592 19.5 -> 12.0 from the cache, 64 x 11096 x 5120 21.8 -> 20.1 / 21.5 -> 13.7.  The margins are for the fits' errors: whole panels, where
-// nothing is exchanged, and weights above 76 MB, where memory bounds both, are predicted less well.  Above 112 MB at most 2 % could be gained (64 x 8192 x 28672
-// 44 us, 50 on tiles).  33 of the 1079 lose more than 3 % from one of the two, 7 more than 8 % (57 x 8192 x 8192 from memory 11 %, and from the cache 10 % faster).
+// nothing is exchanged, and weights above 76 MB, where memory bounds both, are predicted less well.  Twelve of the 1079 lose more than 3 % from one of the two, one more
+// than 8 % (57 x 8192 x 8192 from memory 10 %, and from the cache 10 % faster).  Above 112 MB all stay, though not for want of gains: on their best tile plan
+// the 114 sizes there are 6 % slower in the mean from memory and 21 % faster from the cache (49 x 14744 x 9216 26 and 51 % faster, 19 x 16616 x 13824 33 and 22 % slower;
+// 64 x 8192 x 28672 44 us, 50 on tiles), and the fits do not tell them apart.
 // Three kinds of sizes outside that range stay: k up to 1024 with more tiles than two rounds of compute units (37 x 45056 x 768 13.0 / 14.6 us, weight from the
 // cache; of 260 drawn n from 32776 to 128056 the costs put 16 on tiles, the six of them with k = 768 4 % slower in the mean there, the ten from k = 1280 on 6 % faster), k of
 // one chunk, and, up to 32 rows, k of one or two slabs (34 x 45008 x 256 packed 6.6 / 11.0, 32 x 42896 x 256 packed 5.5 / 11.0, 22 x 16792 x 512 packed 5.8 / 7.0, 30 x

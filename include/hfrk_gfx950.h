@@ -129,7 +129,9 @@ int hfrk_skinny_gemm_validate(int m, int n, int k, int b_stride, int split_k, in
 /* Pure host function: choose the decomposition for a shape (counterpart of infer_skinny_gemm_params,
  * hf_rocm_kernels/operators/skinny_gemm/wrapped.py:42-102).  Returns HFRK_SUCCESS or a shape error.  Where this is the workgroup
  * decomposition (wn >= 1) a call of 17 to 64 rows that names no plan and has none in the table may run on the tiled kernel instead
- * (hfrk_tiled_gemm), as the library's cost estimates of the two have it; every entry point then does, with the same bits. */
+ * (hfrk_tiled_gemm), as the library's cost estimates of the two have it.  Equal calls take the same kernel through every entry point,
+ * with the same bits; but a D or base that is not 16-byte aligned, or a b_stride above 2^21, keeps a call with the skinny kernel, which adds in
+ * another order. */
 int hfrk_skinny_gemm_plan(int m, int n, int k, hfrk_gemm_plan* plan);
 
 /* Plan table (host only, thread-safe): tuned decompositions, keyed (m, n, k, packed), that take the planner's place
@@ -328,8 +330,9 @@ int hfrk_tiled_gemm_plan(int m, int n, int k, hfrk_tiled_plan* plan);
  *   A  fp8 e4m3fn [m,k] row-major     B  the weight: row-major with row stride b_stride (packed == 0) or the buffer
  *   D  16-bit [m,n] row-major            hfrk_pack_weight wrote (packed == 1, b_stride unused)
  *   base  16-bit addend of D's type or NULL; base_stride elements between its rows, 0: one row for all (a bias)
- * fp32 accumulation, one rounding.  Bit-reproducible under one plan; without a plan the split of k, and with it the order of the sums,
- * depends on whether the stream has a workspace.  k % 16 == 0 (256 for a packed weight); n, k and the strides at most 2^21, m at most
+ * fp32 accumulation, one rounding.  Bit-reproducible for equal arguments under one plan; without a plan the split of k, and with it the order
+ * of the sums, depends on whether the stream has a workspace.  Workgroups that share operands start at different places of k, so the order
+ * also depends on which row and column of tiles a result lies in: equal rows of A in different tiles may differ in their last bits.  k % 16 == 0 (256 for a packed weight); n, k and the strides at most 2^21, m at most
  * 2^24, fewer than 2^24 tiles of 64 x 64.
  * A and B 16-byte aligned, b_stride a multiple of 16; D and base may have any alignment, 16 bytes with n % 8 == 0 is the fast one.
  * A plan whose k is split needs the stream's workspace like the skinny GEMMs (see hfrk_init); without a plan k is not split where there is
